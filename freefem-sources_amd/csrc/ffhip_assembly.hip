@@ -1266,16 +1266,125 @@ __global__ __launch_bounds__(256) void k_p1_grad_kappa(
 }
 
 // ---------------------------------------------------------------- CSR mat-vec
-__global__ void k_spmv_csr(int64_t n, const int64_t *__restrict__ rowptr,
-                           const int32_t *__restrict__ colidx, const double *__restrict__ vals,
-                           const int64_t *__restrict__ tmap, const double *__restrict__ x,
-                           double *__restrict__ y) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = 0.;
-  for (int64_t k = rowptr[i]; k < rowptr[i + 1]; ++k)
-    s += (tmap ? vals[tmap[k]] : vals[k]) * x[colidx[k]];
-  y[i] = s;
+// y = A x over a CSR pattern, the value of entry k read as vals[k] (kPlain),
+// vals[slot[k]] (kSlots: the full view of a half matrix) or the entry (j, i)
+// of a symmetric pattern (kTrans: y = A^T x, *missing raised where the pattern
+// holds no such entry).
+//
+// Bound by HBM (12 nnz + 20 n bytes), so every matrix load is coalesced: a wave
+// takes 64 rows, reads their entries consecutively (lane on entry, up to 8
+// independent load pairs per lane in flight), stages the pairs (a, x_j) in LDS
+// and each lane then adds its own row in entry order with fused multiply-adds,
+// the sum that a lane walking its row in memory makes (bit for bit), which took
+// 130 us for A x at cube(72) because the lanes of such a walk lie 120 bytes
+// apart.  Pair i of the stage sits at i + i / 32 (rows of 8 or 16 entries would
+// otherwise meet in the same LDS banks).  Segments over the stage are taken
+// chunk by chunk.
+constexpr int kPlain = 0, kSlots = 1, kTrans = 2;
+constexpr int kSpmvStage = 1024;  // pairs per wave: 16.5 KB, 9 waves per CU (64 P1 rows hold 960)
+__device__ inline int stage_pos(int i) { return i + (i >> 5); }
+
+// slot of column i among the sorted columns [lo, end) of a row, or -1
+__device__ inline int64_t find_entry(int64_t lo, int64_t end, const int32_t *__restrict__ colidx,
+                                     int32_t i) {
+  int64_t hi = end - 1;
+  while (lo <= hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    const int32_t c = colidx[mid];
+    if (c == i) return mid;
+    if (c < i) lo = mid + 1; else hi = mid - 1;
+  }
+  return -1;
+}
+
+template <int MODE>
+__global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__restrict__ rowptr,
+                                                   const int32_t *__restrict__ colidx,
+                                                   const double *__restrict__ vals,
+                                                   const int64_t *__restrict__ slot,
+                                                   const double *__restrict__ x, double *__restrict__ y,
+                                                   int *__restrict__ missing) {
+  constexpr int U = MODE == kTrans ? 4 : 8;
+  __shared__ double2 st[kSpmvStage + kSpmvStage / 32];
+  __shared__ int64_t rs[kWave];  // kTrans: the rows' starts
+  const int lane = threadIdx.x;
+  const int64_t r0 = (int64_t)xcd_block_id() * kWave, r = r0 + lane;
+  if (r0 >= n) return;  // one wave per block
+  const int64_t p0 = rowptr[r < n ? r : n], p1 = rowptr[r + 1 < n ? r + 1 : n];
+  const int64_t seg0 = rowptr[r0], seg1 = rowptr[r0 + kWave < n ? r0 + kWave : n];
+  if constexpr (MODE == kTrans) {
+    rs[lane] = p0;
+    wave_lds_sync();
+  }
+  double acc = 0.;
+  for (int64_t c0 = seg0; c0 < seg1; c0 += kSpmvStage) {
+    const int cnt = (int)(seg1 - c0 < kSpmvStage ? seg1 - c0 : kSpmvStage);
+    for (int i0 = lane; i0 < cnt; i0 += kWave * U) {
+      int32_t j[U];
+      double a[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * kWave;
+        j[u] = i < cnt ? colidx[c0 + i] : 0;
+        if (MODE == kPlain) a[u] = i < cnt ? vals[c0 + i] : 0.;
+        if (MODE == kSlots) a[u] = i < cnt ? vals[slot[c0 + i]] : 0.;
+      }
+      if constexpr (MODE == kTrans) {
+        // Entry k of row i at (i, j): (j, i) is first looked for where it lies
+        // when row j's offsets mirror row i's (structured meshes), so the
+        // chain is row j's ends, one column, one value with U of them in
+        // flight; a binary search finds the others.
+        int64_t q0[U], q1[U], g[U];
+        int32_t ri[U], cg[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int i = i0 + u * kWave;
+          int lo = 0, hi = kWave - 1;  // the row of this entry: the last that starts at or before it
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (rs[mid] <= c0 + i) lo = mid; else hi = mid - 1;
+          }
+          ri[u] = lo;
+          q0[u] = rowptr[j[u]];
+          q1[u] = rowptr[j[u] + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t m = q1[u] - 1 - (c0 + i0 + u * kWave - rs[ri[u]]);
+          g[u] = m > q0[u] ? m : q0[u];
+          ri[u] += (int32_t)r0;
+          cg[u] = g[u] < q1[u] ? colidx[g[u]] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          a[u] = 0.;
+          if (i0 + u * kWave < cnt) {
+            const int64_t s = cg[u] == ri[u] ? g[u] : find_entry(q0[u], q1[u], colidx, ri[u]);
+            if (s >= 0) a[u] = vals[s];
+            else atomicOr(missing, 1);
+          }
+        }
+      }
+      double xv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) xv[u] = x[j[u]];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * kWave;
+        if (i < cnt) st[stage_pos(i)] = double2{a[u], xv[u]};
+      }
+    }
+    wave_lds_sync();
+    const int b0 = (int)((p0 > c0 ? p0 : c0) - c0);
+    const int b1 = (int)((p1 < c0 + cnt ? p1 : c0 + cnt) - c0);
+#pragma unroll 4
+    for (int k = b0; k < b1; ++k) {
+      const double2 q = st[stage_pos(k)];
+      acc = fma(q.x, q.y, acc);
+    }
+    wave_lds_sync();
+  }
+  if (r < n) y[r] = acc;
 }
 
 // slot of the transposed entry: (i,j) at k  ->  (j,i); -1 if absent
@@ -2143,26 +2252,31 @@ int ffhip_spmv(ffhip_ctx ctx, ffhip_mat A, const double *x, double *y, int trans
   return guard([&] {
     FFHIP_REQUIRE(ctx && A && x && y, FFHIP_ERR_ARG, "ffhip_spmv: null argument");
     hipStream_t s = ctx->stream;
+    const unsigned grid = (nblocks(A->n, kWave) + 7) / 8 * 8;  // whole XCD groups
     if (A->half) {  // y = (L + L^T - diag L) x over the full view; symmetric: trans alike
       half_view(A);
       ctx->tic();
-      k_spmv_csr<<<nblocks(A->n, 256), 256, 0, s>>>(A->n, A->fptr, A->fcol, A->vals, A->fslot, x, y);
+      k_spmv_stage<kSlots><<<grid, kWave, 0, s>>>(A->n, A->fptr, A->fcol, A->vals, A->fslot, x, y, nullptr);
       FFHIP_CHECK(hipGetLastError());
       ctx->toc();
       return;
     }
-    int64_t *tmap = nullptr;
-    if (trans) {
-      tmap = dalloc<int64_t>(A->nnz);
-      const bool ok = transpose_map(ctx, A, tmap);
-      if (!ok) dfree(tmap);
-      FFHIP_REQUIRE(ok, FFHIP_ERR_UNSUPPORTED, "ffhip_spmv: transpose needs a symmetric pattern");
+    if (!trans) {
+      ctx->tic();
+      k_spmv_stage<kPlain><<<grid, kWave, 0, s>>>(A->n, A->rowptr, A->colidx, A->vals, nullptr, x, y, nullptr);
+      FFHIP_CHECK(hipGetLastError());
+      ctx->toc();
+      return;
     }
+    int *missing = dalloc<int>(1);
+    FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), s));
     ctx->tic();
-    k_spmv_csr<<<nblocks(A->n, 256), 256, 0, s>>>(A->n, A->rowptr, A->colidx, A->vals, tmap, x, y);
+    k_spmv_stage<kTrans><<<grid, kWave, 0, s>>>(A->n, A->rowptr, A->colidx, A->vals, nullptr, x, y, missing);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
-    dfree(tmap);
+    const int miss = read_flag(ctx, missing);
+    dfree(missing);
+    FFHIP_REQUIRE(miss == 0, FFHIP_ERR_UNSUPPORTED, "ffhip_spmv: transpose needs a symmetric pattern");
   });
 }
 
