@@ -31,6 +31,7 @@
 
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "ffhip_fem.hpp"
@@ -1062,91 +1063,118 @@ __device__ inline double rhs_coef(int kind, double f0, const double *__restrict_
   return f0;
 }
 
-// |K| of every tet, once (the right-hand side gathers it for each of the 4 incidences)
-__global__ void k_tet_mes(int64_t nt, const double *__restrict__ xyz, const int32_t *__restrict__ tets,
-                          double *__restrict__ mes) {
+// LDS position of staged item i of a wave's 64 rows: one item of padding per
+// 32, so that rows of 8, 16 or 24 items do not start in the same banks
+__device__ inline int stage_pos(int i) { return i + (i >> 5); }
+
+// What the row pass below needs of each tet for the terms of its 4 vertices
+// (rule of Tet_5, exact for these products):
+//   kRowScale  f constant on the tet:  E = |K| f, term E / 4
+//   kRowPair   f P1:                   E = (|K| / 20, sum of the 4 f's), term E.x (f_v + E.y)
+//   kRowQuad   f at the 14 points:     E = the 4 integrals, term E[l]
+constexpr int kRowScale = 0, kRowPair = 1, kRowQuad = 2;
+template <int RM>
+__global__ __launch_bounds__(256) void k_p1_load_elem(int64_t nt, const double *__restrict__ xyz,
+                                                      const int32_t *__restrict__ tets, int kind,
+                                                      double f0, const double *__restrict__ fcoef,
+                                                      double *__restrict__ E) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= nt) return;
   double v[4][3];
-  const int4 tv = reinterpret_cast<const int4 *>(tets)[e];
-  const int32_t id[4] = {tv.x, tv.y, tv.z, tv.w};
-  for (int i = 0; i < 4; ++i)
-    for (int k = 0; k < 3; ++k) v[i][k] = xyz[3 * (int64_t)id[i] + k];
-  mes[e] = tet_mesure(v);
-}
-
-// Sum of a row's incidence terms in element order, one row per 32-lane
-// half-wave: lane q computes the term of incidence c0 + q of each chunk of 32
-// into its LDS slot, and every lane then adds the 32 slots in order (the order
-// of the element loop, so the sum rounds as FreeFEM's accumulation into the
-// row).  Slots past the row's end hold +0.0, and adding +0.0 leaves the sum
-// unchanged: a sum that starts at +0.0 is never -0.0 under round-to-nearest.
-template <class F>
-__device__ inline double row_sum_in_order(double *__restrict__ slot, int hl, int64_t deg, F term) {
-  double s = 0.;
-  for (int64_t c0 = 0; c0 < deg; c0 += kHalf) {
-    slot[hl] = c0 + hl < deg ? term(c0 + hl) : 0.;
-    wave_lds_sync();
-#pragma unroll
-    for (int q = 0; q < kHalf; ++q) s += slot[q];
-    wave_lds_sync();
-  }
-  return s;
-}
-
-// b_v = sum over the incident tets of int_K f lambda_v (Tet_5), one row per half-wave
-__global__ __launch_bounds__(256) void k_rhs_p1_3d(int64_t n, const double *__restrict__ xyz,
-                            const int32_t *__restrict__ tets, const double *__restrict__ tmes,
-                            const int64_t *__restrict__ v2e_ptr,
-                            const int32_t *__restrict__ v2e, int kind, double f0,
-                            const double *__restrict__ fcoef, const uint8_t *__restrict__ onbc,
-                            double tgv, double g0, const double *__restrict__ gvals,
-                            double *__restrict__ b) {
-  const int hl = threadIdx.x % kHalf;
-  const int64_t v = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kHalf;
-  if (v >= n) return;  // uniform in the half-wave
-  if (onbc && onbc[v]) {
-    if (hl == 0) b[v] = tgv * (gvals ? gvals[v] : g0);
-    return;
-  }
-  __shared__ double slots[256];
-  const int64_t k0 = v2e_ptr[v];
-  const double s = row_sum_in_order(slots + (threadIdx.x & ~(kHalf - 1)), hl, v2e_ptr[v + 1] - k0,
-                                    [&](int64_t k) {
-    const int32_t idx = v2e[k0 + k];
-    const int64_t e = idx >> 2;
-    const int l = idx & 3;
-    double vv[4][3], fu[4] = {0., 0., 0., 0.};
-    if (kind != FFHIP_COEF_CONST) {  // the points (or the vertex values) are needed for f
-      const int4 tv = reinterpret_cast<const int4 *>(tets)[e];
-      const int32_t id[4] = {tv.x, tv.y, tv.z, tv.w};
-      if (kind == FFHIP_COEF_P1) {
-        for (int i = 0; i < 4; ++i) fu[i] = fcoef[id[i]];
-      } else {
-        for (int i = 0; i < 4; ++i)
-          for (int kk = 0; kk < 3; ++kk) vv[i][kk] = xyz[3 * (int64_t)id[i] + kk];
-      }
-    }
-    const double mes = tmes[e];
-    double r = 0.;
+  int32_t id[4];
+  load_tet(xyz, tets, e, id, v);
+  const double mes = tet_mesure(v);
+  if constexpr (RM == kRowScale) {
+    E[e] = mes * (kind == FFHIP_COEF_P0 ? fcoef[e] : f0);
+  } else if constexpr (RM == kRowPair) {
+    const double se = fcoef[id[0]] + fcoef[id[1]] + fcoef[id[2]] + fcoef[id[3]];
+    reinterpret_cast<double2 *>(E)[e] = double2{mes / 20., se};
+  } else {
+    double r[4] = {0., 0., 0., 0.};
     for (int q = 0; q < 14; ++q) {
       const double px = c_qf5_pts[q][0], py = c_qf5_pts[q][1], pz = c_qf5_pts[q][2];
-      const double l0 = 1. - (px + py + pz);
-      const double lam = l == 0 ? l0 : (l == 1 ? px : (l == 2 ? py : pz));
-      double f = f0;
-      if (kind == FFHIP_COEF_P1) {
-        f = p1_value3(fu, px, py, pz);
-      } else if (kind != FFHIP_COEF_CONST) {
-        double P[3];
-        for (int kk = 0; kk < 3; ++kk)
-          P[kk] = l0 * vv[0][kk] + px * vv[1][kk] + py * vv[2][kk] + pz * vv[3][kk];
-        f = rhs_coef(kind, f0, fcoef, e, q, 14, P[0], P[1], P[2], 3);
-      }
-      r += (mes * qf5_weight(q)) * f * lam;
+      const double l[4] = {1. - (px + py + pz), px, py, pz};
+      double P[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) P[k] = l[0] * v[0][k] + px * v[1][k] + py * v[2][k] + pz * v[3][k];
+      const double W = (mes * qf5_weight(q)) * rhs_coef(kind, f0, fcoef, e, q, 14, P[0], P[1], P[2], 3);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] += W * l[i];
     }
-    return r;
-  });
-  if (hl == 0) b[v] = s;
+    double4 o;
+    o.x = r[0]; o.y = r[1]; o.z = r[2]; o.w = r[3];
+    reinterpret_cast<double4 *>(E)[e] = o;
+  }
+}
+
+// b_v = the sum of v's incidence terms in element order.  A wave takes 64 rows:
+// it reads their incidence lists consecutively (lane on incidence), stages what
+// it gathers in LDS chunk by chunk, and each lane adds its own row from there
+// in order.  Bound by the bytes of the lists and of E (4 + 8..16 per
+// incidence), so the stage is small (4.2 KB: the waves of a CU are limited by
+// registers, not LDS): 187 us for a constant f at cube(160), 98 M incidences,
+// 3.3 TB/s; with 2048 staged items per wave (9 waves per CU) 422 us, with
+// 1024 and 16 in flight 260 us.  A half-wave per row whose 32 lanes each added
+// all 32 slots issued 32 LDS reads for two rows and took 1660 us.  PAIR at
+// cube(96), 21 M incidences: 70 us (half-wave: 378 us with |K| recomputed).
+// PAIR terms need the row's own value (own, minus own2 when given); the
+// product and the sum are rounded on their own, as the term and its addition
+// were.  tgv rows: tgv * (gvals[v] or g0), or 0 with zero_bc.
+template <int RM>
+__global__ __launch_bounds__(64) void k_row_sum(
+    int64_t n, const int64_t *__restrict__ v2e_ptr, const int32_t *__restrict__ v2e,
+    const double *__restrict__ E, const double *__restrict__ own, const double *__restrict__ own2,
+    const uint8_t *__restrict__ onbc, double tgv, double g0, const double *__restrict__ gvals,
+    double *__restrict__ b) {
+  constexpr int U = RM == kRowPair ? 4 : 8, CAP = kWave * U;  // one round of gathers per chunk
+  using T = typename std::conditional<RM == kRowPair, double2, double>::type;
+  __shared__ T st[CAP + CAP / 32];
+  const int lane = threadIdx.x;
+  const int64_t r0 = (int64_t)xcd_block_id() * kWave, r = r0 + lane;
+  if (r0 >= n) return;  // one wave per block
+  const int64_t p0 = v2e_ptr[r < n ? r : n], p1 = v2e_ptr[r + 1 < n ? r + 1 : n];
+  const int64_t seg0 = v2e_ptr[r0], seg1 = v2e_ptr[r0 + kWave < n ? r0 + kWave : n];
+  double me = 0.;
+  if (RM == kRowPair && r < n) me = own2 ? own[r] - own2[r] : own[r];
+  double s = 0.;
+  for (int64_t c0 = seg0; c0 < seg1; c0 += CAP) {
+    const int cnt = (int)(seg1 - c0 < CAP ? seg1 - c0 : CAP);
+    for (int i0 = lane; i0 < cnt; i0 += kWave * U) {
+      int32_t idx[U];
+      T t[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * kWave;
+        idx[u] = i < cnt ? v2e[c0 + i] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        t[u] = reinterpret_cast<const T *>(E)[RM == kRowQuad ? idx[u] : idx[u] >> 2];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * kWave;
+        if (i < cnt) st[stage_pos(i)] = t[u];
+      }
+    }
+    wave_lds_sync();
+    const int b0 = (int)((p0 > c0 ? p0 : c0) - c0);
+    const int b1 = (int)((p1 < c0 + cnt ? p1 : c0 + cnt) - c0);
+#pragma unroll 4
+    for (int k = b0; k < b1; ++k) {
+      if constexpr (RM == kRowPair) {
+        const double2 q = st[stage_pos(k)];
+        double t = q.x * (me + q.y);
+        asm("" : "+v"(t));  // rounded before it is added (no fused multiply-add)
+        s += t;
+      } else {
+        s += RM == kRowScale ? 0.25 * st[stage_pos(k)] : st[stage_pos(k)];
+      }
+    }
+    wave_lds_sync();
+  }
+  if (r >= n) return;
+  if (onbc && onbc[r]) s = tgv * (gvals ? gvals[r] : g0);
+  b[r] = s;
 }
 
 __global__ void k_rhs_p1_2d(int64_t n, const double *__restrict__ xy,
@@ -1191,10 +1219,12 @@ __global__ void k_rhs_p1_2d(int64_t n, const double *__restrict__ xy,
 }
 
 // ---------------------------------------------------------------- adjoint blocks
-// per element: misfit 1/2 int_K e^2 = |K|/40 (sum e_i^2 + (sum e_i)^2), e = u - ud
+// per element: misfit 1/2 int_K e^2 = |K|/40 (sum e_i^2 + (sum e_i)^2), e = u - ud;
+// with pair also (|K|/20, sum e_i), the element's part of M e (kRowPair)
 __global__ __launch_bounds__(256) void k_p1_misfit_elem(
     int64_t nt, const double *__restrict__ xyz, const int32_t *__restrict__ tets,
-    const double *__restrict__ u, const double *__restrict__ ud, double *__restrict__ part) {
+    const double *__restrict__ u, const double *__restrict__ ud, double *__restrict__ part,
+    double2 *__restrict__ pair) {
   __shared__ double lds[256 / kWave];
   double acc = 0.;
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < nt; e += (int64_t)gridDim.x * 256) {
@@ -1209,12 +1239,35 @@ __global__ __launch_bounds__(256) void k_p1_misfit_elem(
     const double s1 = ev[0] + ev[1] + ev[2] + ev[3];
     const double s2 = ev[0] * ev[0] + ev[1] * ev[1] + ev[2] * ev[2] + ev[3] * ev[3];
     acc += mes / 40. * (s2 + s1 * s1);
+    if (pair) pair[e] = double2{mes / 20., s1};
   }
   const double tot = block_sum<256>(acc, lds);
-  if (threadIdx.x == 0) part[blockIdx.x] = tot;
+  if (part && threadIdx.x == 0) part[blockIdx.x] = tot;
 }
 
-// (M e)_v = sum over incident elements of |K|/20 (e_v + sum_K e_j); 0 on Dirichlet rows
+// Sum of a row's incidence terms in element order, one row per 32-lane
+// half-wave: lane q computes the term of incidence c0 + q of each chunk of 32
+// into its LDS slot, and every lane then adds the 32 slots in order (the order
+// of the element loop, so the sum rounds as FreeFEM's accumulation into the
+// row).  Slots past the row's end hold +0.0, and adding +0.0 leaves the sum
+// unchanged: a sum that starts at +0.0 is never -0.0 under round-to-nearest.
+template <class F>
+__device__ inline double row_sum_in_order(double *__restrict__ slot, int hl, int64_t deg, F term) {
+  double s = 0.;
+  for (int64_t c0 = 0; c0 < deg; c0 += kHalf) {
+    slot[hl] = c0 + hl < deg ? term(c0 + hl) : 0.;
+    wave_lds_sync();
+#pragma unroll
+    for (int q = 0; q < kHalf; ++q) s += slot[q];
+    wave_lds_sync();
+  }
+  return s;
+}
+
+// (M e)_v = sum over incident elements of |K|/20 (e_v + sum_K e_j); 0 on
+// Dirichlet rows: the pass of the entry point that may hold no per-element
+// temporary (the other one stores the pairs with the misfit and adds them in
+// k_row_sum, the same terms in the same order)
 __global__ __launch_bounds__(256) void k_p1_mass_apply(
     int64_t n, const double *__restrict__ xyz, const int32_t *__restrict__ tets,
     const int64_t *__restrict__ v2e_ptr, const int32_t *__restrict__ v2e,
@@ -1275,14 +1328,13 @@ __global__ __launch_bounds__(256) void k_p1_grad_kappa(
 // takes 64 rows, reads their entries consecutively (lane on entry, up to 8
 // independent load pairs per lane in flight), stages the pairs (a, x_j) in LDS
 // and each lane then adds its own row in entry order with fused multiply-adds,
-// the sum that a lane walking its row in memory makes (bit for bit), which took
-// 130 us for A x at cube(72) because the lanes of such a walk lie 120 bytes
-// apart.  Pair i of the stage sits at i + i / 32 (rows of 8 or 16 entries would
-// otherwise meet in the same LDS banks).  Segments over the stage are taken
-// chunk by chunk.
+// bit for bit the sum of a lane that walks its row in memory.  The stage is one
+// round of loads (4 or 8 KB, so that LDS does not limit the waves per CU).
+// cube(72) (n = 389,017, nnz = 5.7 M): A x 19 us, half 25 us, A^T x 63 us (29,
+// 41 and 74 us with a 16 KB stage); with a lane per row in memory, the lanes
+// 120 bytes apart, 130 us, 180 us, and 215 us after a 161 us pass that wrote
+// the transposed slots.
 constexpr int kPlain = 0, kSlots = 1, kTrans = 2;
-constexpr int kSpmvStage = 1024;  // pairs per wave: 16.5 KB, 9 waves per CU (64 P1 rows hold 960)
-__device__ inline int stage_pos(int i) { return i + (i >> 5); }
 
 // slot of column i among the sorted columns [lo, end) of a row, or -1
 __device__ inline int64_t find_entry(int64_t lo, int64_t end, const int32_t *__restrict__ colidx,
@@ -1304,8 +1356,8 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
                                                    const int64_t *__restrict__ slot,
                                                    const double *__restrict__ x, double *__restrict__ y,
                                                    int *__restrict__ missing) {
-  constexpr int U = MODE == kTrans ? 4 : 8;
-  __shared__ double2 st[kSpmvStage + kSpmvStage / 32];
+  constexpr int U = MODE == kTrans ? 8 : 4, CAP = kWave * U;  // one round of loads per chunk
+  __shared__ double2 st[CAP + CAP / 32];
   __shared__ int64_t rs[kWave];  // kTrans: the rows' starts
   const int lane = threadIdx.x;
   const int64_t r0 = (int64_t)xcd_block_id() * kWave, r = r0 + lane;
@@ -1317,8 +1369,8 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
     wave_lds_sync();
   }
   double acc = 0.;
-  for (int64_t c0 = seg0; c0 < seg1; c0 += kSpmvStage) {
-    const int cnt = (int)(seg1 - c0 < kSpmvStage ? seg1 - c0 : kSpmvStage);
+  for (int64_t c0 = seg0; c0 < seg1; c0 += CAP) {
+    const int cnt = (int)(seg1 - c0 < CAP ? seg1 - c0 : CAP);
     for (int i0 = lane; i0 < cnt; i0 += kWave * U) {
       int32_t j[U];
       double a[U];
@@ -1407,6 +1459,8 @@ __global__ void k_transpose_map(int64_t n, const int64_t *__restrict__ rowptr,
 }
 
 static unsigned nblocks(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
+// one wave per 64 rows, whole XCD groups
+static unsigned row_sum_grid(int64_t n) { return (nblocks(n, kWave) + 7) / 8 * 8; }
 int read_flag(ffhip_ctx ctx, int *d);
 void half_view(ffhip_mat L);
 
@@ -1573,12 +1627,14 @@ int read_flag(ffhip_ctx ctx, int *d) {
 // J = 1/2 int (u - ud)^2 (partials of kMisfitBlocks blocks, summed on the host
 // in block order) and r = M (u - ud) with the Dirichlet rows zeroed, on the
 // given buffers: part (kMisfitBlocks doubles, when J), onbc (nv bytes) and
-// labs (nlab int32, when r and nlab > 0)
+// labs (nlab int32, when r and nlab > 0), pair (nt, when r; without it r's
+// terms are formed per incidence)
 constexpr int kMisfitBlocks = 1024;
 struct MisfitBuffers {
   double *part = nullptr;
   uint8_t *onbc = nullptr;
   int32_t *labs = nullptr;
+  double2 *pair = nullptr;
 };
 
 __global__ void k_fill_u8(int64_t n, uint8_t *__restrict__ a, uint8_t v) {
@@ -1590,15 +1646,11 @@ void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
                 const int32_t *labels, int nlab, double *J, double *r, const MisfitBuffers &b) {
   hipStream_t s = ctx->stream;
   ctx->tic();
-  if (J) {
-    k_p1_misfit_elem<<<kMisfitBlocks, 256, 0, s>>>(m->nt, m->xyz, m->elems, u, ud, b.part);
+  double h[kMisfitBlocks];
+  if (J || b.pair) {
+    k_p1_misfit_elem<<<kMisfitBlocks, 256, 0, s>>>(m->nt, m->xyz, m->elems, u, ud, b.part, b.pair);
     FFHIP_CHECK(hipGetLastError());
-    double h[kMisfitBlocks];
-    FFHIP_CHECK(hipMemcpyAsync(h, b.part, sizeof(h), hipMemcpyDeviceToHost, s));
-    FFHIP_CHECK(hipStreamSynchronize(s));
-    double tot = 0.;
-    for (int i = 0; i < kMisfitBlocks; ++i) tot += h[i];
-    *J = tot;
+    if (J) FFHIP_CHECK(hipMemcpyAsync(h, b.part, sizeof(h), hipMemcpyDeviceToHost, s));
   }
   if (r) {
     const uint8_t *onbc = nullptr;
@@ -1610,11 +1662,21 @@ void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
                                                        nlab, b.onbc);
       onbc = b.onbc;
     }
-    k_p1_mass_apply<<<nblocks(m->nv * kHalf, 256), 256, 0, s>>>(m->nv, m->xyz, m->elems, m->v2e_ptr, m->v2e,
-                                                        u, ud, onbc, r);
+    if (b.pair)
+      k_row_sum<kRowPair><<<row_sum_grid(m->nv), kWave, 0, s>>>(
+          m->nv, m->v2e_ptr, m->v2e, reinterpret_cast<const double *>(b.pair), u, ud, onbc, 0., 0.,
+          nullptr, r);
+    else
+      k_p1_mass_apply<<<nblocks(m->nv * kHalf, 256), 256, 0, s>>>(m->nv, m->xyz, m->elems, m->v2e_ptr,
+                                                                  m->v2e, u, ud, onbc, r);
     FFHIP_CHECK(hipGetLastError());
   }
   ctx->toc();
+  if (J) {
+    double tot = 0.;
+    for (int i = 0; i < kMisfitBlocks; ++i) tot += h[i];
+    *J = tot;
+  }
 }
 
 // ---------------------------------------------------------------- no-allocation scratch
@@ -2085,14 +2147,23 @@ int ffhip_rhs_p1_form(ffhip_ctx ctx, ffhip_mesh m, int kind, double f0, const do
       gd = gown;
     }
     if (m->dim == 2) upload_t5_once(ctx->device);
-    double *tmes = m->dim == 3 ? dalloc<double>(m->nt) : nullptr;
+    // 3D: one pass over the tets, then one over the rows
+    const int rm = kind == FFHIP_COEF_P1 ? kRowPair
+                   : kind == FFHIP_COEF_SIN3 || kind == FFHIP_COEF_QP ? kRowQuad : kRowScale;
+    double *E = m->dim == 3 ? dalloc<double>(m->nt * (rm == kRowPair ? 2 : rm == kRowQuad ? 4 : 1)) : nullptr;
     ctx->tic();
     if (m->dim == 3) {
-      k_tet_mes<<<nblocks(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, tmes);
-      k_rhs_p1_3d<<<nblocks(n * kHalf, 256), 256, 0, s>>>(n, m->xyz, m->elems, tmes, m->v2e_ptr, m->v2e, kind,
-                                                   f0, fd, onbc, tgv, g0, gd, bd);
-    }
-    else
+#define FFHIP_RHS(RM)                                                                              \
+  do {                                                                                             \
+    k_p1_load_elem<RM><<<nblocks(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, kind, f0, fd, E); \
+    k_row_sum<RM><<<row_sum_grid(n), kWave, 0, s>>>(n, m->v2e_ptr, m->v2e, E, fd, nullptr, onbc, tgv, \
+                                                    g0, gd, bd);                                   \
+  } while (0)
+      if (rm == kRowScale) FFHIP_RHS(kRowScale);
+      else if (rm == kRowPair) FFHIP_RHS(kRowPair);
+      else FFHIP_RHS(kRowQuad);
+#undef FFHIP_RHS
+    } else
       k_rhs_p1_2d<<<nblocks(n, 256), 256, 0, s>>>(n, m->xyz, m->elems, m->v2e_ptr, m->v2e, kind, f0,
                                                    fd, onbc, tgv, g0, gd, bd);
     FFHIP_CHECK(hipGetLastError());
@@ -2106,7 +2177,7 @@ int ffhip_rhs_p1_form(ffhip_ctx ctx, ffhip_mesh m, int kind, double f0, const do
     dfree(labs);
     dfree(fown);
     dfree(gown);
-    dfree(tmes);
+    dfree(E);
   });
 }
 
@@ -2128,14 +2199,15 @@ int ffhip_p1_misfit(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *
       b.onbc = dalloc<uint8_t>(m->nv);
       b.labs = dalloc<int32_t>(nlab);
     }
+    if (r) b.pair = dalloc<double2>(m->nt);
     try {
       misfit_run(ctx, m, u, ud, labels, nlab, J, r, b);
     } catch (...) {
       (void)hipStreamSynchronize(ctx->stream);
-      dfree(b.part); dfree(b.onbc); dfree(b.labs);
+      dfree(b.part); dfree(b.onbc); dfree(b.labs); dfree(b.pair);
       throw;
     }
-    dfree(b.part); dfree(b.onbc); dfree(b.labs);
+    dfree(b.part); dfree(b.onbc); dfree(b.labs); dfree(b.pair);
   });
 }
 
@@ -2252,7 +2324,7 @@ int ffhip_spmv(ffhip_ctx ctx, ffhip_mat A, const double *x, double *y, int trans
   return guard([&] {
     FFHIP_REQUIRE(ctx && A && x && y, FFHIP_ERR_ARG, "ffhip_spmv: null argument");
     hipStream_t s = ctx->stream;
-    const unsigned grid = (nblocks(A->n, kWave) + 7) / 8 * 8;  // whole XCD groups
+    const unsigned grid = row_sum_grid(A->n);
     if (A->half) {  // y = (L + L^T - diag L) x over the full view; symmetric: trans alike
       half_view(A);
       ctx->tic();
