@@ -3,8 +3,7 @@
 // cube(nx,ny,nz) and square(nx,ny) are generated on the GPU with the exact
 // vertex numbering, coordinates, element vertex order, boundary elements and
 // labels of FreeFEM's BuildCube (src/fflib/msh3.cpp:7879-8132) and Carre_
-// (src/fflib/lgmesh.cpp:1229-1384): one thread per vertex / per hex, and a
-// scan for the boundary-element offsets.
+// (src/fflib/lgmesh.cpp:1229-1384), each in one pass.
 #include <hipcub/hipcub.hpp>
 
 #include <cstdarg>
@@ -53,83 +52,90 @@ __constant__ int c_split6[6][4] = {{4, 0, 6, 7}, {0, 4, 5, 7}, {1, 0, 5, 7},
 // Tet faces (Mesh3dn.cpp:72)
 __constant__ int c_tetface[4][3] = {{3, 2, 1}, {0, 2, 3}, {3, 1, 0}, {0, 1, 2}};
 
-__global__ void k_cube_vertices(int nx, int ny, int nz, double xd, double yd,
-                                double zd, double *__restrict__ xyz) {
-  const int64_t nv = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nv) return;
-  const int i = (int)(p % (nx + 1));
-  const int j = (int)((p / (nx + 1)) % (ny + 1));
-  const int k = (int)(p / ((int64_t)(nx + 1) * (ny + 1)));
-  xyz[3 * p + 0] = 0. + xd * i;
-  xyz[3 * p + 1] = 0. + yd * j;
-  xyz[3 * p + 2] = 0. + zd * k;
+struct CubeLabels {
+  int32_t lab[6];
+};
+
+// boundary triangles of the hexes before hex (i, j, k) in hex order: two per
+// hex face on the boundary, counted plane by plane
+__device__ inline int cube_bfaces_before(int i, int j, int k, int nx, int ny, int nz) {
+  const int row = k * ny + j, in_plane = i + nx * j;
+  return 2 * (row + (i > 0) + row +                                        // x = 0, x = 1
+              k * nx + (j > 0 ? nx : i) + k * nx + (j == ny - 1 ? i : 0) +  // y = 0, y = 1
+              (k > 0 ? nx * ny : in_plane) + (k == nz - 1 ? in_plane : 0)); // z = 0, z = 1
 }
 
-__device__ inline int cube_vlab(int64_t v, int nx, int ny, int nz) {
-  const int64_t nj = nx + 1, nk = nj * (ny + 1);
-  const int vi = (int)(v % nj), vj = (int)((v / nj) % (ny + 1)), vk = (int)(v / nk);
-  return 1 * (vi == 0) + 2 * (vi == nx) + 4 * (vj == 0) + 8 * (vj == ny) +
-         16 * (vk == 0) + 32 * (vk == nz);
-}
-
-// one thread per hex: its six tets, and its boundary triangle count
-__global__ void k_cube_tets(int nx, int ny, int nz, int32_t *__restrict__ tets,
-                            int64_t *__restrict__ bcount) {
-  const int64_t nc = (int64_t)nx * ny * nz;
-  const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= nc) return;
-  const int i = (int)(h % nx), j = (int)((h / nx) % ny), k = (int)(h / ((int64_t)nx * ny));
-  const int64_t nj = nx + 1, nk = nj * (ny + 1);
-  int32_t n8[8];
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-        n8[a + 2 * b + 4 * c] = (int32_t)((i + a) + nj * (j + b) + nk * (k + c));
-#pragma unroll
-  for (int d = 0; d < 6; ++d) {
-    int4 t;
-    t.x = n8[c_split6[d][0]]; t.y = n8[c_split6[d][1]];
-    t.z = n8[c_split6[d][2]]; t.w = n8[c_split6[d][3]];
-    reinterpret_cast<int4 *>(tets)[6 * h + d] = t;
+// The whole mesh in one pass: thread p writes vertex p, the block its 256
+// hexes' 1536 tets (consecutive threads on consecutive tets, from the hexes'
+// first vertices in LDS) and each boundary hex its triangles in BuildCube's
+// order, hex, tet, face (msh3.cpp:8090-8110), at the offset counted above.
+// Bound by the tets' store (16 B each): 114 us for 24.6 M tets at cube(160).  A
+// thread per hex that found its triangles by comparing the vertices' labels
+// (64-bit divisions) took 450 us there and about 60 us on the smallest box,
+// after a scan of the hexes' counts.
+__global__ __launch_bounds__(256) void k_cube_mesh(int nx, int ny, int nz, double xd, double yd,
+                                                   double zd, CubeLabels L, double *__restrict__ xyz,
+                                                   int32_t *__restrict__ tets,
+                                                   int32_t *__restrict__ btri,
+                                                   int32_t *__restrict__ blab) {
+  __shared__ int32_t first[256];
+  __shared__ int4 off[6];  // the tets' vertex offsets from the hex's first vertex
+  const int nv = (nx + 1) * (ny + 1) * (nz + 1), nc = nx * ny * nz;
+  const int nj = nx + 1, nk = nj * (ny + 1);
+  const int t = threadIdx.x, p = blockIdx.x * 256 + t;
+  if (p < nv) {
+    const int i = p % nj, r = p / nj, j = r % (ny + 1), k = r / (ny + 1);
+    xyz[3 * (int64_t)p + 0] = 0. + xd * i;
+    xyz[3 * (int64_t)p + 1] = 0. + yd * j;
+    xyz[3 * (int64_t)p + 2] = 0. + zd * k;
   }
-  // each hex face on the boundary carries two boundary triangles
-  bcount[h] = 2 * ((i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1) +
-                   (k == 0) + (k == nz - 1));
-}
-
-// boundary triangles in BuildCube's order: hex, tet, face (msh3.cpp:8090-8110)
-__global__ void k_cube_bfaces(int nx, int ny, int nz, const int32_t *__restrict__ tets,
-                              const int64_t *__restrict__ boff, const int32_t *lab6,
-                              int32_t *__restrict__ btri, int32_t *__restrict__ blab) {
-  const int64_t nc = (int64_t)nx * ny * nz;
-  const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= nc) return;
-  const int i = (int)(h % nx), j = (int)((h / nx) % ny), k = (int)(h / ((int64_t)nx * ny));
-  if (!(i == 0 || i == nx - 1 || j == 0 || j == ny - 1 || k == 0 || k == nz - 1)) return;
+  auto corner = [&](int c) { return (c & 1) + ((c >> 1) & 1) * nj + (c >> 2) * nk; };
+  const int i = p % nx, r = p / nx, j = r % ny, k = r / ny;  // hex p
+  const int f0 = i + nj * j + nk * k;
+  first[t] = f0;
+  if (t < 6)
+    off[t] = int4{corner(c_split6[t][0]), corner(c_split6[t][1]), corner(c_split6[t][2]),
+                  corner(c_split6[t][3])};
+  __syncthreads();
+  const int h0 = blockIdx.x * 256, ntb = 6 * (nc - h0 < 256 ? nc - h0 : 256);
+  for (int q = t; q < ntb; q += 256) {
+    const int h = q / 6, b = first[h];
+    const int4 o = off[q - 6 * h];
+    reinterpret_cast<int4 *>(tets)[6 * (int64_t)h0 + q] = int4{b + o.x, b + o.y, b + o.z, b + o.w};
+  }
+  if (p >= nc) return;
+  // the hex's faces on the boundary, bits as the vertex labels of BuildCube
+  const int on = 1 * (i == 0) + 2 * (i == nx - 1) + 4 * (j == 0) + 8 * (j == ny - 1) + 16 * (k == 0) +
+                 32 * (k == nz - 1);
+  if (!on) return;
   const int nff[6] = {3, 1, 0, 2, 4, 5};  // msh3.cpp:8050
-  int64_t o = boff[h];
-  const int64_t oend = boff[h + 1];  // writes stay inside this hex's scanned range
-  for (int d = 0; d < 6; ++d) {
-    const int32_t *nu = tets + 4 * (6 * h + d);
+  int64_t o = cube_bfaces_before(i, j, k, nx, ny, nz);
+  for (int d = 0; d < 6; ++d)
     for (int f = 0; f < 4; ++f) {
-      const int32_t a = nu[c_tetface[f][0]], b = nu[c_tetface[f][1]], c = nu[c_tetface[f][2]];
-      const int l = cube_vlab(a, nx, ny, nz) & cube_vlab(b, nx, ny, nz) & cube_vlab(c, nx, ny, nz);
-      for (int bit = 0; bit < 6; ++bit)
-        if (l == (1 << bit) && o < oend) {
-          btri[3 * o + 0] = a; btri[3 * o + 1] = b; btri[3 * o + 2] = c;
-          blab[o] = lab6[nff[bit]];
-          ++o;
-        }
+      int c[3], side = on;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        c[q] = c_split6[d][c_tetface[f][q]];
+        // the hex faces that corner c lies on
+        side &= (c[q] & 1 ? 2 : 1) | (c[q] & 2 ? 8 : 4) | (c[q] & 4 ? 32 : 16);
+      }
+      if (!side) continue;  // three corners share at most one face
+      btri[3 * o + 0] = f0 + corner(c[0]);
+      btri[3 * o + 1] = f0 + corner(c[1]);
+      btri[3 * o + 2] = f0 + corner(c[2]);
+      blab[o] = L.lab[nff[__builtin_ctz(side)]];
+      ++o;
     }
-  }
 }
 
 // ---------------------------------------------------------------- square
-__global__ void k_square(int nx, int ny, double *__restrict__ xy, int32_t *__restrict__ tris) {
+struct SquareLabels {
+  int32_t lab[4];
+};
+
+__global__ void k_square(int nx, int ny, SquareLabels L, double *__restrict__ xy,
+                         int32_t *__restrict__ tris, int32_t *__restrict__ bed,
+                         int32_t *__restrict__ blab) {
   const int64_t nv = (int64_t)(nx + 1) * (ny + 1), nc = (int64_t)nx * ny;
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p < nv) {
@@ -143,19 +149,15 @@ __global__ void k_square(int nx, int ny, double *__restrict__ xy, int32_t *__res
     int32_t *t = tris + 6 * p;  // diag 1 (lgmesh.cpp:1300-1306)
     t[0] = i0; t[1] = i1; t[2] = i2; t[3] = i0; t[4] = i2; t[5] = i3;
   }
-}
-
-__global__ void k_square_bedges(int nx, int ny, const int32_t *lab4,
-                                int32_t *__restrict__ bed, int32_t *__restrict__ blab) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nbe = 2 * ((int64_t)nx + ny);
+  // boundary edges (2 (nx + ny) may exceed the vertices of a thin square: the grid covers both)
+  const int64_t b = p, nbe = 2 * ((int64_t)nx + ny);
   if (b >= nbe) return;
   const int nx1 = nx + 1;
   int32_t i1, i2, l;
-  if (b < nx) { i1 = (int32_t)b; i2 = i1 + 1; l = lab4[0]; }                       // bottom
-  else if (b < nx + ny) { int j = (int)(b - nx); i1 = nx + j * nx1; i2 = i1 + nx1; l = lab4[1]; }  // right
-  else if (b < 2 * nx + ny) { int i = (int)(b - nx - ny); i1 = i + ny * nx1; i2 = i1 + 1; l = lab4[2]; }  // up
-  else { int j = (int)(b - 2 * nx - ny); i1 = j * nx1; i2 = i1 + nx1; l = lab4[3]; }  // left
+  if (b < nx) { i1 = (int32_t)b; i2 = i1 + 1; l = L.lab[0]; }                       // bottom
+  else if (b < nx + ny) { int j = (int)(b - nx); i1 = nx + j * nx1; i2 = i1 + nx1; l = L.lab[1]; }  // right
+  else if (b < 2 * nx + ny) { int i = (int)(b - nx - ny); i1 = i + ny * nx1; i2 = i1 + 1; l = L.lab[2]; }  // up
+  else { int j = (int)(b - 2 * nx - ny); i1 = j * nx1; i2 = i1 + nx1; l = L.lab[3]; }  // left
   bed[2 * b] = i1; bed[2 * b + 1] = i2; blab[b] = l;
 }
 
@@ -397,8 +399,8 @@ int ffhip_mesh3_cube(ffhip_ctx ctx, int nx, int ny, int nz, const int32_t labels
     const int64_t nbe = 4 * ((int64_t)nx * ny + (int64_t)nx * nz + (int64_t)ny * nz);
     FFHIP_REQUIRE(nv < (1ll << 31) && 4 * nt < (1ll << 31), FFHIP_ERR_UNSUPPORTED,
                   "ffhip_mesh3_cube: mesh too large for int32 element ids");
-    int32_t lab[6] = {1, 2, 3, 4, 5, 6};
-    if (labels) memcpy(lab, labels, sizeof(lab));
+    CubeLabels lab = {{1, 2, 3, 4, 5, 6}};
+    if (labels) memcpy(lab.lab, labels, sizeof(lab.lab));
     ffhip_mesh m = new ffhip_mesh_s();
     m->ctx = ctx; m->dim = 3; m->nloc = 4; m->nbloc = 3;
     m->nv = nv; m->nt = nt; m->nbe = nbe;
@@ -406,25 +408,11 @@ int ffhip_mesh3_cube(ffhip_ctx ctx, int nx, int ny, int nz, const int32_t labels
     m->elems = dalloc<int32_t>(4 * nt);
     m->belems = dalloc<int32_t>(3 * nbe);
     m->blab = dalloc<int32_t>(nbe);
-    int64_t *cnt = dalloc<int64_t>(nc + 1);
-    int64_t *off = dalloc<int64_t>(nc + 1);
-    int32_t *dlab = dalloc<int32_t>(6);
-    FFHIP_CHECK(hipMemcpyAsync(dlab, lab, sizeof(lab), hipMemcpyHostToDevice, ctx->stream));
-    FFHIP_CHECK(hipMemsetAsync(cnt + nc, 0, sizeof(int64_t), ctx->stream));
     ctx->tic();
-    const int B = 256;
-    k_cube_vertices<<<(unsigned)((nv + B - 1) / B), B, 0, ctx->stream>>>(
-        nx, ny, nz, 1. / nx, 1. / ny, 1. / nz, m->xyz);
-    k_cube_tets<<<(unsigned)((nc + B - 1) / B), B, 0, ctx->stream>>>(nx, ny, nz, m->elems, cnt);
-    exclusive_scan_i64(ctx, cnt, off, nc + 1);
-    k_cube_bfaces<<<(unsigned)((nc + B - 1) / B), B, 0, ctx->stream>>>(
-        nx, ny, nz, m->elems, off, dlab, m->belems, m->blab);
+    k_cube_mesh<<<(unsigned)((nv + 255) / 256), 256, 0, ctx->stream>>>(  // nv > nc
+        nx, ny, nz, 1. / nx, 1. / ny, 1. / nz, lab, m->xyz, m->elems, m->belems, m->blab);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
-    const int64_t got = read_i64(ctx, off + nc);
-    dfree(cnt); dfree(off); dfree(dlab);
-    FFHIP_REQUIRE(got == nbe, FFHIP_ERR_INTERNAL, "cube: %lld boundary faces, expected %lld",
-                  (long long)got, (long long)nbe);
     *out = m;
   });
 }
@@ -437,8 +425,8 @@ int ffhip_mesh2_square(ffhip_ctx ctx, int nx, int ny, const int32_t labels[4],
     const int64_t nbe = 2 * ((int64_t)nx + ny);
     FFHIP_REQUIRE(nv < (1ll << 31) && 3 * nt < (1ll << 31), FFHIP_ERR_UNSUPPORTED,
                   "ffhip_mesh2_square: mesh too large");
-    int32_t lab[4] = {1, 2, 3, 4};
-    if (labels) memcpy(lab, labels, sizeof(lab));
+    SquareLabels lab = {{1, 2, 3, 4}};
+    if (labels) memcpy(lab.lab, labels, sizeof(lab.lab));
     ffhip_mesh m = new ffhip_mesh_s();
     m->ctx = ctx; m->dim = 2; m->nloc = 3; m->nbloc = 2;
     m->nv = nv; m->nt = nt; m->nbe = nbe;
@@ -446,16 +434,12 @@ int ffhip_mesh2_square(ffhip_ctx ctx, int nx, int ny, const int32_t labels[4],
     m->elems = dalloc<int32_t>(3 * nt);
     m->belems = dalloc<int32_t>(2 * nbe);
     m->blab = dalloc<int32_t>(nbe);
-    int32_t *dlab = dalloc<int32_t>(4);
-    FFHIP_CHECK(hipMemcpyAsync(dlab, lab, sizeof(lab), hipMemcpyHostToDevice, ctx->stream));
-    const int B = 256;
-    const int64_t nn = nv > nt / 2 ? nv : nt / 2;
+    const int64_t nn = nv > nbe ? nv : nbe;
     ctx->tic();
-    k_square<<<(unsigned)((nn + B - 1) / B), B, 0, ctx->stream>>>(nx, ny, m->xyz, m->elems);
-    k_square_bedges<<<(unsigned)((nbe + B - 1) / B), B, 0, ctx->stream>>>(nx, ny, dlab, m->belems, m->blab);
+    k_square<<<(unsigned)((nn + 255) / 256), 256, 0, ctx->stream>>>(nx, ny, lab, m->xyz, m->elems,
+                                                                    m->belems, m->blab);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
-    dfree(dlab);
     *out = m;
   });
 }
