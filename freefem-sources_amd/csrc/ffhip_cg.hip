@@ -379,9 +379,14 @@ __global__ void k_bsr_len(int64_t nb, int64_t S3, const int64_t *__restrict__ bp
 // rows (values optionally through tmap; FP32 copy of D^-1/2 A D^-1/2).
 // One block per 64-row slice: the slice's rows are read KC blocks at a time,
 // each of its 3 x 64 scalar rows as one contiguous run of 3 KC values, into
-// LDS, and written out entry-major (the 9 x 64 values of block entry k of the
-// slice at 9 ptr[s] + 9 64 k, placed by bsr_pos); padding entries get value 0
-// and the row's own block column.
+// LDS (the next KC blocks' values already on their way while these are written),
+// and written out entry-major, a thread per block entry (the 9 x 64 values of
+// block entry k of the slice at 9 ptr[s] + 9 64 k, placed by bsr_pos, as
+// 16-byte vectors); padding entries get value 0 and the row's own block column.
+// Bound by HBM: 12 B read and 8 (+ 4) written per value.  cube(32) with both
+// copies: 1175 us with one value per thread and step (two loads in flight, a
+// scaling gather per value and side), now 512 us, 3.1 TB/s (KC = 4: 617 us,
+// KC = 12: 534 us).
 constexpr int kBsrKC = 8;
 // Position of value q (3c + c') of lane li inside one slice entry of the
 // 3x3-block values (9 x 64 values per entry): values 0..7 in vectors of W = 16
@@ -392,18 +397,20 @@ __host__ __device__ constexpr int bsr_pos(int q, int li) {
   constexpr int W = 16 / (int)sizeof(V);
   return q < 8 ? ((q / W) * kSlice + li) * W + q % W : 8 * kSlice + li;
 }
+template <bool TMAP>
 __global__ __launch_bounds__(256) void k_bsr_fill(
-    int64_t nb, int64_t ents, const int64_t *__restrict__ bptr, const int32_t *__restrict__ perm,
+    int64_t nb, const int64_t *__restrict__ bptr, const int32_t *__restrict__ perm,
     const int64_t *__restrict__ sptr, const int32_t *__restrict__ slen,
     const int64_t *__restrict__ rowptr, const int32_t *__restrict__ colidx,
     const double *__restrict__ vals, const int64_t *__restrict__ tmap,
     const double *__restrict__ dsc, int32_t *__restrict__ bcol, double *__restrict__ bval,
     float *__restrict__ bval32) {
   constexpr int KC = kBsrKC, P = kSlice + 1;  // P: padded lane stride (LDS banks)
+  constexpr int NL = kSlice * 9 * KC / 256, NE = KC * kSlice / 256;  // values, block entries per thread
   __shared__ double T[9 * KC * P];
-  __shared__ int32_t Cb[KC * kSlice];
   __shared__ int32_t An[kSlice], Ln[kSlice];
   __shared__ int64_t R0[3 * kSlice];
+  __shared__ double Ds[3 * kSlice];  // the rows' scaling
   const int64_t s = blockIdx.x;
   const int t = threadIdx.x;
   if (t < kSlice) {
@@ -412,47 +419,77 @@ __global__ __launch_bounds__(256) void k_bsr_fill(
     An[t] = a;
     Ln[t] = a >= 0 ? (int32_t)(bptr[a + 1] - bptr[a]) : 0;
 #pragma unroll
-    for (int c = 0; c < 3; ++c) R0[3 * t + c] = a >= 0 ? rowptr[3 * (int64_t)a + c] : 0;
+    for (int c = 0; c < 3; ++c) {
+      R0[3 * t + c] = a >= 0 ? rowptr[3 * (int64_t)a + c] : 0;
+      Ds[3 * t + c] = bval32 && a >= 0 ? dsc[3 * (int64_t)a + c] : 0.;
+    }
   }
   __syncthreads();
   const int W = slen[s];
   const int64_t base = sptr[s];
+  // item u of thread t: t + 256 u = (li * 3 + c) * 3 KC + x, x = 3 kk + cp
+  auto load = [&](int k0, double (&v)[NL], int32_t (&cb)[NE]) {
+#pragma unroll
+    for (int u = 0; u < NL; ++u) {
+      const int it = t + 256 * u, x = it % (3 * KC), rc = it / (3 * KC);
+      const int k = k0 + x / 3;
+      v[u] = 0.;
+      if (k < Ln[rc / 3]) {
+        const int64_t src = R0[rc] + 3 * (int64_t)k0 + x;
+        v[u] = TMAP ? vals[tmap[src]] : vals[src];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NE; ++u) {
+      const int li = (t + 256 * u) % kSlice, k = k0 + (t + 256 * u) / kSlice;
+      cb[u] = k < Ln[li] ? colidx[R0[3 * li] + 3 * (int64_t)k] : -1;
+    }
+  };
+  double v[NL];
+  int32_t cb[NE];
+  load(0, v, cb);
   for (int k0 = 0; k0 < W; k0 += KC) {
-    const int kc = W - k0 < KC ? W - k0 : KC;
-    // read: item = ((li * 3 + c) * 3 KC + x), x = 3 kk + cp
-    for (int it = t; it < kSlice * 9 * KC; it += 256) {
-      const int x = it % (3 * KC), rc = it / (3 * KC), c = rc % 3, li = rc / 3;
-      const int kk = x / 3, cp = x % 3, k = k0 + kk;
-      double v = 0.;
-      if (kk < kc && k < Ln[li]) {
-        const int64_t src = R0[3 * li + c] + 3 * (int64_t)k + cp;
-        v = tmap ? vals[tmap[src]] : vals[src];
-      }
-      T[((3 * c + cp) * KC + kk) * P + li] = v;
+#pragma unroll
+    for (int u = 0; u < NL; ++u) {
+      const int it = t + 256 * u, x = it % (3 * KC), rc = it / (3 * KC);
+      T[((3 * (rc % 3) + x % 3) * KC + x / 3) * P + rc / 3] = v[u];
     }
-    for (int it = t; it < KC * kSlice; it += 256) {
-      const int li = it % kSlice, kk = it / kSlice, k = k0 + kk;
-      Cb[it] = kk < kc && k < Ln[li] ? colidx[R0[3 * li] + 3 * (int64_t)k] / 3 : -1;
-    }
+    int32_t col[NE];
+#pragma unroll
+    for (int u = 0; u < NE; ++u) col[u] = cb[u] < 0 ? -1 : cb[u] / 3;
     __syncthreads();
-    // write: entry kk, value q, lane li (one contiguous run of 9 x 64 kc values)
-    for (int it = t; it < 9 * kc * kSlice; it += 256) {
-      const int li = it % kSlice, q = (it / kSlice) % 9, kk = it / (9 * kSlice);
-      const int64_t eb = 9 * (base + (int64_t)(k0 + kk) * kSlice);
-      const double v = T[(q * KC + kk) * P + li];
-      if (bval) bval[eb + bsr_pos<double>(q, li)] = v;
+    if (k0 + KC < W) load(k0 + KC, v, cb);
+#pragma unroll
+    for (int u = 0; u < NE; ++u) {
+      const int li = (t + 256 * u) % kSlice, kk = (t + 256 * u) / kSlice;
+      if (k0 + kk >= W) continue;
+      const int64_t e = base + (int64_t)(k0 + kk) * kSlice, eb = 9 * e;
+      double w[9];
+#pragma unroll
+      for (int q = 0; q < 9; ++q) w[q] = T[(q * KC + kk) * P + li];
+      if (bval) {
+#pragma unroll
+        for (int q = 0; q < 8; q += 2)
+          *reinterpret_cast<double2 *>(bval + eb + bsr_pos<double>(q, li)) = double2{w[q], w[q + 1]};
+        bval[eb + bsr_pos<double>(8, li)] = w[8];
+      }
       if (bval32) {
-        const int cb = Cb[kk * kSlice + li];
-        bval32[eb + bsr_pos<float>(q, li)] =
-            cb < 0 ? 0.f : (float)(v * dsc[3 * (int64_t)An[li] + q / 3] * dsc[3 * (int64_t)cb + q % 3]);
+        double dc[3] = {0., 0., 0.};
+        if (col[u] >= 0) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) dc[c] = dsc[3 * (int64_t)col[u] + c];
+        }
+        float f[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) f[q] = col[u] < 0 ? 0.f : (float)(w[q] * Ds[3 * li + q / 3] * dc[q % 3]);
+#pragma unroll
+        for (int q = 0; q < 8; q += 4)
+          *reinterpret_cast<float4 *>(bval32 + eb + bsr_pos<float>(q, li)) =
+              float4{f[q], f[q + 1], f[q + 2], f[q + 3]};
+        bval32[eb + bsr_pos<float>(8, li)] = f[8];
       }
+      if (bcol) bcol[e + li] = col[u] >= 0 ? col[u] : (An[li] >= 0 ? An[li] : 0);
     }
-    if (bcol)
-      for (int it = t; it < kc * kSlice; it += 256) {
-        const int li = it % kSlice, kk = it / kSlice;
-        const int cb = Cb[kk * kSlice + li];
-        bcol[base + (int64_t)(k0 + kk) * kSlice + li] = cb >= 0 ? cb : (An[li] >= 0 ? An[li] : 0);
-      }
     __syncthreads();
   }
 }
@@ -1845,9 +1882,9 @@ static void cg_fill_values(ffhip_cg cg, bool transposed, const DiagBufs *db = nu
   if (cg->fmt == kBsr3) {
     if (!dv) dv = dalloc<double>(nval);
     const int64_t nb = A->n / 3, S3 = (nb + kSlice - 1) / kSlice;
-    k_bsr_fill<<<S3, 256, 0, s>>>(
-        nb, cg->ents, A->nodeptr, cg->bperm, cg->sptr, cg->slen, A->rowptr, A->colidx, A->vals, tmap,
-        cg->dsc, transposed ? nullptr : cg->bcol, dv, mixed ? fv : nullptr);
+    auto fill = tmap ? k_bsr_fill<true> : k_bsr_fill<false>;
+    fill<<<S3, 256, 0, s>>>(nb, A->nodeptr, cg->bperm, cg->sptr, cg->slen, A->rowptr, A->colidx, A->vals,
+                            tmap, cg->dsc, transposed ? nullptr : cg->bcol, dv, mixed ? fv : nullptr);
   } else if (cg->fmt != kCsrV) {
     if (!dv) dv = dalloc<double>(cg->ents);
     k_sell_fill<<<cg->S, 256, 0, s>>>(
