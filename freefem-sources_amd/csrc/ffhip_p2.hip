@@ -22,15 +22,13 @@
 //              first-appearance numbering.
 //   pattern    node rows (sorted unique node columns, LDS merge per lane, as
 //              P1), expanded to scalar rows of 3 x 3 blocks.
-//   element    one wave per element: M = D W D^T (30 x 30, D = P2 gradients
-//              at the 14 points, W = |K| w_q) as three 16x16 tiles of
-//              v_mfma_f64_16x16x4f64 over k = 16 (14 points, zero padded);
-//              K[(c,i),(c',j)] = lambda M[ic][jc'] + mu M[ic'][jc]
-//              + mu delta_cc' sum_a M[ia][ja] is formed from M in LDS and
-//              written node-block major (90 doubles per local node).
-//   gather     one wave per node: the incident elements' 90-value blocks are
-//              added in element order into the node's 3 rows staged in LDS,
-//              then written back contiguously.  No atomics, deterministic.
+//   element    the P2 gradients are linear in the barycentrics, so a tet leaves
+//              only its vertex gradients (Lame: |K| and G, 13 doubles; scalar:
+//              their products and the moments of kappa at the Tet_5 points, 25).
+//   rows       one wave per node: the incident tets' blocks of the node's row
+//              are formed from those, added in element order into the rows
+//              staged in LDS, and written back contiguously.  No element
+//              matrices in memory, no atomics, deterministic.
 #include <hipcub/hipcub.hpp>
 
 #include <climits>
@@ -305,254 +303,312 @@ __global__ void k_p2_compact(int64_t nn, const int64_t *__restrict__ nodeptr,
   diag[a] = d < 0 ? -1 : p0 + d;
 }
 
-// ---------------------------------------------------------------- element matrices
-typedef double d4 __attribute__((ext_vector_type(4)));
+// ---------------------------------------------------------------- element integrals, row assembly
+// A P2 gradient is linear in the barycentrics l_v:
+//   vertex i:        4 G_i l_i - G_i
+//   edge (i0, i1):   4 (G_i1 l_i0 + G_i0 l_i1)              (P012_3d.cpp:236-262)
+// so the integral of d_c phi_i d_c' phi_j over a tet is a sum over at most
+// 2 x 2 pairs of vertex gradients, each with a weight that depends on the pair's
+// barycentric indices alone (the mean of l_v l_w is (1 + delta_vw) / 20), or,
+// with a coefficient kappa, on the second moments of kappa.  Tet_5 is exact
+// for these integrands (degree 2; with kappa the moments are taken at its
+// points), so these are the values of Element_Op up to rounding.
+//
+// What the element pass leaves per tet (stride kLame / kLap doubles):
+//   Lame:    G_0..G_3, |K|
+//   Laplace: G_v . G_w (10), m_vw = int kappa l_v l_w (10, both packed by sym4),
+//            M_v = sum_w m_vw (4), M = sum_v M_v
+constexpr int kLame = 13, kLap = 25;
 
-__device__ inline double pick3(const double v[3], int a) { return a == 0 ? v[0] : (a == 1 ? v[1] : v[2]); }
-__device__ inline double pick4(const double v[4], int i) {
-  return i == 0 ? v[0] : (i == 1 ? v[1] : (i == 2 ? v[2] : v[3]));
-}
-
-
-// element rows a node-row gather keeps in flight
-constexpr int kGatherD = 4;
-
-constexpr int kElemBlock = 256;
-constexpr int kElemWaves = kElemBlock / kWave;
-constexpr int kMs = 33;  // LDS row stride of M (doubles)
-
-// Row r = 3 i + a of D (r < 30): gradient component a of P2 basis i,
-//   vertex i:        G_i[a] (4 l_i - 1)
-//   edge (i0, i1):   4 (G_i1[a] l_i0 + G_i0[a] l_i1)        (P012_3d.cpp:236-262)
-struct P2Row {
-  int vert;      // 1: vertex basis
-  int i0, i1;    // vertex index (i0) or edge end points
-  double g0, g1; // G_i0[a], G_i1[a] of the current element
-};
-
-__device__ inline double p2_grad(const P2Row &R, const double l[4]) {
-  if (R.vert) return R.g0 * (4 * pick4(l, R.i0) - 1);
-  return 4 * (R.g1 * pick4(l, R.i0) + R.g0 * pick4(l, R.i1));
-}
-
-// LAP = false: K[(c,i),(c',j)] (row = test function) of the Lame form as 10
-// node blocks of 90 doubles [c][j][c'], block i stored at Ke[90 k] for the
-// incidence k of (e, i).  LAP = true: the scalar P2 stiffness of
-// int3d(kappa grad u . grad v), K(i,j) = sum_a M[(i,a),(j,a)] with kappa(x_q)
-// in the weights, as 10 rows of 10 doubles at Ke[10 k].
-template <bool LAP>
-__global__ __launch_bounds__(kElemBlock) void k_p2_element(
-    int64_t nt, const double *__restrict__ xyz, const int32_t *__restrict__ tets, double lambda,
-    double mu, int kind, double c0, const double *__restrict__ kappa_e,
-    const int32_t *__restrict__ inv, double *__restrict__ Ke) {
-  __shared__ double sM[kElemWaves][32 * kMs];
-  const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int col = lane % 16, kq = lane / 16;
-  // the two rows of D this lane feeds to the matrix cores (r = col, 16 + col)
-  int rr[2] = {col, 16 + col};
-  P2Row R[2];
-  int rvalid[2];
+__global__ __launch_bounds__(256) void k_p2_elem_lame(int64_t nt, const double *__restrict__ xyz,
+                                                      const int32_t *__restrict__ tets,
+                                                      double *__restrict__ E) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nt) return;
+  const int4 tv = reinterpret_cast<const int4 *>(tets)[e];
+  const int32_t id[4] = {tv.x, tv.y, tv.z, tv.w};
+  double v[4][3], G[4][3];
 #pragma unroll
-  for (int I = 0; I < 2; ++I) {
-    const int r = rr[I];
-    rvalid[I] = r < 30;
-    const int i = r < 30 ? r / 3 : 0;
-    R[I].vert = i < 4;
-    const int ed = i < 4 ? 0 : i - 4;
-    R[I].i0 = i < 4 ? i : c_edge[ed][0];
-    R[I].i1 = i < 4 ? i : c_edge[ed][1];
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[i][k] = xyz[3 * (int64_t)id[i] + k];
+  const double mes = tet_geom(v, G);
+  double *o = E + kLame * e;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) o[3 * i + k] = G[i][k];
+  o[12] = mes;
+}
+
+__global__ __launch_bounds__(256) void k_p2_elem_lap(int64_t nt, const double *__restrict__ xyz,
+                                                     const int32_t *__restrict__ tets, int kind,
+                                                     double c0, const double *__restrict__ kappa_e,
+                                                     double *__restrict__ E) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nt) return;
+  const int4 tv = reinterpret_cast<const int4 *>(tets)[e];
+  const int32_t id[4] = {tv.x, tv.y, tv.z, tv.w};
+  double v[4][3], G[4][3], u[4] = {0., 0., 0., 0.};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[i][k] = xyz[3 * (int64_t)id[i] + k];
+    if (kind == FFHIP_COEF_P1) u[i] = kappa_e[id[i]];
   }
-  double* M = sM[w];
-  for (int64_t base = (int64_t)blockIdx.x * kElemWaves; base < nt; base += (int64_t)gridDim.x * kElemWaves) {
-    const int64_t e = base + w;  // wave-uniform
-    if (e < nt) {
-      const int4 tv = reinterpret_cast<const int4 *>(tets)[e];
-      const int32_t id[4] = {tv.x, tv.y, tv.z, tv.w};
-      double v[4][3];
+  const double mes = tet_geom(v, G);
+  const double kc = kind == FFHIP_COEF_P0 ? kappa_e[e] : c0;
+  double m[10] = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
+#pragma unroll 2
+  for (int q = 0; q < 14; ++q) {
+    const double px = c_qf5_pts[q][0], py = c_qf5_pts[q][1], pz = c_qf5_pts[q][2];
+    const double l[4] = {1. - (px + py + pz), px, py, pz};
+    double kq = kc;
+    if (kind == FFHIP_COEF_QP) {
+      kq = kappa_e[14 * e + q];
+    } else if (kind == FFHIP_COEF_P1) {
+      kq = p1_value3(u, px, py, pz);
+    } else if (kind == FFHIP_COEF_SIN3) {
+      double P[3];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int k = 0; k < 3; ++k) P[k] = l[0] * v[0][k] + px * v[1][k] + py * v[2][k] + pz * v[3][k];
+      kq = kappa_sin3(P[0], P[1], P[2]);
+    }
+    const double W = (mes * qf5_weight(q)) * kq;
+    int o = 0;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) v[i][k] = xyz[3 * (int64_t)id[i] + k];
-      double G[4][3];
-      const double mes = tet_geom(v, G);
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int I = 0; I < 2; ++I) {
-        const int a = rr[I] < 30 ? rr[I] % 3 : 0;
-        double ga[4];
+      for (int j = i; j < 4; ++j) m[o++] += (W * l[i]) * l[j];
+  }
+  double *o = E + kLap * e;
+  double M = 0.;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) ga[t] = pick3(G[t], a);
-        R[I].g0 = pick4(ga, R[I].i0);
-        R[I].g1 = pick4(ga, R[I].i1);
-      }
-      d4 acc00 = {0., 0., 0., 0.}, acc01 = {0., 0., 0., 0.}, acc11 = {0., 0., 0., 0.};
+  for (int i = 0; i < 4; ++i) {
+    double Mi = 0.;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const int q = 4 * ks + kq;  // quadrature point of this lane's k index
-        double W = 0., l[4] = {0., 0., 0., 0.};
-        if (q < 14) {
-          const double px = c_qf5_pts[q][0], py = c_qf5_pts[q][1], pz = c_qf5_pts[q][2];
-          l[0] = 1. - (px + py + pz); l[1] = px; l[2] = py; l[3] = pz;
-          W = mes * qf5_weight(q);
-          if (LAP) {
-            double kq = c0;
-            if (kind == FFHIP_COEF_P0) kq = kappa_e[e];
-            else if (kind == FFHIP_COEF_QP) kq = kappa_e[14 * e + q];
-            else if (kind == FFHIP_COEF_P1) {
-              const double u[4] = {kappa_e[id[0]], kappa_e[id[1]], kappa_e[id[2]], kappa_e[id[3]]};
-              kq = p1_value3(u, px, py, pz);
-            }
-            else if (kind == FFHIP_COEF_SIN3) {
-              double P[3];
-#pragma unroll
-              for (int k = 0; k < 3; ++k)
-                P[k] = l[0] * v[0][k] + px * v[1][k] + py * v[2][k] + pz * v[3][k];
-              kq = kappa_sin3(P[0], P[1], P[2]);
-            }
-            W *= kq;
-          }
-        }
-        const double g0 = rvalid[0] ? p2_grad(R[0], l) : 0.;
-        const double g1 = rvalid[1] ? p2_grad(R[1], l) : 0.;
-        acc00 = __builtin_amdgcn_mfma_f64_16x16x4f64(W * g0, g0, acc00, 0, 0, 0);
-        acc01 = __builtin_amdgcn_mfma_f64_16x16x4f64(W * g0, g1, acc01, 0, 0, 0);
-        acc11 = __builtin_amdgcn_mfma_f64_16x16x4f64(W * g1, g1, acc11, 0, 0, 0);
-      }
-      // D[i][j] of a 16x16 tile in lane l, register v: j = l % 16, i = l / 16 + 4 v
-      // (A[i][k] and B[k][j] are taken from lane i + 16 k and j + 16 k)
-#pragma unroll
-      for (int vv = 0; vv < 4; ++vv) {
-        const int i = kq + 4 * vv, j = col;
-        M[i * kMs + j] = acc00[vv];
-        M[i * kMs + 16 + j] = acc01[vv];
-        M[(16 + j) * kMs + i] = acc01[vv];
-        M[(16 + i) * kMs + 16 + j] = acc11[vv];
+    for (int j = 0; j < 4; ++j) {
+      Mi += m[sym4(i, j)];
+      if (j >= i) {
+        o[sym4(i, j)] = G[i][0] * G[j][0] + G[i][1] * G[j][1] + G[i][2] * G[j][2];
+        o[10 + sym4(i, j)] = m[sym4(i, j)];
       }
     }
-    wave_lds_sync();  // M is this wave's own: the waves of the block run independently
-    if (LAP && e < nt) {
-      for (int o = lane; o < 100; o += kWave) {
-        const int i = o / 10, j = o % 10;
-        const double k = M[(3 * i) * kMs + 3 * j] + M[(3 * i + 1) * kMs + 3 * j + 1] +
-                         M[(3 * i + 2) * kMs + 3 * j + 2];
-        Ke[(int64_t)inv[10 * e + i] * 10 + j] = k;
+    o[20 + i] = Mi;
+    M += Mi;
+  }
+  o[24] = M;
+}
+
+// the (at most two) terms of basis i: barycentric l[s] times the gradient of
+// vertex x[s]; a vertex has one (and the constant -G_i, in the weights)
+struct P2Terms {
+  int vert, l[2], x[2];
+};
+__device__ inline P2Terms p2_terms(int i) {
+  P2Terms t;
+  t.vert = i < 4;
+  const int ed = i < 4 ? 0 : i - 4;
+  t.l[0] = i < 4 ? i : c_edge[ed][0];
+  t.l[1] = i < 4 ? i : c_edge[ed][1];
+  t.x[0] = t.l[1];
+  t.x[1] = t.l[0];
+  return t;
+}
+
+// A wave takes kNodesPerWave consecutive node rows, six incidences (60 lanes, one
+// per (incidence, local node j)) at a time: the six tets' integrals are staged
+// in LDS, each lane forms its 3 x 3 block (Laplace: its entry) of the element's
+// row, and the blocks are added to the row in LDS one incidence after the
+// other, in element order.  The next six incidences' integrals and the items
+// after those are loaded meanwhile: one row at a time the chain of dependent
+// loads (list, items, integrals) took 728 us at cube(32) (69.1 M values), this
+// way 352 us with 14 us for the element pass (391 us with a read, add and write
+// per block instead of LDS additions; 4 or 16 nodes per wave within 3 %).  Bound by instruction issue: about
+// 900 instructions per six incidences.  The element matrices formed on the matrix cores
+// (M = D W D^T per tet, 7.2 KB each) and gathered from memory took 606 + 494 us.
+constexpr int kNodesPerWave = 8;
+template <bool LAP>
+__global__ __launch_bounds__(64) void k_p2_rows(
+    int64_t nn, const int64_t *__restrict__ nodeptr, const int64_t *__restrict__ n2e_ptr,
+    const int32_t *__restrict__ n2e, const uint8_t *__restrict__ slot8, const double *__restrict__ E,
+    double lambda, double mu, double *__restrict__ vals) {
+  constexpr int ED = LAP ? kLap : kLame, NB = LAP ? 1 : 9, NV = 10 * NB, GI = 6;
+  constexpr int NE = (GI * ED + kWave - 1) / kWave;
+  __shared__ double acc[NB * kNodeCap];
+  __shared__ double el[NE * kWave];
+  __shared__ double blk[GI * NV];
+  __shared__ uint8_t so[kWave];
+  const int lane = threadIdx.x;
+  const int64_t a0 = (int64_t)xcd_block_id() * kNodesPerWave;
+  if (a0 >= nn) return;  // one wave per block
+  const int cnt = (int)(nn - a0 < kNodesPerWave ? nn - a0 : kNodesPerWave);
+  // this wave's row and list offsets: lane q holds those of node a0 + q
+  const int64_t myp = nodeptr[a0 + (lane < cnt ? lane : cnt)];
+  const int64_t myk = n2e_ptr[a0 + (lane < cnt ? lane : cnt)];
+  auto bcast = [](int64_t v, int q) -> int64_t {
+    const int lo = __builtin_amdgcn_readlane((int)(v & 0xffffffff), q);
+    const int hi = __builtin_amdgcn_readlane((int)(v >> 32), q);
+    return ((int64_t)hi << 32) | (uint32_t)lo;
+  };
+  const int u = lane / 10, j = lane - 10 * u;
+  const P2Terms C = p2_terms(j);
+  // a group: incidences [k, k + n) of node a0 + c (n <= 6; n = 0 past the end)
+  struct Group {
+    int c, n;
+    int64_t k;
+  };
+  auto first = [&](int c) {
+    Group g{c, 0, 0};
+    if (c < cnt) {
+      g.k = bcast(myk, c);
+      const int64_t d = bcast(myk, c + 1) - g.k;
+      g.n = (int)(d < GI ? d : GI);
+    }
+    return g;
+  };
+  auto next = [&](const Group &g) {
+    if (g.c >= cnt) return g;
+    const int64_t left = bcast(myk, g.c + 1) - (g.k + GI);
+    if (left > 0) return Group{g.c, (int)(left < GI ? left : GI), g.k + GI};
+    return first(g.c + 1);
+  };
+  auto load_items = [&](const Group &g, int32_t &item, int &sb) {
+    item = 0;
+    sb = 0;
+    if (u < g.n) {
+      item = n2e[g.k + u];
+      sb = slot8[g.k * 10 + lane];
+    }
+  };
+  auto load_integrals = [&](const Group &g, int32_t item, double (&r)[NE]) {
+    const int32_t e = item / 10;
+#pragma unroll
+    for (int x0 = 0; x0 < NE; ++x0) {
+      const int x = x0 * kWave + lane, uu = x / ED;
+      const int32_t eu = __shfl(e, uu < GI ? 10 * uu : 0, kWave);
+      r[x0] = uu < g.n ? E[(int64_t)eu * ED + (x - uu * ED)] : 0.;
+    }
+  };
+  Group g0 = first(0), g1 = next(g0);
+  int32_t item0, item1;
+  int so0, so1;
+  double r0[NE];
+  load_items(g0, item0, so0);
+  load_items(g1, item1, so1);
+  load_integrals(g0, item0, r0);
+  int64_t p0 = 0;
+  int L = 0, tj[2] = {0, 0}, tdst[2] = {0, 0}, row = -1;
+  while (g0.c < cnt) {
+    if (g0.c != row) {  // the node's row starts
+      row = g0.c;
+      p0 = bcast(myp, row);
+      L = (int)(bcast(myp, row + 1) - p0);
+      for (int t = lane; t < NB * L; t += kWave) acc[t] = 0.;
+      if (!LAP) {  // this lane's two entries of a 90-value block, [c][j][c'] of t = lane, lane + 64
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int t = lane + h * kWave, c = t / 30, r2 = t % 30;
+          tj[h] = r2 / 3;
+          tdst[h] = c * 3 * L + r2 % 3;  // + 3 * offset of node column j
+        }
       }
-    } else if (e < nt) {
-      // entry pairs (rem, rem + 1): a pair stays in its 90-value node-block
-      // row, and rows start at multiples of 720 bytes, so one 16-byte store
-      auto entry = [&](int i, int rem) {
-        const int c = rem / 30, r2 = rem % 30, j = r2 / 3, cp = r2 % 3;
-        double k = lambda * M[(3 * i + c) * kMs + 3 * j + cp] + mu * M[(3 * i + cp) * kMs + 3 * j + c];
-        if (c == cp)
-          k += mu * (M[(3 * i) * kMs + 3 * j] + M[(3 * i + 1) * kMs + 3 * j + 1] +
-                     M[(3 * i + 2) * kMs + 3 * j + 2]);
-        return k;
-      };
-      for (int o = lane; o < 450; o += kWave) {
-        const int i = o / 45, rem = 2 * (o % 45);
-        typedef double f64x2 __attribute__((ext_vector_type(2)));
-        const f64x2 kk = {entry(i, rem), entry(i, rem + 1)};
-        // node block i goes where its incidence entry sits in node i's list
-        // (streamed: non-temporal, the gather reads it once)
-        __builtin_nontemporal_store(kk, reinterpret_cast<f64x2 *>(&Ke[(int64_t)inv[10 * e + i] * 90 + rem]));
+    }
+#pragma unroll
+    for (int x0 = 0; x0 < NE; ++x0) el[x0 * kWave + lane] = r0[x0];
+    so[lane] = (uint8_t)so0;
+    const int i = item0 - 10 * (item0 / 10), ng = g0.n;
+    const Group g2 = next(g1);
+    int32_t item2;
+    int so2;
+    load_integrals(g1, item1, r0);
+    load_items(g2, item2, so2);
+    wave_lds_sync();
+    if (u < ng) {
+      const double *g = el + u * ED;
+      const P2Terms R = p2_terms(i);
+      if constexpr (LAP) {
+        double k = 0.;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            if ((s && R.vert) || (t && C.vert)) continue;
+            double w = 16. * g[10 + sym4(R.l[s], C.l[t])];
+            if (R.vert) w -= 4. * g[20 + C.l[t]];
+            if (C.vert) w -= 4. * g[20 + R.l[s]];
+            if (R.vert && C.vert) w += g[24];
+            k += w * g[sym4(R.x[s], C.x[t])];
+          }
+        blk[lane] = k;
+      } else {
+        // weights of a pair of terms, equal and different barycentrics:
+        // 16 (1 + delta) / 20 for two edges, less 1 with a vertex among them
+        const bool ee = !R.vert && !C.vert;
+        const double hi = ee ? 1.6 : 0.6, lo = ee ? 0.8 : -0.2, mes = g[12];
+        double X[2][3], Y[2][3];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const double w0 = R.l[s] == C.l[0] ? hi : lo;
+          const double w1 = C.vert ? 0. : (R.l[s] == C.l[1] ? hi : lo);
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            X[s][c] = (s && R.vert) ? 0. : mes * g[3 * R.x[s] + c];
+            Y[s][c] = w0 * g[3 * C.x[0] + c] + w1 * g[3 * C.x[1] + c];
+          }
+        }
+        double B[3][3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) B[c][d] = X[0][c] * Y[0][d] + X[1][c] * Y[1][d];
+        const double tr = B[0][0] + B[1][1] + B[2][2];
+        double *o = blk + u * NV + 3 * j;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+            o[30 * c + d] = lambda * B[c][d] + mu * B[d][c] + (c == d ? mu * tr : 0.);
       }
     }
     wave_lds_sync();
-  }
-}
-
-// ---------------------------------------------------------------- row gather
-
-__global__ __launch_bounds__(256) void k_p2v_gather(
-    int64_t nn, const int64_t *__restrict__ nodeptr, const int64_t *__restrict__ n2e_ptr,
-    const uint8_t *__restrict__ slot8, const double *__restrict__ Ke, double *__restrict__ vals) {
-  __shared__ double S[256 / kWave][9 * kNodeCap];
-  const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int64_t a = (int64_t)blockIdx.x * (256 / kWave) + w;
-  if (a >= nn) return;  // wave-uniform; the kernel has no block barrier
-  double *acc = S[w];
-  const int64_t p0 = nodeptr[a];
-  const int L = (int)(nodeptr[a + 1] - p0), Wd = 9 * L;
-  for (int t = lane; t < Wd; t += kWave) acc[t] = 0.;
-  // this lane's two entries of a 90-value block: (c, j, c') of t = lane, lane + 64
-  int tj[2], tdst[2];
+    // element order: a wave's LDS additions are carried out in the order they
+    // are issued, and the lanes of one go to different slots
+    auto add = [](double *p, double v) {
+      (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    };
+    if constexpr (LAP) {
+      const double v = u < ng ? blk[lane] : 0.;
+      for (int uu = 0; uu < ng; ++uu)
+        if (u == uu) add(&acc[so0], v);
+    } else {
+      double v[GI][2];
+      int o[GI][2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int t = lane + h * kWave;
-    const int c = t / 30, r2 = t % 30;
-    tj[h] = r2 / 3;
-    tdst[h] = c * 3 * L + r2 % 3;  // + 3 * offset of node column j
-  }
-  const bool two = lane < 90 - kWave;
-  wave_lds_sync();
-  const int64_t k0 = n2e_ptr[a], k1 = n2e_ptr[a + 1];
-  // the node's blocks are contiguous (incidence order = element order) and
-  // are added one after the other; they are loaded kGatherD at a time, the
-  // next group's loads issued before the current group is added
-  constexpr int D = kGatherD;
-  double va[D], vb[D], na[D], nb[D];
-  int oa[D], ob[D], ma[D], mb[D];
-  auto load = [&](int64_t kg, double (&A)[D], double (&B)[D], int (&OA)[D], int (&OB)[D]) {
+      for (int uu = 0; uu < GI; ++uu)
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int64_t k = kg + d;
-      A[d] = 0.; B[d] = 0.; OA[d] = 0; OB[d] = 0;
-      if (k < k1) {
-        A[d] = __builtin_nontemporal_load(&Ke[k * 90 + lane]);
-        OA[d] = slot8[k * 10 + tj[0]];
-        if (two) { B[d] = __builtin_nontemporal_load(&Ke[k * 90 + lane + kWave]); OB[d] = slot8[k * 10 + tj[1]]; }
-      }
+        for (int h = 0; h < 2; ++h) {
+          const int t = lane + h * kWave;
+          v[uu][h] = t < NV ? blk[uu * NV + t] : 0.;
+          o[uu][h] = tdst[h] + 3 * so[10 * uu + tj[h]];
+        }
+#pragma unroll
+      for (int uu = 0; uu < GI; ++uu)
+        if (uu < ng) {  // uniform
+          add(&acc[o[uu][0]], v[uu][0]);
+          if (lane < NV - kWave) add(&acc[o[uu][1]], v[uu][1]);
+        }
     }
-  };
-  load(k0, va, vb, oa, ob);
-  for (int64_t kg = k0; kg < k1; kg += D) {
-    load(kg + D, na, nb, ma, mb);
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      if (kg + d < k1) {  // wave-uniform
-        acc[tdst[0] + 3 * oa[d]] += va[d];
-        if (two) acc[tdst[1] + 3 * ob[d]] += vb[d];
-        wave_lds_sync();
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < D; ++d) { va[d] = na[d]; vb[d] = nb[d]; oa[d] = ma[d]; ob[d] = mb[d]; }
-  }
-  double *out = vals + 9 * p0;
-  for (int t = lane; t < Wd; t += kWave) out[t] = acc[t];
-}
-
-// scalar P2: one wave per node row; the row's incident element rows (10
-// values each, element order) added slot by slot in LDS
-__global__ __launch_bounds__(256) void k_p2_gather(int64_t nn, const int64_t *__restrict__ nodeptr,
-                                                   const int64_t *__restrict__ n2e_ptr,
-                                                   const uint8_t *__restrict__ slot8,
-                                                   const double *__restrict__ Ke,
-                                                   double *__restrict__ vals) {
-  __shared__ double S[256 / kWave][kNodeCap];
-  const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int64_t a = (int64_t)blockIdx.x * (256 / kWave) + w;
-  if (a >= nn) return;  // wave-uniform; the kernel has no block barrier
-  double *acc = S[w];
-  const int64_t p0 = nodeptr[a];
-  const int L = (int)(nodeptr[a + 1] - p0);
-  for (int t = lane; t < L; t += kWave) acc[t] = 0.;
-  wave_lds_sync();
-  const int64_t k0 = n2e_ptr[a], k1 = n2e_ptr[a + 1];
-  // six incidences per step: lane = 10 u + j takes value j of incidence k + u;
-  // the steps keep element order, and within a step the incidences are added
-  // one after the other
-  const int u = lane / 10, j = lane % 10;
-  for (int64_t k = k0; k < k1; k += 6) {
-    const bool mine = u < 6 && k + u < k1;
-    double v = 0.;
-    int o = 0;
-    if (mine) { v = Ke[(k + u) * 10 + j]; o = slot8[(k + u) * 10 + j]; }
-    for (int uu = 0; uu < 6; ++uu) {
-      if (mine && u == uu) acc[o] += v;
+    wave_lds_sync();
+    if (g1.c != row) {  // the row is complete
+      double *out = vals + NB * p0;
+      for (int t = lane; t < NB * L; t += kWave) out[t] = acc[t];
       wave_lds_sync();
     }
+    g0 = g1; g1 = g2;
+    item0 = item1; item1 = item2;
+    so0 = so1; so1 = so2;
   }
-  for (int t = lane; t < L; t += kWave) vals[p0 + t] = acc[t];
 }
 
 // ---------------------------------------------------------------- Dirichlet
@@ -593,40 +649,82 @@ __global__ void k_p2v_mark_bc(int64_t nbe, const int32_t *__restrict__ btri,
 }
 
 // ---------------------------------------------------------------- right-hand side
-// b_(3a+c) = sum over incident elements (element order) and points q of
-// (|K| w_q f_c) phi_i(x_q), as Element_rhs accumulates it; tgv * g_c on
-// Dirichlet rows
-__global__ void k_p2v_rhs(int64_t nn, const double *__restrict__ xyz, const int32_t *__restrict__ tets,
-                          const int64_t *__restrict__ n2e_ptr, const int32_t *__restrict__ n2e,
-                          int ncomp, double f0, double f1, double f2,
-                          const uint8_t *__restrict__ onbc, double tgv, double g0, double g1,
-                          double g2, double *__restrict__ b) {
-#pragma clang fp contract(off)
-  const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= nn) return;
-  const double fv[3] = {f0, f1, f2};
-  double acc[3] = {0., 0., 0.};
-  for (int64_t k = n2e_ptr[a]; k < n2e_ptr[a + 1]; ++k) {
-    const int32_t item = n2e[k];
-    const int64_t e = item / 10;
-    const int i = item - (int)e * 10;
-    double v[4][3];
-    for (int t = 0; t < 4; ++t)
-      for (int d = 0; d < 3; ++d) v[t][d] = xyz[3 * (int64_t)tets[4 * e + t] + d];
-    const double mes = tet_mesure(v);
-    const int ed = i < 4 ? 0 : i - 4;
-    const int i0 = i < 4 ? i : c_edge[ed][0], i1 = i < 4 ? i : c_edge[ed][1];
-    for (int q = 0; q < 14; ++q) {
-      const double px = c_qf5_pts[q][0], py = c_qf5_pts[q][1], pz = c_qf5_pts[q][2];
-      const double l[4] = {1. - (px + py + pz), px, py, pz};
-      const double coef = mes * qf5_weight(q);
-      const double phi = i < 4 ? l[i] * (2 * l[i] - 1.) : 4. * l[i0] * l[i1];
-      for (int c = 0; c < ncomp; ++c) acc[c] += coef * fv[c] * phi;
-    }
+// |K| of every tet
+__global__ __launch_bounds__(256) void k_p2_mes(int64_t nt, const double *__restrict__ xyz,
+                                                const int32_t *__restrict__ tets,
+                                                double *__restrict__ mes) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nt) return;
+  const int4 tv = reinterpret_cast<const int4 *>(tets)[e];
+  const int32_t id[4] = {tv.x, tv.y, tv.z, tv.w};
+  double v[4][3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[i][k] = xyz[3 * (int64_t)id[i] + k];
+  mes[e] = tet_mesure(v);
+}
+
+// b_(ncomp a + c) = f_c int phi_a, the integral of a P2 basis function over
+// its tets: -|K| / 20 for a vertex, |K| / 5 for an edge (Element_rhs with Tet_5,
+// exact here); the |K| added in element order; tgv * g_c on Dirichlet rows.  A
+// wave takes 64 nodes, reads their incidence lists consecutively and stages the
+// measures in LDS; each lane adds its own node's.  cube(32), 275 k nodes:
+// 10 us and 5 us for the measures; a lane per node that walked its tets with the
+// 14 points took 397 us.
+__global__ __launch_bounds__(64) void k_p2v_rhs(int64_t nn, const double *__restrict__ mes,
+                                                const int64_t *__restrict__ n2e_ptr,
+                                                const int32_t *__restrict__ n2e, int ncomp, double f0,
+                                                double f1, double f2,
+                                                const uint8_t *__restrict__ onbc, double tgv, double g0,
+                                                double g1, double g2, double *__restrict__ b) {
+  constexpr int U = 8, CAP = kWave * U;
+  __shared__ double st[CAP + CAP / 32];
+  auto pos = [](int i) { return i + (i >> 5); };
+  const int lane = threadIdx.x;
+  const int64_t r0 = (int64_t)xcd_block_id() * kWave, a = r0 + lane;
+  if (r0 >= nn) return;  // one wave per block
+  const int64_t p0 = n2e_ptr[a < nn ? a : nn], p1 = n2e_ptr[a + 1 < nn ? a + 1 : nn];
+  const int64_t seg0 = n2e_ptr[r0], seg1 = n2e_ptr[r0 + kWave < nn ? r0 + kWave : nn];
+  const bool vert = p0 < p1 && n2e[p0] % 10 < 4;
+  double s = 0.;
+  for (int64_t c0 = seg0; c0 < seg1; c0 += CAP) {
+    const int cnt = (int)(seg1 - c0 < CAP ? seg1 - c0 : CAP);
+    int32_t e[U];
+    double t[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) e[u] = lane + u * kWave < cnt ? n2e[c0 + lane + u * kWave] / 10 : 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) t[u] = mes[e[u]];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (lane + u * kWave < cnt) st[pos(lane + u * kWave)] = t[u];
+    wave_lds_sync();
+    const int b0 = (int)((p0 > c0 ? p0 : c0) - c0);
+    const int b1 = (int)((p1 < c0 + cnt ? p1 : c0 + cnt) - c0);
+    for (int k = b0; k < b1; ++k) s += st[pos(k)];
+    wave_lds_sync();
   }
-  const double g[3] = {g0, g1, g2};
+  if (a >= nn) return;
+  const double w = vert ? -s / 20. : s / 5.;
+  const double f[3] = {f0, f1, f2}, g[3] = {g0, g1, g2};
   for (int c = 0; c < ncomp; ++c)
-    b[ncomp * a + c] = onbc[ncomp * a + c] ? tgv * g[c] : acc[c];
+    b[ncomp * a + c] = onbc[ncomp * a + c] ? tgv * g[c] : w * f[c];
+}
+
+// the two passes of a right-hand side
+static void p2_rhs(ffhip_ctx ctx, ffhip_p2v sp, int ncomp, const double f[3], const uint8_t *onbc,
+                   double tgv, const double g[3], double *b) {
+  hipStream_t s = ctx->stream;
+  ffhip_mesh m = sp->mesh;
+  Arena ar(ctx, Arena::bytes(m->nt, 8));
+  double *mes = ar.take<double>(m->nt);
+  ctx->tic();
+  k_p2_mes<<<nblk(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, mes);
+  k_p2v_rhs<<<(nblk(sp->nnodes, kWave) + 7) / 8 * 8, kWave, 0, s>>>(
+      sp->nnodes, mes, sp->n2e_ptr, sp->n2e, ncomp, f[0], f[1], f[2], onbc, tgv, g[0], g[1], g[2], b);
+  FFHIP_CHECK(hipGetLastError());
+  ctx->toc();
 }
 
 // onbc (3 nnodes bytes) of the labelled boundary; false if a node was missing
@@ -652,7 +750,7 @@ static bool p2v_mark(ffhip_ctx ctx, ffhip_p2v sp, const int32_t *labels, int nla
 
 static void p2v_release(ffhip_p2v sp) {
   dfree(sp->elem_nodes); dfree(sp->vnode); dfree(sp->ekeys); dfree(sp->enode);
-  dfree(sp->n2e_ptr); dfree(sp->n2e); dfree(sp->n2e_inv);
+  dfree(sp->n2e_ptr); dfree(sp->n2e);
   delete sp;
 }
 
@@ -718,7 +816,7 @@ int ffhip_p2v_create(ffhip_ctx ctx, ffhip_mesh m, ffhip_p2v *out) {
       FFHIP_CHECK(hipStreamSynchronize(s));
       // the arena's temporaries are dead from here on (build_incidence reuses the work buffer)
       build_incidence(ctx, sp->elem_nodes, nt, 10, sp->nnodes, &sp->n2e_ptr, &sp->n2e, nullptr,
-                      &sp->n2e_inv, nullptr);
+                      nullptr, nullptr);
       ctx->toc();
     } catch (...) {
       (void)hipStreamSynchronize(s);
@@ -861,16 +959,12 @@ int ffhip_assemble_p2v_elasticity(ffhip_ctx ctx, ffhip_p2v sp, ffhip_mat A, doub
                   "ffhip_assemble_p2v_elasticity: matrix pattern was not built from this space");
     hipStream_t s = ctx->stream;
     ffhip_mesh m = sp->mesh;
-    Arena ar(ctx, Arena::bytes(900 * m->nt, 8));
-    double *Ke = ar.take<double>(900 * m->nt);
-    int64_t g = (m->nt + kElemWaves - 1) / kElemWaves;
-    const int64_t gmax = 8 * (int64_t)ctx->num_cu;
-    if (g > gmax) g = gmax;
+    Arena ar(ctx, Arena::bytes(kLame * m->nt, 8));
+    double *E = ar.take<double>(kLame * m->nt);
     ctx->tic();
-    k_p2_element<false><<<(unsigned)g, kElemBlock, 0, s>>>(m->nt, m->xyz, m->elems, lambda, mu, 0,
-                                                          0., nullptr, sp->n2e_inv, Ke);
-    k_p2v_gather<<<nblk(sp->nnodes, 256 / kWave), 256, 0, s>>>(sp->nnodes, A->nodeptr, sp->n2e_ptr,
-                                                              A->slot8, Ke, A->vals);
+    k_p2_elem_lame<<<nblk(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, E);
+    k_p2_rows<false><<<(nblk(sp->nnodes, kNodesPerWave) + 7) / 8 * 8, kWave, 0, s>>>(
+        sp->nnodes, A->nodeptr, sp->n2e_ptr, sp->n2e, A->slot8, E, lambda, mu, A->vals);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
   });
@@ -914,7 +1008,6 @@ int ffhip_rhs_p2v(ffhip_ctx ctx, ffhip_p2v sp, const double f[3], const int32_t 
     FFHIP_REQUIRE(ctx && sp && f && b, FFHIP_ERR_ARG, "ffhip_rhs_p2v: null argument");
     FFHIP_REQUIRE(nlab >= 0 && (nlab == 0 || labels), FFHIP_ERR_ARG, "ffhip_rhs_p2v: labels");
     hipStream_t s = ctx->stream;
-    ffhip_mesh m = sp->mesh;
     const int64_t n = 3 * sp->nnodes;
     const double gz[3] = {0., 0., 0.};
     const double *gg = g ? g : gz;
@@ -924,12 +1017,7 @@ int ffhip_rhs_p2v(ffhip_ctx ctx, ffhip_p2v sp, const double f[3], const int32_t 
     try {
       ok = p2v_mark(ctx, sp, labels, nlab, 3, onbc);
       if (!on_device) bd = dalloc<double>(n);
-      ctx->tic();
-      k_p2v_rhs<<<nblk(sp->nnodes, 256), 256, 0, s>>>(sp->nnodes, m->xyz, m->elems, sp->n2e_ptr,
-                                                      sp->n2e, 3, f[0], f[1], f[2], onbc, tgv, gg[0],
-                                                      gg[1], gg[2], bd);
-      FFHIP_CHECK(hipGetLastError());
-      ctx->toc();
+      p2_rhs(ctx, sp, 3, f, onbc, tgv, gg, bd);
       if (!on_device) {
         FFHIP_CHECK(hipMemcpyAsync(b, bd, 8 * n, hipMemcpyDeviceToHost, s));
         FFHIP_CHECK(hipStreamSynchronize(s));
@@ -960,22 +1048,18 @@ int ffhip_assemble_p2(ffhip_ctx ctx, ffhip_p2v sp, ffhip_mat A, int kind, double
     hipStream_t s = ctx->stream;
     ffhip_mesh m = sp->mesh;
     const int64_t cnt = kind == FFHIP_COEF_P1 ? m->nv : kind == FFHIP_COEF_P0 ? m->nt : 14 * m->nt;
-    Arena ar(ctx, Arena::bytes(100 * m->nt, 8) + (arr && !kappa_on_device ? Arena::bytes(cnt, 8) : 0));
-    double *Ke = ar.take<double>(100 * m->nt);
+    Arena ar(ctx, Arena::bytes(kLap * m->nt, 8) + (arr && !kappa_on_device ? Arena::bytes(cnt, 8) : 0));
+    double *E = ar.take<double>(kLap * m->nt);
     const double *kd = kappa_e;
     if (arr && !kappa_on_device) {
       double *kb = ar.take<double>(cnt);
       FFHIP_CHECK(hipMemcpyAsync(kb, kappa_e, 8 * cnt, hipMemcpyHostToDevice, s));
       kd = kb;
     }
-    int64_t g = (m->nt + kElemWaves - 1) / kElemWaves;
-    const int64_t gmax = 8 * (int64_t)ctx->num_cu;
-    if (g > gmax) g = gmax;
     ctx->tic();
-    k_p2_element<true><<<(unsigned)g, kElemBlock, 0, s>>>(m->nt, m->xyz, m->elems, 0., 0., kind, c0,
-                                                          kd, sp->n2e_inv, Ke);
-    k_p2_gather<<<nblk(sp->nnodes, 256 / kWave), 256, 0, s>>>(sp->nnodes, A->nodeptr, sp->n2e_ptr,
-                                                             A->slot8, Ke, A->vals);
+    k_p2_elem_lap<<<nblk(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, kind, c0, kd, E);
+    k_p2_rows<true><<<(nblk(sp->nnodes, kNodesPerWave) + 7) / 8 * 8, kWave, 0, s>>>(
+        sp->nnodes, A->nodeptr, sp->n2e_ptr, sp->n2e, A->slot8, E, 0., 0., A->vals);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
   });
@@ -1018,7 +1102,6 @@ int ffhip_rhs_p2(ffhip_ctx ctx, ffhip_p2v sp, double f, const int32_t *labels, i
     FFHIP_REQUIRE(ctx && sp && b, FFHIP_ERR_ARG, "ffhip_rhs_p2: null argument");
     FFHIP_REQUIRE(nlab >= 0 && (nlab == 0 || labels), FFHIP_ERR_ARG, "ffhip_rhs_p2: labels");
     hipStream_t s = ctx->stream;
-    ffhip_mesh m = sp->mesh;
     const int64_t n = sp->nnodes;
     uint8_t *onbc = dalloc<uint8_t>(n);
     double *bd = on_device ? b : nullptr;
@@ -1026,11 +1109,8 @@ int ffhip_rhs_p2(ffhip_ctx ctx, ffhip_p2v sp, double f, const int32_t *labels, i
     try {
       ok = p2v_mark(ctx, sp, labels, nlab, 1, onbc);
       if (!on_device) bd = dalloc<double>(n);
-      ctx->tic();
-      k_p2v_rhs<<<nblk(n, 256), 256, 0, s>>>(n, m->xyz, m->elems, sp->n2e_ptr, sp->n2e, 1, f, 0., 0.,
-                                             onbc, tgv, g, 0., 0., bd);
-      FFHIP_CHECK(hipGetLastError());
-      ctx->toc();
+      const double fv[3] = {f, 0., 0.}, gv[3] = {g, 0., 0.};
+      p2_rhs(ctx, sp, 1, fv, onbc, tgv, gv, bd);
       if (!on_device) {
         FFHIP_CHECK(hipMemcpyAsync(b, bd, 8 * n, hipMemcpyDeviceToHost, s));
         FFHIP_CHECK(hipStreamSynchronize(s));
