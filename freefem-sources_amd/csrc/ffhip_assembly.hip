@@ -1120,7 +1120,7 @@ __global__ __launch_bounds__(256) void k_p1_load_elem(int64_t nt, const double *
 // PAIR terms need the row's own value (own, minus own2 when given); the
 // product and the sum are rounded on their own, as the term and its addition
 // were.  tgv rows: tgv * (gvals[v] or g0), or 0 with zero_bc.
-template <int RM>
+template <int RM, int ROWS>
 __global__ __launch_bounds__(64) void k_row_sum(
     int64_t n, const int64_t *__restrict__ v2e_ptr, const int32_t *__restrict__ v2e,
     const double *__restrict__ E, const double *__restrict__ own, const double *__restrict__ own2,
@@ -1130,12 +1130,13 @@ __global__ __launch_bounds__(64) void k_row_sum(
   using T = typename std::conditional<RM == kRowPair, double2, double>::type;
   __shared__ T st[CAP + CAP / 32];
   const int lane = threadIdx.x;
-  const int64_t r0 = (int64_t)xcd_block_id() * kWave, r = r0 + lane;
+  const int64_t r0 = (int64_t)xcd_block_id() * ROWS, rend = r0 + ROWS < n ? r0 + ROWS : n;
   if (r0 >= n) return;  // one wave per block
-  const int64_t p0 = v2e_ptr[r < n ? r : n], p1 = v2e_ptr[r + 1 < n ? r + 1 : n];
-  const int64_t seg0 = v2e_ptr[r0], seg1 = v2e_ptr[r0 + kWave < n ? r0 + kWave : n];
+  const int64_t r = r0 + lane;  // lanes past the rows hold an empty range at the end
+  const int64_t p0 = v2e_ptr[r < rend ? r : rend], p1 = v2e_ptr[r + 1 < rend ? r + 1 : rend];
+  const int64_t seg0 = v2e_ptr[r0], seg1 = v2e_ptr[rend];
   double me = 0.;
-  if (RM == kRowPair && r < n) me = own2 ? own[r] - own2[r] : own[r];
+  if (RM == kRowPair && r < rend) me = own2 ? own[r] - own2[r] : own[r];
   double s = 0.;
   for (int64_t c0 = seg0; c0 < seg1; c0 += CAP) {
     const int cnt = (int)(seg1 - c0 < CAP ? seg1 - c0 : CAP);
@@ -1159,20 +1160,20 @@ __global__ __launch_bounds__(64) void k_row_sum(
     wave_lds_sync();
     const int b0 = (int)((p0 > c0 ? p0 : c0) - c0);
     const int b1 = (int)((p1 < c0 + cnt ? p1 : c0 + cnt) - c0);
-#pragma unroll 4
-    for (int k = b0; k < b1; ++k) {
-      if constexpr (RM == kRowPair) {
+    if constexpr (RM == kRowPair) {
+      for (int k = b0; k < b1; ++k) {
         const double2 q = st[stage_pos(k)];
         double t = q.x * (me + q.y);
         asm("" : "+v"(t));  // rounded before it is added (no fused multiply-add)
         s += t;
-      } else {
-        s += RM == kRowScale ? 0.25 * st[stage_pos(k)] : st[stage_pos(k)];
       }
+    } else {
+#pragma unroll 4
+      for (int k = b0; k < b1; ++k) s += RM == kRowScale ? 0.25 * st[stage_pos(k)] : st[stage_pos(k)];
     }
     wave_lds_sync();
   }
-  if (r >= n) return;
+  if (r >= rend) return;
   if (onbc && onbc[r]) s = tgv * (gvals ? gvals[r] : g0);
   b[r] = s;
 }
@@ -1349,7 +1350,7 @@ __device__ inline int64_t find_entry(int64_t lo, int64_t end, const int32_t *__r
   return -1;
 }
 
-template <int MODE>
+template <int MODE, int ROWS>
 __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__restrict__ rowptr,
                                                    const int32_t *__restrict__ colidx,
                                                    const double *__restrict__ vals,
@@ -1360,10 +1361,11 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
   __shared__ double2 st[CAP + CAP / 32];
   __shared__ int64_t rs[kWave];  // kTrans: the rows' starts
   const int lane = threadIdx.x;
-  const int64_t r0 = (int64_t)xcd_block_id() * kWave, r = r0 + lane;
+  const int64_t r0 = (int64_t)xcd_block_id() * ROWS, rend = r0 + ROWS < n ? r0 + ROWS : n;
   if (r0 >= n) return;  // one wave per block
-  const int64_t p0 = rowptr[r < n ? r : n], p1 = rowptr[r + 1 < n ? r + 1 : n];
-  const int64_t seg0 = rowptr[r0], seg1 = rowptr[r0 + kWave < n ? r0 + kWave : n];
+  const int64_t r = r0 + lane;  // lanes past the rows hold an empty range at the end
+  const int64_t p0 = rowptr[r < rend ? r : rend], p1 = rowptr[r + 1 < rend ? r + 1 : rend];
+  const int64_t seg0 = rowptr[r0], seg1 = rowptr[rend];
   if constexpr (MODE == kTrans) {
     rs[lane] = p0;
     wave_lds_sync();
@@ -1391,7 +1393,7 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const int i = i0 + u * kWave;
-          int lo = 0, hi = kWave - 1;  // the row of this entry: the last that starts at or before it
+          int lo = 0, hi = ROWS - 1;  // the row of this entry: the last that starts at or before it
           while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
             if (rs[mid] <= c0 + i) lo = mid; else hi = mid - 1;
@@ -1436,7 +1438,7 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
     }
     wave_lds_sync();
   }
-  if (r < n) y[r] = acc;
+  if (r < rend) y[r] = acc;
 }
 
 // slot of the transposed entry: (i,j) at k  ->  (j,i); -1 if absent
@@ -1459,8 +1461,14 @@ __global__ void k_transpose_map(int64_t n, const int64_t *__restrict__ rowptr,
 }
 
 static unsigned nblocks(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
-// one wave per 64 rows, whole XCD groups
-static unsigned row_sum_grid(int64_t n) { return (nblocks(n, kWave) + 7) / 8 * 8; }
+// Rows per wave of the staged row kernels: 64, or 16 where 64 would leave under
+// 16 waves per CU, each with several chunks one after the other.  PAIR sums and
+// A x, 64 against 16 rows: cube(12) 20.0 / 7.4 and 8.0 / 4.0 us, cube(40) 22.0 /
+// 10.3 and 10.8 / 6.4, cube(60) (227 k rows) 25.8 / 20.8 and 13.9 / 12.6,
+// cube(72) A x 18.9 / 20.1, cube(96) PAIR 70 / 76, cube(160) SCALE 188 / 226.
+static bool few_rows(int64_t n) { return n < 64 * 16 * 256; }
+// one wave per `rows` rows, whole XCD groups
+static unsigned row_grid(int64_t n, int rows) { return (nblocks(n, rows) + 7) / 8 * 8; }
 int read_flag(ffhip_ctx ctx, int *d);
 void half_view(ffhip_mat L);
 
@@ -1650,7 +1658,10 @@ void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
   if (J || b.pair) {
     k_p1_misfit_elem<<<kMisfitBlocks, 256, 0, s>>>(m->nt, m->xyz, m->elems, u, ud, b.part, b.pair);
     FFHIP_CHECK(hipGetLastError());
-    if (J) FFHIP_CHECK(hipMemcpyAsync(h, b.part, sizeof(h), hipMemcpyDeviceToHost, s));
+    if (J) {
+      FFHIP_CHECK(hipMemcpyAsync(h, b.part, sizeof(h), hipMemcpyDeviceToHost, s));
+      FFHIP_CHECK(hipStreamSynchronize(s));
+    }
   }
   if (r) {
     const uint8_t *onbc = nullptr;
@@ -1662,11 +1673,12 @@ void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
                                                        nlab, b.onbc);
       onbc = b.onbc;
     }
-    if (b.pair)
-      k_row_sum<kRowPair><<<row_sum_grid(m->nv), kWave, 0, s>>>(
+    if (b.pair) {
+      auto sum = few_rows(m->nv) ? k_row_sum<kRowPair, 16> : k_row_sum<kRowPair, 64>;
+      sum<<<row_grid(m->nv, few_rows(m->nv) ? 16 : 64), kWave, 0, s>>>(
           m->nv, m->v2e_ptr, m->v2e, reinterpret_cast<const double *>(b.pair), u, ud, onbc, 0., 0.,
           nullptr, r);
-    else
+    } else
       k_p1_mass_apply<<<nblocks(m->nv * kHalf, 256), 256, 0, s>>>(m->nv, m->xyz, m->elems, m->v2e_ptr,
                                                                   m->v2e, u, ud, onbc, r);
     FFHIP_CHECK(hipGetLastError());
@@ -2156,8 +2168,9 @@ int ffhip_rhs_p1_form(ffhip_ctx ctx, ffhip_mesh m, int kind, double f0, const do
 #define FFHIP_RHS(RM)                                                                              \
   do {                                                                                             \
     k_p1_load_elem<RM><<<nblocks(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, kind, f0, fd, E); \
-    k_row_sum<RM><<<row_sum_grid(n), kWave, 0, s>>>(n, m->v2e_ptr, m->v2e, E, fd, nullptr, onbc, tgv, \
-                                                    g0, gd, bd);                                   \
+    auto sum = few_rows(n) ? k_row_sum<RM, 16> : k_row_sum<RM, 64>;                                \
+    sum<<<row_grid(n, few_rows(n) ? 16 : 64), kWave, 0, s>>>(n, m->v2e_ptr, m->v2e, E, fd, nullptr, onbc, \
+                                                             tgv, g0, gd, bd);                     \
   } while (0)
       if (rm == kRowScale) FFHIP_RHS(kRowScale);
       else if (rm == kRowPair) FFHIP_RHS(kRowPair);
@@ -2324,28 +2337,25 @@ int ffhip_spmv(ffhip_ctx ctx, ffhip_mat A, const double *x, double *y, int trans
   return guard([&] {
     FFHIP_REQUIRE(ctx && A && x && y, FFHIP_ERR_ARG, "ffhip_spmv: null argument");
     hipStream_t s = ctx->stream;
-    const unsigned grid = row_sum_grid(A->n);
-    if (A->half) {  // y = (L + L^T - diag L) x over the full view; symmetric: trans alike
-      half_view(A);
+    const unsigned grid = row_grid(A->n, few_rows(A->n) ? 16 : 64);
+    auto product = [&](auto small, auto large, const int64_t *ptr, const int32_t *col, int *missing) {
       ctx->tic();
-      k_spmv_stage<kSlots><<<grid, kWave, 0, s>>>(A->n, A->fptr, A->fcol, A->vals, A->fslot, x, y, nullptr);
+      (few_rows(A->n) ? small : large)<<<grid, kWave, 0, s>>>(A->n, ptr, col, A->vals, A->fslot, x, y, missing);
       FFHIP_CHECK(hipGetLastError());
       ctx->toc();
+    };
+    if (A->half) {  // y = (L + L^T - diag L) x over the full view; symmetric: trans alike
+      half_view(A);
+      product(k_spmv_stage<kSlots, 16>, k_spmv_stage<kSlots, 64>, A->fptr, A->fcol, nullptr);
       return;
     }
     if (!trans) {
-      ctx->tic();
-      k_spmv_stage<kPlain><<<grid, kWave, 0, s>>>(A->n, A->rowptr, A->colidx, A->vals, nullptr, x, y, nullptr);
-      FFHIP_CHECK(hipGetLastError());
-      ctx->toc();
+      product(k_spmv_stage<kPlain, 16>, k_spmv_stage<kPlain, 64>, A->rowptr, A->colidx, nullptr);
       return;
     }
     int *missing = dalloc<int>(1);
     FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), s));
-    ctx->tic();
-    k_spmv_stage<kTrans><<<grid, kWave, 0, s>>>(A->n, A->rowptr, A->colidx, A->vals, nullptr, x, y, missing);
-    FFHIP_CHECK(hipGetLastError());
-    ctx->toc();
+    product(k_spmv_stage<kTrans, 16>, k_spmv_stage<kTrans, 64>, A->rowptr, A->colidx, missing);
     const int miss = read_flag(ctx, missing);
     dfree(missing);
     FFHIP_REQUIRE(miss == 0, FFHIP_ERR_UNSUPPORTED, "ffhip_spmv: transpose needs a symmetric pattern");
