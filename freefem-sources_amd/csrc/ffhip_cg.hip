@@ -27,7 +27,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <vector>
 
 #include "ffhip_internal.hpp"
@@ -1260,11 +1262,18 @@ __global__ __launch_bounds__(kBlock) void k_cg2_update(
 // ---------------------------------------------------------------- GMRES
 // Restarted right-preconditioned GMRES with modified Gram-Schmidt
 // (SolverGMRES::dosolver + fgmres, VirtualSolverCG.hpp:236-255, CG.cpp:347-517).
-// Per inner iteration it: k_gm_prec (V_it = w / ||w|| and Vp_it = C V_it),
-// k_gm_matvec (w = A Vp_it, partial (w, V_0)), then one k_gm_mgs per basis
-// vector i <= it (h_i from the previous partials, w -= h_i V_i, partial
-// (w, V_i+1) or (w, w)); the Hessenberg column, its Givens rotations and the
-// convergence test are the reference's scalar code on the host.
+// Inner iteration it: k_gm_prec (V_it = w / ||w|| and Vp_it = C V_it),
+// k_gm_matvec (w = A Vp_it), then the modified Gram-Schmidt coefficients of all
+// basis vectors from one pass over the basis: h_i = (w - sum_{j<i} h_j V_j, V_i)
+// = (w, V_i) - sum_{j<i} (V_i, V_j) h_j, so k_gm_dots forms the products (w, V_i)
+// and (V_it, V_i), k_gm_coefs solves that unit lower triangular system and
+// k_gm_project subtracts sum h_i V_i with the partial (w, w).  One kernel per
+// basis vector, each waiting for the dot product of the one before, took 5.0 ms
+// for the 36 iterations of a cube(20) system (666 dependent launches), this
+// takes 1.1 ms (22 us of kernels per iteration, launch latency; the host looks
+// every 8 iterations); for large n it reads the basis twice instead of three
+// times and writes w once.  The Hessenberg column's Givens rotations and the convergence
+// test are the reference's scalar code on the host.
 
 // partial (r, r) of the right-hand side off the tgv rows: ||b|| of fgmres
 __global__ __launch_bounds__(kBlock) void k_gm_normb(int64_t n, const double *__restrict__ b,
@@ -1301,11 +1310,15 @@ __global__ FFHIP_MATVEC_ATTR void k_gm_residual(MatFmt<double> M, const double *
   if (threadIdx.x == 0) pout[xcd_block_id()] = tot;
 }
 
-// V = inv * w; Vp = C V (dinv null: the identity)
+// V = w / ||w||, ||w||^2 from the last projection's partials (pin null: the
+// factor inv); Vp = C V (dinv null: the identity)
 __global__ __launch_bounds__(kBlock) void k_gm_prec(int64_t n, double inv,
+                                                    const double *__restrict__ pin,
                                                     const double *__restrict__ w,
                                                     const double *__restrict__ dinv,
                                                     double *__restrict__ V, double *__restrict__ Vp) {
+  __shared__ double lds[kBlock / kWave];
+  if (pin) inv = 1. / sqrt(reduce_partials(pin, gridDim.x, 1, 0, lds));
   int64_t r0, r1;
   block_rows(n, r0, r1);
   for (int64_t r = r0 + threadIdx.x; r < r1; r += kBlock) {
@@ -1315,42 +1328,126 @@ __global__ __launch_bounds__(kBlock) void k_gm_prec(int64_t n, double inv,
   }
 }
 
-// w = A Vp; partial (w, V_0)
+// w = A Vp
 template <int KIND>
 __global__ FFHIP_MATVEC_ATTR void k_gm_matvec(MatFmt<double> M, const double *__restrict__ Vp,
-                                              const double *__restrict__ V0,
-                                              double *__restrict__ w, double *__restrict__ pout) {
-  __shared__ double lds[kBlock / kWave];
-  double part = 0.;
+                                              double *__restrict__ w) {
   matvec_rows<KIND, double, double>(
-      M, [&](int32_t j) { return Vp[j]; },
-      [&](int64_t r, double acc) {
-        w[r] = acc;
-        part += acc * V0[r];
-      });
-  const double tot = block_sum<kBlock>(part, lds);
-  if (threadIdx.x == 0) pout[xcd_block_id()] = tot;
+      M, [&](int32_t j) { return Vp[j]; }, [&](int64_t r, double acc) { w[r] = acc; });
 }
 
-// h_i = (w, V_i) from the partials; w -= h_i V_i; partial (w, Vnext), or
-// (w, w) when Vnext is null (the last basis vector)
-__global__ __launch_bounds__(kBlock) void k_gm_mgs(int i, int64_t n, const double *__restrict__ Vi,
-                                                   const double *__restrict__ Vnext,
-                                                   double *__restrict__ w,
-                                                   const double *__restrict__ pin,
-                                                   double *__restrict__ pout,
-                                                   double *__restrict__ hcol) {
+// partials of (w, V_i) and (V_it, V_i), i <= it, over the rows of block b.x:
+// the waves of the blocks b.x, * share the i (a wave per i while the chip has
+// room); component c of block b.x at part[c gridDim.x + b.x]
+__global__ __launch_bounds__(kBlock) void k_gm_dots(int it, int64_t n, int64_t rows,
+                                                    const double *const *__restrict__ V,
+                                                    const double *__restrict__ w,
+                                                    double *__restrict__ part) {
+  const int lane = threadIdx.x % kWave;
+  const int64_t r0 = blockIdx.x * rows, r1 = r0 + rows < n ? r0 + rows : n;
+  const double *vit = V[it];
+  for (int i = blockIdx.y * kWavesPerBlock + wave_id(); i <= it; i += gridDim.y * kWavesPerBlock) {
+    const double *vi = V[i];
+    double a = 0., b = 0.;
+#pragma unroll 4
+    for (int64_t r = r0 + lane; r < r1; r += kWave) {
+      const double v = vi[r];
+      a += v * w[r];
+      b += v * vit[r];
+    }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (lane == 0) {
+      part[(int64_t)(2 * i) * gridDim.x + blockIdx.x] = a;
+      part[(int64_t)(2 * i + 1) * gridDim.x + blockIdx.x] = b;
+    }
+  }
+}
+
+// The coefficients h_0..h_it (into h) from the P partials per component, one
+// block.  L holds the products (V_i, V_j), j < i, packed by rows (row i at
+// i (i - 1) / 2); row it is written here.
+constexpr int kGmBlock = 1024;
+__global__ __launch_bounds__(kGmBlock) void k_gm_coefs(int it, int P, const double *__restrict__ part,
+                                                       double *__restrict__ L, double *__restrict__ h) {
+  __shared__ double cur;
+  const int t = threadIdx.x, lane = t % kWave;
+  auto row = [&](int64_t i) { return L + i * (i - 1) / 2; };
+  constexpr int NW = kGmBlock / kWave, C = 4;  // components a wave sums at a time
+  for (int c0 = t / kWave; c0 < 2 * (it + 1); c0 += C * NW) {
+    double s[C] = {0., 0., 0., 0.};
+    for (int b = lane; b < P; b += kWave)
+#pragma unroll
+      for (int u = 0; u < C; ++u)
+        if (c0 + u * NW < 2 * (it + 1)) s[u] += part[(int64_t)(c0 + u * NW) * P + b];
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+      const int c = c0 + u * NW, i = c >> 1;
+      s[u] = wave_sum(s[u]);
+      if (lane != 0 || c >= 2 * (it + 1)) continue;
+      if (!(c & 1)) h[i] = s[u];
+      else if (i < it) row(it)[i] = s[u];
+    }
+  }
+  __syncthreads();
+  constexpr int U = 8;  // columns whose entries are loaded ahead
+  if (it < kWave) {  // one wave, the unknowns in its lanes
+    if (t >= kWave) return;
+    double s = lane <= it ? h[lane] : 0.;
+    const double *l = row(lane);
+    for (int j0 = 0; j0 <= it; j0 += U) {
+      double e[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) e[u] = lane <= it && j0 + u < lane ? l[j0 + u] : 0.;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j0 + u < it) s -= e[u] * __shfl(s, j0 + u, kWave);
+    }
+    if (lane <= it) h[lane] = s;
+    return;
+  }
+  // columns in order; thread t holds the unknowns t, t + kGmBlock, ... of one
+  // sweep at a time, so a sweep's unknowns are first freed of the earlier ones
+  for (int i0 = 0; i0 <= it; i0 += kGmBlock) {
+    const int i = i0 + t;
+    double s = i <= it ? h[i] : 0.;
+    if (i <= it)
+      for (int j = 0; j < i0; ++j) s -= row(i)[j] * h[j];
+    const int iend = i0 + kGmBlock - 1 < it ? i0 + kGmBlock - 1 : it;
+    for (int j0 = i0; j0 <= iend; j0 += U) {
+      double e[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) e[u] = i <= it && j0 + u < i ? row(i)[j0 + u] : 0.;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (j0 + u > iend) break;  // uniform
+        if (i == j0 + u) cur = s;
+        __syncthreads();
+        s -= e[u] * cur;
+        __syncthreads();
+      }
+    }
+    if (i <= it) h[i] = s;
+    __syncthreads();
+  }
+}
+
+// w -= sum_{i <= it} h_i V_i, in order; partial (w, w)
+__global__ __launch_bounds__(kBlock) void k_gm_project(int it, int64_t n,
+                                                       const double *const *__restrict__ V,
+                                                       const double *__restrict__ h,
+                                                       double *__restrict__ w,
+                                                       double *__restrict__ pout) {
   __shared__ double lds[kBlock / kWave];
-  const double h = reduce_partials(pin, gridDim.x, 1, 0, lds);
-  if (blockIdx.x == 0 && threadIdx.x == 0) hcol[i] = h;
-  const double a = -h;
   int64_t r0, r1;
   block_rows(n, r0, r1);
   double part = 0.;
   for (int64_t r = r0 + threadIdx.x; r < r1; r += kBlock) {
-    const double v = w[r] + a * Vi[r];
+    double v = w[r];
+#pragma unroll 8
+    for (int i = 0; i <= it; ++i) v -= h[i] * V[i][r];
     w[r] = v;
-    part += v * (Vnext ? Vnext[r] : v);
+    part += v * v;
   }
   const double tot = block_sum<kBlock>(part, lds);
   if (threadIdx.x == 0) pout[xcd_block_id()] = tot;
@@ -1365,6 +1462,7 @@ __global__ __launch_bounds__(kBlock) void k_gm_update(int64_t n, int k, const do
   block_rows(n, r0, r1);
   for (int64_t r = r0 + threadIdx.x; r < r1; r += kBlock) {
     double acc = 0.;
+#pragma unroll 8
     for (int i = 0; i < k; ++i) acc += y[i] * Vp[i][r];
     x[r] = acc + x0[r];
   }
@@ -1620,27 +1718,57 @@ struct ffhip_cg_s {
   MixState *ms = nullptr;
   Cg2State *st2 = nullptr;  // affine CG (LinearCG)
   // GMRES: Krylov basis V_i and C V_i, allocated vector by vector as a solve
-  // first reaches them (as the reference's KN<KN<K>> are) and kept; the
-  // device table of the C V_i pointers; w, x0, the Hessenberg column, y
+  // first reaches them (as the reference's KN<KN<K>> are) and kept; the device
+  // tables of their pointers; w, x0, y, the partials of the dot products, the
+  // packed products (V_i, V_j), and per iteration of a batch the coefficients
+  // with the partials of ||w||^2 (gmOut, and its page-locked host copy)
+  static constexpr int kGmBatch = 8;
   std::vector<double *> gmV, gmVp;
-  double **gmVpDev = nullptr;
-  int gmCap = 0;  // entries of gmVpDev, gmH and gmY
-  double *gmW = nullptr, *gmX0 = nullptr, *gmH = nullptr, *gmY = nullptr;
+  double **gmVDev = nullptr, **gmVpDev = nullptr;
+  int gmCap = 0;  // vectors the tables and the buffers below are sized for
+  double *gmW = nullptr, *gmX0 = nullptr, *gmY = nullptr, *gmS = nullptr, *gmL = nullptr, *gmOut = nullptr;
+  double *gmOutH = nullptr;
+  int gm_blocks() const {  // blocks of the dot products
+    const int64_t b = (n + 255) / 256;
+    return (int)(b < 256 ? b : 256);
+  }
+  int64_t gm_out() const { return (int64_t)gmCap + grid; }  // doubles per iteration of gmOut
   void gm_basis(int k) {
     if (k > gmCap) {
-      const int cap = std::max(k, 2 * gmCap);
-      double **p = dalloc<double *>(cap);
-      double *h = dalloc<double>(cap + 1), *y = dalloc<double>(cap + 1);
-      dfree(gmVpDev); dfree(gmH); dfree(gmY);
-      gmVpDev = p; gmH = h; gmY = y; gmCap = cap;
-      FFHIP_CHECK(hipMemcpy(gmVpDev, gmVp.data(), sizeof(double *) * gmVp.size(),
-                            hipMemcpyHostToDevice));
+      const int cap = std::max(std::max(k, 2 * gmCap), 64);
+      double **pv = dalloc<double *>(cap), **p = dalloc<double *>(cap);
+      double *y = dalloc<double>(cap + 1), *S = dalloc<double>(2 * (int64_t)cap * gm_blocks());
+      double *L = dalloc<double>((int64_t)cap * (cap - 1) / 2);
+      double *out = dalloc<double>(kGmBatch * ((int64_t)cap + grid));
+      if (gmCap)
+        FFHIP_CHECK(hipMemcpy(L, gmL, 8 * (size_t)gmCap * (gmCap - 1) / 2, hipMemcpyDeviceToDevice));
+      dfree(gmVDev); dfree(gmVpDev); dfree(gmY); dfree(gmS); dfree(gmL); dfree(gmOut);
+      if (gmOutH) (void)hipHostFree(gmOutH);
+      gmOutH = nullptr;
+      gmVDev = pv; gmVpDev = p; gmY = y; gmS = S; gmL = L; gmOut = out; gmCap = cap;
+      FFHIP_CHECK(hipHostMalloc((void **)&gmOutH, 8 * kGmBatch * gm_out(), hipHostMallocDefault));
+      FFHIP_CHECK(hipMemcpy(gmVDev, gmV.data(), sizeof(double *) * gmV.size(), hipMemcpyHostToDevice));
+      FFHIP_CHECK(hipMemcpy(gmVpDev, gmVp.data(), sizeof(double *) * gmVp.size(), hipMemcpyHostToDevice));
     }
-    while ((int)gmV.size() < k) {
-      gmV.push_back(dalloc<double>(n));
-      gmVp.push_back(dalloc<double>(n));
-      FFHIP_CHECK(hipMemcpy(gmVpDev + gmVp.size() - 1, &gmVp.back(), sizeof(double *),
-                            hipMemcpyHostToDevice));
+    const size_t k0 = gmV.size();
+    if ((int)k0 < k) {
+      gmV.reserve(k);
+      gmVp.reserve(k);
+      while ((int)gmV.size() < k) {
+        double *v = nullptr, *vp = nullptr;
+        try {
+          v = dalloc<double>(n);
+          vp = dalloc<double>(n);
+        } catch (const Error &) {  // as many as fit: the caller sees how many there are
+          dfree(v);
+          break;
+        }
+        gmV.push_back(v);
+        gmVp.push_back(vp);
+      }
+      const size_t c = gmV.size() - k0;
+      FFHIP_CHECK(hipMemcpy(gmVDev + k0, gmV.data() + k0, sizeof(double *) * c, hipMemcpyHostToDevice));
+      FFHIP_CHECK(hipMemcpy(gmVpDev + k0, gmVp.data() + k0, sizeof(double *) * c, hipMemcpyHostToDevice));
     }
     if (!gmW) { gmW = dalloc<double>(n); gmX0 = dalloc<double>(n); }
   }
@@ -2112,7 +2240,9 @@ static void cg_release(ffhip_cg cg) {
   dfree(cg->st2);
   for (double *&p : cg->gmV) dfree(p);
   for (double *&p : cg->gmVp) dfree(p);
-  dfree(cg->gmVpDev); dfree(cg->gmW); dfree(cg->gmX0); dfree(cg->gmH); dfree(cg->gmY);
+  dfree(cg->gmVDev); dfree(cg->gmVpDev); dfree(cg->gmW); dfree(cg->gmX0); dfree(cg->gmY);
+  dfree(cg->gmS); dfree(cg->gmL); dfree(cg->gmOut);
+  if (cg->gmOutH) (void)hipHostFree(cg->gmOutH);
   delete cg;
 }
 
@@ -2347,7 +2477,7 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
     cg->gm_basis(1);
     FFHIP_CHECK(hipMemcpyAsync(cg->bw, b, 8 * n, kin, s));
     FFHIP_CHECK(hipMemcpyAsync(cg->xw, x, 8 * n, kin, s));
-    std::vector<double> part(G), hcol(m + 1);
+    std::vector<double> part(G);
     // block partials written by the last kernel, added on the host in block order
     auto host_sum = [&](const double *p) {
       FFHIP_CHECK(hipMemcpyAsync(part.data(), p, 8 * G, hipMemcpyDeviceToHost, s));
@@ -2360,9 +2490,13 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
     if (cg->ntgv > 0) k_init_bc<<<nblk(n, 256), 256, 0, s>>>(n, cg->wcl, cg->bw, tgv, cg->xw);
     const int nbitermx = itmax > 0 ? itmax : (int)n;  // SolverGMRES(ds)
     // fgmres (CG.cpp:347-517) with leftC = 0: the scalar part as the reference's
-    std::vector<double> rot0(m + 2), rot1(m + 2), g(m + 1), g1(m + 1), y(m + 1),
-        Hn((size_t)(m + 2) * (m + 1), 0.);
-    auto HN = [&](int i, int j) -> double & { return Hn[(size_t)i * (m + 1) + j]; };
+    std::vector<double> rot0(m + 2), rot1(m + 2), g(m + 1), g1(m + 1), y(m + 1);
+    // (m + 2) x (m + 1), zero; calloc leaves the pages that are never reached
+    // untouched (8 MB for the default restart of 1000)
+    const std::unique_ptr<double, decltype(&std::free)> Hn(
+        (double *)std::calloc((size_t)(m + 2) * (m + 1), sizeof(double)), &std::free);
+    FFHIP_REQUIRE(Hn, FFHIP_ERR_INTERNAL, "ffhip_gmres_solve: out of memory for restart %d", m);
+    auto HN = [&](int i, int j) -> double & { return Hn.get()[(size_t)i * (m + 1) + j]; };
     k_gm_normb<<<G, kBlock, 0, s>>>(n, cg->bw, cg->ntgv > 0 ? cg->wcl : nullptr, cg->pA);
     double normb = std::sqrt(host_sum(cg->pA));
     double relres = 1e100;
@@ -2375,21 +2509,41 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
       g[0] = std::sqrt(host_sum(cg->pA));
       if (normb < 1.e-20 || eps < 0) normb = 1.;
       double inv = 1. / g[0];
-      int it;
+      int it, ahead = 0;  // iterations launched beyond the ones looked at, of the current batch
+      int batch = 0;
+      const int P = cg->gm_blocks();
+      const int64_t rows = (n + P - 1) / P;
       for (it = 0; it < m; it++, iter++) {
-        cg->gm_basis(it + 1);
-        k_gm_prec<<<G, kBlock, 0, s>>>(n, inv, cg->gmW, cg->dinv, cg->gmV[it], cg->gmVp[it]);
-        FFHIP_LAUNCH_FMT(cg, k_gm_matvec, G, s, M, cg->gmVp[it], cg->gmV[0], cg->gmW, cg->pB);
-        double *pin = cg->pB, *pout = cg->pA;
-        for (int i = 0; i <= it; ++i) {  // modified Gram-Schmidt
-          k_gm_mgs<<<G, kBlock, 0, s>>>(i, n, cg->gmV[i], i < it ? cg->gmV[i + 1] : nullptr,
-                                        cg->gmW, pin, pout, cg->gmH);
-          std::swap(pin, pout);
+        if (ahead == 0) {
+          // a batch of iterations in one go, then one copy of what the host
+          // needs of each; those after a convergence are dropped.  Past 2^18
+          // rows an iteration costs more than the wait it saves.
+          batch = std::min(n <= (1 << 18) ? ffhip_cg_s::kGmBatch : 1, m - it);
+          cg->gm_basis(it + batch);
+          batch = std::min(batch, (int)cg->gmV.size() - it);
+          FFHIP_REQUIRE(batch > 0, FFHIP_ERR_HIP, "ffhip_gmres_solve: out of device memory at %d basis vectors", it);
+          const int64_t ld = cg->gm_out();
+          for (int c = 0; c < batch; ++c) {
+            const int j = it + c;
+            double *out = cg->gmOut + c * ld, *norms = out + cg->gmCap;
+            const double *pin = c ? cg->gmOut + (c - 1) * ld + cg->gmCap : nullptr;
+            k_gm_prec<<<G, kBlock, 0, s>>>(n, inv, pin, cg->gmW, cg->dinv, cg->gmV[j], cg->gmVp[j]);
+            FFHIP_LAUNCH_FMT(cg, k_gm_matvec, G, s, M, cg->gmVp[j], cg->gmW);
+            const int share = std::max(1, std::min((j + kWavesPerBlock) / kWavesPerBlock, 2048 / P));
+            k_gm_dots<<<dim3(P, share), kBlock, 0, s>>>(j, n, rows, cg->gmVDev, cg->gmW, cg->gmS);
+            k_gm_coefs<<<1, kGmBlock, 0, s>>>(j, P, cg->gmS, cg->gmL, out);
+            k_gm_project<<<G, kBlock, 0, s>>>(j, n, cg->gmVDev, out, cg->gmW, norms);
+          }
+          FFHIP_CHECK(hipGetLastError());
+          FFHIP_CHECK(hipMemcpyAsync(cg->gmOutH, cg->gmOut, 8 * batch * ld, hipMemcpyDeviceToHost, s));
+          FFHIP_CHECK(hipStreamSynchronize(s));
+          ahead = batch;
         }
-        FFHIP_CHECK(hipGetLastError());
-        FFHIP_CHECK(hipMemcpyAsync(hcol.data(), cg->gmH, 8 * (it + 1), hipMemcpyDeviceToHost, s));
-        const double ww = host_sum(pin);
-        for (int i = 0; i <= it; ++i) HN(i, it) = hcol[i];
+        const double *hc = cg->gmOutH + (batch - ahead) * cg->gm_out(), *wp = hc + cg->gmCap;
+        --ahead;
+        double ww = 0.;
+        for (int i = 0; i < G; ++i) ww += wp[i];
+        for (int i = 0; i <= it; ++i) HN(i, it) = hc[i];
         const double aux = HN(it + 1, it) = std::sqrt(ww);
         inv = 1. / aux;
         for (int i = 0; i < it; i++) {
