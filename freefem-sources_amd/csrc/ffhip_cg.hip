@@ -62,6 +62,13 @@ constexpr int kWavesPerBlock = kBlock / kSlice;
 #define FFHIP_GRID_PER_CU (FFHIP_WPE)
 #endif
 #define FFHIP_MATVEC_ATTR __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FFHIP_WPE, FFHIP_WPE)))
+// A matrix of up to this many bytes per mat-vec is read with plain loads: it
+// stays in the Infinity Cache (256 MiB).  Both sides measured, plain against
+// non-temporal: cube(96) FP64 (134 MB) 25.4 / 32.4 us, cube(112) (214 MB) 40.6 /
+// 49.0, cube(24) [P2,P2,P2] (250 MB) 46 / 61, cube(136) FP32 (229 MB) 41 / 46;
+// beyond: cube(120) FP64 (264 MB) 61.8 / 60.6, cube(144) FP32 (272 MB) 56.7 / 53.9,
+// cube(160) FP64 (644 MB) 150.5 / 139.6.
+constexpr int64_t kCachedMatrix = 256000000;
 constexpr int kU = FFHIP_SELL_U;
 
 // matrix layouts of the mat-vec kernels (described at MatFmt below)
@@ -108,15 +115,22 @@ __device__ inline double reduce_partials(const double *__restrict__ p, int P, in
   return block_sum<kBlock>(s, lds);
 }
 
-template <class T>
-__device__ inline T ntload(const T *p) { return __builtin_nontemporal_load(p); }
+// Loads of the streamed matrix: NT past every cache (a matrix that does not
+// fit in the Infinity Cache would only push the vectors out of it), else
+// plain, so that a matrix that fits stays there from one mat-vec to the next
+// (MatFmt::nt).
+template <bool NT, class T>
+__device__ inline T mload(const T *p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
 
 // One row of a slice: sum_k a_k * X(j_k) over the L (wave-uniform) entries of
 // this lane's row.  Unrolled by U: the U column and value loads of a round
 // are all issued before any gather, so every wave keeps 2U streaming loads
 // and U (or 2U) gathers in flight instead of one dependent chain per entry.
 // IT = int32_t: absolute columns; IT = int16_t: deltas to the row (row0 + d).
-template <int U, class V, class ACC, class IT, class F>
+template <bool NT, int U, class V, class ACC, class IT, class F>
 __device__ inline ACC sell_row(const IT *__restrict__ colp, const V *__restrict__ valp, int L,
                                int32_t row0, F xval) {
   ACC acc = 0;
@@ -128,9 +142,9 @@ __device__ inline ACC sell_row(const IT *__restrict__ colp, const V *__restrict_
       j[u] = row0;  // past the row end: a valid column with a zero value
       a[u] = 0;
       if (k + u < L) {
-        const IT c = ntload(colp + (int64_t)(k + u) * kSlice);
+        const IT c = mload<NT>(colp + (int64_t)(k + u) * kSlice);
         j[u] = sizeof(IT) == 2 ? row0 + (int32_t)c : (int32_t)c;
-        a[u] = ntload(valp + (int64_t)(k + u) * kSlice);
+        a[u] = mload<NT>(valp + (int64_t)(k + u) * kSlice);
       }
     }
     ACC xv[U];
@@ -159,7 +173,7 @@ __host__ __device__ inline int64_t pair_pos(int L, int k, int lane) {
   return (k >> 1) < h ? ((int64_t)(k >> 1) * kSlice + lane) * 2 + (k & 1) : (int64_t)h * 2 * kSlice + lane;
 }
 
-template <int U, class V, class ACC, class F>
+template <bool NT, int U, class V, class ACC, class F>
 __device__ inline ACC sell_row16(const int16_t *__restrict__ colp, const V *__restrict__ valp,
                                  int L, int32_t row0, F xval) {
   static_assert(U % 4 == 0, "unroll by whole index groups");
@@ -171,7 +185,7 @@ __device__ inline ACC sell_row16(const int16_t *__restrict__ colp, const V *__re
     for (int g = 0; g < U / 4; ++g) {
       u32x2 pk = {0u, 0u};  // past the row end: deltas 0 (the row itself)
       if (k + 4 * g < L)
-        pk = ntload(reinterpret_cast<const u32x2 *>(colp + (int64_t)((k >> 2) + g) * (4 * kSlice)));
+        pk = mload<NT>(reinterpret_cast<const u32x2 *>(colp + (int64_t)((k >> 2) + g) * (4 * kSlice)));
       j[4 * g + 0] = row0 + (int32_t)(int16_t)(pk.x & 0xffffu);
       j[4 * g + 1] = row0 + (int32_t)(int16_t)(pk.x >> 16);
       j[4 * g + 2] = row0 + (int32_t)(int16_t)(pk.y & 0xffffu);
@@ -180,7 +194,7 @@ __device__ inline ACC sell_row16(const int16_t *__restrict__ colp, const V *__re
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       a[u] = 0;
-      if (k + u < L) a[u] = ntload(valp + (int64_t)(k + u) * kSlice);
+      if (k + u < L) a[u] = mload<NT>(valp + (int64_t)(k + u) * kSlice);
     }
     ACC xv[U];
 #pragma unroll
@@ -208,7 +222,7 @@ __device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadId
 // FP32 mat-vec 6 % faster).  Otherwise each block walks its own contiguous
 // chunk of slices — kept for the [P2,P2,P2] block layout, whose node rows are
 // sorted by length in windows and ran 1.8x slower with the cyclic walk.
-constexpr bool kCyclicSell = true, kCyclicBsr = false;
+constexpr bool kCyclicSell = true;
 template <bool CYCLIC>
 __device__ inline void wave_slices(int64_t S, int64_t &first, int64_t &end, int64_t &stride) {
   if (CYCLIC) {
@@ -496,8 +510,8 @@ __global__ __launch_bounds__(256) void k_bsr_fill(
   }
 }
 
-// First slice of each of nw waves when the S3 slices are split over them by
-// entries: wave w takes the slices that start in [w E / nw, (w+1) E / nw),
+// First slice of each of nw blocks when the S3 slices are split over them by
+// entries: block w takes the slices that start in [w E / nw, (w+1) E / nw),
 // E = sptr[S3].
 __global__ void k_bsr_waves(int64_t S3, const int64_t *__restrict__ sptr, int nw,
                             int32_t *__restrict__ wstart) {
@@ -659,8 +673,9 @@ struct MatFmt {
   const V *val;          // kBsr3: 9 ents values, entry k of slice s at 9 ptr[s] + 9 64 k (bsr_pos)
   int64_t nb, ents;      // kBsr3: node rows, slice entries (ptr/len/col: slices, perm: rows)
   const int32_t *perm;   // kBsr3: node row of each sorted position
-  const int32_t *wstart; // kBsr3: first slice of each of the nw waves (nw + 1), split by entries
+  const int32_t *wstart; // kBsr3: first slice of each of the nw blocks (nw + 1), split by entries
   int nw;
+  bool nt;  // the matrix's loads bypass the caches
 };
 
 // Buffer resource over [p, p + bytes): a buffer load at a byte offset past
@@ -668,20 +683,20 @@ struct MatFmt {
 __device__ inline __amdgpu_buffer_rsrc_t slice_rsrc(const void *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
 }
-constexpr int kBufNT = 2;  // cache policy of the streamed matrix loads: non-temporal
+constexpr int kBufNT = 2;  // cache policy of a non-temporal buffer load
 
 // Entries k >= U of a kSell16 FP64 row (rows longer than U), summed into acc
 // in entry order, four per round (one packed delta group).
-template <class ACC, class F>
+template <bool NT, class ACC, class F>
 __device__ inline ACC sell16_tail(const int16_t *__restrict__ col16, const double *__restrict__ val,
                                   int L, int lane, int32_t row0, F xval, ACC acc) {
   for (int k = kU; k < L; k += 4) {
-    const u32x2 pk = ntload(reinterpret_cast<const u32x2 *>(col16 + (int64_t)(k >> 2) * (4 * kSlice) + 4 * lane));
+    const u32x2 pk = mload<NT>(reinterpret_cast<const u32x2 *>(col16 + (int64_t)(k >> 2) * (4 * kSlice) + 4 * lane));
     const int32_t j[4] = {row0 + (int32_t)(int16_t)(pk.x & 0xffffu), row0 + (int32_t)(int16_t)(pk.x >> 16),
                           row0 + (int32_t)(int16_t)(pk.y & 0xffffu), row0 + (int32_t)(int16_t)(pk.y >> 16)};
     double a[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) a[t] = k + t < L ? ntload(val + pair_pos(L, k + t, lane)) : 0.;
+    for (int t = 0; t < 4; ++t) a[t] = k + t < L ? mload<NT>(val + pair_pos(L, k + t, lane)) : 0.;
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc += (ACC)a[t] * xval(j[t]);
   }
@@ -696,7 +711,7 @@ __device__ inline ACC sell16_tail(const int16_t *__restrict__ col16, const doubl
 // the gathers.  epi(r, acc, pre(r), r < n) is called for every lane (rows
 // past n only in the last slice, whose pre was given a clamped row).  The
 // products are summed in entry order.
-template <class ACC, class F, class P, class E>
+template <bool NT, class ACC, class F, class P, class E>
 __device__ inline void sell16_walk(const MatFmt<double> &M, F xval, P pre, E epi) {
   constexpr int U = kU, G4 = kU / 4, NP = kU / 2;
   static_assert(kU % 4 == 0, "unroll by whole index groups");
@@ -716,12 +731,12 @@ __device__ inline void sell16_walk(const MatFmt<double> &M, F xval, P pre, E epi
     u32x2 pk[G4];
 #pragma unroll
     for (int g = 0; g < G4; ++g)
-      pk[g] = __builtin_amdgcn_raw_buffer_load_b64(rc, (g * kSlice + lane) * 8, 0, kBufNT);
+      pk[g] = __builtin_amdgcn_raw_buffer_load_b64(rc, (g * kSlice + lane) * 8, 0, NT ? kBufNT : 0);
     u32x4 q[NP];
 #pragma unroll
     for (int m = 0; m < NP; ++m)
-      q[m] = __builtin_amdgcn_raw_buffer_load_b128(rp, (m * kSlice + lane) * 16, 0, kBufNT);
-    const u32x2 odd = __builtin_amdgcn_raw_buffer_load_b64(r1, lane * 8, 0, kBufNT);
+      q[m] = __builtin_amdgcn_raw_buffer_load_b128(rp, (m * kSlice + lane) * 16, 0, NT ? kBufNT : 0);
+    const u32x2 odd = __builtin_amdgcn_raw_buffer_load_b64(r1, lane * 8, 0, NT ? kBufNT : 0);
     int32_t j[U];
 #pragma unroll
     for (int g = 0; g < G4; ++g) {
@@ -744,17 +759,17 @@ __device__ inline void sell16_walk(const MatFmt<double> &M, F xval, P pre, E epi
     ACC acc = 0;
 #pragma unroll
     for (int u = 0; u < U; ++u) acc += (ACC)a[u] * xv[u];
-    if (L > U) acc = sell16_tail(M.col16 + cb, M.val + vb, L, lane, r32, xval, acc);
+    if (L > U) acc = sell16_tail<NT>(M.col16 + cb, M.val + vb, L, lane, r32, xval, acc);
     epi(r, acc, pv, r < M.n);
   }
 }
 
 // Calls epi(r, sum_k a_rk X(j_k)) once for every row r of this block's range;
 // for kCsrV only the first lane of each 16-lane group calls it.
-template <int KIND, class V, class ACC, class F, class E>
-__device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
+template <bool NT, int KIND, class V, class ACC, class F, class E>
+__device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
   if constexpr (KIND == kSell16 && sizeof(V) == 8) {
-    sell16_walk<ACC>(M, xval, [](int32_t) { return 0; },
+    sell16_walk<NT, ACC>(M, xval, [](int32_t) { return 0; },
                      [&](int64_t r, ACC acc, int, bool row) { if (row) epi(r, acc); });
   } else if constexpr (KIND == kSell || KIND == kSell16) {
     int64_t s0, s1, ds;
@@ -768,45 +783,56 @@ __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
       const int32_t r32 = (int32_t)(r < M.n ? r : M.n - 1);
       ACC acc;
       if constexpr (KIND == kSell16)
-        acc = sell_row16<kU, V, ACC>(M.col16 + uniform(M.ptr16[s]) + 4 * lane, M.val + base, L, r32,
+        acc = sell_row16<NT, kU, V, ACC>(M.col16 + uniform(M.ptr16[s]) + 4 * lane, M.val + base, L, r32,
                                      xval);
       else
-        acc = sell_row<kU, V, ACC, int32_t>(M.col + base, M.val + base, L, r32, xval);
+        acc = sell_row<NT, kU, V, ACC, int32_t>(M.col + base, M.val + base, L, r32, xval);
       if (r < M.n) epi(r, acc);
     }
   } else if constexpr (KIND == kBsr3) {
-    // Groups of U block entries; the next group's block columns are loaded
+    // The block's four waves share each slice, a quarter of its entries each
+    // (a wave per slice left one serial chain of 14-32 rounds per SIMD at
+    // cube(20), 1077 slices: 50 us, now 29 with the matrix kept in the caches,
+    // 41 without; cube(8) 18 -> 9.6 us); their sums meet in LDS, added in entry order, and
+    // 192 threads finish the slice's rows.  Groups of U block entries; the
+    // next group's block columns are loaded
     // with the current group's values, so the gathers of x need no second
     // round trip.  The slice's columns and values are read through buffer
     // resources bounded to the slice: past its width they read 0 without a
     // memory access, and those blocks' sums are dropped by a uniform select.
     constexpr int U = sizeof(V) == 8 ? FFHIP_BSR_U : FFHIP_BSR_U32;
+    __shared__ ACC red[2][kWavesPerBlock][3 * kSlice];
     const int64_t S3 = (M.nb + kSlice - 1) / kSlice;
-    int64_t s0, s1, ds;
-    if (M.wstart && (int)gridDim.x * kWavesPerBlock == M.nw) {
-      // slices split over the waves by entries (rows of vertex and of edge
+    int64_t s0, s1;
+    if (M.wstart && (int)gridDim.x == M.nw) {
+      // slices split over the blocks by entries (rows of vertex and of edge
       // nodes differ in length by about 2.5x)
-      const int wg = xcd_block_id() * kWavesPerBlock + wave_id();
-      s0 = __builtin_amdgcn_readfirstlane(M.wstart[wg]);
-      s1 = __builtin_amdgcn_readfirstlane(M.wstart[wg + 1]);
-      ds = 1;
+      const int lb = xcd_block_id();
+      s0 = __builtin_amdgcn_readfirstlane(M.wstart[lb]);
+      s1 = __builtin_amdgcn_readfirstlane(M.wstart[lb + 1]);
     } else {
-      wave_slices<kCyclicBsr>(S3, s0, s1, ds);
+      const int64_t G = gridDim.x, lb = xcd_block_id();
+      s0 = (lb * S3) / G;
+      s1 = ((lb + 1) * S3) / G;
     }
-    const int lane = threadIdx.x % kSlice;
-    for (int64_t s = s0; s < s1; s += ds) {
-      const int64_t i = s * kSlice + lane;
-      const int32_t a = i < M.nb ? M.perm[i] : -1;
+    const int lane = threadIdx.x % kSlice, wv = wave_id();
+    int buf = 0;
+    for (int64_t s = s0; s < s1; ++s, buf ^= 1) {
       const int64_t sb = uniform(M.ptr[s]);
       const int L = __builtin_amdgcn_readfirstlane(M.len[s]);
+      const int part = (L + kWavesPerBlock * U - 1) / (kWavesPerBlock * U) * U;  // entries per wave
+      const int k0 = wv * part < L ? wv * part : L, k1 = k0 + part < L ? k0 + part : L;
       const auto rc = slice_rsrc(M.col + sb, (uint32_t)L * kSlice * 4);
       const auto rv = slice_rsrc(M.val + 9 * sb, (uint32_t)L * (9 * kSlice) * (uint32_t)sizeof(V));
+      // the row that this thread finishes: component t / 64 of the lane's node
+      const int64_t i = s * kSlice + lane;
+      const int32_t a = wv < 3 && i < M.nb ? M.perm[i] : -1;
       ACC s0v = 0, s1v = 0, s2v = 0;
       int32_t bn[U];
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        bn[u] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rc, (u * kSlice + lane) * 4, 0, kBufNT);
-      for (int k = 0; k < L; k += U) {
+        bn[u] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rc, ((k0 + u) * kSlice + lane) * 4, 0, NT ? kBufNT : 0);
+      for (int k = k0; k < k1; k += U) {
         int32_t b[U];
         ACC xv[U][3];
 #pragma unroll
@@ -815,43 +841,42 @@ __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
 #pragma unroll
           for (int c = 0; c < 3; ++c) xv[u][c] = xval(3 * b[u] + c);
         }
-        V wv[U][9];
+        V wv9[U][9];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           constexpr int W = 16 / (int)sizeof(V), Z = (int)sizeof(V);
           const int eb = 9 * kSlice * (k + u);
 #pragma unroll
           for (int g = 0; g < 8 / W; ++g) {
-            const u32x4 r = __builtin_amdgcn_raw_buffer_load_b128(rv, (eb + bsr_pos<V>(g * W, lane)) * Z, 0, kBufNT);
+            const u32x4 r = __builtin_amdgcn_raw_buffer_load_b128(rv, (eb + bsr_pos<V>(g * W, lane)) * Z, 0, NT ? kBufNT : 0);
             if constexpr (sizeof(V) == 8) {
-              wv[u][2 * g] = __builtin_bit_cast(V, u32x2{r.x, r.y});
-              wv[u][2 * g + 1] = __builtin_bit_cast(V, u32x2{r.z, r.w});
+              wv9[u][2 * g] = __builtin_bit_cast(V, u32x2{r.x, r.y});
+              wv9[u][2 * g + 1] = __builtin_bit_cast(V, u32x2{r.z, r.w});
             } else {
               // the whole vector is reinterpreted (a bit cast of one component
               // lvalue, r.y, reads the vector's first component)
               const f32x4 f = __builtin_bit_cast(f32x4, r);
-              wv[u][4 * g] = f.x;
-              wv[u][4 * g + 1] = f.y;
-              wv[u][4 * g + 2] = f.z;
-              wv[u][4 * g + 3] = f.w;
+              wv9[u][4 * g] = f.x;
+              wv9[u][4 * g + 1] = f.y;
+              wv9[u][4 * g + 2] = f.z;
+              wv9[u][4 * g + 3] = f.w;
             }
           }
           const int o8 = (eb + bsr_pos<V>(8, lane)) * Z;
           if constexpr (sizeof(V) == 8)
-            wv[u][8] = __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rv, o8, 0, kBufNT));
+            wv9[u][8] = __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rv, o8, 0, NT ? kBufNT : 0));
           else
-            wv[u][8] = __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(rv, o8, 0, kBufNT));
+            wv9[u][8] = __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(rv, o8, 0, NT ? kBufNT : 0));
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          bn[u] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rc, ((k + U + u) * kSlice + lane) * 4, 0,
-                                                                kBufNT);
+          bn[u] = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(rc, ((k + U + u) * kSlice + lane) * 4, 0, NT ? kBufNT : 0);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const ACC t0 = (ACC)wv[u][0] * xv[u][0] + (ACC)wv[u][1] * xv[u][1] + (ACC)wv[u][2] * xv[u][2];
-          const ACC t1 = (ACC)wv[u][3] * xv[u][0] + (ACC)wv[u][4] * xv[u][1] + (ACC)wv[u][5] * xv[u][2];
-          const ACC t2 = (ACC)wv[u][6] * xv[u][0] + (ACC)wv[u][7] * xv[u][1] + (ACC)wv[u][8] * xv[u][2];
-          const bool in = k + u < L;
+          const ACC t0 = (ACC)wv9[u][0] * xv[u][0] + (ACC)wv9[u][1] * xv[u][1] + (ACC)wv9[u][2] * xv[u][2];
+          const ACC t1 = (ACC)wv9[u][3] * xv[u][0] + (ACC)wv9[u][4] * xv[u][1] + (ACC)wv9[u][5] * xv[u][2];
+          const ACC t2 = (ACC)wv9[u][6] * xv[u][0] + (ACC)wv9[u][7] * xv[u][1] + (ACC)wv9[u][8] * xv[u][2];
+          const bool in = k + u < k1;
           s0v += in ? t0 : (ACC)0;
           s1v += in ? t1 : (ACC)0;
           s2v += in ? t2 : (ACC)0;
@@ -862,10 +887,17 @@ __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
 #pragma unroll
         for (int u = 0; u < U; ++u) asm volatile("" : "+v"(bn[u]));
       }
+      red[buf][wv][lane] = s0v;
+      red[buf][wv][kSlice + lane] = s1v;
+      red[buf][wv][2 * kSlice + lane] = s2v;
+      // two buffers: the next slice's sums go to the other one, and the one
+      // after that comes behind the next barrier
+      __syncthreads();
       if (a >= 0) {
-        epi(3 * (int64_t)a, s0v);
-        epi(3 * (int64_t)a + 1, s1v);
-        epi(3 * (int64_t)a + 2, s2v);
+        ACC acc = red[buf][0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < kWavesPerBlock; ++w) acc += red[buf][w][threadIdx.x];
+        epi(3 * (int64_t)a + wv, acc);
       }
     }
   } else {
@@ -886,7 +918,7 @@ __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
             const int64_t kk = k + u * kLanesPerRow;
             j[u] = 0;
             a[u] = 0;
-            if (kk < k1) { j[u] = ntload(M.col + kk); a[u] = ntload(M.val + kk); }
+            if (kk < k1) { j[u] = mload<NT>(M.col + kk); a[u] = mload<NT>(M.val + kk); }
           }
           ACC xv[4];
 #pragma unroll
@@ -902,6 +934,12 @@ __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
   }
 }
 
+template <int KIND, class V, class ACC, class F, class E>
+__device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
+  if (M.nt) matvec_rows_as<true, KIND, V, ACC>(M, xval, epi);
+  else matvec_rows_as<false, KIND, V, ACC>(M, xval, epi);
+}
+
 // Calls epi(r, sum_k a_rk X(j_k), pre(r), row) for the rows r of this block's
 // range, row = false for the padding lanes of the last kSell16 slice (their
 // r is past n: epi stores nothing there, and pre was given a clamped row);
@@ -910,7 +948,8 @@ __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
 template <int KIND, class V, class ACC, class F, class P, class E>
 __device__ inline void matvec_rows_pre(const MatFmt<V> &M, F xval, P pre, E epi) {
   if constexpr (KIND == kSell16 && sizeof(V) == 8) {
-    sell16_walk<ACC>(M, xval, pre, epi);
+    if (M.nt) sell16_walk<true, ACC>(M, xval, pre, epi);
+    else sell16_walk<false, ACC>(M, xval, pre, epi);
   } else {
     matvec_rows<KIND, V, ACC>(M, xval, [&](int64_t r, ACC acc) { epi(r, acc, pre(r), true); });
   }
@@ -1697,7 +1736,7 @@ struct ffhip_cg_s {
   int64_t *sptr16 = nullptr;  // kSell16 slice offsets of scol16
   int32_t *bcol = nullptr;    // kBsr3 block columns (slices over sorted node rows)
   int32_t *bperm = nullptr;   // kBsr3 node row of each sorted position
-  int32_t *bwave = nullptr;   // kBsr3 first slice of each mat-vec wave (grid x 4 + 1)
+  int32_t *bwave = nullptr;   // kBsr3 first slice of each mat-vec block (grid + 1)
   // values in the solver's layout; for kCsrV, sval is A's value array (borrowed)
   double *sval = nullptr;    // A
   double *svalT = nullptr;   // A^T (built on first transposed solve)
@@ -1820,6 +1859,11 @@ struct ffhip_cg_s {
       t_dv += d; t_mv += a; t_up += b; ++n_timed;
     }
   }
+  // bytes of the matrix that one mat-vec streams, with values of `size` bytes
+  int64_t matrix_bytes(size_t size) const {
+    if (fmt == kBsr3) return ents * (int64_t)(9 * size + 4);
+    return ents * (int64_t)(size + (fmt == kSell16 ? 2 : 4));
+  }
   template <class V>
   MatFmt<V> fmt_of(const V *val) const {
     MatFmt<V> M;
@@ -1834,8 +1878,9 @@ struct ffhip_cg_s {
     else if (fmt == kBsr3) { M.ptr = sptr; M.len = slen; M.col = bcol; M.nb = n / 3; }
     else { M.ptr = A->rowptr; M.len = nullptr; M.col = A->colidx; }
     M.wstart = fmt == kBsr3 ? bwave : nullptr;
-    M.nw = fmt == kBsr3 && bwave ? grid * kWavesPerBlock : 0;
+    M.nw = fmt == kBsr3 && bwave ? grid : 0;
     M.val = val;
+    M.nt = matrix_bytes(sizeof(V)) > kCachedMatrix;
     return M;
   }
 };
@@ -1952,7 +1997,7 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
   }
   int64_t g;
   if (cg->fmt == kBsr3) {
-    g = ((A->n / 3 + kSlice - 1) / kSlice + kWavesPerBlock - 1) / kWavesPerBlock;
+    g = (A->n / 3 + kSlice - 1) / kSlice;  // a block per slice
   } else if (cg->fmt != kCsrV) {
     g = (cg->S + kWavesPerBlock - 1) / kWavesPerBlock;
   } else {
@@ -1965,7 +2010,7 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
   if (g < 1) g = 1;
   cg->grid = (int)g;
   if (cg->fmt == kBsr3) {
-    const int nw = cg->grid * kWavesPerBlock;
+    const int nw = cg->grid;
     cg->bwave = dalloc<int32_t>(nw + 1);
     k_bsr_waves<<<nblk(nw + 1, 256), 256, 0, s>>>((A->n / 3 + kSlice - 1) / kSlice, cg->sptr, nw,
                                                   cg->bwave);
