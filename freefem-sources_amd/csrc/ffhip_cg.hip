@@ -2004,7 +2004,11 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
     cg->ents = A->nnz;
     g = (A->n + kBlock / kLanesPerRow - 1) / (kBlock / kLanesPerRow);
   }
-  const int64_t gmax = FFHIP_GRID_PER_CU * (int64_t)ctx->num_cu;
+  // resident blocks per CU: 3 of an FP32 solver, 2 of an FP64 one (FP64 mat-vecs at
+  // 2 against 3: cube(160) 136.9 / 139.4 us, cube(96) 24.8 / 25.4, cube(20) 3x3 blocks
+  // 29.1 / 29.7, the vector kernels within 3 %; FP32 cube(64) 6.6 / 5.6, cube(128)
+  // 32.4 / 30.1)
+  const int64_t gmax = (cg->mode == FFHIP_CG_MIXED ? FFHIP_GRID_PER_CU : 2) * (int64_t)ctx->num_cu;
   if (g > gmax) g = gmax;
   if (g >= 64) g -= g % 8;  // whole XCD groups
   if (g < 1) g = 1;
