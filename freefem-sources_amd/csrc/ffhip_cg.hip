@@ -703,65 +703,102 @@ __device__ inline ACC sell16_tail(const int16_t *__restrict__ col16, const doubl
   return acc;
 }
 
-// The FP64 kSell16 walk over this wave's slices.  A slice's values (entry
-// pairs, 16-byte loads) and packed deltas are read through buffer resources
-// that end at the slice's last entry, so the loads of a round are issued
-// unconditionally: entries past the slice width read as value 0, delta 0
-// (the row itself).  pre(r) (the row's own epilogue operands) is issued with
-// the gathers.  epi(r, acc, pre(r), r < n) is called for every lane (rows
-// past n only in the last slice, whose pre was given a clamped row).  The
-// products are summed in entry order.
-template <bool NT, class ACC, class F, class P, class E>
-__device__ inline void sell16_walk(const MatFmt<double> &M, F xval, P pre, E epi) {
+// Row r32 (lane `lane` of slice s) of an FP64 kSell16 matrix times X.  A slice's
+// values (entry pairs, 16-byte loads) and packed deltas are read through buffer
+// resources that end at the slice's last entry, so the loads of a round are
+// issued unconditionally: entries past the slice width read as value 0, delta 0
+// (the row itself).  pre(r32) (the row's own epilogue operands, into pv) is
+// issued with the gathers.  The products are summed in entry order.
+template <bool NT, class ACC, class F, class P, class PV>
+__device__ inline ACC sell16_slice_row(const MatFmt<double> &M, int64_t s, int lane, int32_t r32, F xval,
+                                       P pre, PV &pv) {
   constexpr int U = kU, G4 = kU / 4, NP = kU / 2;
   static_assert(kU % 4 == 0, "unroll by whole index groups");
+  const int64_t vb = uniform(M.ptr[s]), cb = uniform(M.ptr16[s]);
+  const int L = __builtin_amdgcn_readfirstlane(M.len[s]);
+  const int Lh = L >> 1;
+  const auto rc = slice_rsrc(M.col16 + cb, (uint32_t)((L + 3) >> 2) * (4 * kSlice) * 2);
+  const auto rp = slice_rsrc(M.val + vb, (uint32_t)Lh * (2 * kSlice) * 8);
+  const auto r1 = slice_rsrc(M.val + vb + (int64_t)Lh * (2 * kSlice), (uint32_t)(L & 1) * kSlice * 8);
+  u32x2 pk[G4];
+#pragma unroll
+  for (int g = 0; g < G4; ++g)
+    pk[g] = __builtin_amdgcn_raw_buffer_load_b64(rc, (g * kSlice + lane) * 8, 0, NT ? kBufNT : 0);
+  u32x4 q[NP];
+#pragma unroll
+  for (int m = 0; m < NP; ++m)
+    q[m] = __builtin_amdgcn_raw_buffer_load_b128(rp, (m * kSlice + lane) * 16, 0, NT ? kBufNT : 0);
+  const u32x2 odd = __builtin_amdgcn_raw_buffer_load_b64(r1, lane * 8, 0, NT ? kBufNT : 0);
+  int32_t j[U];
+#pragma unroll
+  for (int g = 0; g < G4; ++g) {
+    j[4 * g + 0] = r32 + (int32_t)(int16_t)(pk[g].x & 0xffffu);
+    j[4 * g + 1] = r32 + (int32_t)(int16_t)(pk[g].x >> 16);
+    j[4 * g + 2] = r32 + (int32_t)(int16_t)(pk[g].y & 0xffffu);
+    j[4 * g + 3] = r32 + (int32_t)(int16_t)(pk[g].y >> 16);
+  }
+  double a[U];
+#pragma unroll
+  for (int m = 0; m < NP; ++m) {
+    const u32x2 lo = m == Lh ? odd : u32x2{q[m].x, q[m].y};
+    a[2 * m] = __builtin_bit_cast(double, lo);
+    a[2 * m + 1] = __builtin_bit_cast(double, u32x2{q[m].z, q[m].w});
+  }
+  ACC xv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) xv[u] = xval(j[u]);
+  pv = pre(r32);
+  ACC acc = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) acc += (ACC)a[u] * xv[u];
+  if (L > U) acc = sell16_tail<NT>(M.col16 + cb, M.val + vb, L, lane, r32, xval, acc);
+  return acc;
+}
+
+// The FP64 kSell16 walk over this wave's slices.  epi(r, acc, pre(r), r < n) is
+// called for every lane (rows past n only in the last slice, whose pre was
+// given a clamped row).
+template <bool NT, class ACC, class F, class P, class E>
+__device__ inline void sell16_walk(const MatFmt<double> &M, F xval, P pre, E epi) {
   int64_t s, s1, ds;
   wave_slices<kCyclicSell>(M.S, s, s1, ds);
   const int lane = threadIdx.x % kSlice;
   for (; s < s1; s += ds) {
-    const int64_t vb = uniform(M.ptr[s]), cb = uniform(M.ptr16[s]);
-    const int L = __builtin_amdgcn_readfirstlane(M.len[s]);
-    const int Lh = L >> 1;
     const int64_t r = s * kSlice + lane;
     // rows past n (last slice) have only padding: their column is clamped
     const int32_t r32 = (int32_t)(r < M.n ? r : M.n - 1);
-    const auto rc = slice_rsrc(M.col16 + cb, (uint32_t)((L + 3) >> 2) * (4 * kSlice) * 2);
-    const auto rp = slice_rsrc(M.val + vb, (uint32_t)Lh * (2 * kSlice) * 8);
-    const auto r1 = slice_rsrc(M.val + vb + (int64_t)Lh * (2 * kSlice), (uint32_t)(L & 1) * kSlice * 8);
-    u32x2 pk[G4];
-#pragma unroll
-    for (int g = 0; g < G4; ++g)
-      pk[g] = __builtin_amdgcn_raw_buffer_load_b64(rc, (g * kSlice + lane) * 8, 0, NT ? kBufNT : 0);
-    u32x4 q[NP];
-#pragma unroll
-    for (int m = 0; m < NP; ++m)
-      q[m] = __builtin_amdgcn_raw_buffer_load_b128(rp, (m * kSlice + lane) * 16, 0, NT ? kBufNT : 0);
-    const u32x2 odd = __builtin_amdgcn_raw_buffer_load_b64(r1, lane * 8, 0, NT ? kBufNT : 0);
-    int32_t j[U];
-#pragma unroll
-    for (int g = 0; g < G4; ++g) {
-      j[4 * g + 0] = r32 + (int32_t)(int16_t)(pk[g].x & 0xffffu);
-      j[4 * g + 1] = r32 + (int32_t)(int16_t)(pk[g].x >> 16);
-      j[4 * g + 2] = r32 + (int32_t)(int16_t)(pk[g].y & 0xffffu);
-      j[4 * g + 3] = r32 + (int32_t)(int16_t)(pk[g].y >> 16);
-    }
-    double a[U];
-#pragma unroll
-    for (int m = 0; m < NP; ++m) {
-      const u32x2 lo = m == Lh ? odd : u32x2{q[m].x, q[m].y};
-      a[2 * m] = __builtin_bit_cast(double, lo);
-      a[2 * m + 1] = __builtin_bit_cast(double, u32x2{q[m].z, q[m].w});
-    }
-    ACC xv[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) xv[u] = xval(j[u]);
-    const auto pv = pre(r32);
-    ACC acc = 0;
-#pragma unroll
-    for (int u = 0; u < U; ++u) acc += (ACC)a[u] * xv[u];
-    if (L > U) acc = sell16_tail<NT>(M.col16 + cb, M.val + vb, L, lane, r32, xval, acc);
+    decltype(pre(r32)) pv;
+    const ACC acc = sell16_slice_row<NT, ACC>(M, s, lane, r32, xval, pre, pv);
     epi(r, acc, pv, r < M.n);
   }
+}
+
+// One CSR row over the 16 lanes of a group, the sum in every lane.
+template <bool NT, class V, class ACC, class F>
+__device__ inline ACC csr_row_sum(const MatFmt<V> &M, int64_t r, bool in, int lane, F xval) {
+  ACC acc = 0;
+  if (in) {
+    const int64_t k0 = M.ptr[r], k1 = M.ptr[r + 1];
+    for (int64_t k = k0 + lane; k < k1; k += 4 * kLanesPerRow) {
+      int32_t j[4];
+      V a[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t kk = k + u * kLanesPerRow;
+        j[u] = 0;
+        a[u] = 0;
+        if (kk < k1) { j[u] = mload<NT>(M.col + kk); a[u] = mload<NT>(M.val + kk); }
+      }
+      ACC xv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) xv[u] = xval(j[u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc += (ACC)a[u] * xv[u];
+    }
+  }
+#pragma unroll
+  for (int off = kLanesPerRow / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
+  return acc;
 }
 
 // Calls epi(r, sum_k a_rk X(j_k)) once for every row r of this block's range;
@@ -907,28 +944,7 @@ __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
     constexpr int NG = kBlock / kLanesPerRow;
     for (int64_t rb = r0; rb < r1; rb += NG) {
       const int64_t r = rb + g;
-      ACC acc = 0;
-      if (r < r1) {
-        const int64_t k0 = M.ptr[r], k1 = M.ptr[r + 1];
-        for (int64_t k = k0 + lane; k < k1; k += 4 * kLanesPerRow) {
-          int32_t j[4];
-          V a[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int64_t kk = k + u * kLanesPerRow;
-            j[u] = 0;
-            a[u] = 0;
-            if (kk < k1) { j[u] = mload<NT>(M.col + kk); a[u] = mload<NT>(M.val + kk); }
-          }
-          ACC xv[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) xv[u] = xval(j[u]);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) acc += (ACC)a[u] * xv[u];
-        }
-      }
-#pragma unroll
-      for (int off = kLanesPerRow / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
+      const ACC acc = csr_row_sum<NT, V, ACC>(M, r, r < r1, lane, xval);
       if (r < r1 && lane == 0) epi(r, acc);
     }
   }
@@ -1149,6 +1165,218 @@ __global__ FFHIP_MATVEC_ATTR void k_residual(MatFmt<double> M, const double *__r
   if (threadIdx.x == 0) {
     const int lb = xcd_block_id();
     pout[3 * lb] = a; pout[3 * lb + 1] = c; pout[3 * lb + 2] = e;
+  }
+}
+
+// ---------------------------------------------------------------- small systems
+// A whole FP64 solve of a small system in one workgroup: the start
+// (SetInitWithBC, G = A x - b), the iterations of the three kernels above and
+// the residual sums.  Up to some thousand rows an iteration is nothing but the
+// latency of three launches (12 us with the gaps between them) and a solve
+// waits for the set-up of a captured chunk; here it is three barriers, with h,
+// A h and x in LDS and g and D^-1 in registers, bound by the latency of a row
+// (slice offsets, entries from L2, gathers from LDS).  us per iteration, this
+// against launches (set-up included): 216 rows 2.3 / 17.7, 1000 rows 4.0 / 15.1,
+// 1728 rows 6.9 / 13.2, 4096 rows 10.9 / 12.4 (P1 cubes); CSR 216 rows 5.6 / 19.4.
+//
+// The sums are those of the launches, bit for bit: virtual block vb of the G
+// that the launches would use is played by four waves (up to four blocks at a
+// time, the others in turn), rows and slices go to the same threads, and
+// partials are added in the same order.
+constexpr int kSmallBlocks = 16;                         // virtual blocks
+constexpr int kSmallRows = kSmallBlocks * kBlock;        // kSell16: 256 rows each
+constexpr int kSmallRowsCsr = kSmallBlocks * kBlock / kLanesPerRow;  // kCsrV: 16 rows
+struct SmallOut {
+  CgState st;
+  double res[3 * kSmallBlocks];  // k_residual's partials
+};
+template <int KIND, int Q>  // Q: rows of a thread in the vector passes
+__global__ __launch_bounds__(1024) void k_pcg_small(MatFmt<double> M, int G, const double *b, double *x,
+                                                    const double *__restrict__ dinv,
+                                                    const uint8_t *__restrict__ wcl, double tgv,
+                                                    double eps, int itmax, SmallOut *__restrict__ out) {
+  constexpr bool SELL = KIND == kSell16;
+  constexpr int T = SELL ? Q : 4;  // virtual blocks that a wave plays in a mat-vec
+  __shared__ double H[Q * 1024], A[Q * 1024], X[Q * 1024];
+  __shared__ double ws[3][kSmallBlocks * kWavesPerBlock];  // wave sums
+  const int n = (int)M.n, S = (int)M.S, t = threadIdx.x % kBlock, lane = threadIdx.x % kWave;
+  const int W = wave_id(), w = W % kWavesPerBlock, nv = blockDim.x / kBlock;
+  int row[Q];  // this thread's rows in the vector passes; -1: none
+  double g[Q], di[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    // block_rows; a kCsrV block's up to 16 rows take 16 lanes here
+    const int vb = SELL ? q * nv + W / kWavesPerBlock : threadIdx.x / kLanesPerRow;
+    const int r = vb * n / G + (SELL ? t : threadIdx.x % kLanesPerRow);
+    row[q] = vb < G && r < (vb + 1) * n / G ? r : -1;
+    di[q] = 0.; g[q] = 0.;
+    if (row[q] >= 0) {
+      di[q] = dinv[row[q]];
+      const double x0 = wcl && wcl[row[q]] ? b[row[q]] / tgv : x[row[q]];
+      X[row[q]] = x0;
+      H[row[q]] = x0;
+    }
+  }
+  // the rows of A H of this wave in turn q: epi(r, acc, row) as in matvec_rows_pre
+  auto matvec = [&](int q, auto epi) {
+    const auto xval = [&](int32_t j) { return H[j]; };
+    const int vb = q * nv + W / kWavesPerBlock;
+    if (vb >= G) return;
+    if constexpr (SELL) {  // wave_slices: at most one slice
+      const int groups = G % 8 ? 1 : 8, nloc = G / groups, grp = vb / nloc, loc = vb - grp * nloc;
+      const int s = grp * S / groups + loc * kWavesPerBlock + w;
+      if (s >= (grp + 1) * S / groups) return;
+      const int r = s * kSlice + lane, rc = r < n ? r : n - 1;
+      int pv;
+      const double acc =
+          sell16_slice_row<false, double>(M, s, lane, rc, xval, [](int32_t) { return 0; }, pv);
+      epi(r, acc, r < n);
+    } else {
+      const int r = vb * n / G + t / kLanesPerRow;
+      const bool in = r < (vb + 1) * n / G;
+      const double acc = csr_row_sum<false, double, double>(M, r, in, t % kLanesPerRow, xval);
+      if (in && t % kLanesPerRow == 0) epi(r, acc, true);
+    }
+  };
+  // wave sums of one value per thread: of a mat-vec's turn q, of a vector pass
+  auto put = [&](int k, int q, double v) {
+    v = wave_sum(v);
+    const int vb = q * nv + W / kWavesPerBlock;
+    if (lane == 0 && vb < G) ws[k][vb * kWavesPerBlock + w] = v;
+  };
+  auto put_rows = [&](int k, int q, double v) {
+    if constexpr (SELL) put(k, q, v);
+    else {  // the first wave of the block, its other lanes and the other waves without rows
+      v = row16_sum(v);
+      const int vb = threadIdx.x / kLanesPerRow, l = threadIdx.x % kLanesPerRow;
+      if (vb < G && l < kWavesPerBlock) ws[k][vb * kWavesPerBlock + l] = l == 0 ? v : 0.;
+    }
+  };
+  auto partial = [&](int k) {  // block_sum of virtual block `lane`
+    double p = 0.;
+    if (lane < G) {
+#pragma unroll
+      for (int i = 0; i < kWavesPerBlock; ++i) p += ws[k][lane * kWavesPerBlock + i];
+    }
+    return p;
+  };
+  auto total = [&](int k) { return 0. + wave_sum(partial(k)); };  // reduce_partials
+  __syncthreads();
+#pragma unroll 1
+  for (int q = 0; q < T; ++q) {  // k_pcg_init
+    double part = 0.;
+    matvec(q, [&](int r, double acc, bool in) {
+      if (!in) return;
+      const double gv = acc + -1. * b[r];
+      const double c = dinv[r] * gv;
+      A[r] = gv;
+      part += gv * c;
+    });
+    put(0, q, part);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (row[q] >= 0) g[q] = A[row[q]];
+  double gcg0 = 0., eps2 = 0., gcgp = 0., gcg, rho = 0.;
+  int it = 1, done = 0;
+  for (;; ++it) {
+    // pcg_begin
+    gcg = total(0);
+    double gamma = 0.;
+    if (it == 1) {
+      gcg0 = gcg;
+      eps2 = eps > 0 ? eps * eps * gcg : eps * eps;
+      if (gcg != gcg) done = 4;
+      else if (gcg < 1e-30) done = 2;
+    } else {
+      gamma = gcg / gcgp;
+      if (gcg != gcg) done = 4;
+      else if (gcg < eps2) done = 1;
+      else if (it - 1 >= itmax) done = 3;
+    }
+    gcgp = gcg;
+    if (done) break;  // the same in every thread
+    // k_pcg_dirvec
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      double part = 0.;
+      if (row[q] >= 0) {
+        const double h = it > 1 ? H[row[q]] : 0.;
+        if (it > 1) X[row[q]] += rho * h;
+        const double hn = gamma * h - __dmul_rn(di[q], g[q]);
+        H[row[q]] = hn;
+        part += g[q] * hn;
+      }
+      put_rows(1, q, part);
+    }
+    __syncthreads();
+    // k_pcg_matvec
+#pragma unroll 1
+    for (int q = 0; q < T; ++q) {
+      double part = 0.;
+      matvec(q, [&](int r, double acc, bool in) {
+        if (in) A[r] = acc;
+        part += (in ? H[r] : 0.) * acc;
+      });
+      put(2, q, part);
+    }
+    __syncthreads();
+    // k_pcg_update
+    const double hah = total(2), gh = total(1);
+    rho = -gh / hah;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      double part = 0.;
+      if (row[q] >= 0) {
+        const double gn = g[q] + rho * A[row[q]];
+        g[q] = gn;
+        const double c = __dmul_rn(di[q], gn);
+        part += gn * c;
+      }
+      put_rows(0, q, part);
+    }
+    __syncthreads();
+  }
+  // the stopping launch's step, then the residual of the solution
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (row[q] >= 0) {
+      if (it > 1) X[row[q]] += rho * H[row[q]];
+      H[row[q]] = X[row[q]];
+    }
+  __syncthreads();
+#pragma unroll 1
+  for (int q = 0; q < T; ++q) {  // k_residual
+    double rr = 0., bb = 0., rc = 0.;
+    matvec(q, [&](int r, double acc, bool in) {
+      if (!in) return;
+      const double v = b[r] - acc;
+      rr += v * v;
+      bb += b[r] * b[r];
+      rc += v * (dinv[r] * v);
+    });
+    put(0, q, rr);
+    put(1, q, bb);
+    put(2, q, rc);
+  }
+  __syncthreads();  // b has been read: x may be the same array
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (row[q] >= 0) x[row[q]] = X[row[q]];
+  if (W == 0) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double p = partial(c);
+      if (lane < G) out->res[3 * lane + c] = p;
+    }
+    if (lane == 0) {
+      out->st.gcg0 = gcg0;
+      out->st.eps2 = eps2;
+      out->st.gcg_prev[it & 1] = gcg;
+      out->st.done = done;
+      out->st.iters = it - 1;
+    }
   }
 }
 
@@ -2276,6 +2504,76 @@ int ffhip_cg_solve_mixed(ffhip_cg cg, const double *sval, const float *sval32, d
   }
 }
 
+// the figures of a finished solve for the caller, and the errors of one that
+// did not converge (res: the sums of k_residual)
+static void solve_result(ffhip_cg cg, const CgState &hs, const double res[3], double ms, int itmax,
+                         ffhip_cg_stats *stats) {
+  if (stats) {
+    stats->iters = hs.iters;
+    stats->converged = hs.done == 1 ? 1 : (hs.done == 2 ? 2 : 0);
+    stats->refinements = hs.refinements;
+    stats->gcg0 = hs.gcg0;
+    stats->gcg = cg->mode == FFHIP_CG_FP64 ? hs.gcg_prev[(hs.iters + 1) & 1] : res[2];
+    stats->true_gcg = res[2];
+    stats->true_relres = res[1] > 0 ? std::sqrt(res[0] / res[1]) : std::sqrt(res[0]);
+    stats->ms_solve = ms;
+    stats->timed = cg->n_timed;
+    stats->ms_matvec_avg = cg->n_timed ? cg->t_mv / cg->n_timed : 0.;
+    stats->ms_update_avg = cg->n_timed ? cg->t_up / cg->n_timed : 0.;
+    stats->ms_direction_avg = cg->n_timed ? cg->t_dv / cg->n_timed : 0.;
+  }
+  FFHIP_REQUIRE(hs.done != 4, FFHIP_ERR_NAN, "ffhip_cg_solve: NaN in CG (bad matrix)");
+  FFHIP_REQUIRE(hs.done != 3, FFHIP_ERR_NOCONV,
+                "ffhip_cg_solve: ConjugueGradient did not converge in %d iterations", itmax);
+}
+
+// Systems that k_pcg_small solves: FP64 in the 16-bit sliced layout up to
+// kSmallRows rows, in CSR (taken where slices would pad) up to kSmallRowsCsr,
+// unless kernel-by-kernel launches are asked for.  One CU reads the matrix at
+// about 64 bytes a cycle: past 2^16 entries (the 4096 rows of a P1 cube) the
+// launches win.  The iteration cap bounds the one launch.
+static bool pcg_small(ffhip_cg cg, int itmax) {
+  const bool fits = (cg->fmt == kSell16 && cg->n <= kSmallRows) || (cg->fmt == kCsrV && cg->n <= kSmallRowsCsr);
+  return cg->mode == FFHIP_CG_FP64 && fits && cg->ents <= 1 << 16 && cg->grid <= kSmallBlocks &&
+         cg->use_graph && !cg->profile && itmax <= 65536;
+}
+static void pcg_solve_small(ffhip_cg cg, const double *b, double *x, int on_device, const double *sval,
+                            double eps, int itmax, double tgv, ffhip_cg_stats *stats) {
+  ffhip_ctx ctx = cg->ctx;
+  hipStream_t s = ctx->stream;
+  const int64_t n = cg->n;
+  const double *bd = b;
+  double *xd = x;
+  if (!on_device) {
+    FFHIP_CHECK(hipMemcpyAsync(cg->bw, b, 8 * n, hipMemcpyHostToDevice, s));
+    FFHIP_CHECK(hipMemcpyAsync(cg->xw, x, 8 * n, hipMemcpyHostToDevice, s));
+    bd = cg->bw;
+    xd = cg->xw;
+  }
+  static_assert(sizeof(SmallOut) <= ffhip_ctx_s::kPinned, "page-locked read-back");
+  SmallOut *out = static_cast<SmallOut *>(ctx->pinned);
+  memset(out, 0, sizeof(*out));
+  const int G = cg->grid;
+  ctx->tic();
+  const auto kernel = cg->fmt == kCsrV ? k_pcg_small<kCsrV, 1>
+                      : G <= 4         ? k_pcg_small<kSell16, 1>
+                                       : k_pcg_small<kSell16, kSmallBlocks / 4>;
+  kernel<<<1, kBlock * std::min(G, 4), 0, s>>>(cg->fmt_of(sval), G, bd, xd, cg->dinv,
+                                               cg->ntgv > 0 ? cg->wcl : nullptr, tgv, eps, itmax, out);
+  FFHIP_CHECK(hipGetLastError());
+  ctx->toc();
+  if (!on_device) {
+    FFHIP_CHECK(hipMemcpyAsync(x, cg->xw, 8 * n, hipMemcpyDeviceToHost, s));
+    FFHIP_CHECK(hipStreamSynchronize(s));
+  }
+  double res[3] = {0., 0., 0.};
+  for (int i = 0; i < G; ++i)
+    for (int c = 0; c < 3; ++c) res[c] += out->res[3 * i + c];
+  cg->t_dv = cg->t_mv = cg->t_up = 0.;
+  cg->n_timed = 0;
+  solve_result(cg, out->st, res, ctx->last_ms, itmax, stats);
+}
+
 static void cg_release(ffhip_cg cg) {
   for (hipEvent_t e : cg->ev) (void)hipEventDestroy(e);
   for (auto &g : cg->graphs) (void)hipGraphExecDestroy(g.exec);
@@ -2389,6 +2687,10 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
     const double *sval = trans ? cg->svalT : cg->sval;
     const float *sval32 = trans ? cg->sval32T : cg->sval32;
     if (itmax <= 0) itmax = (int)n;  // SolverCG(ds): itmax > 0 ? itmax : n
+    if (pcg_small(cg, itmax)) {
+      pcg_solve_small(cg, b, x, on_device, sval, eps, itmax, tgv, stats);
+      return;
+    }
     // captured before this solve's first launch (kept for later solves)
     if (cg->mode == FFHIP_CG_FP64) (void)pcg_chunk_graph(cg, sval);
     else { (void)mix_chunk_graph(cg, sval32, 0); (void)mix_chunk_graph(cg, sval32, 1); }
@@ -2431,23 +2733,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
     residual_sums(cg, sval, cg->xw, cg->bw, nullptr, res);
     FFHIP_CHECK(hipMemcpyAsync(x, cg->xw, 8 * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
     FFHIP_CHECK(hipStreamSynchronize(s));
-    if (stats) {
-      stats->iters = hs.iters;
-      stats->converged = hs.done == 1 ? 1 : (hs.done == 2 ? 2 : 0);
-      stats->refinements = hs.refinements;
-      stats->gcg0 = hs.gcg0;
-      stats->gcg = cg->mode == FFHIP_CG_FP64 ? hs.gcg_prev[(hs.iters + 1) & 1] : res[2];
-      stats->true_gcg = res[2];
-      stats->true_relres = res[1] > 0 ? std::sqrt(res[0] / res[1]) : std::sqrt(res[0]);
-      stats->ms_solve = ms;
-      stats->timed = cg->n_timed;
-      stats->ms_matvec_avg = cg->n_timed ? cg->t_mv / cg->n_timed : 0.;
-      stats->ms_update_avg = cg->n_timed ? cg->t_up / cg->n_timed : 0.;
-      stats->ms_direction_avg = cg->n_timed ? cg->t_dv / cg->n_timed : 0.;
-    }
-    FFHIP_REQUIRE(hs.done != 4, FFHIP_ERR_NAN, "ffhip_cg_solve: NaN in CG (bad matrix)");
-    FFHIP_REQUIRE(hs.done != 3, FFHIP_ERR_NOCONV,
-                  "ffhip_cg_solve: ConjugueGradient did not converge in %d iterations", itmax);
+    solve_result(cg, hs, res, ms, itmax, stats);
   });
 }
 

@@ -339,6 +339,7 @@ int ffhip_init(int device, ffhip_ctx *out) {
     FFHIP_CHECK(hipStreamCreate(&c->stream));
     FFHIP_CHECK(hipEventCreate(&c->ev0));
     FFHIP_CHECK(hipEventCreate(&c->ev1));
+    FFHIP_CHECK(hipHostMalloc(&c->pinned, ffhip_ctx_s::kPinned, hipHostMallocDefault));
     hipDeviceProp_t prop;
     FFHIP_CHECK(hipGetDeviceProperties(&prop, device));
     c->num_cu = prop.multiProcessorCount;
@@ -353,6 +354,7 @@ int ffhip_ctx_free(ffhip_ctx c) {
     (void)hipStreamSynchronize(c->stream);
     if (c->scratch) (void)hipFree(c->scratch);
     if (c->work) (void)hipFree(c->work);
+    if (c->pinned) (void)hipHostFree(c->pinned);
     (void)hipEventDestroy(c->ev0);
     (void)hipEventDestroy(c->ev1);
     (void)hipStreamDestroy(c->stream);

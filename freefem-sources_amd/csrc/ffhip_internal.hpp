@@ -92,6 +92,10 @@ struct ffhip_ctx_s {
   void *work = nullptr;
   size_t work_bytes = 0;
   void *ensure_work(size_t bytes);
+  // page-locked host memory that kernels write small results to (read after the
+  // call's wait; one call at a time per context)
+  static constexpr size_t kPinned = 4096;
+  void *pinned = nullptr;
   double last_ms = 0.;  // device time of the last timed call
   void tic();           // record ev0 on the stream
   void toc();           // record ev1, synchronise, set last_ms
@@ -188,6 +192,13 @@ __device__ inline double dpp_row(double v) {
 __device__ inline double join_halves(unsigned lo, unsigned hi) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
+__device__ inline double row16_sum(double v) {  // over each 16 lanes
+  v += dpp_row<0x128>(v);                       // row_ror:8
+  v += dpp_row<0x124>(v);
+  v += dpp_row<0x122>(v);
+  v += dpp_row<0x121>(v);
+  return v;
+}
 __device__ inline double wave_sum(double v) {
   {
     const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
@@ -201,11 +212,7 @@ __device__ inline double wave_sum(double v) {
     const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
     v = join_halves(l[0], h[0]) + join_halves(l[1], h[1]);
   }
-  v += dpp_row<0x128>(v);  // row_ror:8
-  v += dpp_row<0x124>(v);
-  v += dpp_row<0x122>(v);
-  v += dpp_row<0x121>(v);
-  return v;
+  return row16_sum(v);
 }
 
 // Deterministic block reduction of one double; result valid in every thread.

@@ -356,7 +356,8 @@ enum { FFHIP_CG_INDEX16 = 0x40, FFHIP_CG_INDEX32 = 0x80 };
 /* The solve loops replay one captured chunk of 16 iterations (a hipGraph per
  * solver, value array and parity, captured on first use); FFHIP_CG_EAGER in
  * mode launches the kernels one by one instead (as does per-kernel
- * profiling). */
+ * profiling).  A small FP64 system (up to 4096 rows) is solved by one launch
+ * of one workgroup otherwise, with the same bits. */
 enum { FFHIP_CG_EAGER = 0x200 };
 typedef struct {
   int iters;          /* CG iterations (inner FP32 iterations for MIXED)   */
