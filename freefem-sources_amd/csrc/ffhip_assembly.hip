@@ -65,6 +65,7 @@ __global__ void k_v2e_bucket(const int32_t *__restrict__ elems, int64_t m,
 __global__ void k_u32_to_i64(int64_t n, const uint32_t *__restrict__ a, int64_t *__restrict__ b) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) b[i] = a[i];
+  if (i == 0) b[n] = 0;  // the scan's last input
 }
 
 __global__ void k_v2e_fill(const int32_t *__restrict__ elems, int64_t m,
@@ -513,6 +514,7 @@ __global__ void k_link_len(int64_t n, int dim, const int64_t *__restrict__ v2e_p
   if (dim == 3) l = b == 0 ? 3 + deg / 2 : 2 + (deg + b) / 2;
   else l = b == 0 ? 1 + deg : 2 + deg;
   len[v] = deg == 0 ? 0 : l;
+  if (v == 0) len[n] = 0;  // the scan's last input
 }
 
 // buffered columns to their CSR place; diagonal slots.  One lane per row:
@@ -1025,14 +1027,9 @@ __global__ __launch_bounds__(256) void k_p1_values_rows(
 
 // ---------------------------------------------------------------- Dirichlet
 __global__ void k_mark_bc(int64_t nbe, int nbloc, const int32_t *__restrict__ belems,
-                          const int32_t *__restrict__ blab, const int32_t *__restrict__ labs,
-                          int nlab, uint8_t *__restrict__ onbc) {
+                          const int32_t *__restrict__ blab, Labels labels, uint8_t *__restrict__ onbc) {
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nbe) return;
-  const int32_t lab = blab[f];
-  bool on = false;
-  for (int k = 0; k < nlab; ++k) on |= (lab == labs[k]);
-  if (!on) return;
+  if (f >= nbe || !labels.has(blab[f])) return;
   for (int q = 0; q < nbloc; ++q) onbc[belems[nbloc * f + q]] = 1;  // same value from every writer
 }
 
@@ -1042,7 +1039,7 @@ __global__ void k_set_diag(int64_t n, const uint8_t *__restrict__ onbc,
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n || !onbc[i]) return;
   const int64_t s = diag[i];
-  if (s < 0) { atomicMax(missing, 1); return; }
+  if (s < 0) { *missing = 1; return; }
   vals[s] = tgv;
 }
 
@@ -1415,7 +1412,7 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
           if (i0 + u * kWave < cnt) {
             const int64_t s = cg[u] == ri[u] ? g[u] : find_entry(q0[u], q1[u], colidx, ri[u]);
             if (s >= 0) a[u] = vals[s];
-            else atomicOr(missing, 1);
+            else *missing = 1;
           }
         }
       }
@@ -1469,7 +1466,6 @@ static unsigned nblocks(int64_t n, int b) { return (unsigned)((n + b - 1) / b); 
 static bool few_rows(int64_t n) { return n < 64 * 16 * 256; }
 // one wave per `rows` rows, whole XCD groups
 static unsigned row_grid(int64_t n, int rows) { return (nblocks(n, rows) + 7) / 8 * 8; }
-int read_flag(ffhip_ctx ctx, int *d);
 void half_view(ffhip_mat L);
 
 // once per device (__constant__ memory is per device): the context's device,
@@ -1504,8 +1500,7 @@ void v2e_fill_sort(ffhip_ctx ctx, const int32_t *elems, int64_t M, int64_t n, co
   hipStream_t s = ctx->stream;
   int32_t *cur = dalloc<int32_t>(n);
   int *flag = dalloc<int>(1);
-  FFHIP_CHECK(hipMemsetAsync(cur, 0, 4 * n, s));
-  FFHIP_CHECK(hipMemsetAsync(flag, 0, sizeof(int), s));
+  clear(ctx, {{cur, 4 * (size_t)n}, {flag, sizeof(int)}});
   k_v2e_fill<<<nblocks(M, 256), 256, 0, s>>>(elems, M, ptr, cur, list);
   k_v2e_sort_half<<<nblocks(n * kHalf, 256), 256, 0, s>>>(n, ptr, list, flag);
   k_v2e_sort<<<nblocks(n, 256), 256, 0, s>>>(n, ptr, list);
@@ -1532,9 +1527,7 @@ void build_incidence(ffhip_ctx ctx, const int32_t *elems, int64_t nt, int nloc, 
   int64_t *ptr = dalloc<int64_t>(n + 1);
   int32_t *list = dalloc<int32_t>(M);
   int32_t *inv = inv_out ? dalloc<int32_t>(M) : nullptr;
-  FFHIP_CHECK(hipMemsetAsync(deg, 0, 4 * n, s));
-  FFHIP_CHECK(hipMemsetAsync(deg64 + n, 0, 8, s));
-  FFHIP_CHECK(hipMemsetAsync(flag, 0, sizeof(int), s));
+  clear(ctx, {{deg, 4 * (size_t)n}, {flag, sizeof(int)}});
   if (sc && nloc == 4)  // the element scales computed in the same pass
     k_v2e_bucket_scale<<<nblocks(nt, 256), 256, 0, s>>>(elems, nt, *sc, deg, bucket, flag);
   else
@@ -1615,7 +1608,7 @@ void set_diag_rows(ffhip_ctx ctx, int64_t n, const uint8_t *onbc, const int64_t 
 // tmap[k] = slot of the transposed entry; false if the pattern is not symmetric
 bool transpose_map(ffhip_ctx ctx, ffhip_mat A, int64_t *tmap) {
   int *missing = dalloc<int>(1);
-  FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), ctx->stream));
+  clear(ctx, {{missing, sizeof(int)}});
   k_transpose_map<<<nblocks(A->n, 256), 256, 0, ctx->stream>>>(A->n, A->rowptr, A->colidx, tmap,
                                                                 missing);
   FFHIP_CHECK(hipGetLastError());
@@ -1624,53 +1617,41 @@ bool transpose_map(ffhip_ctx ctx, ffhip_mat A, int64_t *tmap) {
   return miss == 0;
 }
 
-int read_flag(ffhip_ctx ctx, int *d) {
-  int h = 0;
-  FFHIP_CHECK(hipMemcpyAsync(&h, d, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  FFHIP_CHECK(hipStreamSynchronize(ctx->stream));
-  return h;
-}
-
 // ---------------------------------------------------------------- misfit
 // J = 1/2 int (u - ud)^2 (partials of kMisfitBlocks blocks, summed on the host
-// in block order) and r = M (u - ud) with the Dirichlet rows zeroed, on the
-// given buffers: part (kMisfitBlocks doubles, when J), onbc (nv bytes) and
-// labs (nlab int32, when r and nlab > 0), pair (nt, when r; without it r's
-// terms are formed per incidence)
+// in block order; they go to page-locked memory) and r = M (u - ud) with the
+// Dirichlet rows zeroed, on the given buffers: onbc (nv bytes, when r and
+// nlab > 0), labs (nlab int32, where there are more labels than kernels take
+// by value), pair (nt, when r; without it r's terms are formed per incidence)
 constexpr int kMisfitBlocks = 1024;
+static_assert(8 * kMisfitBlocks <= ffhip_ctx_s::kPinnedData, "page-locked partials");
 struct MisfitBuffers {
-  double *part = nullptr;
   uint8_t *onbc = nullptr;
   int32_t *labs = nullptr;
   double2 *pair = nullptr;
 };
 
-__global__ void k_fill_u8(int64_t n, uint8_t *__restrict__ a, uint8_t v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = v;
+// the vertices of the boundary elements with these labels
+void mark_bc(ffhip_ctx ctx, ffhip_mesh m, const Labels &labels, uint8_t *onbc) {
+  clear(ctx, {{onbc, (size_t)m->nv}});
+  if (m->nbe)
+    k_mark_bc<<<nblocks(m->nbe, 256), 256, 0, ctx->stream>>>(m->nbe, m->nbloc, m->belems, m->blab, labels, onbc);
+  FFHIP_CHECK(hipGetLastError());
 }
 
 void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
                 const int32_t *labels, int nlab, double *J, double *r, const MisfitBuffers &b) {
   hipStream_t s = ctx->stream;
   ctx->tic();
-  double h[kMisfitBlocks];
+  double *part = J ? static_cast<double *>(ctx->pinned_data()) : nullptr;
   if (J || b.pair) {
-    k_p1_misfit_elem<<<kMisfitBlocks, 256, 0, s>>>(m->nt, m->xyz, m->elems, u, ud, b.part, b.pair);
+    k_p1_misfit_elem<<<kMisfitBlocks, 256, 0, s>>>(m->nt, m->xyz, m->elems, u, ud, part, b.pair);
     FFHIP_CHECK(hipGetLastError());
-    if (J) {
-      FFHIP_CHECK(hipMemcpyAsync(h, b.part, sizeof(h), hipMemcpyDeviceToHost, s));
-      FFHIP_CHECK(hipStreamSynchronize(s));
-    }
   }
   if (r) {
     const uint8_t *onbc = nullptr;
     if (nlab > 0) {
-      FFHIP_CHECK(hipMemcpyAsync(b.labs, labels, 4 * nlab, hipMemcpyHostToDevice, s));
-      k_fill_u8<<<nblocks(m->nv, 256), 256, 0, s>>>(m->nv, b.onbc, 0);
-      if (m->nbe)
-        k_mark_bc<<<nblocks(m->nbe, 256), 256, 0, s>>>(m->nbe, m->nbloc, m->belems, m->blab, b.labs,
-                                                       nlab, b.onbc);
+      mark_bc(ctx, m, LabelArg(ctx, labels, nlab, b.labs).L, b.onbc);
       onbc = b.onbc;
     }
     if (b.pair) {
@@ -1686,7 +1667,7 @@ void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
   ctx->toc();
   if (J) {
     double tot = 0.;
-    for (int i = 0; i < kMisfitBlocks; ++i) tot += h[i];
+    for (int i = 0; i < kMisfitBlocks; ++i) tot += part[i];
     *J = tot;
   }
 }
@@ -1695,12 +1676,11 @@ void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
 // The scratch of ffhip_p1_misfit_noalloc: a file-scope device array, one copy
 // per device, reached through the address hipGetSymbolAddress gives on that
 // device (the array's name is a host-side stand-in in host code).  Layout:
-// misfit partials | labels | Dirichlet marks.  Every call on a device shares
+// labels | Dirichlet marks.  Every call on a device shares
 // it: overlapping calls on one device race.
 constexpr int64_t kNoallocMaxVertices = (int64_t)1 << 24;
 constexpr int kNoallocMaxLabels = 64;
-constexpr size_t kScratchPartOff = 0;
-constexpr size_t kScratchLabelsOff = 8 * kMisfitBlocks;
+constexpr size_t kScratchLabelsOff = 0;
 constexpr size_t kScratchOnbcOff = kScratchLabelsOff + 4 * kNoallocMaxLabels;
 constexpr size_t kScratchBytes = kScratchOnbcOff + (size_t)kNoallocMaxVertices;
 constexpr int kMaxDevices = 64;
@@ -1755,7 +1735,7 @@ ffhip_mat pattern_p1(ffhip_ctx ctx, ffhip_mesh m, const double *Ce, bool *values
   if (vals_pass) {
     bool scaled = false;
     ovf = dalloc<int>(1);
-    FFHIP_CHECK(hipMemsetAsync(ovf, 0, sizeof(int), s));
+    clear(ctx, {{ovf, sizeof(int)}});
     bucket = build_v2e_unsorted(m, sc, &scaled, ovf);
     if (sc && !scaled) {
       k_p1_scale_3d<<<nblocks(m->nt, 256), 256, 0, s>>>(m->nt, sc->xyz, m->elems, sc->kind, sc->c0,
@@ -1787,9 +1767,7 @@ ffhip_mat pattern_p1(ffhip_ctx ctx, ffhip_mesh m, const double *Ce, bool *values
       uint32_t *bcnt = ar.take<uint32_t>(n);
       int64_t *len = ar.take<int64_t>(n + 1);
       int *flags = ar.take<int>(2);  // any big row, any row unlike its link count
-      FFHIP_CHECK(hipMemsetAsync(bcnt, 0, 4 * n, s));
-      FFHIP_CHECK(hipMemsetAsync(len + n, 0, 8, s));
-      FFHIP_CHECK(hipMemsetAsync(flags, 0, 2 * sizeof(int), s));
+      clear(ctx, {{bcnt, 4 * (size_t)n}, {flags, 2 * sizeof(int)}});
       if (m->nbe)
         k_bcount<<<nblocks(m->nbe * m->nbloc, 256), 256, 0, s>>>(m->nbe * m->nbloc, m->belems, bcnt);
       k_link_len<<<nblocks(n, 256), 256, 0, s>>>(n, m->dim, m->v2e_ptr, bcnt, len);
@@ -1798,9 +1776,7 @@ ffhip_mat pattern_p1(ffhip_ctx ctx, ffhip_mesh m, const double *Ce, bool *values
       if (bucket) {  // the entry count and the bucket overflow flag in one wait
         int64_t nnz = 0;
         int of = 0;
-        FFHIP_CHECK(hipMemcpyAsync(&nnz, A->rowptr + n, sizeof(nnz), hipMemcpyDeviceToHost, s));
-        FFHIP_CHECK(hipMemcpyAsync(&of, ovf, sizeof(of), hipMemcpyDeviceToHost, s));
-        FFHIP_CHECK(hipStreamSynchronize(s));
+        fetch(ctx, {{&nnz, A->rowptr + n, sizeof(nnz)}, {&of, ovf, sizeof(of)}});
         A->nnz = nnz;
         if (of) {  // some list exceeds its bucket: the lists by the atomic fill
           dfree(bucket);
@@ -1826,8 +1802,7 @@ ffhip_mat pattern_p1(ffhip_ctx ctx, ffhip_mesh m, const double *Ce, bool *values
             n, m->elems, m->v2e_ptr, m->v2e, A->slotmap, A->big, flags, out);
       FFHIP_CHECK(hipGetLastError());
       int h[2] = {0, 0};
-      FFHIP_CHECK(hipMemcpyAsync(h, flags, sizeof(h), hipMemcpyDeviceToHost, s));
-      FFHIP_CHECK(hipStreamSynchronize(s));
+      fetch(ctx, {{h, flags, sizeof(h)}});
       direct_ok = !h[0] && !h[1];
       if (!direct_ok) { dfree(A->colidx); dfree(A->vals); }
       if (direct_ok) dfree(bucket);  // every list sorted by the pass
@@ -2099,21 +2074,16 @@ int ffhip_set_bc(ffhip_ctx ctx, ffhip_mesh m, ffhip_mat A, const int32_t *labels
     FFHIP_REQUIRE(tgv > 0, FFHIP_ERR_UNSUPPORTED, "ffhip_set_bc: only tgv > 0 is supported");
     hipStream_t s = ctx->stream;
     uint8_t *onbc = dalloc<uint8_t>(A->n);
-    int32_t *labs = dalloc<int32_t>(nlab > 0 ? nlab : 1);
-    int *missing = dalloc<int>(1);
-    if (nlab) FFHIP_CHECK(hipMemcpyAsync(labs, labels, 4 * nlab, hipMemcpyHostToDevice, s));
-    FFHIP_CHECK(hipMemsetAsync(onbc, 0, A->n, s));
-    FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), s));
+    const LabelArg labs(ctx, labels, nlab);
+    int *missing = ctx->flag(0);
     ctx->tic();
-    if (m->nbe)
-      k_mark_bc<<<nblocks(m->nbe, 256), 256, 0, s>>>(m->nbe, m->nbloc, m->belems, m->blab, labs,
-                                                     nlab, onbc);
+    mark_bc(ctx, m, labs.L, onbc);
     k_set_diag<<<nblocks(A->n, 256), 256, 0, s>>>(A->n, onbc, A->diag, tgv, A->vals, missing);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
     if (onbc_out) FFHIP_CHECK(hipMemcpy(onbc_out, onbc, A->n, hipMemcpyDeviceToHost));
-    const int miss = read_flag(ctx, missing);
-    dfree(onbc); dfree(labs); dfree(missing);
+    const int miss = *missing;
+    dfree(onbc);
     FFHIP_REQUIRE(miss == 0, FFHIP_ERR_INTERNAL, "ffhip_set_bc: a Dirichlet row has no diagonal");
   });
 }
@@ -2132,15 +2102,10 @@ int ffhip_rhs_p1_form(ffhip_ctx ctx, ffhip_mesh m, int kind, double f0, const do
     build_v2e(m);
     const int64_t n = m->nv;
     uint8_t *onbc = nullptr;
-    int32_t *labs = nullptr;
+    const LabelArg labs(ctx, labels, nlab > 0 ? nlab : 0);
     if (nlab > 0) {
       onbc = dalloc<uint8_t>(n);
-      labs = dalloc<int32_t>(nlab);
-      FFHIP_CHECK(hipMemcpyAsync(labs, labels, 4 * nlab, hipMemcpyHostToDevice, s));
-      FFHIP_CHECK(hipMemsetAsync(onbc, 0, n, s));
-      if (m->nbe)
-        k_mark_bc<<<nblocks(m->nbe, 256), 256, 0, s>>>(m->nbe, m->nbloc, m->belems, m->blab, labs,
-                                                       nlab, onbc);
+      mark_bc(ctx, m, labs.L, onbc);
     }
     double *bd = on_device ? b : dalloc<double>(n);
     const double *fd = fcoef, *gd = gvals;
@@ -2187,7 +2152,6 @@ int ffhip_rhs_p1_form(ffhip_ctx ctx, ffhip_mesh m, int kind, double f0, const do
     }
     FFHIP_CHECK(hipStreamSynchronize(s));
     dfree(onbc);
-    dfree(labs);
     dfree(fown);
     dfree(gown);
     dfree(E);
@@ -2207,7 +2171,6 @@ int ffhip_p1_misfit(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *
     FFHIP_REQUIRE(nlab >= 0 && (nlab == 0 || labels), FFHIP_ERR_ARG, "ffhip_p1_misfit: labels");
     build_v2e(m);
     MisfitBuffers b;
-    b.part = J ? dalloc<double>(kMisfitBlocks) : nullptr;
     if (r && nlab > 0) {
       b.onbc = dalloc<uint8_t>(m->nv);
       b.labs = dalloc<int32_t>(nlab);
@@ -2217,10 +2180,10 @@ int ffhip_p1_misfit(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *
       misfit_run(ctx, m, u, ud, labels, nlab, J, r, b);
     } catch (...) {
       (void)hipStreamSynchronize(ctx->stream);
-      dfree(b.part); dfree(b.onbc); dfree(b.labs); dfree(b.pair);
+      dfree(b.onbc); dfree(b.labs); dfree(b.pair);
       throw;
     }
-    dfree(b.part); dfree(b.onbc); dfree(b.labs); dfree(b.pair);
+    dfree(b.onbc); dfree(b.labs); dfree(b.pair);
   });
 }
 
@@ -2240,7 +2203,6 @@ int ffhip_p1_misfit_noalloc(ffhip_ctx ctx, ffhip_mesh m, const double *u, const 
                   "or ffhip_p1_misfit on this mesh builds it; this entry point allocates nothing)");
     unsigned char *base = noalloc_scratch(ctx->device);
     MisfitBuffers b;
-    b.part = reinterpret_cast<double *>(base + kScratchPartOff);
     b.labs = reinterpret_cast<int32_t *>(base + kScratchLabelsOff);
     b.onbc = base + kScratchOnbcOff;
     misfit_run(ctx, m, u, ud, labels, nlab, J, r, b);
@@ -2353,12 +2315,9 @@ int ffhip_spmv(ffhip_ctx ctx, ffhip_mat A, const double *x, double *y, int trans
       product(k_spmv_stage<kPlain, 16>, k_spmv_stage<kPlain, 64>, A->rowptr, A->colidx, nullptr);
       return;
     }
-    int *missing = dalloc<int>(1);
-    FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), s));
-    product(k_spmv_stage<kTrans, 16>, k_spmv_stage<kTrans, 64>, A->rowptr, A->colidx, missing);
-    const int miss = read_flag(ctx, missing);
-    dfree(missing);
-    FFHIP_REQUIRE(miss == 0, FFHIP_ERR_UNSUPPORTED, "ffhip_spmv: transpose needs a symmetric pattern");
+    const int *missing = ctx->flag(0);
+    product(k_spmv_stage<kTrans, 16>, k_spmv_stage<kTrans, 64>, A->rowptr, A->colidx, ctx->flag(0));
+    FFHIP_REQUIRE(*missing == 0, FFHIP_ERR_UNSUPPORTED, "ffhip_spmv: transpose needs a symmetric pattern");
   });
 }
 

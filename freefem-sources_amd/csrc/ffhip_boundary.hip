@@ -28,7 +28,6 @@
 
 namespace ffhip {
 
-int read_flag(ffhip_ctx ctx, int *d);
 
 namespace {
 
@@ -82,7 +81,7 @@ __device__ inline double coef_at(int kind, double c0, const double *__restrict__
 template <int NB, bool MAT>
 __global__ __launch_bounds__(256) void k_p1_boundary(
     int64_t n, const double *__restrict__ xyz, const int32_t *__restrict__ belems,
-    const int32_t *__restrict__ blab, const int32_t *__restrict__ labs, int nlab,
+    const int32_t *__restrict__ blab, Labels labels,
     const int64_t *__restrict__ bptr, const int32_t *__restrict__ blist, BndRule R, int kind,
     double c0, const double *__restrict__ coef, const int64_t *__restrict__ rowptr,
     const int32_t *__restrict__ colidx, double *__restrict__ vals, const uint8_t *__restrict__ skip,
@@ -98,10 +97,7 @@ __global__ __launch_bounds__(256) void k_p1_boundary(
     const int32_t item = blist[k];
     const int64_t e = item / NB;
     const int l = item - (int)e * NB;
-    bool on = false;
-    const int32_t lab = blab[e];
-    for (int i = 0; i < nlab; ++i) on |= lab == labs[i];
-    if (!on) continue;
+    if (!labels.has(blab[e])) continue;
     double B[NB][D];
     int32_t vid[NB];
 #pragma unroll
@@ -160,24 +156,13 @@ __global__ __launch_bounds__(256) void k_p1_boundary(
           if (colidx[mid] < vid[m]) lo = mid + 1; else hi = mid;
         }
         if (lo < r1 && colidx[lo] == vid[m]) vals[lo] += row[m];
-        else atomicOr(missing, 1);
+        else *missing = 1;
       }
     } else {
       bv += r;
     }
   }
   if (!MAT) b[v] = bv;
-}
-
-__global__ void k_mark_labels(int64_t nbe, int nbloc, const int32_t *__restrict__ belems,
-                              const int32_t *__restrict__ blab, const int32_t *__restrict__ labs,
-                              int nlab, uint8_t *__restrict__ onbc) {
-  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nbe) return;
-  bool on = false;
-  for (int k = 0; k < nlab; ++k) on |= blab[f] == labs[k];
-  if (!on) return;
-  for (int q = 0; q < nbloc; ++q) onbc[belems[nbloc * f + q]] = 1;  // same value from every writer
 }
 
 // vertex -> (boundary element * nbloc + local) lists, boundary-element order
@@ -223,24 +208,22 @@ int ffhip_assemble_p1_boundary(ffhip_ctx ctx, ffhip_mesh m, ffhip_mat A, const i
     build_b2v(m);
     double *owned;
     const double *cd = coef_device(m, kind, coef, on_device, &owned);
-    int32_t *labs = dalloc<int32_t>(nlab);
-    int *missing = dalloc<int>(1);
-    FFHIP_CHECK(hipMemcpyAsync(labs, labels, 4 * (size_t)nlab, hipMemcpyHostToDevice, s));
-    FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), s));
+    const LabelArg labs(ctx, labels, nlab);
+    int *missing = ctx->flag(0);
     const BndRule R = rule(m->dim);
     ctx->tic();
     if (m->dim == 3)
       k_p1_boundary<3, true><<<nblocks(m->nv, 256), 256, 0, s>>>(
-          m->nv, m->xyz, m->belems, m->blab, labs, nlab, m->b2e_ptr, m->b2e, R, kind, c0, cd,
+          m->nv, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, c0, cd,
           A->rowptr, A->colidx, A->vals, nullptr, nullptr, missing);
     else
       k_p1_boundary<2, true><<<nblocks(m->nv, 256), 256, 0, s>>>(
-          m->nv, m->xyz, m->belems, m->blab, labs, nlab, m->b2e_ptr, m->b2e, R, kind, c0, cd,
+          m->nv, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, c0, cd,
           A->rowptr, A->colidx, A->vals, nullptr, nullptr, missing);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
-    const int miss = read_flag(ctx, missing);
-    dfree(labs); dfree(missing); dfree(owned);
+    const int miss = *missing;
+    dfree(owned);
     FFHIP_REQUIRE(miss == 0, FFHIP_ERR_ARG,
                   "ffhip_assemble_p1_boundary: a boundary element is not a face of the mesh");
   });
@@ -261,16 +244,11 @@ int ffhip_rhs_p1_boundary(ffhip_ctx ctx, ffhip_mesh m, const int32_t *labels, in
     build_b2v(m);
     double *owned;
     const double *cd = coef_device(m, kind, coef, on_device, &owned);
-    int32_t *labs = dalloc<int32_t>(nlab + ndlab);
-    FFHIP_CHECK(hipMemcpyAsync(labs, labels, 4 * (size_t)nlab, hipMemcpyHostToDevice, s));
-    if (ndlab)
-      FFHIP_CHECK(hipMemcpyAsync(labs + nlab, dlabels, 4 * (size_t)ndlab, hipMemcpyHostToDevice, s));
+    const LabelArg labs(ctx, labels, nlab), dlabs(ctx, dlabels, ndlab);
     uint8_t *skip = nullptr;
     if (ndlab) {
       skip = dalloc<uint8_t>(n);
-      FFHIP_CHECK(hipMemsetAsync(skip, 0, n, s));
-      k_mark_labels<<<nblocks(m->nbe, 256), 256, 0, s>>>(m->nbe, m->nbloc, m->belems, m->blab,
-                                                         labs + nlab, ndlab, skip);
+      mark_bc(ctx, m, dlabs.L, skip);
     }
     double *bd = b;
     if (!on_device) {
@@ -281,11 +259,11 @@ int ffhip_rhs_p1_boundary(ffhip_ctx ctx, ffhip_mesh m, const int32_t *labels, in
     ctx->tic();
     if (m->dim == 3)
       k_p1_boundary<3, false><<<nblocks(n, 256), 256, 0, s>>>(
-          n, m->xyz, m->belems, m->blab, labs, nlab, m->b2e_ptr, m->b2e, R, kind, g0, cd, nullptr,
+          n, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, g0, cd, nullptr,
           nullptr, nullptr, skip, bd, nullptr);
     else
       k_p1_boundary<2, false><<<nblocks(n, 256), 256, 0, s>>>(
-          n, m->xyz, m->belems, m->blab, labs, nlab, m->b2e_ptr, m->b2e, R, kind, g0, cd, nullptr,
+          n, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, g0, cd, nullptr,
           nullptr, nullptr, skip, bd, nullptr);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
@@ -293,7 +271,7 @@ int ffhip_rhs_p1_boundary(ffhip_ctx ctx, ffhip_mesh m, const int32_t *labels, in
       FFHIP_CHECK(hipMemcpy(b, bd, 8 * n, hipMemcpyDeviceToHost));
       dfree(bd);
     }
-    dfree(labs); dfree(skip); dfree(owned);
+    dfree(skip); dfree(owned);
   });
 }
 

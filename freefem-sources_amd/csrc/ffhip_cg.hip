@@ -36,7 +36,6 @@
 
 namespace ffhip {
 void build_v2e(ffhip_mesh m);
-int read_flag(ffhip_ctx ctx, int *d);
 bool transpose_map(ffhip_ctx ctx, ffhip_mat A, int64_t *tmap);
 
 constexpr int kSlice = 64;
@@ -255,6 +254,7 @@ __global__ void k_sell_len(int64_t n, int64_t S, const int64_t *__restrict__ row
   }
   len[s] = (int32_t)m;
   cnt[s] = m * kSlice;
+  if (s == 0) cnt[S] = 0;  // the scan's last input
 }
 
 // vals_src may be permuted through tmap (transposed values)
@@ -359,6 +359,7 @@ __global__ __launch_bounds__(256) void k_sell_fill(
 __global__ void k_sell_len4(int64_t S, const int32_t *__restrict__ len, int64_t *__restrict__ cnt) {
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s < S) cnt[s] = (int64_t)((len[s] + 3) & ~3) * kSlice;
+  if (s == 0) cnt[S] = 0;
 }
 
 // node-row sort keys: window of 4096 rows in the high bits, longer rows first
@@ -388,6 +389,7 @@ __global__ void k_bsr_len(int64_t nb, int64_t S3, const int64_t *__restrict__ bp
   }
   len[s] = (int32_t)m;
   cnt[s] = m * kSlice;
+  if (s == 0) cnt[S3] = 0;
 }
 
 // 3x3 blocks of a vector-P2 matrix from its scalar CSR: entry k of sorted node
@@ -621,12 +623,12 @@ __global__ __launch_bounds__(kBlock) void k_tgv_reduce(int GB, const double *__r
 }
 
 // the layout sizes for the host (entries of the sliced layout and of the
-// packed deltas: the last slice offsets) and the far-column flag
+// packed deltas: the last slice offsets) and the far-column flag's start
 __global__ void k_setup_sizes(SetupRb *__restrict__ rb, const int64_t *__restrict__ ents,
-                              const int64_t *__restrict__ ents16, const int *__restrict__ far) {
+                              const int64_t *__restrict__ ents16, int far) {
   rb->ents = ents ? *ents : 0;
   rb->ents16 = ents16 ? *ents16 : 0;
-  rb->far = far ? *far : 1;
+  rb->far = far;
 }
 
 __global__ void k_jacobi(int64_t n, const double *__restrict__ d, const uint8_t *__restrict__ has,
@@ -1881,9 +1883,17 @@ __global__ __launch_bounds__(kBlock) void k_mix_update(
   if (threadIdx.x == 0) pout[xcd_block_id()] = tot;
 }
 
-// end of a chunk of CG launches: the next chunk starts `chunk` iterations on
-__global__ void k_cg_advance(CgState *st, int chunk) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->it0 += chunk;
+// end of a chunk of CG launches: the next chunk starts `chunk` iterations on;
+// the state goes to the host's copy
+__global__ void k_cg_advance(CgState *st, int chunk, CgState *host) {
+  if (threadIdx.x != 0) return;
+  st->it0 += chunk;
+  *host = *st;
+}
+// a small struct from the launch's arguments to the device
+template <class T>
+__global__ void k_put(T *dst, T v) {
+  *dst = v;
 }
 
 // fold the FP32 correction into the FP64 solution: x += D^-1/2 (sigma y32); y32 = 0
@@ -1980,7 +1990,7 @@ struct ffhip_cg_s {
   double *xw = nullptr, *bw = nullptr, *G = nullptr, *CG = nullptr, *H[2] = {nullptr, nullptr},
          *AH = nullptr;
   float *r32 = nullptr, *p32[2] = {nullptr, nullptr}, *q32 = nullptr, *y32 = nullptr;
-  double *pA = nullptr, *pB = nullptr, *pC = nullptr;
+  double *pA = nullptr, *pB = nullptr;
   CgState *st = nullptr;
   MixState *ms = nullptr;
   Cg2State *st2 = nullptr;  // affine CG (LinearCG)
@@ -2087,6 +2097,8 @@ struct ffhip_cg_s {
       t_dv += d; t_mv += a; t_up += b; ++n_timed;
     }
   }
+  // the state as the host reads it after a chunk (k_cg_advance writes it)
+  CgState *host_state() const { return static_cast<CgState *>(ctx->pinned_data()); }
   // bytes of the matrix that one mat-vec streams, with values of `size` bytes
   int64_t matrix_bytes(size_t size) const {
     if (fmt == kBsr3) return ents * (int64_t)(9 * size + 4);
@@ -2138,8 +2150,7 @@ struct ffhip_cg_s {
 // the tgv figures into the solver
 static SetupRb setup_readback(ffhip_cg cg) {
   SetupRb h;
-  FFHIP_CHECK(hipMemcpyAsync(&h, cg->rb, sizeof(h), hipMemcpyDeviceToHost, cg->ctx->stream));
-  FFHIP_CHECK(hipStreamSynchronize(cg->ctx->stream));
+  fetch(cg->ctx, {{&h, cg->rb, sizeof(h)}});
   cg->tgvm = h.ttgv;
   cg->ntgv = (int)h.ntgv;
   return h;
@@ -2171,10 +2182,9 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
     cg->sptr = dalloc<int64_t>(S3 + 1);
     cg->slen = dalloc<int32_t>(S3);
     int64_t *cnt = dalloc<int64_t>(S3 + 1);
-    FFHIP_CHECK(hipMemsetAsync(cnt + S3, 0, 8, s));
     k_bsr_len<<<nblk(S3, 256), 256, 0, s>>>(nb, S3, A->nodeptr, cg->bperm, cg->slen, cnt);
     exclusive_scan_i64(ctx, cnt, cg->sptr, S3 + 1);
-    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + S3, nullptr, nullptr);
+    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + S3, nullptr, 1);
     cg->ents = setup_readback(cg).ents;
     dfree(cnt); dfree(tmp); dfree(keys); dfree(skeys); dfree(vals);
     cg->bcol = dalloc<int32_t>(cg->ents);
@@ -2184,23 +2194,19 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
     // slice widths and offsets and the offsets of the packed 16-bit deltas,
     // then one read-back decides among sliced ELL with 16-bit deltas (the fill
     // then checks them), with int32 columns, and CSR
-    Arena ar(ctx, 3 * Arena::bytes(cg->S + 1, 8) + Arena::bytes(1, 4));
+    Arena ar(ctx, 2 * Arena::bytes(cg->S + 1, 8));
     cg->sptr = dalloc<int64_t>(cg->S + 1);
     cg->slen = dalloc<int32_t>(cg->S);
     cg->sptr16 = dalloc<int64_t>(cg->S + 1);
     int64_t *cnt = ar.take<int64_t>(cg->S + 1);
     int64_t *cnt4 = ar.take<int64_t>(cg->S + 1);
-    int *fard = ar.take<int>(1);
-    FFHIP_CHECK(hipMemsetAsync(cnt + cg->S, 0, 8, s));
-    FFHIP_CHECK(hipMemsetAsync(cnt4 + cg->S, 0, 8, s));
-    FFHIP_CHECK(hipMemsetAsync(fard, 0, sizeof(int), s));
     k_sell_len<<<nblk(cg->S, 256), 256, 0, s>>>(A->n, cg->S, A->rowptr, cg->slen, cnt);
     exclusive_scan_i64(ctx, cnt, cg->sptr, cg->S + 1);
     // 16-bit column deltas unless index32: the fill checks every delta
     // against 2^15 and falls back to int32 columns (far_pending)
     k_sell_len4<<<nblk(cg->S, 256), 256, 0, s>>>(cg->S, cg->slen, cnt4);
     exclusive_scan_i64(ctx, cnt4, cg->sptr16, cg->S + 1);
-    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + cg->S, cg->sptr16 + cg->S, index32 ? nullptr : fard);
+    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + cg->S, cg->sptr16 + cg->S, index32);
     FFHIP_CHECK(hipGetLastError());
     const SetupRb h = setup_readback(cg);
     cg->ents = h.ents;
@@ -2315,8 +2321,8 @@ static void cg_fill_values(ffhip_cg cg, bool transposed, const DiagBufs *db = nu
   }
   FFHIP_CHECK(hipGetLastError());
   SetupRb h{};
-  if (read_rb || check_far) FFHIP_CHECK(hipMemcpyAsync(&h, cg->rb, sizeof(h), hipMemcpyDeviceToHost, s));
-  FFHIP_CHECK(hipStreamSynchronize(s));
+  if (read_rb || check_far) fetch(ctx, {{&h, cg->rb, sizeof(h)}});
+  else FFHIP_CHECK(hipStreamSynchronize(s));
   if (read_rb) {
     cg->tgvm = h.ttgv;
     cg->ntgv = (int)h.ntgv;
@@ -2365,10 +2371,10 @@ static void cg_jacobi_tail(ffhip_cg cg, const DiagBufs &b) {
 static void residual_sums(ffhip_cg cg, const double *val, const double *x, const double *b,
                           double *rout, double out[3]) {
   hipStream_t s = cg->ctx->stream;
-  FFHIP_LAUNCH_FMT(cg, k_residual, cg->grid, s, cg->fmt_of(val), x, b, cg->dinv, rout, cg->pC);
+  FFHIP_REQUIRE(24 * (size_t)cg->grid <= ffhip_ctx_s::kPinnedData, FFHIP_ERR_INTERNAL, "residual partials");
+  double *h = static_cast<double *>(cg->ctx->pinned_data());
+  FFHIP_LAUNCH_FMT(cg, k_residual, cg->grid, s, cg->fmt_of(val), x, b, cg->dinv, rout, h);
   FFHIP_CHECK(hipGetLastError());
-  std::vector<double> h(3 * (size_t)cg->grid);
-  FFHIP_CHECK(hipMemcpyAsync(h.data(), cg->pC, 24 * cg->grid, hipMemcpyDeviceToHost, s));
   FFHIP_CHECK(hipStreamSynchronize(s));
   out[0] = out[1] = out[2] = 0.;
   for (int i = 0; i < cg->grid; ++i)
@@ -2398,7 +2404,7 @@ static void launch_pcg_chunk(ffhip_cg cg, const double *sval, bool marks) {
     k_pcg_update<<<G, kBlock, 0, s>>>(cg->n, cg->AH, cg->dinv, cg->G, cg->pB, cg->pA, cg->st);
     if (marks) cg->mark(4 * c + 3);
   }
-  k_cg_advance<<<1, 64, 0, s>>>(cg->st, kChunk);
+  k_cg_advance<<<1, 64, 0, s>>>(cg->st, kChunk, cg->host_state());
 }
 
 // One chunk of MIXED inner iterations it0 + c, par = it0 & 1.
@@ -2418,7 +2424,7 @@ static void launch_mix_chunk(ffhip_cg cg, const float *sval32, int par, bool mar
                                       cg->st, cg->ms);
     if (marks) cg->mark(4 * c + 3);
   }
-  k_cg_advance<<<1, 64, 0, s>>>(cg->st, kChunk);
+  k_cg_advance<<<1, 64, 0, s>>>(cg->st, kChunk, cg->host_state());
 }
 
 static hipGraphExec_t pcg_chunk_graph(ffhip_cg cg, const double *sval) {
@@ -2437,9 +2443,7 @@ int ffhip_cg_solve_mixed(ffhip_cg cg, const double *sval, const float *sval32, d
   const int G = cg->grid;
   const int chunk = kChunk;
   hipGraphExec_t gx[2] = {mix_chunk_graph(cg, sval32, 0), mix_chunk_graph(cg, sval32, 1)};
-  FFHIP_CHECK(hipMemsetAsync(cg->p32[0], 0, 4 * n, s));
-  FFHIP_CHECK(hipMemsetAsync(cg->p32[1], 0, 4 * n, s));
-  FFHIP_CHECK(hipMemsetAsync(cg->y32, 0, 4 * n, s));
+  clear(ctx, {{cg->p32[0], 4 * (size_t)n}, {cg->p32[1], 4 * (size_t)n}, {cg->y32, 4 * (size_t)n}});
   memset(&hs, 0, sizeof(hs));
   MixState hm;
   memset(&hm, 0, sizeof(hm));
@@ -2463,8 +2467,8 @@ int ffhip_cg_solve_mixed(ffhip_cg cg, const double *sval, const float *sval32, d
     hs.it0 = it;
     hs.itmax = itmax;
     hs.eps = eps;
-    FFHIP_CHECK(hipMemcpyAsync(cg->st, &hs, sizeof(hs), hipMemcpyHostToDevice, s));
-    FFHIP_CHECK(hipMemcpyAsync(cg->ms, &hm, sizeof(hm), hipMemcpyHostToDevice, s));
+    k_put<<<1, 1, 0, s>>>(cg->st, hs);
+    k_put<<<1, 1, 0, s>>>(cg->ms, hm);
     cg->ensure_events(4 * chunk);
     const int par = it & 1;
     for (;;) {
@@ -2473,8 +2477,8 @@ int ffhip_cg_solve_mixed(ffhip_cg cg, const double *sval, const float *sval32, d
       else launch_mix_chunk(cg, sval32, par, cg->profile != 0);
       it += chunk;
       FFHIP_CHECK(hipGetLastError());
-      FFHIP_CHECK(hipMemcpyAsync(&hs, cg->st, sizeof(hs), hipMemcpyDeviceToHost, s));
       FFHIP_CHECK(hipStreamSynchronize(s));
+      hs = *cg->host_state();
       cg->collect(it0, chunk, hs.iters);
       if (hs.done || hs.need_update) break;
     }
@@ -2550,8 +2554,8 @@ static void pcg_solve_small(ffhip_cg cg, const double *b, double *x, int on_devi
     bd = cg->bw;
     xd = cg->xw;
   }
-  static_assert(sizeof(SmallOut) <= ffhip_ctx_s::kPinned, "page-locked read-back");
-  SmallOut *out = static_cast<SmallOut *>(ctx->pinned);
+  static_assert(sizeof(SmallOut) <= ffhip_ctx_s::kPinnedData, "page-locked read-back");
+  SmallOut *out = static_cast<SmallOut *>(ctx->pinned_data());
   memset(out, 0, sizeof(*out));
   const int G = cg->grid;
   ctx->tic();
@@ -2583,7 +2587,7 @@ static void cg_release(ffhip_cg cg) {
   dfree(cg->sval32); dfree(cg->sval32T); dfree(cg->dinv); dfree(cg->dsc); dfree(cg->wcl);
   dfree(cg->xw); dfree(cg->bw); dfree(cg->G); dfree(cg->CG); dfree(cg->H[0]); dfree(cg->H[1]);
   dfree(cg->AH); dfree(cg->r32); dfree(cg->q32); dfree(cg->y32); dfree(cg->p32[0]);
-  dfree(cg->p32[1]); dfree(cg->pA); dfree(cg->pB); dfree(cg->pC); dfree(cg->st); dfree(cg->ms);
+  dfree(cg->p32[1]); dfree(cg->pA); dfree(cg->pB); dfree(cg->st); dfree(cg->ms);
   dfree(cg->st2);
   for (double *&p : cg->gmV) dfree(p);
   for (double *&p : cg->gmVp) dfree(p);
@@ -2621,7 +2625,7 @@ int ffhip_cg_create(ffhip_ctx ctx, ffhip_mat A, int mode, ffhip_cg *out) {
         cg_plan_layout(cg, layout, index32);  // reads the tgv figures back with its sizes
         cg_fill_values(cg, false);
       } else {  // FP64: the Jacobi set-up after the layout, from the fill's diagonal on sliced ELL
-        FFHIP_CHECK(hipMemsetAsync(cg->rb, 0, sizeof(SetupRb), ctx->stream));
+        clear(ctx, {{cg->rb, sizeof(SetupRb)}});
         cg_plan_layout(cg, layout, index32);
         Arena ar(ctx, DiagBufs::bytes(n));
         const DiagBufs b(ar, n);
@@ -2642,7 +2646,6 @@ int ffhip_cg_create(ffhip_ctx ctx, ffhip_mat A, int mode, ffhip_cg *out) {
       }
       cg->pA = dalloc<double>(3 * (int64_t)cg->grid);
       cg->pB = dalloc<double>(3 * (int64_t)cg->grid);
-      cg->pC = dalloc<double>(3 * (int64_t)cg->grid);
       cg->st = dalloc<CgState>(1);
       cg->ms = dalloc<MixState>(1);
       cg->st2 = dalloc<Cg2State>(1);
@@ -2710,7 +2713,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
       hs.it0 = 1;
       hs.itmax = itmax;
       hs.eps = eps;
-      FFHIP_CHECK(hipMemcpyAsync(cg->st, &hs, sizeof(hs), hipMemcpyHostToDevice, s));
+      k_put<<<1, 1, 0, s>>>(cg->st, hs);
       FFHIP_LAUNCH_FMT(cg, k_pcg_init, G, s, M, cg->xw, cg->bw, cg->dinv, cg->G, cg->CG, cg->H[0],
                        cg->pA, cg->st);
       FFHIP_CHECK(hipGetLastError());
@@ -2719,8 +2722,8 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
         if (gx) FFHIP_CHECK(hipGraphLaunch(gx, s));
         else launch_pcg_chunk(cg, sval, cg->profile != 0);
         FFHIP_CHECK(hipGetLastError());
-        FFHIP_CHECK(hipMemcpyAsync(&hs, cg->st, sizeof(hs), hipMemcpyDeviceToHost, s));
         FFHIP_CHECK(hipStreamSynchronize(s));
+        hs = *cg->host_state();
         cg->collect(it, chunk, hs.done ? hs.iters : it + chunk - 1);
         if (hs.done) break;
       }
@@ -2767,8 +2770,7 @@ int ffhip_cg_solve_affine(ffhip_cg cg, const double *b, double *x, int on_device
                                         cg->pA, cg->st2);
       if ((it + 1) % chunk == 0) {
         FFHIP_CHECK(hipGetLastError());
-        FFHIP_CHECK(hipMemcpyAsync(&hs, cg->st2, sizeof(hs), hipMemcpyDeviceToHost, s));
-        FFHIP_CHECK(hipStreamSynchronize(s));
+        fetch(ctx, {{&hs, cg->st2, sizeof(hs)}});
         if (hs.done) break;
       }
     }

@@ -36,11 +36,77 @@ void exclusive_scan_i64(ffhip_ctx ctx, const int64_t *in, int64_t *out,
                                                ctx->stream));
 }
 
+struct FetchArgs {
+  const uint32_t *src[4];
+  int end[4];  // words up to and with this source
+};
+__global__ __launch_bounds__(64) void k_fetch(FetchArgs a, uint32_t *__restrict__ dst) {
+  const int i = threadIdx.x;
+  int k = 0, base = 0;
+  while (k < 4 && i >= a.end[k]) base = a.end[k++];
+  if (k < 4) dst[i] = a.src[k][i - base];
+}
+void fetch(ffhip_ctx ctx, std::initializer_list<Fetch> list) {
+  FetchArgs a{};
+  int k = 0, words = 0;
+  for (const Fetch &f : list) {
+    a.src[k] = static_cast<const uint32_t *>(f.src);
+    a.end[k++] = words += f.bytes / 4;
+  }
+  FFHIP_REQUIRE(list.size() <= 4 && words <= 64, FFHIP_ERR_INTERNAL, "fetch: %d words", words);
+  for (; k < 4; ++k) a.end[k] = words;
+  k_fetch<<<1, 64, 0, ctx->stream>>>(a, static_cast<uint32_t *>(ctx->pinned_data()));
+  FFHIP_CHECK(hipGetLastError());
+  FFHIP_CHECK(hipStreamSynchronize(ctx->stream));
+  const char *p = static_cast<const char *>(ctx->pinned_data());
+  for (const Fetch &f : list) {
+    memcpy(f.dst, p, f.bytes);
+    p += f.bytes;
+  }
+}
 int64_t read_i64(ffhip_ctx ctx, const int64_t *p) {
   int64_t v = 0;
-  FFHIP_CHECK(hipMemcpyAsync(&v, p, sizeof(v), hipMemcpyDeviceToHost, ctx->stream));
-  FFHIP_CHECK(hipStreamSynchronize(ctx->stream));
+  fetch(ctx, {{&v, p, sizeof(v)}});
   return v;
+}
+int read_flag(ffhip_ctx ctx, const int *p) {
+  int v = 0;
+  fetch(ctx, {{&v, p, sizeof(v)}});
+  return v;
+}
+
+struct ClearArgs {
+  char *p[4];
+  size_t bytes[4];
+  int64_t end[4];  // 16-byte units up to and with this buffer
+};
+__global__ __launch_bounds__(256) void k_clear(ClearArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int k = 0;
+  int64_t base = 0;
+  while (k < 4 && i >= a.end[k]) base = a.end[k++];
+  if (k == 4) return;
+  const size_t o = 16 * (size_t)(i - base);
+  if (o + 16 <= a.bytes[k]) {
+    *reinterpret_cast<uint4 *>(a.p[k] + o) = make_uint4(0, 0, 0, 0);
+  } else {
+    for (size_t b = o; b < a.bytes[k]; ++b) a.p[k][b] = 0;
+  }
+}
+void clear(ffhip_ctx ctx, std::initializer_list<Clear> list) {
+  ClearArgs a{};
+  int k = 0;
+  int64_t units = 0;
+  for (const Clear &c : list) {
+    FFHIP_REQUIRE(k < 4 && (uintptr_t)c.p % 16 == 0, FFHIP_ERR_INTERNAL, "clear: buffers");
+    a.p[k] = static_cast<char *>(c.p);
+    a.bytes[k] = c.bytes;
+    a.end[k++] = units += (int64_t)((c.bytes + 15) / 16);
+  }
+  for (; k < 4; ++k) a.end[k] = units;
+  if (!units) return;
+  k_clear<<<(unsigned)((units + 255) / 256), 256, 0, ctx->stream>>>(a);
+  FFHIP_CHECK(hipGetLastError());
 }
 
 // ---------------------------------------------------------------- cube
@@ -339,7 +405,7 @@ int ffhip_init(int device, ffhip_ctx *out) {
     FFHIP_CHECK(hipStreamCreate(&c->stream));
     FFHIP_CHECK(hipEventCreate(&c->ev0));
     FFHIP_CHECK(hipEventCreate(&c->ev1));
-    FFHIP_CHECK(hipHostMalloc(&c->pinned, ffhip_ctx_s::kPinned, hipHostMallocDefault));
+    FFHIP_CHECK(hipHostMalloc(&c->pinned, ffhip_ctx_s::kPinnedFlags + ffhip_ctx_s::kPinnedData, hipHostMallocDefault));
     hipDeviceProp_t prop;
     FFHIP_CHECK(hipGetDeviceProperties(&prop, device));
     c->num_cu = prop.multiProcessorCount;

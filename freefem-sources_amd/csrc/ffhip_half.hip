@@ -24,7 +24,6 @@
 
 namespace ffhip {
 
-int read_flag(ffhip_ctx ctx, int *d);
 
 namespace {
 

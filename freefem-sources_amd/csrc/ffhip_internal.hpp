@@ -9,6 +9,8 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
+#include <initializer_list>
 #include <string>
 
 #include "../../include/ffhip.h"
@@ -92,10 +94,18 @@ struct ffhip_ctx_s {
   void *work = nullptr;
   size_t work_bytes = 0;
   void *ensure_work(size_t bytes);
-  // page-locked host memory that kernels write small results to (read after the
-  // call's wait; one call at a time per context)
-  static constexpr size_t kPinned = 4096;
+  // page-locked host memory that kernels write small results to, read after the
+  // call's wait (a context serves one call at a time): 16 flags, then data.  A
+  // read-back this way is a launch and a wait; a copy to pageable memory cost
+  // about 15 us more.
+  static constexpr size_t kPinnedFlags = 64, kPinnedData = 65536;
   void *pinned = nullptr;
+  int *flag(int i) {  // cleared flag i: kernels store 1 (plain stores: no atomics on host memory)
+    int *p = static_cast<int *>(pinned) + i;
+    *p = 0;
+    return p;
+  }
+  void *pinned_data() { return static_cast<char *>(pinned) + kPinnedFlags; }
   double last_ms = 0.;  // device time of the last timed call
   void tic();           // record ev0 on the stream
   void toc();           // record ev1, synchronise, set last_ms
@@ -281,6 +291,59 @@ struct Arena {
   }
 };
 int64_t read_i64(ffhip_ctx ctx, const int64_t *p);
+int read_flag(ffhip_ctx ctx, const int *p);
+// Small device values to the host: one launch that writes them to page-locked
+// memory, then a wait for the stream (bytes: multiples of 4, 256 at most in all).
+struct Fetch {
+  void *dst;
+  const void *src;
+  unsigned bytes;
+};
+void fetch(ffhip_ctx ctx, std::initializer_list<Fetch> list);
+// Clears up to 4 buffers in one launch (16-byte aligned; a memset each was a
+// launch each).
+struct Clear {
+  void *p;
+  size_t bytes;
+};
+void clear(ffhip_ctx ctx, std::initializer_list<Clear> list);
+
+// Boundary labels as a kernel takes them: up to kNear by value (no copy to the
+// device), more in an array that lives as long as the LabelArg.
+struct Labels {
+  static constexpr int kNear = 16;
+  int n;
+  int32_t near_[kNear];
+  const int32_t *far;
+  __device__ bool has(int32_t lab) const {
+    bool on = false;
+    for (int k = 0; k < n; ++k) on |= lab == (far ? far[k] : near_[k]);
+    return on;
+  }
+};
+struct LabelArg {
+  Labels L{};
+  int32_t *own = nullptr;
+  // buf: device room for the labels (else allocated where needed)
+  LabelArg(ffhip_ctx ctx, const int32_t *labels, int nlab, int32_t *buf = nullptr) {
+    L.n = nlab;
+    if (nlab <= Labels::kNear) {
+      for (int k = 0; k < nlab; ++k) L.near_[k] = labels[k];
+      return;
+    }
+    if (!buf) buf = own = dalloc<int32_t>(nlab);
+    L.far = buf;
+    if (hipError_t e = hipMemcpyAsync(buf, labels, 4 * (size_t)nlab, hipMemcpyHostToDevice, ctx->stream)) {
+      dfree(own);
+      FFHIP_CHECK(e);
+    }
+  }
+  LabelArg(const LabelArg &) = delete;
+  LabelArg &operator=(const LabelArg &) = delete;
+  ~LabelArg() { dfree(own); }
+};
+// the vertices of the boundary elements with these labels
+void mark_bc(ffhip_ctx ctx, ffhip_mesh m, const Labels &labels, uint8_t *onbc);
 
 // the per-device address of the no-allocation entry points' scratch array
 // (ffhip_assembly.hip); set up by ffhip_init with the device current

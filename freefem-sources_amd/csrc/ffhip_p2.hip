@@ -39,7 +39,6 @@
 namespace ffhip {
 void set_diag_rows(ffhip_ctx ctx, int64_t n, const uint8_t *onbc, const int64_t *diag, double tgv,
                    double *vals, int *missing);
-int read_flag(ffhip_ctx ctx, int *d);
 
 // Tet::nvedge (local vertex pairs of the 6 edges)
 static __constant__ int c_edge[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
@@ -88,6 +87,7 @@ __global__ void k_p2_edge_heads(int64_t E, const uint64_t *__restrict__ skeys,
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= E) return;
   const int64_t h = (p == 0 || skeys[p] != skeys[p - 1]) ? 1 : 0;
+  if (p == 0) head[E] = mark[E / 6 * 10] = 0;  // the scans' last inputs
   head[p] = h;
   mark[sitems[p]] = h;
 }
@@ -627,23 +627,20 @@ __device__ inline int32_t find_edge_node(const uint64_t *__restrict__ ekeys,
 // dofs of the labelled boundary triangles: 3 vertex nodes and 3 edge nodes,
 // all components
 __global__ void k_p2v_mark_bc(int64_t nbe, const int32_t *__restrict__ btri,
-                              const int32_t *__restrict__ blab, const int32_t *__restrict__ labs,
-                              int nlab, const int32_t *__restrict__ vnode,
+                              const int32_t *__restrict__ blab, Labels labels,
+                              const int32_t *__restrict__ vnode,
                               const uint64_t *__restrict__ ekeys, const int32_t *__restrict__ enode,
                               int64_t ne, int ncomp, uint8_t *__restrict__ onbc,
                               int *__restrict__ missing) {
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nbe) return;
-  int on = 0;
-  for (int q = 0; q < nlab; ++q) on |= blab[f] == labs[q];
-  if (!on) return;
+  if (f >= nbe || !labels.has(blab[f])) return;
   const int32_t *t = btri + 3 * f;
   int32_t nodes[6] = {vnode[t[0]], vnode[t[1]], vnode[t[2]],
                       find_edge_node(ekeys, enode, ne, edge_key(t[0], t[1])),
                       find_edge_node(ekeys, enode, ne, edge_key(t[1], t[2])),
                       find_edge_node(ekeys, enode, ne, edge_key(t[0], t[2]))};
   for (int i = 0; i < 6; ++i) {
-    if (nodes[i] < 0) { atomicMax(missing, 1); continue; }
+    if (nodes[i] < 0) { *missing = 1; continue; }
     for (int c = 0; c < ncomp; ++c) onbc[ncomp * (int64_t)nodes[i] + c] = 1;
   }
 }
@@ -727,25 +724,17 @@ static void p2_rhs(ffhip_ctx ctx, ffhip_p2v sp, int ncomp, const double f[3], co
   ctx->toc();
 }
 
-// onbc (3 nnodes bytes) of the labelled boundary; false if a node was missing
-static bool p2v_mark(ffhip_ctx ctx, ffhip_p2v sp, const int32_t *labels, int nlab, int ncomp,
-                     uint8_t *onbc) {
-  hipStream_t s = ctx->stream;
+// onbc (ncomp nnodes bytes) of the labelled boundary; *missing (host, read
+// after the stream's wait) raised if a node was missing
+static void p2v_mark(ffhip_ctx ctx, ffhip_p2v sp, const Labels &labels, int ncomp, uint8_t *onbc,
+                     int *missing) {
   ffhip_mesh m = sp->mesh;
-  int32_t *labs = dalloc<int32_t>(nlab > 0 ? nlab : 1);
-  int *missing = dalloc<int>(1);
-  if (nlab) FFHIP_CHECK(hipMemcpyAsync(labs, labels, 4 * nlab, hipMemcpyHostToDevice, s));
-  FFHIP_CHECK(hipMemsetAsync(onbc, 0, ncomp * sp->nnodes, s));
-  FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), s));
+  clear(ctx, {{onbc, (size_t)(ncomp * sp->nnodes)}});
   if (m->nbe)
-    k_p2v_mark_bc<<<nblk(m->nbe, 256), 256, 0, s>>>(m->nbe, m->belems, m->blab, labs, nlab,
-                                                    sp->vnode, sp->ekeys, sp->enode, sp->ne, ncomp,
-                                                    onbc, missing);
+    k_p2v_mark_bc<<<nblk(m->nbe, 256), 256, 0, ctx->stream>>>(m->nbe, m->belems, m->blab, labels, sp->vnode,
+                                                              sp->ekeys, sp->enode, sp->ne, ncomp, onbc,
+                                                              missing);
   FFHIP_CHECK(hipGetLastError());
-  const int miss = read_flag(ctx, missing);
-  dfree(labs);
-  dfree(missing);
-  return miss == 0;
 }
 
 static void p2v_release(ffhip_p2v sp) {
@@ -792,19 +781,16 @@ int ffhip_p2v_create(ffhip_ctx ctx, ffhip_mesh m, ffhip_p2v *out) {
                                                      2 * vb, s));
       int64_t *head = ar.take<int64_t>(E + 1), *hscan = ar.take<int64_t>(E + 1);
       int64_t *mark = ar.take<int64_t>(NI + 1), *rank = ar.take<int64_t>(NI + 1);
-      FFHIP_CHECK(hipMemsetAsync(head + E, 0, 8, s));
-      FFHIP_CHECK(hipMemsetAsync(mark + NI, 0, 8, s));
       k_p2_edge_heads<<<nblk(E, 256), 256, 0, s>>>(E, skeys, sitems, head, mark);
       k_p2_vmark<<<nblk(4 * nt, 256), 256, 0, s>>>(nt, m->elems, firstv, mark);
       exclusive_scan_i64(ctx, head, hscan, E + 1);
-      sp->ne = read_i64(ctx, hscan + E);
+      exclusive_scan_i64(ctx, mark, rank, NI + 1);
+      fetch(ctx, {{&sp->ne, hscan + E, 8}, {&sp->nnodes, rank + NI, 8}});
       int32_t *item_seg = ar.take<int32_t>(E);
       int32_t *segfirst = ar.take<int32_t>(E);  // ne <= E
       sp->ekeys = dalloc<uint64_t>(sp->ne);
       k_p2_edge_seg<<<nblk(E, 256), 256, 0, s>>>(E, skeys, vb, sitems, hscan, head, item_seg, sp->ekeys,
                                                  segfirst);
-      exclusive_scan_i64(ctx, mark, rank, NI + 1);
-      sp->nnodes = read_i64(ctx, rank + NI);
       sp->elem_nodes = dalloc<int32_t>(NI);
       k_p2_assign<<<nblk(NI, 256), 256, 0, s>>>(nt, m->elems, firstv, item_seg, segfirst, rank,
                                                 sp->elem_nodes);
@@ -877,27 +863,29 @@ static void p2_pattern(ffhip_ctx ctx, ffhip_p2v sp, int ncomp, ffhip_mat *out) {
       int32_t *rowbuf = ar.take<int32_t>(kNodeCap * nn);
       int8_t *dposr = ar.take<int8_t>(nn);
       A->slot8 = dalloc<uint8_t>(m->nt * 100);
-      FFHIP_CHECK(hipMemsetAsync(len, 0, 8 * (nn + 1), s));
-      FFHIP_CHECK(hipMemsetAsync(ovf, 0, sizeof(int), s));
+      clear(ctx, {{len, 8 * (size_t)(nn + 1)}, {ovf, sizeof(int)}});
       // one wave per node row (hash set in LDS); the lane-per-row merge if a
       // row does not fit
       k_p2_pattern_wave<<<nblk(nn * kWave, 256), 256, 0, s>>>(nn, sp->elem_nodes, sp->n2e_ptr, sp->n2e,
                                                               len, rowbuf, dposr, A->slot8, ovf);
       FFHIP_CHECK(hipGetLastError());
-      const bool wave_ok = read_flag(ctx, ovf) == 0;
+      exclusive_scan_i64(ctx, len, A->nodeptr, nn + 1);
+      int over = 0;
+      int64_t nnz_nodes = 0;
+      fetch(ctx, {{&over, ovf, sizeof(over)}, {&nnz_nodes, A->nodeptr + nn, 8}});
+      const bool wave_ok = over == 0;
       constexpr int B = 128, CAP = kNodeCap;
       if (!wave_ok) {
-        FFHIP_CHECK(hipMemsetAsync(len, 0, 8 * (nn + 1), s));
-        FFHIP_CHECK(hipMemsetAsync(ovf, 0, sizeof(int), s));
+        clear(ctx, {{len, 8 * (size_t)(nn + 1)}, {ovf, sizeof(int)}});
         k_pattern_rows<B, CAP, false><<<nblk(nn, B), B, 0, s>>>(
             nn, 10, sp->elem_nodes, sp->n2e_ptr, sp->n2e, len, nullptr, nullptr, nullptr, nullptr,
             nullptr, ovf);
         FFHIP_CHECK(hipGetLastError());
         FFHIP_REQUIRE(read_flag(ctx, ovf) == 0, FFHIP_ERR_UNSUPPORTED,
                       "ffhip_pattern_p2v: a node couples to more than %d nodes", CAP);
+        exclusive_scan_i64(ctx, len, A->nodeptr, nn + 1);
+        nnz_nodes = read_i64(ctx, A->nodeptr + nn);
       }
-      exclusive_scan_i64(ctx, len, A->nodeptr, nn + 1);
-      const int64_t nnz_nodes = read_i64(ctx, A->nodeptr + nn);
       int32_t *ncol = nullptr;
       if (!wave_ok) {
         ncol = rowbuf;  // the row buffers are free: nnz_nodes <= kNodeCap * nn
@@ -978,25 +966,25 @@ int ffhip_set_bc_p2v(ffhip_ctx ctx, ffhip_p2v sp, ffhip_mat A, const int32_t *la
     FFHIP_REQUIRE(nlab >= 0 && (nlab == 0 || labels), FFHIP_ERR_ARG, "ffhip_set_bc_p2v: labels");
     FFHIP_REQUIRE(tgv > 0, FFHIP_ERR_UNSUPPORTED, "ffhip_set_bc_p2v: only tgv > 0 is supported");
     uint8_t *onbc = dalloc<uint8_t>(A->n);
-    int *missing = dalloc<int>(1);
-    bool ok = false;
-    int miss = 0;
+    const LabelArg labs(ctx, labels, nlab);
+    const int *unknown = ctx->flag(0), *missing = ctx->flag(1);
     try {
       ctx->tic();
-      ok = p2v_mark(ctx, sp, labels, nlab, 3, onbc);
-      FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), ctx->stream));
-      set_diag_rows(ctx, A->n, onbc, A->diag, tgv, A->vals, missing);
+      p2v_mark(ctx, sp, labs.L, 3, onbc, ctx->flag(0));
+      set_diag_rows(ctx, A->n, onbc, A->diag, tgv, A->vals, ctx->flag(1));
       ctx->toc();
       if (onbc_out) {
         FFHIP_CHECK(hipMemcpyAsync(onbc_out, onbc, A->n, hipMemcpyDeviceToHost, ctx->stream));
+        FFHIP_CHECK(hipStreamSynchronize(ctx->stream));
       }
-      miss = read_flag(ctx, missing);
     } catch (...) {
       (void)hipStreamSynchronize(ctx->stream);
-      dfree(onbc); dfree(missing);
+      dfree(onbc);
       throw;
     }
-    dfree(onbc); dfree(missing);
+    const bool ok = !*unknown;
+    const int miss = *missing;
+    dfree(onbc);
     FFHIP_REQUIRE(ok, FFHIP_ERR_INTERNAL, "ffhip_set_bc_p2v: a boundary edge is no element edge");
     FFHIP_REQUIRE(miss == 0, FFHIP_ERR_INTERNAL, "ffhip_set_bc_p2v: a Dirichlet row has no diagonal");
   });
@@ -1013,9 +1001,10 @@ int ffhip_rhs_p2v(ffhip_ctx ctx, ffhip_p2v sp, const double f[3], const int32_t 
     const double *gg = g ? g : gz;
     uint8_t *onbc = dalloc<uint8_t>(n);
     double *bd = on_device ? b : nullptr;
-    bool ok = false;
+    const LabelArg labs(ctx, labels, nlab);
+    const int *unknown = ctx->flag(0);
     try {
-      ok = p2v_mark(ctx, sp, labels, nlab, 3, onbc);
+      p2v_mark(ctx, sp, labs.L, 3, onbc, ctx->flag(0));
       if (!on_device) bd = dalloc<double>(n);
       p2_rhs(ctx, sp, 3, f, onbc, tgv, gg, bd);
       if (!on_device) {
@@ -1030,7 +1019,7 @@ int ffhip_rhs_p2v(ffhip_ctx ctx, ffhip_p2v sp, const double f[3], const int32_t 
     }
     dfree(onbc);
     if (!on_device) dfree(bd);
-    FFHIP_REQUIRE(ok, FFHIP_ERR_INTERNAL, "ffhip_rhs_p2v: a boundary edge is no element edge");
+    FFHIP_REQUIRE(!*unknown, FFHIP_ERR_INTERNAL, "ffhip_rhs_p2v: a boundary edge is no element edge");
   });
 }
 
@@ -1073,24 +1062,25 @@ int ffhip_set_bc_p2(ffhip_ctx ctx, ffhip_p2v sp, ffhip_mat A, const int32_t *lab
     FFHIP_REQUIRE(nlab >= 0 && (nlab == 0 || labels), FFHIP_ERR_ARG, "ffhip_set_bc_p2: labels");
     FFHIP_REQUIRE(tgv > 0, FFHIP_ERR_UNSUPPORTED, "ffhip_set_bc_p2: only tgv > 0 is supported");
     uint8_t *onbc = dalloc<uint8_t>(A->n);
-    int *missing = dalloc<int>(1);
-    bool ok = false;
-    int miss = 0;
+    const LabelArg labs(ctx, labels, nlab);
+    const int *unknown = ctx->flag(0), *missing = ctx->flag(1);
     try {
       ctx->tic();
-      ok = p2v_mark(ctx, sp, labels, nlab, 1, onbc);
-      FFHIP_CHECK(hipMemsetAsync(missing, 0, sizeof(int), ctx->stream));
-      set_diag_rows(ctx, A->n, onbc, A->diag, tgv, A->vals, missing);
+      p2v_mark(ctx, sp, labs.L, 1, onbc, ctx->flag(0));
+      set_diag_rows(ctx, A->n, onbc, A->diag, tgv, A->vals, ctx->flag(1));
       ctx->toc();
-      if (onbc_out)
+      if (onbc_out) {
         FFHIP_CHECK(hipMemcpyAsync(onbc_out, onbc, A->n, hipMemcpyDeviceToHost, ctx->stream));
-      miss = read_flag(ctx, missing);
+        FFHIP_CHECK(hipStreamSynchronize(ctx->stream));
+      }
     } catch (...) {
       (void)hipStreamSynchronize(ctx->stream);
-      dfree(onbc); dfree(missing);
+      dfree(onbc);
       throw;
     }
-    dfree(onbc); dfree(missing);
+    const bool ok = !*unknown;
+    const int miss = *missing;
+    dfree(onbc);
     FFHIP_REQUIRE(ok, FFHIP_ERR_INTERNAL, "ffhip_set_bc_p2: a boundary edge is no element edge");
     FFHIP_REQUIRE(miss == 0, FFHIP_ERR_INTERNAL, "ffhip_set_bc_p2: a Dirichlet row has no diagonal");
   });
@@ -1105,9 +1095,10 @@ int ffhip_rhs_p2(ffhip_ctx ctx, ffhip_p2v sp, double f, const int32_t *labels, i
     const int64_t n = sp->nnodes;
     uint8_t *onbc = dalloc<uint8_t>(n);
     double *bd = on_device ? b : nullptr;
-    bool ok = false;
+    const LabelArg labs(ctx, labels, nlab);
+    const int *unknown = ctx->flag(0);
     try {
-      ok = p2v_mark(ctx, sp, labels, nlab, 1, onbc);
+      p2v_mark(ctx, sp, labs.L, 1, onbc, ctx->flag(0));
       if (!on_device) bd = dalloc<double>(n);
       const double fv[3] = {f, 0., 0.}, gv[3] = {g, 0., 0.};
       p2_rhs(ctx, sp, 1, fv, onbc, tgv, gv, bd);
@@ -1123,7 +1114,7 @@ int ffhip_rhs_p2(ffhip_ctx ctx, ffhip_p2v sp, double f, const int32_t *labels, i
     }
     dfree(onbc);
     if (!on_device) dfree(bd);
-    FFHIP_REQUIRE(ok, FFHIP_ERR_INTERNAL, "ffhip_rhs_p2: a boundary edge is no element edge");
+    FFHIP_REQUIRE(!*unknown, FFHIP_ERR_INTERNAL, "ffhip_rhs_p2: a boundary edge is no element edge");
   });
 }
 
