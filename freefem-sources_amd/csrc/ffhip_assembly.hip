@@ -232,19 +232,19 @@ __global__ void k_v2e_sort(int64_t n, const int64_t *__restrict__ ptr, int32_t *
 }
 
 // ---------------------------------------------------------------- pattern (half-wave rows)
-// One row per 32-lane half-wave: lane q loads incidence q's element vertices
-// (4 candidates per lane), inserts them into an open-addressing set in LDS
-// (atomicCAS; the lane that claims a slot appends the column), and the
-// unique columns are ordered by a counting sort (rank = number of smaller
-// columns).  One pass writes the row length, the sorted columns to a 64-entry
-// row buffer, the relative diagonal slot and the element-to-row map (each
-// candidate's offset by binary search in the sorted columns); after the scan,
-// k_pattern_compact moves the buffered columns to their CSR place.  Rows with
-// more than 32 incident elements or 64 columns are flagged in big[] for the
-// lane-per-row merge (k_pattern_rows).
+// One row per 32-lane half-wave: lane q loads incidence q's element vertices,
+// places those other than the row's own in an open-addressing set in LDS (all
+// of them step together: read, write where free, read back), the set is
+// compacted by ballots and the columns are ordered by a counting sort (rank =
+// number of smaller columns).  One pass writes the row length, the sorted
+// columns to a 64-entry row buffer, the relative diagonal slot and the
+// element-to-row map (each lane kept its columns' slots in the set, which get
+// their ranks); after the scan, k_pattern_compact moves the buffered columns to
+// their CSR place.  Rows with more than 32 incident elements or 64 columns are
+// flagged in big[] for the lane-per-row merge (k_pattern_rows).
 constexpr int kRowBuf = 64;
 
-constexpr int kHash = 128;  // LDS hash slots per row (a row has at most 1 + 3 * 32 columns)
+constexpr int kHash = 128;  // LDS hash slots per row (a row has at most 3 * 32 columns besides its own)
 
 // Where the pass writes a row it builds.  Buffered: the 64-entry row
 // buffers (rowbuf, rowval), the length and the diagonal offset, moved to CSR
@@ -271,25 +271,31 @@ struct PatternOut {
 // With bucket (the incidence lists unsorted, 32 entries per row, every list
 // within its bucket; VALS only): each lane ranks its incidence among the
 // row's and writes it to v2e at that rank, in place of k_v2e_sort_bucket.
+// Bound by its vector instructions (cube(160): 600 per wave, nine tenths of the
+// issue slots).  cube(160), 2.84 -> 2.27 ms: an atomic compare-and-swap per
+// candidate, an atomic count and a second search per column took 770; a third of
+// the rest is the values' geometry and sums.
 template <int NLOC, bool VALS, bool DIRECT>
 __global__ __launch_bounds__(256) void k_pattern_half(
     int64_t n, const int32_t *__restrict__ elems, const int64_t *__restrict__ v2e_ptr,
     int32_t *__restrict__ v2e, uint32_t *__restrict__ slotmap, uint8_t *__restrict__ big,
     int *__restrict__ any_big, PatternOut out, const double *__restrict__ xyz = nullptr,
     const double *__restrict__ Ce = nullptr, const int32_t *__restrict__ bucket = nullptr) {
-  constexpr int NH = 256 / kHalf;
+  constexpr int NH = 256 / kHalf, R = NLOC - 1, kFree = INT_MAX;
   // every LDS array below is per row (half-wave), so a wave orders its own
   // accesses (wave_lds_sync) and the waves of a block run independently
-  __shared__ int32_t hk[NH][kHash];      // open-addressing set of the row's columns
-  __shared__ uint8_t hslot[NH][kRowBuf];  // the set slot of each unique column
-  __shared__ uint8_t hrank[NH][kHash];    // the offset in the row of the column in each set slot
-  __shared__ int32_t ucol[NH][kRowBuf];  // unique columns, then sorted
-  __shared__ int32_t ucnt[NH];
-  __shared__ double sv[VALS ? NH : 1][VALS ? 4 * kHalf : 1];   // incidence rows (VALS)
-  __shared__ __align__(16) uint32_t so[VALS ? NH : 1][VALS ? kHalf : 1];  // their slot bytes (VALS)
-  __shared__ __align__(16) double dq[VALS ? NH : 1][VALS ? kHalf : 1];    // their diagonal entries (VALS)
-  __shared__ uint32_t smask[VALS ? NH : 1][VALS ? kHalf : 1];  // per off-diagonal slot: its incidences (VALS)
+  __shared__ __align__(16) int32_t hk[NH][kHash];     // open-addressing set of the row's columns but its own
+  __shared__ uint8_t hrank[NH][kHash];                // the offset in the row of the column in each set slot
+  __shared__ __align__(16) int32_t ucol[NH][kRowBuf];  // the set's columns
+  __shared__ uint8_t uslot[NH][kRowBuf];              // and their slots
+  // VALS: incidence q's entries at [(column - own - 1) mod 4][q] ([3]: the diagonal),
+  // its slot bytes in that order (own first), and for every slot of the row and each
+  // of the three the incidences that hold it there
+  __shared__ __align__(16) double sv[VALS ? NH : 1][VALS ? 4 * kHalf : 1];
+  __shared__ __align__(16) uint32_t so[VALS ? NH : 1][VALS ? kHalf : 1];
+  __shared__ uint32_t smask[VALS ? NH : 1][VALS ? 3 : 1][VALS ? kHalf + 1 : 1];
   const int hl = threadIdx.x % kHalf, hid = threadIdx.x / kHalf;
+  const bool upper = threadIdx.x % kWave >= kHalf;
   const int64_t v = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kHalf;
   int64_t k0 = 0, p0 = 0, p1 = 0;
   int deg = 0;
@@ -300,14 +306,21 @@ __global__ __launch_bounds__(256) void k_pattern_half(
   }
   bool mine = v < n && deg <= kHalf;
   if (!mine) deg = 0;
-  for (int i = hl; i < kHash; i += kHalf) hk[hid][i] = INT_MAX;
-  if (hl == 0) ucnt[hid] = 0;
-  if constexpr (VALS) smask[hid][hl] = 0;
-  int32_t c[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX};
+  // this half's bits of a wave's ballot
+  const auto half = [&](bool x) {
+    const uint64_t w = __builtin_amdgcn_ballot_w64(x);
+    return upper ? (uint32_t)(w >> 32) : (uint32_t)w;
+  };
+  *reinterpret_cast<int4 *>(&hk[hid][4 * hl]) = make_int4(kFree, kFree, kFree, kFree);
+  *reinterpret_cast<int2 *>(&ucol[hid][2 * hl]) = make_int2(kFree, kFree);
+  if constexpr (VALS) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r) smask[hid][r][hl] = 0;
+  }
+  int32_t c[4] = {kFree, kFree, kFree, kFree};
   int64_t e = 0;
   int lv = 0;
-  double vv[VALS ? 4 : 1][3], Cv = 0.;
-  int32_t idx = INT_MAX;
+  int32_t idx = kFree;
   int qp = hl;  // the incidence's position in the row's list (element order)
   bool ranked = false;
   if constexpr (VALS) {
@@ -315,17 +328,20 @@ __global__ __launch_bounds__(256) void k_pattern_half(
       // unsorted bucket: each lane's rank among the row's entries (element
       // ids are distinct) places its incidence, and everything it stores
       // per incidence below, in element order
-      idx = hl < deg ? bucket[32 * v + hl] : INT_MAX;
+      idx = hl < deg ? bucket[32 * v + hl] : kFree;
       so[hid][hl] = (uint32_t)idx;
       wave_lds_sync();
       int rho = 0;
 #pragma unroll
       for (int g = 0; g < kHalf / 4; ++g) {
+        if (__builtin_amdgcn_ballot_w64(deg > 4 * g) == 0) break;
         const uint4 w = *reinterpret_cast<const uint4 *>(&so[hid][4 * g]);
         rho += ((int32_t)w.x < idx) + ((int32_t)w.y < idx) + ((int32_t)w.z < idx) + ((int32_t)w.w < idx);
       }
-      qp = rho;
-      if (hl < deg) v2e[k0 + qp] = idx;
+      if (hl < deg) {
+        qp = rho;
+        v2e[k0 + qp] = idx;
+      }
       ranked = true;
     }
   }
@@ -340,154 +356,189 @@ __global__ __launch_bounds__(256) void k_pattern_half(
 #pragma unroll
       for (int m = 0; m < NLOC; ++m) c[m] = elems[e * NLOC + m];
     }
-    if constexpr (VALS) {  // issued now, used after the set and sort phases (their latency hidden)
-#pragma unroll
-      for (int i = 0; i < (VALS ? 4 : 1); ++i)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) vv[i][k] = xyz[3 * (int64_t)c[i] + k];
-      Cv = Ce[e];
-    }
   }
-  wave_lds_sync();
-  // insert the candidates; the lane that claims a free slot appends the column.
-  // The row's own vertex is in every incident element: only lane 0 inserts it
-  // (a quarter fewer atomics; c[] keeps it for the element-to-row map below)
+  // the other vertices, from the one after the row's own on (cyclic)
+  int32_t key[R];
+  if (NLOC == 4) {
+    const int32_t b0 = lv & 1 ? c[1] : c[0], b1 = lv & 1 ? c[2] : c[1], b2 = lv & 1 ? c[3] : c[2],
+                  b3 = lv & 1 ? c[0] : c[3];
+    key[0] = lv & 2 ? b3 : b1;
+    key[1] = lv & 2 ? b0 : b2;
+    key[R - 1] = lv & 2 ? b1 : b3;
+  } else {
+    key[0] = lv == 0 ? c[1] : lv == 1 ? c[2] : c[0];
+    key[1] = lv == 0 ? c[2] : lv == 1 ? c[0] : c[1];
+  }
+  // Equal keys are at the same slot in every step: a slot that was free is
+  // written by all of them, and they all see it taken by theirs or by another.
+  // Ends: the set holds at most 96 columns of its 128 slots.
+  uint32_t slot[R];
+  bool open[R];  // still looking (a repeated own vertex is no other column)
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    if (c[r] == INT_MAX || (c[r] == (int32_t)v && hl != 0)) continue;
-    uint32_t h = ((uint32_t)c[r] * 2654435761u) >> (32 - 7);
-    for (;;) {  // ends: the set holds at most 97 columns of its 128 slots
-      const int32_t old = atomicCAS(&hk[hid][h], INT_MAX, c[r]);
-      if (old == INT_MAX) {
-        const int idx = atomicAdd(&ucnt[hid], 1);
-        if (idx < kRowBuf) { ucol[hid][idx] = c[r]; hslot[hid][idx] = (uint8_t)h; }
-        break;
+  for (int r = 0; r < R; ++r) {
+    slot[r] = ((uint32_t)__umul24((uint32_t)key[r], 0x9e3779u) >> 17) % kHash;
+    open[r] = key[r] != kFree && key[r] != (int32_t)v;
+  }
+  const auto at = [&](int r) -> int32_t & { return hk[hid][slot[r]]; };
+  for (;;) {
+    int32_t was[R], is[R];
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < R; ++r) was[r] = __hip_atomic_load(&at(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (open[r] && was[r] == kFree)
+        __hip_atomic_store(&at(r), key[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    wave_lds_sync();
+    bool more = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) is[r] = __hip_atomic_load(&at(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      open[r] = open[r] && is[r] != key[r];
+      if (open[r]) slot[r] = (slot[r] + 1) % kHash;
+      more |= open[r];
+    }
+    if (__builtin_amdgcn_ballot_w64(more) == 0) break;
+  }
+  // compaction: lane hl's four slots
+  int nset = 0;  // columns in the set
+  {
+    const int4 w = *reinterpret_cast<const int4 *>(&hk[hid][4 * hl]);
+    const int32_t k4[4] = {w.x, w.y, w.z, w.w};
+    const uint32_t below = (1u << hl) - 1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bool full = k4[j] != kFree;
+      const uint32_t mk = half(full);
+      const int at_ = nset + __builtin_popcount(mk & below);
+      if (full && at_ < kRowBuf) {
+        ucol[hid][at_] = k4[j];
+        uslot[hid][at_] = (uint8_t)(4 * hl + j);
       }
-      if (old == c[r]) break;
-      h = (h + 1) & (kHash - 1);
+      nset += __builtin_popcount(mk);
     }
   }
   wave_lds_sync();
-  const int len = ucnt[hid];
+  const int len = nset + (deg > 0);  // and the row's own column
   if (len > kRowBuf) mine = false;
-  const int64_t r0 = p0;
-  const bool wrong = DIRECT && mine && p1 - p0 != len;  // the row's length is not its pointers' 
+  const bool wrong = DIRECT && mine && p1 - p0 != len;  // the row's length is not its pointers'
+  const bool write = mine && !wrong;
   // counting sort: the rank of a column is the number of smaller columns
-  int32_t u[2] = {INT_MAX, INT_MAX};
-  int rk[2] = {0, 0};
-  if (mine) {
+  int dpos = 0;
 #pragma unroll
-    for (int h2 = 0; h2 < 2; ++h2) {
-      const int j = hl + h2 * kHalf;
-      if (j < len) {
-        u[h2] = ucol[hid][j];
-        int r = 0;
-        for (int i = 0; i < len; ++i) r += ucol[hid][i] < u[h2] ? 1 : 0;
-        rk[h2] = r;
-      }
+  for (int h2 = 0; h2 < 2; ++h2) {
+    const int j = hl + h2 * kHalf;
+    if (h2 == 1 && __builtin_amdgcn_ballot_w64(mine && nset > kHalf) == 0) break;
+    const bool on = mine && j < nset;
+    const int32_t u = on ? ucol[hid][j] : kFree;
+    const bool less = u < (int32_t)v;  // before the row's own column
+    int rk = less ? 0 : 1;
+    for (int g = 0; __builtin_amdgcn_ballot_w64(on && 4 * g < nset); ++g) {  // past nset: kFree
+      const int4 w = *reinterpret_cast<const int4 *>(&ucol[hid][(4 * g) % kRowBuf]);
+      rk += (w.x < u) + (w.y < u) + (w.z < u) + (w.w < u);
     }
-  }
-  wave_lds_sync();
-  int dpos = -1;
-  if (mine) {
-#pragma unroll
-    for (int h2 = 0; h2 < 2; ++h2)
-      if (hl + h2 * kHalf < len) {
-        hrank[hid][hslot[hid][hl + h2 * kHalf]] = (uint8_t)rk[h2];
-        ucol[hid][rk[h2]] = u[h2];
-        if (!DIRECT) out.rowbuf[kRowBuf * v + rk[h2]] = u[h2];
-        else if (!wrong) out.colidx[r0 + rk[h2]] = u[h2];
-        if ((int64_t)u[h2] == v) dpos = rk[h2];
-      }
-  }
-#pragma unroll
-  for (int off = 1; off < kHalf; off <<= 1) {
-    const int t = __shfl_xor(dpos, off, kWave);
-    dpos = t > dpos ? t : dpos;
+    dpos += __builtin_popcount(half(on && less));
+    if (on) {
+      hrank[hid][uslot[hid][j]] = (uint8_t)rk;
+      if (!DIRECT) out.rowbuf[kRowBuf * v + rk] = u;
+      else if (write) out.colidx[p0 + rk] = u;
+    }
   }
   wave_lds_sync();
   if (v < n && hl == 0) {
     big[v] = mine ? 0 : 1;
     if (!mine) atomicOr(any_big, 1);
     if (DIRECT && wrong) atomicOr(out.mismatch, 1);
-    if (mine && !DIRECT) { out.rowlen[v] = len; out.dposr[v] = (int8_t)dpos; }
-    if (mine && DIRECT && !wrong) out.diag[v] = dpos < 0 ? -1 : r0 + dpos;
+    if (mine && len) {
+      if (!DIRECT) out.rowbuf[kRowBuf * v + dpos] = (int32_t)v;
+      else if (write) out.colidx[p0 + dpos] = (int32_t)v;
+    }
+    if (mine && !DIRECT) { out.rowlen[v] = len; out.dposr[v] = (int8_t)(len ? dpos : -1); }
+    if (write && DIRECT) out.diag[v] = len ? p0 + dpos : -1;
   }
   if (mine && hl < deg) {
-    uint32_t pk = 0;
+    uint32_t pk = (uint32_t)dpos, rank[R];  // own first
 #pragma unroll
-    for (int m = 0; m < NLOC; ++m) {
-      // the column is in the set: its slot holds its offset in the row
-      uint32_t h = ((uint32_t)c[m] * 2654435761u) >> (32 - 7);
-      while (hk[hid][h] != c[m]) h = (h + 1) & (kHash - 1);
-      pk |= (uint32_t)hrank[hid][h] << (8 * m);
+    for (int r = 0; r < R; ++r) {
+      rank[r] = key[r] == (int32_t)v ? dpos : hrank[hid][slot[r]];
+      pk |= rank[r] << (8 * r + 8);
     }
-    slotmap[k0 + qp] = pk;
+    if (NLOC == 4) slotmap[k0 + qp] = __builtin_rotateleft32(pk, 8 * lv);
+    else
+      slotmap[k0 + qp] = lv == 0 ? pk : lv == 1 ? (pk << 8 & 0xffff00u) | pk >> 16
+                                                : (pk << 16 & 0xff0000u) | pk >> 8;
     if constexpr (VALS) {
-      double r[4];
-      p1_row_entries(vv, lv, Cv, r);
+      // the vertices are read here, not with the element: the registers that they
+      // held through the passes above left 6 waves per SIMD instead of 8
+      double vv[4][3], r4[4];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        sv[hid][4 * qp + m] = r[m];
-        const uint32_t slot = (pk >> (8 * m)) & 0xffu;
-        if (m != lv && slot < kHalf) atomicOr(&smask[hid][slot], 1u << qp);
-      }
-      dq[hid][qp] = r[lv];
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) vv[m][k] = xyz[3 * (int64_t)c[m] + k];
+      p1_row_entries(vv, lv, Ce[e], r4);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) sv[hid][((m - lv - 1) & 3) * kHalf + qp] = r4[m];
+#pragma unroll
+      for (int r = 0; r < 3; ++r)  // slots past 32 to the word that nobody reads
+        atomicOr(&smask[hid][r][min(rank[r < R ? r : 0], (uint32_t)kHalf)], 1u << qp);
       so[hid][qp] = pk;
     }
   }
   if constexpr (VALS) {  // the row's values, each slot summed by its lane in element order
-    wave_lds_sync();
     const int nq = mine ? deg : 0;
-    const uint32_t me0 = (uint32_t)hl * 0x01010101u, me1 = (uint32_t)(hl + kHalf) * 0x01010101u;
+    if (hl >= nq) sv[hid][3 * kHalf + hl] = 0.;
+    wave_lds_sync();
     double acc0 = 0., acc1 = 0.;
     // Every incidence holds the diagonal slot: its lane adds the incidences'
-    // diagonal entries in order, 8 per round (reads before adds; past the
-    // row's count +0.0, which leaves the sum unchanged: it starts at +0.0
-    // and is never -0.0).  Another slot's lane adds the entries of the
-    // incidences in its mask (bit q: incidence q holds the slot), lowest
-    // first, 4 per round.  Both orders are the element order.
+    // diagonal entries in order, 8 per round (past the row's count +0.0, which
+    // leaves the sum unchanged: it starts at +0.0 and is never -0.0).  Another
+    // slot's lane adds the entries of the incidences in its masks (bit q:
+    // incidence q holds the slot), lowest first, 3 per round.  Both orders are
+    // the element order.
     if (hl == dpos) {
       for (int q0 = 0; q0 < nq; q0 += 8) {
         double a[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) a[i] = dq[hid][q0 + i];
+        for (int i = 0; i < 8; ++i) a[i] = sv[hid][3 * kHalf + q0 + i];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc0 += q0 + i < nq ? a[i] : 0.;
+        for (int i = 0; i < 8; ++i) acc0 += a[i];
       }
-    } else if (hl < len) {
-      uint32_t mask = mine ? smask[hid][hl] : 0u;
+    } else if (mine && hl < len) {
+      const uint32_t m1 = smask[hid][1][hl], m2 = smask[hid][2][hl];
+      uint32_t mask = smask[hid][0][hl] | m1 | m2;
       while (mask) {
-        int q[4];
-        bool ok[4];
+        constexpr int U = 3;
+        double a[U];
+        bool ok[U];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < U; ++i) {
           ok[i] = mask != 0;
-          q[i] = ok[i] ? __builtin_ctz(mask) : 0;
+          const int q = (__ffs(mask) - 1) & (kHalf - 1);
+          const int r = (int)(m1 >> q & 1) + 2 * (int)(m2 >> q & 1);
+          a[i] = sv[hid][r * kHalf + q];
           mask &= mask - 1;
         }
-        double a[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t t0 = so[hid][q[i]] ^ me0, z0 = (t0 - 0x01010101u) & ~t0 & 0x80808080u;
-          a[i] = sv[hid][4 * q[i] + (z0 ? __builtin_ctz(z0) >> 3 : 0)];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc0 += ok[i] ? a[i] : 0.;
+        for (int i = 0; i < U; ++i) acc0 += ok[i] ? a[i] : 0.;
       }
     }
-    if (len > kHalf)  // rows of more than 32 columns: the second slot of each lane
-      for (int q = 0; q < nq; ++q) {
-        const uint32_t t1 = so[hid][q] ^ me1, z1 = (t1 - 0x01010101u) & ~t1 & 0x80808080u;
-        if (z1) acc1 += sv[hid][4 * q + (__builtin_ctz(z1) >> 3)];
-      }
+    if (__builtin_amdgcn_ballot_w64(mine && len > kHalf)) {  // rows of more than 32 columns: the second slot of each lane
+      const uint32_t me1 = (uint32_t)(hl + kHalf) * 0x01010101u;
+      if (len > kHalf)
+        for (int q = 0; q < nq; ++q) {
+          const uint32_t t1 = so[hid][q] ^ me1, z1 = (t1 - 0x01010101u) & ~t1 & 0x80808080u;
+          if (z1) acc1 += sv[hid][(((__builtin_ctz(z1) >> 3) - 1) & 3) * kHalf + q];
+        }
+    }
     if (mine && !DIRECT) {
       if (hl < len) out.rowval[kRowBuf * v + hl] = acc0;
       if (hl + kHalf < len) out.rowval[kRowBuf * v + hl + kHalf] = acc1;
     }
-    if (mine && DIRECT && !wrong) {
-      if (hl < len) out.vals[r0 + hl] = acc0;
-      if (hl + kHalf < len) out.vals[r0 + hl + kHalf] = acc1;
+    if (write && DIRECT) {
+      if (hl < len) out.vals[p0 + hl] = acc0;
+      if (hl + kHalf < len) out.vals[p0 + hl + kHalf] = acc1;
     }
   }
 }
@@ -576,7 +627,7 @@ __device__ inline double p1_kappa_integral(int64_t e, const int32_t id[4], const
     for (int q = 0; q < 14; ++q)
       S += (mes * qf5_weight(q)) * p1_value3(u, c_qf5_pts[q][0], c_qf5_pts[q][1], c_qf5_pts[q][2]);
   } else if (kind == FFHIP_COEF_SIN3) {
-#pragma unroll 2
+#pragma unroll 1
     for (int q = 0; q < 14; ++q) {
       const double px = c_qf5_pts[q][0], py = c_qf5_pts[q][1], pz = c_qf5_pts[q][2];
       const double l0 = 1. - (px + py + pz);
@@ -900,7 +951,8 @@ __global__ __launch_bounds__(256) void k_p1_scale_3d(int64_t nt, const double *_
 // block's global count atomics are issued before the tet's scale is
 // computed (their round trip hidden by the arithmetic), and the items are
 // placed after it.  The scale is the same computation as k_p1_scale_3d's.
-// (5 waves per SIMD: 86 VGPRs, no spills; uncapped it takes 108 and runs 4)
+// (5 waves per SIMD, no spills; uncapped it takes 108 registers and runs 4.  One
+// point of the rule at a time: cube(160) 1256 -> 1150 us, two at a time 1210)
 constexpr int kFuseLog = 11;
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 5))) void k_v2e_bucket_scale(const int32_t *__restrict__ tets, int64_t nt,
                                                           ScaleArgs sc, uint32_t *__restrict__ deg,

@@ -115,16 +115,16 @@ __device__ inline double tet_mesure(const double v[4][3]) {
   return det3_pivot(AB, AC, AD) / 6.;
 }
 
-// sin(2 pi x): t = 2x = k + r with k = rint(t) and |r| <= 1/2 (exact), then
-// sin(pi r) from its Taylor series truncated after r^21 (coefficients
-// (-1)^j pi^(2j+1) / (2j+1)!, Horner in r^2; truncation below 3e-16 on
-// |r| <= 1/2) and the sign (-1)^k.  About 16 FP64 operations, a third of a
-// general sinpi with its quadrant branches: the 42 evaluations per tet are
-// most of the element kernel's work.
+// sin(2 pi x): u = x - rint(x) and b = min(|u|, 1/2 - |u|), both exact, then
+// sin(pi r), r = 2b <= 1/2, from its Taylor series truncated after r^21
+// (coefficients (-1)^j pi^(2j+1) / (2j+1)!, Horner in r^2; truncation below
+// 3e-16) with u's sign.  17 FP64 operations, a third of a general sinpi with its
+// quadrant branches: the 42 evaluations per tet are most of the element kernel's
+// work.  (The sign from the parity of rint(2x) took a conversion to 64-bit
+// integers, 9 more operations.)
 __device__ inline double sin2pi(double x) {
-  const double t = 2. * x;
-  const double k = rint(t);
-  const double r = t - k;
+  const double u = x - rint(x), a = fabs(u), b = fmin(a, 0.5 - a);
+  const double r = b + b;
   const double s = r * r;
   double p = 5.39266466260812848935e-10;
   p = fma(p, s, -2.29484289972698731102e-8);
@@ -137,8 +137,7 @@ __device__ inline double sin2pi(double x) {
   p = fma(p, s, 2.55016403987734544386);
   p = fma(p, s, -5.16771278004997002925);
   p = fma(p, s, 3.14159265358979323846);
-  const double y = r * p;
-  return ((int64_t)k & 1) ? -y : y;
+  return copysign(r * p, u);
 }
 
 // kappa = 1+0.5*sin(2*pi*x)*sin(2*pi*y)*sin(2*pi*z), the script's product
