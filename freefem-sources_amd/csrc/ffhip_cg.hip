@@ -1120,6 +1120,256 @@ __global__ FFHIP_MATVEC_ATTR void k_pcg_matvec(MatFmt<double> M, const double *_
   if (threadIdx.x == 0) pout[2 * xcd_block_id()] = a;  // (g, h) comes from the direction kernel
 }
 
+// ---------------------------------------------------------------- symmetric values
+// K2 over half of the values.  The mat-vec is bound by the bytes of the matrix,
+// 10 per entry.  Where A is symmetric (bit for bit) and its rows follow few
+// patterns (the rows of a box: the same column distances inside, others at its
+// faces), a row needs its entries from the diagonal on from memory and no
+// index: the entries before it are those of the rows above, read a short while
+// ago, and a byte names the row's pattern.  65 bytes a row for 147 (P1 on a
+// cube).  The same entries in the same order: the bits of k_pcg_matvec.
+//
+// us per mat-vec, half against whole: cube(64) 8.9 / 10.9, cube(96) 18.8 / 24.6,
+// cube(112) 26.2 / 39.0, cube(128) 38.1 / 70.9, cube(160) 96 / 137 (366 MB from
+// HBM; the vector kernels lose 18 us there, their vectors in the Infinity Cache
+// no more).  Not faster at cube(160): non-temporal loads of the values (111), of
+// some of the planes (98 to 103), the next slice's values loaded ahead (102), 3
+// blocks per CU (102), slices in columns that keep a plane's values in the L2
+// (98: a fifth fewer misses).
+//
+// Up to 8 entries before the diagonal and NU from it on, NU 4 or 8:
+// [slice][entry from the diagonal on][64 rows].
+constexpr int kSymHalf = 8, kSymSlots = 256, kSymMax = 192;  // patterns: slots of the table, most taken
+constexpr uint16_t kSymNone = 0xffffu;
+struct SymPattern {
+  uint16_t off[kSymHalf];   // entry i before the diagonal: its owner's entry, in bytes; kSymNone: none
+  int16_t d[2 * kSymHalf];  // column distances before the diagonal, from it on (0: none)
+};
+struct SymFmt {
+  int64_t n, S;
+  const double *val;
+  const uint8_t *cls;
+  const SymPattern *table;
+};
+
+template <int NL, int NU>
+__global__ FFHIP_MATVEC_ATTR void k_pcg_matvec_sym(SymFmt M, const double *__restrict__ H,
+                                                   double *__restrict__ AH, double *__restrict__ pout,
+                                                   CgState *st) {
+  __shared__ double lds[kBlock / kWave];
+  __shared__ __align__(16) SymPattern tab[kSymSlots];
+  if (st->stop) {  // the direction kernel stopped the solve: publish it
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->done = st->stop;
+    return;
+  }
+  if (st->done) return;
+  for (int i = threadIdx.x; i < (int)(sizeof(tab) / 16); i += kBlock)
+    reinterpret_cast<u32x4 *>(tab)[i] = reinterpret_cast<const u32x4 *>(M.table)[i];
+  __syncthreads();
+  const auto hr = slice_rsrc(H, (uint32_t)(M.n * 8));
+  const auto vr = slice_rsrc(M.val, (uint32_t)(M.S * (NU * kSlice * 8)));
+  // a load past the values' end gives 0
+  const auto val = [&](uint32_t o, uint32_t plane) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(vr, o, plane, 0));
+  };
+  // byte offset of row r's diagonal
+  const auto at = [](uint32_t r) { return r * 8u + (r / kSlice) * ((NU - 1) * kSlice * 8u); };
+  double p_hah = 0.;
+  int64_t s, s1, ds;
+  wave_slices<kCyclicSell>(M.S, s, s1, ds);
+  const int lane = threadIdx.x % kSlice;
+  for (; s < s1; s += ds) {
+    const int64_t r = s * kSlice + lane;
+    const uint32_t rc = (uint32_t)(r < M.n ? r : M.n - 1);  // past n: the last row's sum, not stored
+    const int c = M.cls[rc];
+    const uint32_t own = at(rc);
+    double u[NU];
+#pragma unroll
+    for (int k = 0; k < NU; ++k) u[k] = val(own, k * (kSlice * 8));
+    const u32x4 *t = reinterpret_cast<const u32x4 *>(&tab[c]);
+    const u32x4 w = t[0], e0 = t[1], e1 = t[2];
+    const uint32_t oo[4] = {w.x, w.y, w.z, w.w};
+    const uint32_t dd[8] = {e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w};
+    const auto off = [&](int k) { return k & 1 ? oo[k >> 1] >> 16 : oo[k >> 1] & 0xffffu; };
+    const auto col = [&](int k) {
+      return rc + (uint32_t)(k & 1 ? (int32_t)dd[k >> 1] >> 16 : (int32_t)(int16_t)dd[k >> 1]);
+    };
+    const auto xof = [&](int k) {
+      return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(hr, col(k) * 8u, 0, 0));
+    };
+    double a[NL], xl[NL], xu[NU];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) a[k] = val(off(k) == kSymNone ? 0xffffffffu : off(k) + at(col(k)), 0);
+#pragma unroll
+    for (int k = 0; k < NL; ++k) xl[k] = xof(k);
+#pragma unroll
+    for (int k = 0; k < NU; ++k) xu[k] = xof(kSymHalf + k);
+    const double h = H[rc];
+    double acc = 0.;
+#pragma unroll
+    for (int k = 0; k < NL; ++k) acc += a[k] * xl[k];
+#pragma unroll
+    for (int k = 0; k < NU; ++k) acc += u[k] * xu[k];
+    if (r < M.n) AH[r] = acc;
+    p_hah += (r < M.n ? h : 0.) * acc;
+  }
+  const double tot = block_sum<kBlock>(p_hah, lds);
+  if (threadIdx.x == 0) pout[2 * xcd_block_id()] = tot;
+}
+
+// A row of the kSell16 layout as the pattern search sees it: its distances as
+// stored (4 packed groups: rows of up to 16 entries), the counts before the
+// diagonal and from it on.
+struct SymRow {
+  u32x2 pk[4];
+  int nl, nu, L;
+  __device__ int32_t delta(int k) const {
+    const uint32_t w = k & 2 ? pk[k >> 2].y : pk[k >> 2].x;
+    return k & 1 ? (int32_t)w >> 16 : (int32_t)(int16_t)w;
+  }
+};
+__device__ inline SymRow sym_row(const MatFmt<double> &M, int64_t r) {
+  SymRow R;
+  const int64_t s = r / kSlice;
+  const int lane = (int)(r % kSlice);
+  R.L = M.len[s];
+  const int64_t cb = M.ptr16[s];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    R.pk[g] = u32x2{0u, 0u};
+    if (4 * g < R.L) R.pk[g] = *reinterpret_cast<const u32x2 *>(M.col16 + cb + ((int64_t)g * kSlice + lane) * 4);
+  }
+  R.nl = R.nu = 0;
+  bool past = false;  // the diagonal or a column after it was seen: distance 0 is padding
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int32_t d = R.delta(k);
+    R.nl += d < 0;
+    R.nu += d > 0 || (d == 0 && !past && k < R.L);
+    past |= d >= 0;
+  }
+  return R;
+}
+// the positions, from the diagonal on, that row r's entries before the diagonal
+// have in the rows of their columns (4 bits each); *ok: all there, with the same value
+__device__ inline uint32_t sym_owners(const MatFmt<double> &M, int64_t r, const SymRow &R, bool &ok) {
+  const int64_t vb = M.ptr[r / kSlice];
+  uint32_t pw = 0;
+#pragma unroll 1
+  for (int k = 0; k < R.nl; ++k) {
+    const u32x2 g = k < 4 ? R.pk[0] : R.pk[1];  // nl <= 8
+    const uint32_t w = k & 2 ? g.y : g.x;
+    const int32_t d = k & 1 ? (int32_t)w >> 16 : (int32_t)(int16_t)w;
+    const int64_t j = r + d;
+    const SymRow J = sym_row(M, j);
+    int kj = -1;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) kj = J.delta(q) == -d ? q : kj;
+    if (kj < 0 || J.L > 16 || kj - J.nl >= kSymHalf) { ok = false; return 0; }
+    const double mine = M.val[vb + pair_pos(R.L, k, (int)(r % kSlice))];
+    const double theirs = M.val[M.ptr[j / kSlice] + pair_pos(J.L, kj, (int)(j % kSlice))];
+    if (__builtin_bit_cast(uint64_t, mine) != __builtin_bit_cast(uint64_t, theirs)) { ok = false; return 0; }
+    pw |= (uint32_t)(kj - J.nl) << (4 * k);
+  }
+  return pw;
+}
+struct SymTables {
+  unsigned long long key[kSymSlots];  // hash of the pattern, 0: free
+  int64_t rep[kSymSlots];             // a row of the pattern
+  SymRow row[kSymSlots];
+  uint32_t owners[kSymSlots];
+  int bad, count, nl, nu;  // some row does not fit; patterns; most entries before a diagonal, from it on
+};
+// every row's slot in the table of patterns.  Once a row fails (or the table
+// fills, as on an unstructured mesh within its first blocks) the rest is left.
+__global__ __launch_bounds__(256) void k_sym_rows(MatFmt<double> M, SymTables *T, uint8_t *__restrict__ cls,
+                                                  uint32_t *__restrict__ owners) {
+  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (r >= M.n || __hip_atomic_load(&T->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  const SymRow R = sym_row(M, r);
+  bool ok = R.L <= 16 && R.nl <= kSymHalf && R.nu <= kSymHalf;
+  const uint32_t pw = ok ? sym_owners(M, r, R, ok) : 0;
+  if (ok) {
+    unsigned long long h = 0x9e3779b97f4a7c15ull ^ ((unsigned long long)pw << 16 | R.nl << 8 | R.nu);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      h = (h ^ ((unsigned long long)R.pk[g].y << 32 | R.pk[g].x)) * 0xbf58476d1ce4e5b9ull;
+      h ^= h >> 29;
+    }
+    h |= 1;
+    ok = false;
+    for (int p = 0; p < 16 && !ok; ++p) {
+      const int t = (int)(((h >> 8) + p) & (kSymSlots - 1));
+      unsigned long long k = __hip_atomic_load(&T->key[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (k == 0) {
+        k = atomicCAS(&T->key[t], 0ull, h);
+        if (k == 0) {
+          T->rep[t] = r;
+          if (atomicAdd(&T->count, 1) >= kSymMax) break;
+          k = h;
+        }
+      }
+      if (k == h) {
+        cls[r] = (uint8_t)t;
+        owners[r] = pw;
+        ok = true;
+      }
+    }
+  }
+  if (!ok) atomicOr(&T->bad, 1);
+}
+// the patterns from their rows
+__global__ __launch_bounds__(kSymSlots) void k_sym_table(MatFmt<double> M, SymTables *T,
+                                                         const uint32_t *__restrict__ owners,
+                                                         SymPattern *__restrict__ table) {
+  const int t = threadIdx.x;
+  SymPattern P;
+  for (int k = 0; k < kSymHalf; ++k) {
+    P.off[k] = kSymNone;
+    P.d[k] = P.d[kSymHalf + k] = 0;
+  }
+  if (T->key[t] && !T->bad) {
+    const int64_t r = T->rep[t];
+    const SymRow R = sym_row(M, r);
+    const uint32_t pw = owners[r];
+    T->row[t] = R;
+    T->owners[t] = pw;
+    atomicMax(&T->nl, R.nl);
+    atomicMax(&T->nu, R.nu);
+    for (int k = 0; k < 16; ++k) {
+      const int32_t d = R.delta(k);
+      if (k < R.nl) {
+        P.d[k] = (int16_t)d;
+        P.off[k] = (uint16_t)((pw >> (4 * k) & 15u) * (kSlice * 8u));
+      } else if (k - R.nl < R.nu) {
+        P.d[kSymHalf + k - R.nl] = (int16_t)d;
+      }
+    }
+  }
+  table[t] = P;
+}
+// the values from the diagonal on; every row compared with its pattern's
+__global__ __launch_bounds__(256) void k_sym_fill(MatFmt<double> M, SymTables *T, const uint8_t *__restrict__ cls,
+                                                  const uint32_t *__restrict__ owners, int NU,
+                                                  double *__restrict__ val) {
+  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (r >= M.n || __hip_atomic_load(&T->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  const SymRow R = sym_row(M, r);
+  const int t = cls[r];
+  const SymRow &Q = T->row[t];
+  bool same = owners[r] == T->owners[t] && R.nl == Q.nl && R.nu == Q.nu;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) same &= R.pk[g].x == Q.pk[g].x && R.pk[g].y == Q.pk[g].y;
+  if (!same) {  // a hash met twice
+    atomicOr(&T->bad, 1);
+    return;
+  }
+  const int64_t vb = M.ptr[r / kSlice];
+  for (int p = 0; p < NU; ++p)
+    val[(r / kSlice * NU + p) * kSlice + r % kSlice] =
+        p < R.nu ? M.val[vb + pair_pos(R.L, R.nl + p, (int)(r % kSlice))] : 0.;
+}
+
 __global__ __launch_bounds__(kBlock) void k_pcg_update(
     int64_t n, const double *__restrict__ AH, const double *__restrict__ dinv,
     double *__restrict__ G, const double *__restrict__ pin, double *__restrict__ pout, CgState *st) {
@@ -2060,6 +2310,12 @@ struct ffhip_cg_s {
   };
   std::vector<Chunk> graphs;
   int use_graph = 1;
+  // symmetric values of an FP64 kSell16 solver (k_pcg_matvec_sym): 0 not looked
+  // for since the values changed, 1 there, -1 the matrix has not that form
+  int sym = 0, sym_nl = 0, sym_nu = 0;
+  double *symval = nullptr;
+  uint8_t *symcls = nullptr;
+  SymPattern *symtab = nullptr;
   template <class F>
   hipGraphExec_t graph(int kind, const void *val, int par, F launch) {
     if (!use_graph || profile) return nullptr;
@@ -2390,7 +2646,7 @@ static double mix_residual(ffhip_cg cg, const double *sval) {
 
 // One chunk of FP64 PCG iterations it0 + c, c < kChunk, it0 = 1 (mod kChunk):
 // the H buffer parity follows c.
-static void launch_pcg_chunk(ffhip_cg cg, const double *sval, bool marks) {
+static void launch_pcg_chunk(ffhip_cg cg, const double *sval, bool sym, bool marks) {
   hipStream_t s = cg->ctx->stream;
   const int G = cg->grid;
   const MatFmt<double> M = cg->fmt_of(sval);
@@ -2399,7 +2655,13 @@ static void launch_pcg_chunk(ffhip_cg cg, const double *sval, bool marks) {
     k_pcg_dirvec<<<G, kBlock, 0, s>>>(c, cg->n, cg->H[c & 1], cg->dinv, cg->G, cg->H[(c + 1) & 1],
                                       cg->xw, cg->pA, cg->pB, cg->st);
     if (marks) cg->mark(4 * c + 1);
-    FFHIP_LAUNCH_FMT(cg, k_pcg_matvec, G, s, M, cg->H[(c + 1) & 1], cg->AH, cg->pB, cg->st);
+    if (sym)
+      (cg->sym_nu == 4              ? k_pcg_matvec_sym<3, 4>
+       : cg->sym_nl == kSymHalf - 1 ? k_pcg_matvec_sym<kSymHalf - 1, kSymHalf>
+                                    : k_pcg_matvec_sym<kSymHalf, kSymHalf>)<<<G, kBlock, 0, s>>>(
+          SymFmt{cg->n, cg->S, cg->symval, cg->symcls, cg->symtab}, cg->H[(c + 1) & 1], cg->AH, cg->pB, cg->st);
+    else
+      FFHIP_LAUNCH_FMT(cg, k_pcg_matvec, G, s, M, cg->H[(c + 1) & 1], cg->AH, cg->pB, cg->st);
     if (marks) cg->mark(4 * c + 2);
     k_pcg_update<<<G, kBlock, 0, s>>>(cg->n, cg->AH, cg->dinv, cg->G, cg->pB, cg->pA, cg->st);
     if (marks) cg->mark(4 * c + 3);
@@ -2427,8 +2689,65 @@ static void launch_mix_chunk(ffhip_cg cg, const float *sval32, int par, bool mar
   k_cg_advance<<<1, 64, 0, s>>>(cg->st, kChunk, cg->host_state());
 }
 
-static hipGraphExec_t pcg_chunk_graph(ffhip_cg cg, const double *sval) {
-  return cg->graph(0, sval, 1, [&] { launch_pcg_chunk(cg, sval, false); });
+static hipGraphExec_t pcg_chunk_graph(ffhip_cg cg, const double *sval, bool sym) {
+  return cg->graph(sym ? 2 : 0, sval, 1, [&] { launch_pcg_chunk(cg, sval, sym, false); });
+}
+
+// The symmetric values of a solver in its kSymAfter-th iteration of a solve; true
+// when they are there.  The search and the copy cost 0.2 to 0.6 ms (cube(96),
+// cube(160)) and give 6 to 23 us an iteration: worth it in a solve that has run
+// a while, for a matrix past kSymMinBytes (cube(64), 39 MB, would gain 2 us an
+// iteration for 0.15 ms).  A matrix of another form is seen as one within the
+// search's first blocks, once per solver.
+constexpr int kSymAfter = 4 * kChunk;
+constexpr int64_t kSymMinBytes = 64000000;
+static bool sym_build(ffhip_cg cg) {
+  if (cg->sym) return cg->sym > 0;
+  ffhip_ctx ctx = cg->ctx;
+  hipStream_t s = ctx->stream;
+  const int64_t n = cg->n;
+  cg->sym = -1;
+  // 32-bit byte offsets of the values
+  if (cg->fmt != kSell16 || cg->mode != FFHIP_CG_FP64 || cg->matrix_bytes(8) <= kSymMinBytes ||
+      cg->S * (kSymHalf * kSlice * 8) >= (int64_t)UINT32_MAX)
+    return false;
+  SymTables *T = nullptr;
+  uint32_t *owners = nullptr;
+  const MatFmt<double> M = cg->fmt_of(cg->sval);
+  int end[4] = {1, 0, 0, 0};  // SymTables' bad, count, nl, nu
+  try {
+    T = dalloc<SymTables>(1);
+    owners = dalloc<uint32_t>(n);
+    if (!cg->symcls) cg->symcls = dalloc<uint8_t>(n);
+    if (!cg->symtab) cg->symtab = dalloc<SymPattern>(kSymSlots);
+    clear(ctx, {{T, sizeof(SymTables)}});
+    k_sym_rows<<<nblk(n, 256), 256, 0, s>>>(M, T, cg->symcls, owners);
+    k_sym_table<<<1, kSymSlots, 0, s>>>(M, T, owners, cg->symtab);
+    FFHIP_CHECK(hipGetLastError());
+    fetch(ctx, {{end, &T->bad, sizeof(end)}});
+    if (!end[0]) {
+      cg->sym_nl = end[2];
+      cg->sym_nu = end[2] <= 3 && end[3] <= 4 ? 4 : kSymHalf;
+      if (!cg->symval) cg->symval = dalloc<double>(cg->S * cg->sym_nu * kSlice);
+      k_sym_fill<<<nblk(n, 256), 256, 0, s>>>(M, T, cg->symcls, owners, cg->sym_nu, cg->symval);
+      FFHIP_CHECK(hipGetLastError());
+      fetch(ctx, {{end, &T->bad, sizeof(end)}});
+    }
+  } catch (const Error &) {  // no room for them: the solve goes on without
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(s);
+    end[0] = 1;
+  }
+  dfree(T);
+  dfree(owners);
+  if (end[0]) {
+    dfree(cg->symval);
+    dfree(cg->symcls);
+    dfree(cg->symtab);
+    return false;
+  }
+  cg->sym = 1;
+  return true;
 }
 static hipGraphExec_t mix_chunk_graph(ffhip_cg cg, const float *sval32, int par) {
   return cg->graph(1, sval32, par, [&] { launch_mix_chunk(cg, sval32, par, false); });
@@ -2589,6 +2908,7 @@ static void cg_release(ffhip_cg cg) {
   dfree(cg->AH); dfree(cg->r32); dfree(cg->q32); dfree(cg->y32); dfree(cg->p32[0]);
   dfree(cg->p32[1]); dfree(cg->pA); dfree(cg->pB); dfree(cg->st); dfree(cg->ms);
   dfree(cg->st2);
+  dfree(cg->symval); dfree(cg->symcls); dfree(cg->symtab);
   for (double *&p : cg->gmV) dfree(p);
   for (double *&p : cg->gmVp) dfree(p);
   dfree(cg->gmVDev); dfree(cg->gmVpDev); dfree(cg->gmW); dfree(cg->gmX0); dfree(cg->gmY);
@@ -2672,6 +2992,7 @@ int ffhip_cg_layout(ffhip_cg cg, int *layout, int64_t *entries) {
 int ffhip_cg_update_values(ffhip_cg cg) {
   return guard([&] {
     FFHIP_REQUIRE(cg, FFHIP_ERR_ARG, "ffhip_cg_update_values: null solver");
+    if (cg->sym > 0) cg->sym = 0;
     cg_setup_jacobi(cg);
     setup_readback(cg);
     cg_fill_values(cg, false);
@@ -2695,7 +3016,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
       return;
     }
     // captured before this solve's first launch (kept for later solves)
-    if (cg->mode == FFHIP_CG_FP64) (void)pcg_chunk_graph(cg, sval);
+    if (cg->mode == FFHIP_CG_FP64) (void)pcg_chunk_graph(cg, sval, !trans && cg->sym > 0);
     else { (void)mix_chunk_graph(cg, sval32, 0); (void)mix_chunk_graph(cg, sval32, 1); }
     FFHIP_CHECK(hipMemcpyAsync(cg->bw, b, 8 * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
     FFHIP_CHECK(hipMemcpyAsync(cg->xw, x, 8 * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
@@ -2709,7 +3030,8 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
       const int G = cg->grid;
       const MatFmt<double> M = cg->fmt_of(sval);
       const int chunk = kChunk;
-      hipGraphExec_t gx = pcg_chunk_graph(cg, sval);
+      bool sym = !trans && cg->sym > 0;
+      hipGraphExec_t gx = pcg_chunk_graph(cg, sval, sym);
       hs.it0 = 1;
       hs.itmax = itmax;
       hs.eps = eps;
@@ -2720,12 +3042,16 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
       cg->ensure_events(4 * chunk);
       for (int it = 1;; it += chunk) {
         if (gx) FFHIP_CHECK(hipGraphLaunch(gx, s));
-        else launch_pcg_chunk(cg, sval, cg->profile != 0);
+        else launch_pcg_chunk(cg, sval, sym, cg->profile != 0);
         FFHIP_CHECK(hipGetLastError());
         FFHIP_CHECK(hipStreamSynchronize(s));
         hs = *cg->host_state();
         cg->collect(it, chunk, hs.done ? hs.iters : it + chunk - 1);
         if (hs.done) break;
+        if (!sym && !trans && it + chunk > kSymAfter && sym_build(cg)) {
+          sym = true;
+          gx = pcg_chunk_graph(cg, sval, sym);
+        }
       }
     } else {
       ffhip_cg_solve_mixed(cg, sval, sval32, eps, itmax, hs);
