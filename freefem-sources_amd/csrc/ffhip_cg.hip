@@ -1049,7 +1049,7 @@ __device__ inline void block_rows4(int64_t r0, int64_t r1, int64_t &a4, int64_t 
 // K1: the direction H = gamma H_prev - Cg, written by an elementwise pass so
 // that the mat-vec gathers one vector (forming H on the fly from two gathered
 // vectors per column made the cube(160) mat-vec 17 % slower and the
-// [P2,P2,P2] block mat-vec 50 % slower).
+// [P2,P2,P2] block mat-vec 50 % slower; smaller systems: k_pcg_dir_matvec).
 // It also applies the last update's step x += rho H_prev (ConjugueGradient's
 // x += ro*h, CG.cpp:241), moved here from the update kernel: this pass reads
 // H_prev anyway, so the step costs 16 instead of 24 bytes per row.  x enters
@@ -1118,6 +1118,64 @@ __global__ FFHIP_MATVEC_ATTR void k_pcg_matvec(MatFmt<double> M, const double *_
   }
   const double a = block_sum<kBlock>(p_hah, lds);
   if (threadIdx.x == 0) pout[2 * xcd_block_id()] = a;  // (g, h) comes from the direction kernel
+}
+
+// K1 and K2 in one launch: the direction formed for every gathered column from
+// two vectors, H_prev and C g (which the update then keeps).  For systems in
+// the caches, whose iterations are bound by the latency of their launches
+// (cube(24): 3 of about 5 us with the gaps); the rule is at ffhip_cg_s::fuse.
+template <int KIND>
+__global__ FFHIP_MATVEC_ATTR void k_pcg_dir_matvec(int c, MatFmt<double> M, const double *__restrict__ Hold,
+                                                   const double *__restrict__ CG,
+                                                   const double *__restrict__ G, double *__restrict__ Hnew,
+                                                   double *__restrict__ AH, double *__restrict__ x,
+                                                   const double *__restrict__ pin,
+                                                   double *__restrict__ pout, CgState *st) {
+  __shared__ double lds[kBlock / kWave];
+  if (st->done) return;  // set by an earlier launch only: every block of this one agrees
+  double gamma;
+  const bool go = pcg_begin(c, pin, st, lds, gamma);
+  const bool step = st->it0 + c > 1;  // an update ran before this direction
+  const double rho = st->rho;
+  if (!go) {  // the update publishes the stop
+    int64_t r0, r1;
+    block_rows(M.n, r0, r1);
+    if (step)
+      for (int64_t r = r0 + threadIdx.x; r < r1; r += kBlock) x[r] += rho * Hold[r];
+    return;
+  }
+  double p_hah = 0., p_gh = 0.;
+  struct Own {
+    double h, cg, g, x;
+  };
+  const auto pre = [&](int64_t r) { return Own{Hold[r], CG[r], G[r], x[r]}; };
+  const auto epi = [&](int64_t r, double acc, const Own &o, bool row) {
+    if (!row) return;
+    const double hn = gamma * o.h - o.cg;
+    Hnew[r] = hn;
+    AH[r] = acc;
+    if (step) x[r] = o.x + rho * o.h;
+    p_gh += o.g * hn;
+    p_hah += hn * acc;
+  };
+  if constexpr (KIND == kSell16) {
+    const auto hr = slice_rsrc(Hold, (uint32_t)(M.n * 8)), cr = slice_rsrc(CG, (uint32_t)(M.n * 8));
+    matvec_rows_pre<KIND, double, double>(
+        M,
+        [&](int32_t j) {
+          const double h = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(hr, j * 8, 0, 0));
+          return gamma * h - __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(cr, j * 8, 0, 0));
+        },
+        pre, epi);
+  } else {
+    matvec_rows_pre<KIND, double, double>(M, [&](int32_t j) { return gamma * Hold[j] - CG[j]; }, pre, epi);
+  }
+  const double a = block_sum<kBlock>(p_hah, lds);
+  const double b = block_sum<kBlock>(p_gh, lds);
+  if (threadIdx.x == 0) {
+    pout[2 * xcd_block_id()] = a;
+    pout[2 * xcd_block_id() + 1] = b;
+  }
 }
 
 // ---------------------------------------------------------------- symmetric values
@@ -1372,8 +1430,13 @@ __global__ __launch_bounds__(256) void k_sym_fill(MatFmt<double> M, SymTables *T
 
 __global__ __launch_bounds__(kBlock) void k_pcg_update(
     int64_t n, const double *__restrict__ AH, const double *__restrict__ dinv,
-    double *__restrict__ G, const double *__restrict__ pin, double *__restrict__ pout, CgState *st) {
+    double *__restrict__ G, double *__restrict__ CG, const double *__restrict__ pin,
+    double *__restrict__ pout, CgState *st) {
   __shared__ double lds[kBlock / kWave];
+  if (st->stop) {  // k_pcg_dir_matvec stopped the solve: publish it
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->done = st->stop;
+    return;
+  }
   if (st->done) return;
   const int P = gridDim.x;
   const double hah = reduce_partials(pin, P, 2, 0, lds);
@@ -1387,6 +1450,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(
     const double g = G[r] + rho * AH[r];
     G[r] = g;
     const double c = __dmul_rn(dinv[r], g);  // C g, formed again by the next direction kernel
+    if (CG) CG[r] = c;                        // but kept for k_pcg_dir_matvec
     part += g * c;
   }
   const double tot = block_sum<kBlock>(part, lds);
@@ -2090,6 +2154,30 @@ __global__ FFHIP_MATVEC_ATTR void k_mix_matvec(MatFmt<float> M, const float *__r
   if (threadIdx.x == 0) pout[xcd_block_id()] = tot;
 }
 
+// K_m1 and K_m2 in one launch: p formed for every gathered column
+template <int KIND>
+__global__ FFHIP_MATVEC_ATTR void k_mix_dir_matvec(int c, MatFmt<float> M, const float *__restrict__ pold,
+                                                   const float *__restrict__ r32, float *__restrict__ pnew,
+                                                   float *__restrict__ q, const double *__restrict__ pin,
+                                                   double *__restrict__ pout, CgState *st, MixState *ms) {
+  __shared__ double lds[kBlock / kWave];
+  if (st->done || st->need_update) return;
+  float cbf;
+  if (!mix_begin(c, pin, st, ms, lds, cbf)) return;
+  const auto p = [&](int64_t j) { return r32[j] + cbf * pold[j]; };
+  double part = 0.;
+  matvec_rows<KIND, float, float>(
+      M, [&](int32_t j) { return p(j); },
+      [&](int64_t r, float acc) {
+        const float pr = p(r);
+        pnew[r] = pr;
+        q[r] = acc;
+        part += (double)pr * (double)acc;
+      });
+  const double tot = block_sum<kBlock>(part, lds);
+  if (threadIdx.x == 0) pout[xcd_block_id()] = tot;
+}
+
 // K_m3: alpha = rho/(p,q); y32 += alpha p; r32 -= alpha q; partial (r32, r32)
 __global__ __launch_bounds__(kBlock) void k_mix_update(
     int c, int64_t n, const float *__restrict__ p, const float *__restrict__ q,
@@ -2352,6 +2440,17 @@ struct ffhip_cg_s {
       FFHIP_CHECK(hipEventElapsedTime(&b, ev[4 * c + 2], ev[4 * c + 3]));
       t_dv += d; t_mv += a; t_up += b; ++n_timed;
     }
+  }
+  // The direction formed in the mat-vec (not for 3x3 blocks, whose mat-vec gains
+  // little from one launch less): up to where the second gathered vector costs
+  // what the launch did.  us per solve, apart / together, FP64 cube(24) 1474 /
+  // 1233, cube(48) 3495 / 3212, cube(64) 7181 / 6864, cube(72) 8876 / 8802, cube(80)
+  // 10601 / 12184; MIXED cube(24) 2097 / 1897, cube(64) 6204 / 5768, cube(96) 16574 /
+  // 15730, cube(112) 24958 / 24649, cube(128) 36932 / 37865.  FP64 systems of one
+  // workgroup's size keep the launches' bits of k_pcg_small.
+  bool fuse() const {
+    if (fmt == kBsr3) return false;
+    return mode == FFHIP_CG_MIXED ? n <= 1 << 20 : n > kSmallRows && n <= 5 << 16;
   }
   // the state as the host reads it after a chunk (k_cg_advance writes it)
   CgState *host_state() const { return static_cast<CgState *>(ctx->pinned_data()); }
@@ -2649,13 +2748,18 @@ static double mix_residual(ffhip_cg cg, const double *sval) {
 static void launch_pcg_chunk(ffhip_cg cg, const double *sval, bool sym, bool marks) {
   hipStream_t s = cg->ctx->stream;
   const int G = cg->grid;
+  const bool fused = cg->fuse();
   const MatFmt<double> M = cg->fmt_of(sval);
   for (int c = 0; c < kChunk; ++c) {
     if (marks) cg->mark(4 * c);
-    k_pcg_dirvec<<<G, kBlock, 0, s>>>(c, cg->n, cg->H[c & 1], cg->dinv, cg->G, cg->H[(c + 1) & 1],
-                                      cg->xw, cg->pA, cg->pB, cg->st);
+    if (!fused)
+      k_pcg_dirvec<<<G, kBlock, 0, s>>>(c, cg->n, cg->H[c & 1], cg->dinv, cg->G, cg->H[(c + 1) & 1],
+                                        cg->xw, cg->pA, cg->pB, cg->st);
     if (marks) cg->mark(4 * c + 1);
-    if (sym)
+    if (fused)
+      FFHIP_LAUNCH_FMT(cg, k_pcg_dir_matvec, G, s, c, M, cg->H[c & 1], cg->CG, cg->G, cg->H[(c + 1) & 1],
+                       cg->AH, cg->xw, cg->pA, cg->pB, cg->st);
+    else if (sym)
       (cg->sym_nu == 4              ? k_pcg_matvec_sym<3, 4>
        : cg->sym_nl == kSymHalf - 1 ? k_pcg_matvec_sym<kSymHalf - 1, kSymHalf>
                                     : k_pcg_matvec_sym<kSymHalf, kSymHalf>)<<<G, kBlock, 0, s>>>(
@@ -2663,7 +2767,8 @@ static void launch_pcg_chunk(ffhip_cg cg, const double *sval, bool sym, bool mar
     else
       FFHIP_LAUNCH_FMT(cg, k_pcg_matvec, G, s, M, cg->H[(c + 1) & 1], cg->AH, cg->pB, cg->st);
     if (marks) cg->mark(4 * c + 2);
-    k_pcg_update<<<G, kBlock, 0, s>>>(cg->n, cg->AH, cg->dinv, cg->G, cg->pB, cg->pA, cg->st);
+    k_pcg_update<<<G, kBlock, 0, s>>>(cg->n, cg->AH, cg->dinv, cg->G, fused ? cg->CG : nullptr, cg->pB,
+                                      cg->pA, cg->st);
     if (marks) cg->mark(4 * c + 3);
   }
   k_cg_advance<<<1, 64, 0, s>>>(cg->st, kChunk, cg->host_state());
@@ -2674,13 +2779,18 @@ static void launch_mix_chunk(ffhip_cg cg, const float *sval32, int par, bool mar
   hipStream_t s = cg->ctx->stream;
   const int G = cg->grid;
   const MatFmt<float> M32 = cg->fmt_of(sval32);
+  const bool fused = cg->fuse();
   for (int c = 0; c < kChunk; ++c) {
     const float *pold = cg->p32[(par + c + 1) & 1];
     float *pnew = cg->p32[(par + c) & 1];
     if (marks) cg->mark(4 * c);
-    k_mix_dirvec<<<G, kBlock, 0, s>>>(c, cg->n, pold, cg->r32, pnew, cg->pA, cg->st, cg->ms);
+    if (!fused) k_mix_dirvec<<<G, kBlock, 0, s>>>(c, cg->n, pold, cg->r32, pnew, cg->pA, cg->st, cg->ms);
     if (marks) cg->mark(4 * c + 1);
-    FFHIP_LAUNCH_FMT(cg, k_mix_matvec, G, s, M32, pnew, cg->q32, cg->pB, cg->st);
+    if (fused)
+      FFHIP_LAUNCH_FMT(cg, k_mix_dir_matvec, G, s, c, M32, pold, cg->r32, pnew, cg->q32, cg->pA, cg->pB, cg->st,
+                       cg->ms);
+    else
+      FFHIP_LAUNCH_FMT(cg, k_mix_matvec, G, s, M32, pnew, cg->q32, cg->pB, cg->st);
     if (marks) cg->mark(4 * c + 2);
     k_mix_update<<<G, kBlock, 0, s>>>(c, cg->n, pnew, cg->q32, cg->y32, cg->r32, cg->pB, cg->pA,
                                       cg->st, cg->ms);
