@@ -11,7 +11,8 @@
 //      bitonic sort of the first 32 in a half-wave, insertion sort beyond.
 //   2. pattern: one half-wave per row loads the vertices of the row's
 //      incident elements (4 per lane), deduplicates them in an LDS hash set
-//      and orders the unique columns by a counting sort.  One pass writes
+//      (the lanes step together: no atomics) and orders the unique columns by
+//      a counting sort.  One pass writes
 //      each row's sorted columns to a row buffer, its length and, for every
 //      incidence entry, the offsets of that element's vertices inside the row
 //      (the element-to-row map); after a scan of the lengths the buffers are
@@ -27,6 +28,10 @@
 //      (src/femlib/HashMatrix.cpp:1294-1332).  2D triangles and the rows with
 //      more than 32 elements use a lane-per-row walk with the row staged in
 //      LDS.
+//   4. right-hand sides, the adjoint's M (u - u_d) and CSR products: a pass over
+//      the elements leaves each its terms, and a wave per 16 or 64 rows stages
+//      the rows' entries in LDS with coalesced loads, added by a lane per row in
+//      their order.
 #include <hipcub/hipcub.hpp>
 
 #include <cstring>

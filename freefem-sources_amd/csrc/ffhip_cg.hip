@@ -9,9 +9,12 @@
 // (FP64) segment and no cross-lane reduction is needed per row.
 //
 // Iteration (same recurrences as ConjugueGradient):
-//   K1: H = gamma*H_prev - C g  (formed on the fly for every gathered column)
-//       AH = A H, partial sums of (H,AH) and (g,H)
-//   K2: rho = -(g,H)/(H,AH); x += rho H; g += rho AH; Cg = D^-1 g; (g,Cg)
+//   K1: x += rho H_prev; H = gamma*H_prev - C g, partial sum of (g,H)
+//   K2: AH = A H, partial sum of (H,AH)
+//   K3: rho = -(g,H)/(H,AH); g += rho AH; (g, D^-1 g)
+// Systems in the caches form H in K2, for every gathered column (k_pcg_dir_matvec,
+// k_mix_dir_matvec); long solves of large box matrices read half of the values
+// (k_pcg_matvec_sym); small systems are solved by one workgroup (k_pcg_small).
 // Each kernel starts by re-reducing the previous kernel's per-block partial
 // sums in a fixed order, so all blocks derive identical scalars with no
 // cross-block atomics or fences, and the result is bitwise reproducible.
@@ -2941,11 +2944,12 @@ int ffhip_cg_solve_mixed(ffhip_cg cg, const double *sval, const float *sval32, d
 // the figures of a finished solve for the caller, and the errors of one that
 // did not converge (res: the sums of k_residual)
 static void solve_result(ffhip_cg cg, const CgState &hs, const double res[3], double ms, int itmax,
-                         ffhip_cg_stats *stats) {
+                         int half_from, ffhip_cg_stats *stats) {
   if (stats) {
     stats->iters = hs.iters;
     stats->converged = hs.done == 1 ? 1 : (hs.done == 2 ? 2 : 0);
     stats->refinements = hs.refinements;
+    stats->half_from = half_from;
     stats->gcg0 = hs.gcg0;
     stats->gcg = cg->mode == FFHIP_CG_FP64 ? hs.gcg_prev[(hs.iters + 1) & 1] : res[2];
     stats->true_gcg = res[2];
@@ -3005,7 +3009,7 @@ static void pcg_solve_small(ffhip_cg cg, const double *b, double *x, int on_devi
     for (int c = 0; c < 3; ++c) res[c] += out->res[3 * i + c];
   cg->t_dv = cg->t_mv = cg->t_up = 0.;
   cg->n_timed = 0;
-  solve_result(cg, out->st, res, ctx->last_ms, itmax, stats);
+  solve_result(cg, out->st, res, ctx->last_ms, itmax, 0, stats);
 }
 
 static void cg_release(ffhip_cg cg) {
@@ -3134,6 +3138,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
     ctx->tic();
     if (cg->ntgv > 0) k_init_bc<<<nblk(n, 256), 256, 0, s>>>(n, cg->wcl, cg->bw, tgv, cg->xw);
     CgState hs;
+    int half_from = 0;
     memset(&hs, 0, sizeof(hs));
     cg->t_dv = cg->t_mv = cg->t_up = 0.;
     cg->n_timed = 0;
@@ -3142,6 +3147,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
       const MatFmt<double> M = cg->fmt_of(sval);
       const int chunk = kChunk;
       bool sym = !trans && cg->sym > 0;
+      half_from = sym ? 1 : 0;
       hipGraphExec_t gx = pcg_chunk_graph(cg, sval, sym);
       hs.it0 = 1;
       hs.itmax = itmax;
@@ -3161,6 +3167,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
         if (hs.done) break;
         if (!sym && !trans && it + chunk > kSymAfter && sym_build(cg)) {
           sym = true;
+          half_from = it + chunk;
           gx = pcg_chunk_graph(cg, sval, sym);
         }
       }
@@ -3173,7 +3180,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
     residual_sums(cg, sval, cg->xw, cg->bw, nullptr, res);
     FFHIP_CHECK(hipMemcpyAsync(x, cg->xw, 8 * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
     FFHIP_CHECK(hipStreamSynchronize(s));
-    solve_result(cg, hs, res, ms, itmax, stats);
+    solve_result(cg, hs, res, ms, itmax, half_from, stats);
   });
 }
 

@@ -1,5 +1,5 @@
 // ffhip_p2.hip — vector P2 ([P2,P2,P2]) linear elasticity on tetrahedra:
-// node numbering, matrix pattern, Lame element matrices on the matrix cores,
+// node numbering, matrix pattern, rows from the elements' vertex gradients,
 // atomic-free row assembly, clamped boundary rows and body-force right-hand
 // side.
 //
@@ -20,7 +20,7 @@
 //              with atomicMin over vertices, a radix sort of the edge keys and
 //              one scan over the items — equal to FreeFEM's sequential
 //              first-appearance numbering.
-//   pattern    node rows (sorted unique node columns, LDS merge per lane, as
+//   pattern    node rows (sorted unique node columns, a wave per row, as
 //              P1), expanded to scalar rows of 3 x 3 blocks.
 //   element    the P2 gradients are linear in the barycentrics, so a tet leaves
 //              only its vertex gradients (Lame: |K| and G, 13 doubles; scalar:

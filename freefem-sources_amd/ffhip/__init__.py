@@ -42,7 +42,7 @@ class FFHipError(RuntimeError):
 
 class CGStats(ctypes.Structure):
     _fields_ = [("iters", ctypes.c_int), ("converged", ctypes.c_int),
-                ("refinements", ctypes.c_int), ("reserved", ctypes.c_int),
+                ("refinements", ctypes.c_int), ("half_from", ctypes.c_int),
                 ("gcg0", ctypes.c_double), ("gcg", ctypes.c_double),
                 ("true_gcg", ctypes.c_double), ("true_relres", ctypes.c_double),
                 ("ms_solve", ctypes.c_double), ("ms_matvec_avg", ctypes.c_double),

@@ -282,7 +282,8 @@ int ffhip_mat_device_ptrs(ffhip_mat mat, int64_t **rowptr, int32_t **colidx,
 int ffhip_mat_free(ffhip_mat mat);
 
 /* y = A x (trans = 0) or A^T x (trans = 1) on device vectors:
- * HashMatrix::addMatMul (HashMatrix.cpp:1086-1154) without the accumulate. */
+ * HashMatrix::addMatMul (HashMatrix.cpp:1086-1154) without the accumulate.
+ * A^T of a pattern that is not symmetric is refused; y is then undefined. */
 int ffhip_spmv(ffhip_ctx ctx, ffhip_mat mat, const double *x, double *y,
                int trans);
 
@@ -302,7 +303,7 @@ int ffhip_pattern_p2v(ffhip_ctx ctx, ffhip_p2v space, ffhip_mat *mat);
 /* Values of int3d(Th)(lambda*div(u)*div(v) + 2*mu*(epsilon(u)'*epsilon(v)))
  * with Tet_5: Element_Op (problem.cpp:6337-6437) with the P2 basis of
  * TypeOfFE_P2Lagrange3d (P012_3d.cpp:199-270), accumulated in element order.
- * Local matrices on the FP64 matrix cores. */
+ * The element integrals as sums over products of vertex gradients. */
 int ffhip_assemble_p2v_elasticity(ffhip_ctx ctx, ffhip_p2v space, ffhip_mat mat,
                                   double lambda, double mu);
 /* on(labels, u1=.., u2=.., u3=..): all components of the vertex and edge nodes
@@ -363,7 +364,7 @@ typedef struct {
   int iters;          /* CG iterations (inner FP32 iterations for MIXED)   */
   int converged;      /* ConjugueGradient's nret: 1 converged, 2 gCg0<1e-30, 0 no */
   int refinements;    /* MIXED: FP64 residual recomputations              */
-  int reserved;
+  int half_from;      /* FP64: first iteration whose mat-vec read half of the values, 0: none */
   double gcg0;        /* (g0, D^-1 g0), g0 = A x0 - b                       */
   double gcg;         /* final (g, D^-1 g) (recurrence for FP64, true for MIXED) */
   double true_gcg;    /* final (g, D^-1 g) recomputed in FP64 from x         */
@@ -376,7 +377,7 @@ typedef struct {
   double ms_update_avg;
   int timed;
   int reserved2;
-  double ms_direction_avg; /* the same for the direction kernel */
+  double ms_direction_avg; /* the same for the direction kernel (about 0 where the mat-vec forms it) */
 } ffhip_cg_stats;
 /* Solver setup for a matrix (SolverCG ctor + HMatVirtPrecon,
  * src/femlib/VirtualSolverCG.hpp:27-69, 157-167): tgv detection
