@@ -965,7 +965,7 @@ __global__ __launch_bounds__(256) void k_p1_scale_3d(int64_t nt, const double *_
 // computed (their round trip hidden by the arithmetic), and the items are
 // placed after it.  The scale is the same computation as k_p1_scale_3d's.
 // (5 waves per SIMD, no spills; uncapped it takes 108 registers and runs 4.  One
-// point of the rule at a time: cube(160) 1256 -> 1150 us, two at a time 1210)
+// point of the rule at a time: cube(160) 1150 us for 1210 with two, now 1107)
 constexpr int kFuseLog = 11;
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 5))) void k_v2e_bucket_scale(const int32_t *__restrict__ tets, int64_t nt,
                                                           ScaleArgs sc, uint32_t *__restrict__ deg,
