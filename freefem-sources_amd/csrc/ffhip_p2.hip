@@ -259,7 +259,8 @@ __global__ __launch_bounds__(256) void k_p2_pattern_wave(
 // scalar rows 3a + c of node a: for every node column b, columns 3b, 3b+1, 3b+2
 // (node columns from ncol at nodeptr, or from the row buffers when rowbuf != null).
 // One wave per node: the node's 3 rows are one run of 9 L columns at 9 p0,
-// written with consecutive lanes on consecutive entries.
+// written with consecutive lanes on consecutive entries (each column formed once
+// for the three rows: cube(32) 149 -> 113 us).
 __global__ __launch_bounds__(256) void k_p2v_expand(int64_t nn, const int64_t *__restrict__ nodeptr,
                                                     const int32_t *__restrict__ ncol,
                                                     const int64_t *__restrict__ ndiag,
@@ -271,14 +272,17 @@ __global__ __launch_bounds__(256) void k_p2v_expand(int64_t nn, const int64_t *_
   const int lane = threadIdx.x % kWave;
   const int64_t a = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   if (a >= nn) return;  // uniform in the wave
-  const int64_t p0 = nodeptr[a], L = nodeptr[a + 1] - p0;
+  const int64_t p0 = nodeptr[a];
+  const int L = (int)(nodeptr[a + 1] - p0);
   const int32_t *cols = rowbuf ? rowbuf + kNodeCap * a : ncol + p0;
   const int64_t base0 = 9 * p0;
-  for (int c = 0; c < 3; ++c)
-    for (int64_t j = lane; j < 3 * L; j += kWave) {
-      const int64_t q = j / 3;
-      colidx[base0 + c * 3 * L + j] = 3 * cols[q] + (int32_t)(j - 3 * q);
-    }
+  for (int j = lane; j < 3 * L; j += kWave) {
+    const int q = j / 3;
+    const int32_t col = 3 * cols[q] + (j - 3 * q);
+    colidx[base0 + j] = col;
+    colidx[base0 + 3 * L + j] = col;
+    colidx[base0 + 6 * L + j] = col;
+  }
   if (lane < 3) {
     const int c = lane;
     const int64_t r = 3 * a + c, base = base0 + c * 3 * L;
