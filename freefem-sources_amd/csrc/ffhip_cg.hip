@@ -2352,44 +2352,65 @@ struct ffhip_cg_s {
     return (int)(b < 256 ? b : 256);
   }
   int64_t gm_out() const { return (int64_t)gmCap + grid; }  // doubles per iteration of gmOut
-  void gm_basis(int k) {
-    if (k > gmCap) {
-      const int cap = std::max(std::max(k, 2 * gmCap), 64);
-      double **pv = dalloc<double *>(cap), **p = dalloc<double *>(cap);
-      double *y = dalloc<double>(cap + 1), *S = dalloc<double>(2 * (int64_t)cap * gm_blocks());
-      double *L = dalloc<double>((int64_t)cap * (cap - 1) / 2);
-      double *out = dalloc<double>(kGmBatch * ((int64_t)cap + grid));
-      if (gmCap)
-        FFHIP_CHECK(hipMemcpy(L, gmL, 8 * (size_t)gmCap * (gmCap - 1) / 2, hipMemcpyDeviceToDevice));
-      dfree(gmVDev); dfree(gmVpDev); dfree(gmY); dfree(gmS); dfree(gmL); dfree(gmOut);
-      if (gmOutH) (void)hipHostFree(gmOutH);
-      gmOutH = nullptr;
-      gmVDev = pv; gmVpDev = p; gmY = y; gmS = S; gmL = L; gmOut = out; gmCap = cap;
-      FFHIP_CHECK(hipHostMalloc((void **)&gmOutH, 8 * kGmBatch * gm_out(), hipHostMallocDefault));
-      FFHIP_CHECK(hipMemcpy(gmVDev, gmV.data(), sizeof(double *) * gmV.size(), hipMemcpyHostToDevice));
-      FFHIP_CHECK(hipMemcpy(gmVpDev, gmVp.data(), sizeof(double *) * gmVp.size(), hipMemcpyHostToDevice));
-    }
-    const size_t k0 = gmV.size();
-    if ((int)k0 < k) {
-      gmV.reserve(k);
-      gmVp.reserve(k);
-      while ((int)gmV.size() < k) {
-        double *v = nullptr, *vp = nullptr;
-        try {
-          v = dalloc<double>(n);
-          vp = dalloc<double>(n);
-        } catch (const Error &) {  // as many as fit: the caller sees how many there are
-          dfree(v);
-          break;
-        }
-        gmV.push_back(v);
-        gmVp.push_back(vp);
+  // room for `need` vectors, and for up to `want` while device memory lasts
+  void gm_basis(int need, int want) {
+    if (!gmW) gmW = dalloc<double>(n);
+    if (!gmX0) gmX0 = dalloc<double>(n);
+    if (want > gmCap) {
+      try {
+        gm_tables(std::max(std::max(want, 2 * gmCap), 64));
+      } catch (const Error &) {
+        if (need > gmCap) throw;
       }
-      const size_t c = gmV.size() - k0;
+    }
+    const size_t k0 = gmV.size(), k = (size_t)std::min(want, gmCap);
+    if (k <= k0) return;
+    gmV.reserve(k);
+    gmVp.reserve(k);
+    while (gmV.size() < k) {
+      double *v = nullptr, *vp = nullptr;
+      try {
+        v = dalloc<double>(n);
+        vp = dalloc<double>(n);
+      } catch (const Error &) {
+        dfree(v);
+        break;
+      }
+      gmV.push_back(v);
+      gmVp.push_back(vp);
+    }
+    if (const size_t c = gmV.size() - k0) {
       FFHIP_CHECK(hipMemcpy(gmVDev + k0, gmV.data() + k0, sizeof(double *) * c, hipMemcpyHostToDevice));
       FFHIP_CHECK(hipMemcpy(gmVpDev + k0, gmVp.data() + k0, sizeof(double *) * c, hipMemcpyHostToDevice));
     }
-    if (!gmW) { gmW = dalloc<double>(n); gmX0 = dalloc<double>(n); }
+    FFHIP_REQUIRE((int)gmV.size() >= need, FFHIP_ERR_HIP,
+                  "ffhip_gmres_solve: out of device memory at %d basis vectors", (int)gmV.size());
+  }
+  // the tables and buffers for cap vectors: all of them, or as they were
+  void gm_tables(int cap) {
+    double **pv = nullptr, **p = nullptr, *y = nullptr, *S = nullptr, *L = nullptr, *out = nullptr;
+    void *outH = nullptr;
+    try {
+      pv = dalloc<double *>(cap);
+      p = dalloc<double *>(cap);
+      y = dalloc<double>(cap + 1);
+      S = dalloc<double>(2 * (int64_t)cap * gm_blocks());
+      L = dalloc<double>((int64_t)cap * (cap - 1) / 2);
+      out = dalloc<double>(kGmBatch * ((int64_t)cap + grid));
+      FFHIP_CHECK(hipHostMalloc(&outH, 8 * kGmBatch * ((int64_t)cap + grid), hipHostMallocDefault));
+      if (gmCap) {
+        FFHIP_CHECK(hipMemcpy(L, gmL, 8 * (size_t)gmCap * (gmCap - 1) / 2, hipMemcpyDeviceToDevice));
+        FFHIP_CHECK(hipMemcpy(pv, gmV.data(), sizeof(double *) * gmV.size(), hipMemcpyHostToDevice));
+        FFHIP_CHECK(hipMemcpy(p, gmVp.data(), sizeof(double *) * gmVp.size(), hipMemcpyHostToDevice));
+      }
+    } catch (...) {
+      dfree(pv); dfree(p); dfree(y); dfree(S); dfree(L); dfree(out);
+      if (outH) (void)hipHostFree(outH);
+      throw;
+    }
+    dfree(gmVDev); dfree(gmVpDev); dfree(gmY); dfree(gmS); dfree(gmL); dfree(gmOut);
+    if (gmOutH) (void)hipHostFree(gmOutH);
+    gmVDev = pv; gmVpDev = p; gmY = y; gmS = S; gmL = L; gmOut = out; gmOutH = (double *)outH; gmCap = cap;
   }
   // captured chunks of CG launches, keyed by (mode, value array, parity of the
   // chunk's first iteration); kernel by kernel when eager or profiling (event
@@ -3255,7 +3276,7 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
     const double *sval = trans ? cg->svalT : cg->sval;
     const MatFmt<double> M = cg->fmt_of(sval);
     const hipMemcpyKind kin = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    cg->gm_basis(1);
+    cg->gm_basis(1, 1);
     FFHIP_CHECK(hipMemcpyAsync(cg->bw, b, 8 * n, kin, s));
     FFHIP_CHECK(hipMemcpyAsync(cg->xw, x, 8 * n, kin, s));
     std::vector<double> part(G);
@@ -3300,9 +3321,8 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
           // needs of each; those after a convergence are dropped.  Past 2^18
           // rows an iteration costs more than the wait it saves.
           batch = std::min(n <= (1 << 18) ? ffhip_cg_s::kGmBatch : 1, m - it);
-          cg->gm_basis(it + batch);
+          cg->gm_basis(it + 1, it + batch);
           batch = std::min(batch, (int)cg->gmV.size() - it);
-          FFHIP_REQUIRE(batch > 0, FFHIP_ERR_HIP, "ffhip_gmres_solve: out of device memory at %d basis vectors", it);
           const int64_t ld = cg->gm_out();
           for (int c = 0; c < batch; ++c) {
             const int j = it + c;

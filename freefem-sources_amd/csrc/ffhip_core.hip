@@ -338,6 +338,7 @@ void *block_alloc(size_t bytes) {
     e = hipMalloc(&p, want);
   }
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     set_error("hipMalloc(%zu bytes) -> %s", want, hipGetErrorString(e));
     throw Error{FFHIP_ERR_HIP};
   }

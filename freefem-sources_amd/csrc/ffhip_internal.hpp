@@ -24,10 +24,13 @@ struct Error {
   int code;
 };
 
+// (A failed call's error stays the thread's last error until it is read, also
+// over calls that succeed: read here, so that no later launch check reports it.)
 #define FFHIP_CHECK(expr)                                                      \
   do {                                                                         \
     hipError_t e_ = (expr);                                                    \
     if (e_ != hipSuccess) {                                                    \
+      (void)hipGetLastError();                                                 \
       ::ffhip::set_error("%s:%d: %s -> %s", __FILE__, __LINE__, #expr,         \
                          hipGetErrorString(e_));                               \
       throw ::ffhip::Error{FFHIP_ERR_HIP};                                     \

@@ -1,0 +1,136 @@
+"""Calls on a device whose memory has run out.  hipMalloc and hipHostMalloc as
+libffhip calls them go through Python here (their slots in the library's table
+of imported functions), which fails the chosen requests by asking the runtime
+for 2^60 bytes: the error, and the last error it leaves, are the runtime's own."""
+import ctypes
+import struct
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ffhip = pytest.importorskip("ffhip")
+ERR_HIP = -2
+
+
+def import_slots(path):
+    """offset of each imported function's slot from the library's load address"""
+    f = open(path, "rb").read()
+    shoff, = struct.unpack_from("<Q", f, 0x28)
+    shentsize, shnum = struct.unpack_from("<HH", f, 0x3A)
+    sections = [struct.unpack_from("<IIQQQQIIQQ", f, shoff + i * shentsize) for i in range(shnum)]
+    slots = {}
+    for _, kind, _, _, off, size, link, _, _, _ in sections:
+        if kind != 4:  # SHT_RELA
+            continue
+        symoff, strlink = sections[link][4], sections[link][6]
+        stroff = sections[strlink][4] if strlink else 0
+        for o in range(off, off + size, 24):
+            where, info, _ = struct.unpack_from("<QQq", f, o)
+            if info & 0xffffffff == 7:  # R_X86_64_JUMP_SLOT
+                name, = struct.unpack_from("<I", f, symoff + 24 * (info >> 32))
+                slots[f[stroff + name:f.index(b"\0", stroff + name)].decode()] = where
+    return slots
+
+
+class Allocator:
+    def __init__(self):
+        L = ffhip.lib()
+        ffhip.context()
+        path = ffhip.LIBPATH
+        base = min(int(l.split("-")[0], 16) for l in open("/proc/self/maps") if l.rstrip().endswith(path))
+        slots = import_slots(path)
+        self.fail = lambda size: False
+        self.fail_host = lambda size: False
+        self.kept = []
+        for name, sig, rule in (("hipMalloc", ctypes.c_size_t, "fail"),
+                                ("hipHostMalloc", ctypes.c_size_t, "fail_host")):
+            real = getattr(L, name)
+            extra = [ctypes.c_uint] if name == "hipHostMalloc" else []
+            real.argtypes = [ctypes.c_void_p, sig] + extra
+            real.restype = ctypes.c_int
+            proto = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, sig, *extra)
+
+            def call(p, size, *flags, real=real, rule=rule):
+                return real(p, (1 << 60) if getattr(self, rule)(size) else size, *flags)
+            slot = ctypes.c_void_p.from_address(base + slots[name])
+            self.kept.append((slot, slot.value, proto(call)))
+            slot.value = ctypes.cast(self.kept[-1][2], ctypes.c_void_p).value
+
+    def drop_cache(self):
+        """the library gives its cached blocks back when a request fails"""
+        self.fail = lambda size: True
+        with pytest.raises(ffhip.FFHipError) as e:
+            ffhip.cube(183, 171, 167)  # larger than any block kept
+        assert e.value.code == ERR_HIP
+        self.fail = lambda size: False
+
+    def limit(self, size, count):
+        """requests for a block of `size` bytes fail after `count` of them"""
+        left = [count]
+
+        def fail(s):
+            if size <= s < size + 256:
+                left[0] -= 1
+            return left[0] < 0 and size <= s < size + 256
+        self.fail = fail
+
+    def close(self):
+        for slot, old, _ in self.kept:
+            slot.value = old
+
+
+@pytest.fixture
+def alloc():
+    a = Allocator()
+    yield a
+    a.close()
+
+
+def rotation(n):
+    rng = np.random.default_rng(n)
+    i = np.arange(n)
+    M = np.zeros((n, n))
+    M[i, i] = 1.5 + 0.05 * rng.standard_normal(n)
+    M[i[:-1], i[:-1] + 1] = 1.0
+    M[i[1:], i[1:] - 1] = -0.9
+    rows, ci = np.nonzero(M)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int64)
+    return ffhip.Matrix.upload(rp, ci.astype(np.int32), M[rows, ci]), rng.standard_normal(n)
+
+
+def test_gmres_takes_the_vectors_that_fit(alloc):
+    n = 3000
+    A, b = rotation(n)
+    x0, s0 = ffhip.CG(A).gmres(b, eps=1e-10)
+    its = s0["iters"]
+    assert s0["converged"] == 1 and its > 12
+    for pairs in (its + 1, its + 3, 5):
+        cg = ffhip.CG(A)
+        alloc.drop_cache()
+        alloc.limit(8 * n, 2 + 2 * pairs + 1)  # w and x0, the pairs, and half of one more
+        if pairs > its:  # a batch cut short, the same arithmetic
+            x, st = cg.gmres(b, eps=1e-10)
+            assert st["iters"] == its and np.array_equal(x, x0)
+        else:
+            with pytest.raises(ffhip.FFHipError) as e:
+                cg.gmres(b, eps=1e-10)
+            assert e.value.code == ERR_HIP
+            alloc.fail = lambda size: False
+            x, st = cg.gmres(b, eps=1e-10)  # room again
+            assert st["iters"] == its and np.array_equal(x, x0)
+        alloc.fail = lambda size: False
+
+
+def test_gmres_after_a_failed_page_locked_buffer(alloc):
+    n = 3000
+    A, b = rotation(n)
+    x0, _ = ffhip.CG(A).gmres(b, eps=1e-10)
+    cg = ffhip.CG(A)
+    alloc.fail_host = lambda size: True
+    with pytest.raises(ffhip.FFHipError) as e:
+        cg.gmres(b, eps=1e-10)
+    assert e.value.code == ERR_HIP
+    alloc.fail_host = lambda size: False
+    assert np.array_equal(cg.gmres(b, eps=1e-10)[0], x0)
