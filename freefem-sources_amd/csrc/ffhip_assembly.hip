@@ -1328,9 +1328,10 @@ __device__ inline double row_sum_in_order(double *__restrict__ slot, int hl, int
 }
 
 // (M e)_v = sum over incident elements of |K|/20 (e_v + sum_K e_j); 0 on
-// Dirichlet rows: the pass of the entry point that may hold no per-element
-// temporary (the other one stores the pairs with the misfit and adds them in
-// k_row_sum, the same terms in the same order)
+// Dirichlet rows: the pass where there is no per-element temporary (the entry
+// point that allocates nothing, a device without room for one; else the pairs
+// are stored with the misfit and added in k_row_sum, the same terms in the same
+// order)
 __global__ __launch_bounds__(256) void k_p1_mass_apply(
     int64_t n, const double *__restrict__ xyz, const int32_t *__restrict__ tets,
     const int64_t *__restrict__ v2e_ptr, const int32_t *__restrict__ v2e,
@@ -2236,12 +2237,17 @@ int ffhip_p1_misfit(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *
     FFHIP_REQUIRE(nlab >= 0 && (nlab == 0 || labels), FFHIP_ERR_ARG, "ffhip_p1_misfit: labels");
     build_v2e(m);
     MisfitBuffers b;
-    if (r && nlab > 0) {
-      b.onbc = dalloc<uint8_t>(m->nv);
-      b.labs = dalloc<int32_t>(nlab);
-    }
-    if (r) b.pair = dalloc<double2>(m->nt);
     try {
+      if (r && nlab > 0) {
+        b.onbc = dalloc<uint8_t>(m->nv);
+        b.labs = dalloc<int32_t>(nlab);
+      }
+      if (r) {
+        try {
+          b.pair = dalloc<double2>(m->nt);
+        } catch (const Error &) {  // no room for the pairs: r without them, the same bits
+        }
+      }
       misfit_run(ctx, m, u, ud, labels, nlab, J, r, b);
     } catch (...) {
       (void)hipStreamSynchronize(ctx->stream);

@@ -134,3 +134,16 @@ def test_gmres_after_a_failed_page_locked_buffer(alloc):
     assert e.value.code == ERR_HIP
     alloc.fail_host = lambda size: False
     assert np.array_equal(cg.gmres(b, eps=1e-10)[0], x0)
+
+
+@pytest.mark.parametrize("labels", [(), (1, 3, 5), tuple(range(3, 40))])
+def test_misfit_without_room_for_the_element_pairs(alloc, labels):
+    import torch
+    M = ffhip.cube(13, 11, 9)
+    g = torch.Generator().manual_seed(3)
+    u, ud = (torch.randn(M.nv, generator=g, dtype=torch.float64).cuda() for _ in range(2))
+    J0, r0 = ffhip.p1_misfit(M, u, ud, labels)
+    alloc.drop_cache()
+    alloc.limit(16 * M.nt, 0)
+    J, r = ffhip.p1_misfit(M, u, ud, labels)
+    assert J == J0 and torch.equal(r, r0)
