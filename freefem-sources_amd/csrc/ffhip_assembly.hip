@@ -1181,13 +1181,19 @@ __global__ __launch_bounds__(256) void k_p1_load_elem(int64_t nt, const double *
 // cube(96), 21 M incidences: 70 us (half-wave: 378 us with |K| recomputed).
 // PAIR terms need the row's own value (own, minus own2 when given); the
 // product and the sum are rounded on their own, as the term and its addition
-// were.  tgv rows: tgv * (gvals[v] or g0), or 0 with zero_bc.
-template <int RM, int ROWS>
+// were.  tgv rows: tgv * (gvals[v] or g0).
+// PART (a device without room for every tet's E): E holds the tets [e0, e1), the
+// row's sum goes on from b, and the last part (e1 = nt) writes the tgv rows.  A
+// row's list is in element order, so the additions are the same.
+struct RowPart {
+  int64_t e0, e1, nt;
+};
+template <int RM, int ROWS, bool PART = false>
 __global__ __launch_bounds__(64) void k_row_sum(
     int64_t n, const int64_t *__restrict__ v2e_ptr, const int32_t *__restrict__ v2e,
     const double *__restrict__ E, const double *__restrict__ own, const double *__restrict__ own2,
     const uint8_t *__restrict__ onbc, double tgv, double g0, const double *__restrict__ gvals,
-    double *__restrict__ b) {
+    double *__restrict__ b, RowPart part = {}) {
   constexpr int U = RM == kRowPair ? 4 : 8, CAP = kWave * U;  // one round of gathers per chunk
   using T = typename std::conditional<RM == kRowPair, double2, double>::type;
   __shared__ T st[CAP + CAP / 32];
@@ -1195,11 +1201,25 @@ __global__ __launch_bounds__(64) void k_row_sum(
   const int64_t r0 = (int64_t)xcd_block_id() * ROWS, rend = r0 + ROWS < n ? r0 + ROWS : n;
   if (r0 >= n) return;  // one wave per block
   const int64_t r = r0 + lane;  // lanes past the rows hold an empty range at the end
-  const int64_t p0 = v2e_ptr[r < rend ? r : rend], p1 = v2e_ptr[r + 1 < rend ? r + 1 : rend];
+  int64_t p0 = v2e_ptr[r < rend ? r : rend], p1 = v2e_ptr[r + 1 < rend ? r + 1 : rend];
   const int64_t seg0 = v2e_ptr[r0], seg1 = v2e_ptr[rend];
   double me = 0.;
   if (RM == kRowPair && r < rend) me = own2 ? own[r] - own2[r] : own[r];
   double s = 0.;
+  if constexpr (PART) {
+    auto first = [&](int64_t e) {  // the row's first incidence of a tet >= e
+      int64_t lo = p0, hi = p1;
+      while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (v2e[mid] >> 2 < e) lo = mid + 1; else hi = mid;
+      }
+      return lo;
+    };
+    const int64_t a = first(part.e0), z = first(part.e1);
+    p0 = a;
+    p1 = z;
+    if (part.e0 > 0 && r < rend) s = b[r];
+  }
   for (int64_t c0 = seg0; c0 < seg1; c0 += CAP) {
     const int cnt = (int)(seg1 - c0 < CAP ? seg1 - c0 : CAP);
     for (int i0 = lane; i0 < cnt; i0 += kWave * U) {
@@ -1209,6 +1229,10 @@ __global__ __launch_bounds__(64) void k_row_sum(
       for (int u = 0; u < U; ++u) {
         const int i = i0 + u * kWave;
         idx[u] = i < cnt ? v2e[c0 + i] : 0;
+        if (PART) {  // another part's tets are staged too, but not added
+          const int64_t e = idx[u] >> 2;
+          idx[u] = e >= part.e0 && e < part.e1 ? idx[u] - 4 * (int32_t)part.e0 : 0;
+        }
       }
 #pragma unroll
       for (int u = 0; u < U; ++u)
@@ -1236,7 +1260,10 @@ __global__ __launch_bounds__(64) void k_row_sum(
     wave_lds_sync();
   }
   if (r >= rend) return;
-  if (onbc && onbc[r]) s = tgv * (gvals ? gvals[r] : g0);
+  if (onbc && onbc[r]) {
+    if (PART && part.e1 < part.nt) return;
+    s = tgv * (gvals ? gvals[r] : g0);
+  }
   b[r] = s;
 }
 
@@ -1724,7 +1751,7 @@ void misfit_run(ffhip_ctx ctx, ffhip_mesh m, const double *u, const double *ud,
       auto sum = few_rows(m->nv) ? k_row_sum<kRowPair, 16> : k_row_sum<kRowPair, 64>;
       sum<<<row_grid(m->nv, few_rows(m->nv) ? 16 : 64), kWave, 0, s>>>(
           m->nv, m->v2e_ptr, m->v2e, reinterpret_cast<const double *>(b.pair), u, ud, onbc, 0., 0.,
-          nullptr, r);
+          nullptr, r, RowPart{});
     } else
       k_p1_mass_apply<<<nblocks(m->nv * kHalf, 256), 256, 0, s>>>(m->nv, m->xyz, m->elems, m->v2e_ptr,
                                                                   m->v2e, u, ud, onbc, r);
@@ -2190,18 +2217,36 @@ int ffhip_rhs_p1_form(ffhip_ctx ctx, ffhip_mesh m, int kind, double f0, const do
       gd = gown;
     }
     if (m->dim == 2) upload_t5_once(ctx->device);
-    // 3D: one pass over the tets, then one over the rows
+    // 3D: one pass over the tets, then one over the rows; part by part where a
+    // device has no room for every tet's terms (8 to 32 bytes each)
     const int rm = kind == FFHIP_COEF_P1 ? kRowPair
                    : kind == FFHIP_COEF_SIN3 || kind == FFHIP_COEF_QP ? kRowQuad : kRowScale;
-    double *E = m->dim == 3 ? dalloc<double>(m->nt * (rm == kRowPair ? 2 : rm == kRowQuad ? 4 : 1)) : nullptr;
+    const int ed = rm == kRowPair ? 2 : rm == kRowQuad ? 4 : 1;
+    double *E = nullptr;
+    int64_t part = m->nt;
+    while (m->dim == 3 && !E) {
+      try {
+        E = dalloc<double>(part * ed);
+      } catch (const Error &) {
+        if (part <= 256) throw;
+        part = (part + 1) / 2;
+      }
+    }
     ctx->tic();
     if (m->dim == 3) {
 #define FFHIP_RHS(RM)                                                                              \
   do {                                                                                             \
-    k_p1_load_elem<RM><<<nblocks(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, kind, f0, fd, E); \
-    auto sum = few_rows(n) ? k_row_sum<RM, 16> : k_row_sum<RM, 64>;                                \
-    sum<<<row_grid(n, few_rows(n) ? 16 : 64), kWave, 0, s>>>(n, m->v2e_ptr, m->v2e, E, fd, nullptr, onbc, \
-                                                             tgv, g0, gd, bd);                     \
+    int64_t e0 = 0;                                                                                \
+    do {                                                                                           \
+      const int64_t cnt = m->nt - e0 < part ? m->nt - e0 : part;                                   \
+      const double *fe = !fd || kind == FFHIP_COEF_P1 ? fd                                         \
+                                                      : fd + e0 * (kind == FFHIP_COEF_QP ? 14 : 1); \
+      k_p1_load_elem<RM><<<nblocks(cnt, 256), 256, 0, s>>>(cnt, m->xyz, m->elems + 4 * e0, kind, f0, fe, E); \
+      auto sum = part < m->nt ? k_row_sum<RM, 64, true>                                            \
+                 : few_rows(n) ? k_row_sum<RM, 16> : k_row_sum<RM, 64>;                            \
+      sum<<<row_grid(n, part == m->nt && few_rows(n) ? 16 : 64), kWave, 0, s>>>(                   \
+          n, m->v2e_ptr, m->v2e, E, fd, nullptr, onbc, tgv, g0, gd, bd, RowPart{e0, e0 + cnt, m->nt}); \
+    } while ((e0 += part) < m->nt);                                                                \
   } while (0)
       if (rm == kRowScale) FFHIP_RHS(kRowScale);
       else if (rm == kRowPair) FFHIP_RHS(kRowPair);

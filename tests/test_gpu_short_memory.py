@@ -147,3 +147,24 @@ def test_misfit_without_room_for_the_element_pairs(alloc, labels):
     alloc.limit(16 * M.nt, 0)
     J, r = ffhip.p1_misfit(M, u, ud, labels)
     assert J == J0 and torch.equal(r, r0)
+
+
+@pytest.mark.parametrize("kind,entries,size", [(ffhip.COEF_CONST, 0, 1), (ffhip.COEF_P0, 1, 1), (ffhip.COEF_P1, -1, 2),
+                                               (ffhip.COEF_SIN3, 0, 4), (ffhip.COEF_QP, 14, 4)])
+@pytest.mark.parametrize("labels", [(), (2, 5)])
+def test_rhs_without_room_for_every_tet(alloc, kind, entries, size, labels):
+    import torch
+    M = ffhip.cube(13, 11, 9)  # 7722 tets
+    g = torch.Generator().manual_seed(4)
+    f = torch.randn(M.nv if entries < 0 else entries * M.nt, generator=g, dtype=torch.float64).cuda() if entries else None
+    gv = torch.randn(M.nv, generator=g, dtype=torch.float64).cuda()
+    b0, b = (torch.full((M.nv,), float("nan"), dtype=torch.float64, device="cuda") for _ in range(2))
+    ffhip.rhs_p1_form(M, kind, 1.5, f, labels, gvals=gv, out=b0)
+    alloc.drop_cache()
+    for parts in (1, 3):  # halves, then eighths
+        sizes = [8 * size * (-(-M.nt // 2 ** k)) for k in range(parts)]
+        alloc.fail = lambda s: any(q <= s < q + 256 for q in sizes)
+        ffhip.rhs_p1_form(M, kind, 1.5, f, labels, gvals=gv, out=b)
+        assert torch.equal(b, b0)
+        b.fill_(float("nan"))
+        alloc.drop_cache()
