@@ -1413,7 +1413,7 @@ __global__ __launch_bounds__(256) void k_p1_grad_kappa(
 // y = A x over a CSR pattern, the value of entry k read as vals[k] (kPlain),
 // vals[slot[k]] (kSlots: the full view of a half matrix) or the entry (j, i)
 // of a symmetric pattern (kTrans: y = A^T x, *missing raised where the pattern
-// holds no such entry).
+// holds no such entry; y's old values go to keep, for a call that is refused).
 //
 // Bound by HBM (12 nnz + 20 n bytes), so every matrix load is coalesced: a wave
 // takes 64 rows, reads their entries consecutively (lane on entry, up to 8
@@ -1446,7 +1446,7 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
                                                    const double *__restrict__ vals,
                                                    const int64_t *__restrict__ slot,
                                                    const double *__restrict__ x, double *__restrict__ y,
-                                                   int *__restrict__ missing) {
+                                                   int *__restrict__ missing, double *__restrict__ keep) {
   constexpr int U = MODE == kTrans ? 8 : 4, CAP = kWave * U;  // one round of loads per chunk
   __shared__ double2 st[CAP + CAP / 32];
   __shared__ int64_t rs[kWave];  // kTrans: the rows' starts
@@ -1528,7 +1528,9 @@ __global__ __launch_bounds__(64) void k_spmv_stage(int64_t n, const int64_t *__r
     }
     wave_lds_sync();
   }
-  if (r < rend) y[r] = acc;
+  if (r >= rend) return;
+  if (MODE == kTrans) keep[r] = y[r];
+  y[r] = acc;
 }
 
 // slot of the transposed entry: (i,j) at k  ->  (j,i); -1 if absent
@@ -2416,23 +2418,35 @@ int ffhip_spmv(ffhip_ctx ctx, ffhip_mat A, const double *x, double *y, int trans
     FFHIP_REQUIRE(ctx && A && x && y, FFHIP_ERR_ARG, "ffhip_spmv: null argument");
     hipStream_t s = ctx->stream;
     const unsigned grid = row_grid(A->n, few_rows(A->n) ? 16 : 64);
-    auto product = [&](auto small, auto large, const int64_t *ptr, const int32_t *col, int *missing) {
+    auto product = [&](auto small, auto large, const int64_t *ptr, const int32_t *col, int *missing, double *keep) {
       ctx->tic();
-      (few_rows(A->n) ? small : large)<<<grid, kWave, 0, s>>>(A->n, ptr, col, A->vals, A->fslot, x, y, missing);
+      (few_rows(A->n) ? small : large)<<<grid, kWave, 0, s>>>(A->n, ptr, col, A->vals, A->fslot, x, y, missing, keep);
       FFHIP_CHECK(hipGetLastError());
       ctx->toc();
     };
     if (A->half) {  // y = (L + L^T - diag L) x over the full view; symmetric: trans alike
       half_view(A);
-      product(k_spmv_stage<kSlots, 16>, k_spmv_stage<kSlots, 64>, A->fptr, A->fcol, nullptr);
+      product(k_spmv_stage<kSlots, 16>, k_spmv_stage<kSlots, 64>, A->fptr, A->fcol, nullptr, nullptr);
       return;
     }
     if (!trans) {
-      product(k_spmv_stage<kPlain, 16>, k_spmv_stage<kPlain, 64>, A->rowptr, A->colidx, nullptr);
+      product(k_spmv_stage<kPlain, 16>, k_spmv_stage<kPlain, 64>, A->rowptr, A->colidx, nullptr, nullptr);
       return;
     }
-    const int *missing = ctx->flag(0);
-    product(k_spmv_stage<kTrans, 16>, k_spmv_stage<kTrans, 64>, A->rowptr, A->colidx, ctx->flag(0));
+    int *missing = ctx->flag(0);
+    double *keep = dalloc<double>(A->n);
+    try {
+      product(k_spmv_stage<kTrans, 16>, k_spmv_stage<kTrans, 64>, A->rowptr, A->colidx, missing, keep);
+      if (*missing) {
+        FFHIP_CHECK(hipMemcpyAsync(y, keep, 8 * A->n, hipMemcpyDeviceToDevice, s));
+        FFHIP_CHECK(hipStreamSynchronize(s));
+      }
+    } catch (...) {
+      (void)hipStreamSynchronize(s);
+      dfree(keep);
+      throw;
+    }
+    dfree(keep);
     FFHIP_REQUIRE(*missing == 0, FFHIP_ERR_UNSUPPORTED, "ffhip_spmv: transpose needs a symmetric pattern");
   });
 }

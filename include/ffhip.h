@@ -283,7 +283,7 @@ int ffhip_mat_free(ffhip_mat mat);
 
 /* y = A x (trans = 0) or A^T x (trans = 1) on device vectors:
  * HashMatrix::addMatMul (HashMatrix.cpp:1086-1154) without the accumulate.
- * A^T of a pattern that is not symmetric is refused; y is then undefined. */
+ * A^T of a pattern that is not symmetric is refused, y left as it was. */
 int ffhip_spmv(ffhip_ctx ctx, ffhip_mat mat, const double *x, double *y,
                int trans);
 
