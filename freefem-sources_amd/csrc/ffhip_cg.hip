@@ -569,6 +569,9 @@ struct SetupRb {
   double ttgv, ntgv;      // the tgv value (0: none) and the count of rows holding it
   int64_t ents, ents16;   // entries of the sliced layout, of its packed 16-bit deltas
   int far;                // some column is more than 2^15 from its row
+  // of sampled rows: entries, those whose place in the next row holds the next
+  // column, and those where it holds one within kNear columns
+  int entries, next, near_;
 };
 
 // pass 1: max diagonal; pass 2: count of the max (*top), max of the rest
@@ -627,12 +630,38 @@ __global__ __launch_bounds__(kBlock) void k_tgv_reduce(int GB, const double *__r
 }
 
 // the layout sizes for the host (entries of the sliced layout and of the
-// packed deltas: the last slice offsets) and the far-column flag's start
-__global__ void k_setup_sizes(SetupRb *__restrict__ rb, const int64_t *__restrict__ ents,
-                              const int64_t *__restrict__ ents16, int far) {
+// packed deltas: the last slice offsets), the far-column flag's start and, with
+// sample, how far apart the values lie that lanes on consecutive rows gather
+// (1024 rows, 4 per thread)
+constexpr int kSetupBlock = 256, kNear = 64;
+__global__ __launch_bounds__(kSetupBlock) void k_setup_sizes(
+    SetupRb *__restrict__ rb, const int64_t *__restrict__ ents, const int64_t *__restrict__ ents16, int far,
+    bool sample, int64_t n, const int64_t *__restrict__ rowptr, const int32_t *__restrict__ colidx) {
+  __shared__ double lds[kSetupBlock / kWave];
+  int entries = 0, next = 0, near_ = 0;
+  if (sample) {  // n > 1
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t r = (q * kSetupBlock + threadIdx.x) * (n - 1) / (4 * kSetupBlock);
+      const int64_t p0 = rowptr[r], p1 = rowptr[r + 1], p2 = rowptr[r + 2];
+      const int L = (int)(p1 - p0 < 32 ? p1 - p0 : 32);
+      entries += L;
+      for (int k = 0; k < L && p1 + k < p2; ++k) {
+        const int d = colidx[p1 + k] - colidx[p0 + k];
+        next += d == 1;
+        near_ += d >= -kNear && d <= kNear;
+      }
+    }
+  }
+  const double e = block_sum<kSetupBlock>(entries, lds), m = block_sum<kSetupBlock>(next, lds),
+               w = block_sum<kSetupBlock>(near_, lds);
+  if (threadIdx.x != 0) return;
   rb->ents = ents ? *ents : 0;
   rb->ents16 = ents16 ? *ents16 : 0;
   rb->far = far;
+  rb->entries = (int)e;
+  rb->next = (int)m;
+  rb->near_ = (int)w;
 }
 
 __global__ void k_jacobi(int64_t n, const double *__restrict__ d, const uint8_t *__restrict__ has,
@@ -2467,15 +2496,28 @@ struct ffhip_cg_s {
     }
   }
   // The direction formed in the mat-vec (not for 3x3 blocks, whose mat-vec gains
-  // little from one launch less): up to where the second gathered vector costs
-  // what the launch did.  us per solve, apart / together, FP64 cube(24) 1474 /
-  // 1233, cube(48) 3495 / 3212, cube(64) 7181 / 6864, cube(72) 8876 / 8802, cube(80)
-  // 10601 / 12184; MIXED cube(24) 2097 / 1897, cube(64) 6204 / 5768, cube(96) 16574 /
-  // 15730, cube(112) 24958 / 24649, cube(128) 36932 / 37865.  FP64 systems of one
-  // workgroup's size keep the launches' bits of k_pcg_small.
+  // little from one launch less), up to where the second gathered vector costs
+  // what the launch did.  That depends on the gathers: a wave's 64 of them take 4
+  // lines where consecutive rows hold consecutive columns (box meshes), up to 64
+  // in an arbitrary numbering.  us per iteration, apart / together, FP64 on
+  // cubes: 15.6 k rows 12.7 / 10.6, 69 k 15.4 / 14.3, 314 k 24.6 / 23.5 (531 k 42 /
+  // 48); the vertices shuffled within 30: 97 k 15.6 / 14.6, 227 k 21.7 / 20.9, within
+  // 300: 227 k 22.6 / 22.8; numbered at random: 9.3 k 14.0 / 13.8, 15.6 k 14.3 / 14.2,
+  // 30 k 16.5 / 17.7, 69 k 20.5 / 24.7, 314 k 41.3 / 66.5; scalar P2 (CSR) 24 k 16.0 /
+  // 15.1, 69 k 26.4 / 27.7, 275 k 73.4 / 86.4.  MIXED on cubes: 69 k 19.3 / 16.4, 1.03 M
+  // 35.6 / 34.1 (cube(128) 36.9 / 37.9 ms a solve); within 30: 227 k 21.0 / 19.4, 531 k
+  // 28.3 / 28.6, 1.03 M 36.7 / 39.9; at random 30 k 20.8 / 20.7, 69 k 23.8 / 25.7, 1.03 M
+  // 102 / 230; P2 24 k 21.1 / 18.6, 149 k 41.3 / 41.4.  FP64 systems of one workgroup's
+  // size keep the launches' bits of k_pcg_small.
+  // order (kSell16): most sampled entries are followed by the next column (2), by
+  // one near it (1), or not (0)
+  int order = 0;
+  int64_t fuse_small() const { return mode == FFHIP_CG_MIXED ? 1 << 15 : 1 << 14; }
+  int64_t fuse_large() const { return mode == FFHIP_CG_MIXED ? 1 << 20 : 5 << 16; }
   bool fuse() const {
-    if (fmt == kBsr3) return false;
-    return mode == FFHIP_CG_MIXED ? n <= 1 << 20 : n > kSmallRows && n <= 5 << 16;
+    if (fmt == kBsr3 || (mode == FFHIP_CG_FP64 && n <= kSmallRows)) return false;
+    const int64_t most = fmt != kSell16 || order == 0 ? fuse_small() : order == 1 ? 1 << 18 : fuse_large();
+    return n <= most;
   }
   // the state as the host reads it after a chunk (k_cg_advance writes it)
   CgState *host_state() const { return static_cast<CgState *>(ctx->pinned_data()); }
@@ -2564,7 +2606,7 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
     int64_t *cnt = dalloc<int64_t>(S3 + 1);
     k_bsr_len<<<nblk(S3 * kSlice, 256), 256, 0, s>>>(nb, S3, A->nodeptr, cg->bperm, cg->slen, cnt);
     exclusive_scan_i64(ctx, cnt, cg->sptr, S3 + 1);
-    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + S3, nullptr, 1);
+    k_setup_sizes<<<1, kSetupBlock, 0, s>>>(cg->rb, cg->sptr + S3, nullptr, 1, false, A->n, A->rowptr, A->colidx);
     cg->ents = setup_readback(cg).ents;
     dfree(cnt); dfree(tmp); dfree(keys); dfree(skeys); dfree(vals);
     cg->bcol = dalloc<int32_t>(cg->ents);
@@ -2586,10 +2628,13 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
     // against 2^15 and falls back to int32 columns (far_pending)
     k_sell_len4<<<nblk(cg->S, 256), 256, 0, s>>>(cg->S, cg->slen, cnt4);
     exclusive_scan_i64(ctx, cnt4, cg->sptr16, cg->S + 1);
-    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + cg->S, cg->sptr16 + cg->S, index32);
+    const bool sample = cg->n > cg->fuse_small() && cg->n <= cg->fuse_large();
+    k_setup_sizes<<<1, kSetupBlock, 0, s>>>(cg->rb, cg->sptr + cg->S, cg->sptr16 + cg->S, index32, sample, A->n,
+                                            A->rowptr, A->colidx);
     FFHIP_CHECK(hipGetLastError());
     const SetupRb h = setup_readback(cg);
     cg->ents = h.ents;
+    if (sample) cg->order = 2 * h.next >= h.entries ? 2 : 2 * h.near_ >= h.entries ? 1 : 0;
     if (layout == FFHIP_CG_LAYOUT_SELL || 4 * cg->ents <= 5 * A->nnz) {
       // 16-bit deltas, and gathers through buffer resources with 32-bit byte offsets
       if (h.far || A->n >= ((int64_t)1 << 28)) {
@@ -2965,7 +3010,7 @@ int ffhip_cg_solve_mixed(ffhip_cg cg, const double *sval, const float *sval32, d
 // the figures of a finished solve for the caller, and the errors of one that
 // did not converge (res: the sums of k_residual)
 static void solve_result(ffhip_cg cg, const CgState &hs, const double res[3], double ms, int itmax,
-                         int half_from, ffhip_cg_stats *stats) {
+                         int half_from, bool small, ffhip_cg_stats *stats) {
   if (stats) {
     stats->iters = hs.iters;
     stats->converged = hs.done == 1 ? 1 : (hs.done == 2 ? 2 : 0);
@@ -2979,6 +3024,7 @@ static void solve_result(ffhip_cg cg, const CgState &hs, const double res[3], do
     stats->timed = cg->n_timed;
     stats->ms_matvec_avg = cg->n_timed ? cg->t_mv / cg->n_timed : 0.;
     stats->ms_update_avg = cg->n_timed ? cg->t_up / cg->n_timed : 0.;
+    stats->fused = small ? 0 : cg->fuse();
     stats->ms_direction_avg = cg->n_timed ? cg->t_dv / cg->n_timed : 0.;
   }
   FFHIP_REQUIRE(hs.done != 4, FFHIP_ERR_NAN, "ffhip_cg_solve: NaN in CG (bad matrix)");
@@ -3030,7 +3076,7 @@ static void pcg_solve_small(ffhip_cg cg, const double *b, double *x, int on_devi
     for (int c = 0; c < 3; ++c) res[c] += out->res[3 * i + c];
   cg->t_dv = cg->t_mv = cg->t_up = 0.;
   cg->n_timed = 0;
-  solve_result(cg, out->st, res, ctx->last_ms, itmax, 0, stats);
+  solve_result(cg, out->st, res, ctx->last_ms, itmax, 0, true, stats);
 }
 
 static void cg_release(ffhip_cg cg) {
@@ -3201,7 +3247,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
     residual_sums(cg, sval, cg->xw, cg->bw, nullptr, res);
     FFHIP_CHECK(hipMemcpyAsync(x, cg->xw, 8 * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
     FFHIP_CHECK(hipStreamSynchronize(s));
-    solve_result(cg, hs, res, ms, itmax, half_from, stats);
+    solve_result(cg, hs, res, ms, itmax, half_from, false, stats);
   });
 }
 

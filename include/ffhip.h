@@ -376,7 +376,7 @@ typedef struct {
   double ms_matvec_avg;
   double ms_update_avg;
   int timed;
-  int reserved2;
+  int fused;          /* 1: the mat-vec formed the direction (no direction kernel) */
   double ms_direction_avg; /* the same for the direction kernel (about 0 where the mat-vec forms it) */
 } ffhip_cg_stats;
 /* Solver setup for a matrix (SolverCG ctor + HMatVirtPrecon,
