@@ -516,8 +516,8 @@ __global__ __launch_bounds__(256) void k_bsr_fill(
   }
 }
 
-// First slice of each of nw blocks when the S3 slices are split over them by
-// entries: block w takes the slices that start in [w E / nw, (w+1) E / nw),
+// First slice of each of nw blocks (or waves) when the S3 slices are split over
+// them by entries: w takes the slices that start in [w E / nw, (w+1) E / nw),
 // E = sptr[S3].
 __global__ void k_bsr_waves(int64_t S3, const int64_t *__restrict__ sptr, int nw,
                             int32_t *__restrict__ wstart) {
@@ -708,8 +708,8 @@ struct MatFmt {
   const V *val;          // kBsr3: 9 ents values, entry k of slice s at 9 ptr[s] + 9 64 k (bsr_pos)
   int64_t nb, ents;      // kBsr3: node rows, slice entries (ptr/len/col: slices, perm: rows)
   const int32_t *perm;   // kBsr3: node row of each sorted position
-  const int32_t *wstart; // kBsr3: first slice of each of the nw blocks (nw + 1), split by entries
-  int nw;
+  const int32_t *wstart; // kBsr3: first slice of each block (share) or wave, and the end, split by entries
+  bool share;            // kBsr3: a block's waves take its slices together
   bool nt;  // the matrix's loads bypass the caches
 };
 
@@ -838,7 +838,7 @@ __device__ inline ACC csr_row_sum(const MatFmt<V> &M, int64_t r, bool in, int la
 
 // Calls epi(r, sum_k a_rk X(j_k)) once for every row r of this block's range;
 // for kCsrV only the first lane of each 16-lane group calls it.
-template <bool NT, int KIND, class V, class ACC, class F, class E>
+template <bool NT, bool SHARE, int KIND, class V, class ACC, class F, class E>
 __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
   if constexpr (KIND == kSell16 && sizeof(V) == 8) {
     sell16_walk<NT, ACC>(M, xval, [](int32_t) { return 0; },
@@ -862,43 +862,44 @@ __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
       if (r < M.n) epi(r, acc);
     }
   } else if constexpr (KIND == kBsr3) {
-    // The block's four waves share each slice, a quarter of its entries each
-    // (a wave per slice left one serial chain of 14-32 rounds per SIMD at
-    // cube(20), 1077 slices: 50 us, now 29 with the matrix kept in the caches,
-    // 41 without; cube(8) 18 -> 9.6 us); their sums meet in LDS, added in entry order, and
-    // 192 threads finish the slice's rows.  Groups of U block entries; the
-    // next group's block columns are loaded
+    // While there are fewer slices than waves or the matrix stays in the caches
+    // (SHARE), the block's four waves take each slice together, a quarter of its entries each (a wave per slice
+    // left one serial chain of 14-32 rounds per SIMD at cube(20), 1077 slices: 50 us,
+    // now 29 with the matrix kept in the caches, 41 without; cube(8) 18 -> 9.6 us);
+    // their sums meet in LDS, added in entry order, and 192 threads finish the
+    // slice's rows.  Else a wave per slice: no barrier, no wave without entries
+    // (slices of 16 to 24 are two to three groups of 8).  Shared / a wave each, us
+    // FP64 (at 2 / 3 blocks per CU): cube(28), 2894 slices, 102.8 / 105.2, cube(30),
+    // 3547, 118.0 / 111.9, cube(34) 175.4 / 164.8; FP32 cube(28) 39.3 / 50.0 (in the
+    // caches), cube(30) 54.2 / 52.0, cube(32) 68.5 / 64.0, cube(40) 136.1 / 125.6.
+    // Groups of U block entries; the next group's block columns are loaded
     // with the current group's values, so the gathers of x need no second
     // round trip.  The slice's columns and values are read through buffer
     // resources bounded to the slice: past its width they read 0 without a
     // memory access, and those blocks' sums are dropped by a uniform select.
     constexpr int U = sizeof(V) == 8 ? FFHIP_BSR_U : FFHIP_BSR_U32;
-    __shared__ ACC red[2][kWavesPerBlock][3 * kSlice];
-    const int64_t S3 = (M.nb + kSlice - 1) / kSlice;
-    int64_t s0, s1;
-    if (M.wstart && (int)gridDim.x == M.nw) {
-      // slices split over the blocks by entries (rows of vertex and of edge
-      // nodes differ in length by about 2.5x)
-      const int lb = xcd_block_id();
-      s0 = __builtin_amdgcn_readfirstlane(M.wstart[lb]);
-      s1 = __builtin_amdgcn_readfirstlane(M.wstart[lb + 1]);
-    } else {
-      const int64_t G = gridDim.x, lb = xcd_block_id();
-      s0 = (lb * S3) / G;
-      s1 = ((lb + 1) * S3) / G;
-    }
+    __shared__ ACC red[SHARE ? 2 : 1][SHARE ? kWavesPerBlock : 1][SHARE ? 3 * kSlice : 1];
+    // slices split over the blocks or the waves by entries (rows of vertex and
+    // of edge nodes differ in length by about 2.5x)
+    const int wk = SHARE ? xcd_block_id() : xcd_block_id() * kWavesPerBlock + wave_id();
+    const int64_t s0 = __builtin_amdgcn_readfirstlane(M.wstart[wk]);
+    const int64_t s1 = __builtin_amdgcn_readfirstlane(M.wstart[wk + 1]);
     const int lane = threadIdx.x % kSlice, wv = wave_id();
     int buf = 0;
     for (int64_t s = s0; s < s1; ++s, buf ^= 1) {
       const int64_t sb = uniform(M.ptr[s]);
       const int L = __builtin_amdgcn_readfirstlane(M.len[s]);
-      const int part = (L + kWavesPerBlock * U - 1) / (kWavesPerBlock * U) * U;  // entries per wave
-      const int k0 = wv * part < L ? wv * part : L, k1 = k0 + part < L ? k0 + part : L;
+      int k0 = 0, k1 = L;  // this wave's entries
+      if constexpr (SHARE) {
+        const int part = (L + kWavesPerBlock * U - 1) / (kWavesPerBlock * U) * U;
+        k0 = wv * part < L ? wv * part : L;
+        k1 = k0 + part < L ? k0 + part : L;
+      }
       const auto rc = slice_rsrc(M.col + sb, (uint32_t)L * kSlice * 4);
       const auto rv = slice_rsrc(M.val + 9 * sb, (uint32_t)L * (9 * kSlice) * (uint32_t)sizeof(V));
-      // the row that this thread finishes: component t / 64 of the lane's node
+      // shared: the row that this thread finishes is component t / 64 of the lane's node
       const int64_t i = s * kSlice + lane;
-      const int32_t a = wv < 3 && i < M.nb ? M.perm[i] : -1;
+      const int32_t a = (wv < 3 || !SHARE) && i < M.nb ? M.perm[i] : -1;
       ACC s0v = 0, s1v = 0, s2v = 0;
       int32_t bn[U];
 #pragma unroll
@@ -959,17 +960,23 @@ __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
 #pragma unroll
         for (int u = 0; u < U; ++u) asm volatile("" : "+v"(bn[u]));
       }
-      red[buf][wv][lane] = s0v;
-      red[buf][wv][kSlice + lane] = s1v;
-      red[buf][wv][2 * kSlice + lane] = s2v;
-      // two buffers: the next slice's sums go to the other one, and the one
-      // after that comes behind the next barrier
-      __syncthreads();
-      if (a >= 0) {
-        ACC acc = red[buf][0][threadIdx.x];
+      if constexpr (SHARE) {
+        red[buf][wv][lane] = s0v;
+        red[buf][wv][kSlice + lane] = s1v;
+        red[buf][wv][2 * kSlice + lane] = s2v;
+        // two buffers: the next slice's sums go to the other one, and the one
+        // after that comes behind the next barrier
+        __syncthreads();
+        if (a >= 0) {
+          ACC acc = red[buf][0][threadIdx.x];
 #pragma unroll
-        for (int w = 1; w < kWavesPerBlock; ++w) acc += red[buf][w][threadIdx.x];
-        epi(3 * (int64_t)a + wv, acc);
+          for (int w = 1; w < kWavesPerBlock; ++w) acc += red[buf][w][threadIdx.x];
+          epi(3 * (int64_t)a + wv, acc);
+        }
+      } else if (a >= 0) {
+        epi(3 * (int64_t)a, s0v);
+        epi(3 * (int64_t)a + 1, s1v);
+        epi(3 * (int64_t)a + 2, s2v);
       }
     }
   } else {
@@ -987,8 +994,14 @@ __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
 
 template <int KIND, class V, class ACC, class F, class E>
 __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
-  if (M.nt) matvec_rows_as<true, KIND, V, ACC>(M, xval, epi);
-  else matvec_rows_as<false, KIND, V, ACC>(M, xval, epi);
+  if constexpr (KIND == kBsr3) {
+    if (!M.share) {  // larger than the caches
+      matvec_rows_as<true, false, KIND, V, ACC>(M, xval, epi);
+      return;
+    }
+  }
+  if (M.nt) matvec_rows_as<true, true, KIND, V, ACC>(M, xval, epi);
+  else matvec_rows_as<false, true, KIND, V, ACC>(M, xval, epi);
 }
 
 // Calls epi(r, sum_k a_rk X(j_k), pre(r), row) for the rows r of this block's
@@ -2345,7 +2358,8 @@ struct ffhip_cg_s {
   int64_t *sptr16 = nullptr;  // kSell16 slice offsets of scol16
   int32_t *bcol = nullptr;    // kBsr3 block columns (slices over sorted node rows)
   int32_t *bperm = nullptr;   // kBsr3 node row of each sorted position
-  int32_t *bwave = nullptr;   // kBsr3 first slice of each mat-vec block (grid + 1)
+  bool bshare = false;        // kBsr3 a mat-vec block's waves take its slices together
+  int32_t *bwave = nullptr;   // kBsr3 first slice of each mat-vec block or wave, and the end
   // values in the solver's layout; for kCsrV, sval is A's value array (borrowed)
   double *sval = nullptr;    // A
   double *svalT = nullptr;   // A^T (built on first transposed solve)
@@ -2539,8 +2553,8 @@ struct ffhip_cg_s {
     if (fmt == kSell || fmt == kSell16) { M.ptr = sptr; M.len = slen; M.col = scol; }
     else if (fmt == kBsr3) { M.ptr = sptr; M.len = slen; M.col = bcol; M.nb = n / 3; }
     else { M.ptr = A->rowptr; M.len = nullptr; M.col = A->colidx; }
-    M.wstart = fmt == kBsr3 ? bwave : nullptr;
-    M.nw = fmt == kBsr3 && bwave ? grid : 0;
+    M.wstart = bwave;
+    M.share = bshare;
     M.val = val;
     M.nt = matrix_bytes(sizeof(V)) > kCachedMatrix;
     return M;
@@ -2656,24 +2670,29 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
   }
   int64_t g;
   if (cg->fmt == kBsr3) {
-    g = (A->n / 3 + kSlice - 1) / kSlice;  // a block per slice
+    g = (A->n / 3 + kSlice - 1) / kSlice;  // a block per slice, or a wave
+    cg->bshare = g <= (int64_t)kWavesPerBlock * FFHIP_GRID_PER_CU * ctx->num_cu ||
+                 cg->matrix_bytes(cg->mode == FFHIP_CG_MIXED ? 4 : 8) <= kCachedMatrix;
+    if (!cg->bshare) g = (g + kWavesPerBlock - 1) / kWavesPerBlock;
   } else if (cg->fmt != kCsrV) {
     g = (cg->S + kWavesPerBlock - 1) / kWavesPerBlock;
   } else {
     cg->ents = A->nnz;
     g = (A->n + kBlock / kLanesPerRow - 1) / (kBlock / kLanesPerRow);
   }
-  // resident blocks per CU: 3 of an FP32 solver, 2 of an FP64 one (FP64 mat-vecs at
+  // resident blocks per CU: 3 of an FP32 solver and of 3x3-block slices that are not
+  // shared, 2 of another FP64 one (FP64 mat-vecs at
   // 2 against 3: cube(160) 136.9 / 139.4 us, cube(96) 24.8 / 25.4, cube(20) 3x3 blocks
   // 29.1 / 29.7, the vector kernels within 3 %; FP32 cube(64) 6.6 / 5.6, cube(128)
   // 32.4 / 30.1)
-  const int64_t gmax = (cg->mode == FFHIP_CG_MIXED ? FFHIP_GRID_PER_CU : 2) * (int64_t)ctx->num_cu;
+  const bool three = cg->mode == FFHIP_CG_MIXED || (cg->fmt == kBsr3 && !cg->bshare);
+  const int64_t gmax = (three ? FFHIP_GRID_PER_CU : 2) * (int64_t)ctx->num_cu;
   if (g > gmax) g = gmax;
   if (g >= 64) g -= g % 8;  // whole XCD groups
   if (g < 1) g = 1;
   cg->grid = (int)g;
   if (cg->fmt == kBsr3) {
-    const int nw = cg->grid;
+    const int nw = cg->bshare ? cg->grid : cg->grid * kWavesPerBlock;
     cg->bwave = dalloc<int32_t>(nw + 1);
     k_bsr_waves<<<nblk(nw + 1, 256), 256, 0, s>>>((A->n / 3 + kSlice - 1) / kSlice, cg->sptr, nw,
                                                   cg->bwave);
