@@ -368,29 +368,42 @@ __global__ __launch_bounds__(256) void k_p2_elem_lap(int64_t nt, const double *_
     if (kind == FFHIP_COEF_P1) u[i] = kappa_e[id[i]];
   }
   const double mes = tet_geom(v, G);
-  const double kc = kind == FFHIP_COEF_P0 ? kappa_e[e] : c0;
+  // kappa constant or linear: the integrals of l_i l_j l_k, |K| / 120 (2 and 6 times
+  // that with two and three equal).  The rule's 14 points otherwise: a chain of
+  // 7 us, unrolled so that the points' loads are not waited for one by one.
   double m[10] = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
-#pragma unroll 2
-  for (int q = 0; q < 14; ++q) {
-    const double px = c_qf5_pts[q][0], py = c_qf5_pts[q][1], pz = c_qf5_pts[q][2];
-    const double l[4] = {1. - (px + py + pz), px, py, pz};
-    double kq = kc;
-    if (kind == FFHIP_COEF_QP) {
-      kq = kappa_e[14 * e + q];
-    } else if (kind == FFHIP_COEF_P1) {
-      kq = p1_value3(u, px, py, pz);
-    } else if (kind == FFHIP_COEF_SIN3) {
-      double P[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) P[k] = l[0] * v[0][k] + px * v[1][k] + py * v[2][k] + pz * v[3][k];
-      kq = kappa_sin3(P[0], P[1], P[2]);
-    }
-    const double W = (mes * qf5_weight(q)) * kq;
+  if (kind != FFHIP_COEF_SIN3 && kind != FFHIP_COEF_QP) {
+    if (kind != FFHIP_COEF_P1) u[0] = u[1] = u[2] = u[3] = kind == FFHIP_COEF_P0 ? kappa_e[e] : c0;
+    const double w = mes * (1. / 120.), S = (u[0] + u[1]) + (u[2] + u[3]);
     int o = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = i; j < 4; ++j) m[o++] += (W * l[i]) * l[j];
+      for (int j = i; j < 4; ++j) {
+        const double t = S + u[i] + u[j];
+        m[o++] = w * (i == j ? t + t : t);
+      }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 14; ++q) {
+      const double px = c_qf5_pts[q][0], py = c_qf5_pts[q][1], pz = c_qf5_pts[q][2];
+      const double l[4] = {1. - (px + py + pz), px, py, pz};
+      double kq;
+      if (kind == FFHIP_COEF_QP) {
+        kq = kappa_e[14 * e + q];
+      } else {
+        double P[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) P[k] = l[0] * v[0][k] + px * v[1][k] + py * v[2][k] + pz * v[3][k];
+        kq = kappa_sin3(P[0], P[1], P[2]);
+      }
+      const double W = (mes * qf5_weight(q)) * kq;
+      int o = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = i; j < 4; ++j) m[o++] += (W * l[i]) * l[j];
+    }
   }
   double *o = E + kLap * e;
   double M = 0.;
@@ -427,7 +440,7 @@ __device__ inline P2Terms p2_terms(int i) {
   return t;
 }
 
-// A wave takes kNodesPerWave consecutive node rows, six incidences (60 lanes, one
+// A wave takes `nodes` consecutive node rows, six incidences (60 lanes, one
 // per (incidence, local node j)) at a time: the six tets' integrals are staged
 // in LDS, each lane forms its 3 x 3 block (Laplace: its entry) of the element's
 // row, and the blocks are added to the row in LDS one incidence after the
@@ -438,10 +451,9 @@ __device__ inline P2Terms p2_terms(int i) {
 // per block instead of LDS additions; 4 or 16 nodes per wave within 3 %).  Bound by instruction issue: about
 // 900 instructions per six incidences.  The element matrices formed on the matrix cores
 // (M = D W D^T per tet, 7.2 KB each) and gathered from memory took 606 + 494 us.
-constexpr int kNodesPerWave = 8;
 template <bool LAP>
 __global__ __launch_bounds__(64) void k_p2_rows(
-    int64_t nn, const int64_t *__restrict__ nodeptr, const int64_t *__restrict__ n2e_ptr,
+    int64_t nn, int nodes, const int64_t *__restrict__ nodeptr, const int64_t *__restrict__ n2e_ptr,
     const int32_t *__restrict__ n2e, const uint8_t *__restrict__ slot8, const double *__restrict__ E,
     double lambda, double mu, double *__restrict__ vals) {
   constexpr int ED = LAP ? kLap : kLame, NB = LAP ? 1 : 9, NV = 10 * NB, GI = 6;
@@ -451,9 +463,9 @@ __global__ __launch_bounds__(64) void k_p2_rows(
   __shared__ double blk[GI * NV];
   __shared__ uint8_t so[kWave];
   const int lane = threadIdx.x;
-  const int64_t a0 = (int64_t)xcd_block_id() * kNodesPerWave;
+  const int64_t a0 = (int64_t)xcd_block_id() * nodes;
   if (a0 >= nn) return;  // one wave per block
-  const int cnt = (int)(nn - a0 < kNodesPerWave ? nn - a0 : kNodesPerWave);
+  const int cnt = (int)(nn - a0 < nodes ? nn - a0 : nodes);
   // this wave's row and list offsets: lane q holds those of node a0 + q
   const int64_t myp = nodeptr[a0 + (lane < cnt ? lane : cnt)];
   const int64_t myk = n2e_ptr[a0 + (lane < cnt ? lane : cnt)];
@@ -621,6 +633,13 @@ __global__ __launch_bounds__(64) void k_p2_rows(
     so0 = so1; so1 = so2;
   }
 }
+
+// Nodes of a wave of k_p2_rows: 8, fewer where that leaves the chip without waves
+// and a call waits for one wave's chain.  1 / 2 / 4 / 8, us per assembly, elasticity
+// on cubes: 343 nodes 24.3 / 27.2 / 30.8 / 36.6, 9261 40.1 / 36.8 / 37.3 / 43.2, 35.9 k 89 /
+// 72.3 / 67.5 / 72.4, 118 k 253 / 193 / 162 / 160, 275 k 588 / 465 / 374 / 364; scalar 343
+// 27.1 / 29.3 / 32.4 / 37.7, 9261 33.4 / 33.4 / 36.4 / 42.5, 68.9 k 81.7 / 70.7 / 65.5 / 70.6.
+static int nodes_per_wave(int64_t nn) { return nn <= 1 << 12 ? 1 : nn <= 1 << 14 ? 2 : nn <= 100000 ? 4 : 8; }
 
 // ---------------------------------------------------------------- Dirichlet
 __device__ inline int32_t find_edge_node(const uint64_t *__restrict__ ekeys,
@@ -962,8 +981,9 @@ int ffhip_assemble_p2v_elasticity(ffhip_ctx ctx, ffhip_p2v sp, ffhip_mat A, doub
     double *E = ar.take<double>(kLame * m->nt);
     ctx->tic();
     k_p2_elem_lame<<<nblk(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, E);
-    k_p2_rows<false><<<(nblk(sp->nnodes, kNodesPerWave) + 7) / 8 * 8, kWave, 0, s>>>(
-        sp->nnodes, A->nodeptr, sp->n2e_ptr, sp->n2e, A->slot8, E, lambda, mu, A->vals);
+    const int nodes = nodes_per_wave(sp->nnodes);
+    k_p2_rows<false><<<(nblk(sp->nnodes, nodes) + 7) / 8 * 8, kWave, 0, s>>>(
+        sp->nnodes, nodes, A->nodeptr, sp->n2e_ptr, sp->n2e, A->slot8, E, lambda, mu, A->vals);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
   });
@@ -1058,8 +1078,9 @@ int ffhip_assemble_p2(ffhip_ctx ctx, ffhip_p2v sp, ffhip_mat A, int kind, double
     }
     ctx->tic();
     k_p2_elem_lap<<<nblk(m->nt, 256), 256, 0, s>>>(m->nt, m->xyz, m->elems, kind, c0, kd, E);
-    k_p2_rows<true><<<(nblk(sp->nnodes, kNodesPerWave) + 7) / 8 * 8, kWave, 0, s>>>(
-        sp->nnodes, A->nodeptr, sp->n2e_ptr, sp->n2e, A->slot8, E, 0., 0., A->vals);
+    const int nodes = nodes_per_wave(sp->nnodes);
+    k_p2_rows<true><<<(nblk(sp->nnodes, nodes) + 7) / 8 * 8, kWave, 0, s>>>(
+        sp->nnodes, nodes, A->nodeptr, sp->n2e_ptr, sp->n2e, A->slot8, E, 0., 0., A->vals);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
   });
