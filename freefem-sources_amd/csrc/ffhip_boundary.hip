@@ -75,7 +75,7 @@ __device__ inline double coef_at(int kind, double c0, const double *__restrict__
   return c0;
 }
 
-// A wave takes kBndRows vertices: their (boundary element, local vertex) items
+// A wave takes ROWS vertices: their (boundary element, local vertex) items
 // are one run of blist, a lane each, 64 at a time (the integral and the slots of
 // the vertex's row), then the vertices' lanes add them in their order.  MAT: add
 // the rows of alpha*u*v into vals (slots of row v); otherwise add g*v into b[v]
@@ -83,9 +83,16 @@ __device__ inline double coef_at(int kind, double c0, const double *__restrict__
 // overwrites afterwards).  Bound by the chain of a lane (points, searches): a
 // lane per vertex with all its items took 42 us (matrix) and 15 (right-hand side)
 // on a 61 x 50 x 43 box, now 26 and 10.
-constexpr int kBndRows = 16;
-template <int NB, bool MAT>
-__global__ __launch_bounds__(64) void k_p1_boundary(
+// Most waves find no item, so what a mesh's inside costs is the number of blocks,
+// and what its boundary costs is a wave's chain.  us, 64 threads and 16 vertices a
+// wave / 256 and 16 / 256 and 32 / 256 and 64: right-hand side square(300) 6.3 / 6.2 /
+// 6.2 / 6.9, square(1000) 18.4 / 9.1 / 7.6 / 7.1, square(2000) 58.6 / 25.0 / 15.5 / 10.1,
+// cube(64) 12.1 / 12.0 / 12.4 / 18.2, cube(160) 64.9 / 49.9 / 45.0 / 45.6, cube(200) 117 /
+// 79.0 / 65.3 / 63.6 (with a sine 131 / 138 / 119 / 121); matrix square(1000) 20.7 / 11.8 /
+// 10.1 / 12.3, square(2000) 61.9 / 28.6 / 19.6 / 15.8, cube(30) 20.5 / 21.2 / 27.5 / 49.6,
+// cube(200) 200 / 257 / 241 / 252.
+template <int NB, bool MAT, int BLOCK, int ROWS>
+__global__ __launch_bounds__(BLOCK) void k_p1_boundary(
     int64_t n, const double *__restrict__ xyz, const int32_t *__restrict__ belems,
     const int32_t *__restrict__ blab, Labels labels,
     const int64_t *__restrict__ bptr, const int32_t *__restrict__ blist, BndRule R, int kind,
@@ -93,17 +100,22 @@ __global__ __launch_bounds__(64) void k_p1_boundary(
     const int32_t *__restrict__ colidx, double *__restrict__ vals, const uint8_t *__restrict__ skip,
     double *__restrict__ b, int *__restrict__ missing) {
   constexpr int D = NB;  // coordinates per vertex: 3 for faces of a 3D mesh, 2 for edges
-  __shared__ double sv[kWave][MAT ? NB : 1];  // an item's entries
-  __shared__ int32_t so[kWave][MAT ? NB : 1];  // their slots in the row, -1: none
-  const int lane = threadIdx.x;
-  const int64_t v0 = (int64_t)blockIdx.x * kBndRows, v1 = v0 + kBndRows < n ? v0 + kBndRows : n;
+  constexpr int NW = BLOCK / kWave;  // the waves run on their own: no block barrier
+  __shared__ double sv_[NW][kWave][MAT ? NB : 1];   // an item's entries
+  __shared__ int32_t so_[NW][kWave][MAT ? NB : 1];  // their slots in the row, -1: none
+  const int lane = NW == 1 ? threadIdx.x : threadIdx.x % kWave;
+  const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  auto &sv = sv_[w];
+  auto &so = so_[w];
+  const int64_t v0 = ((int64_t)blockIdx.x * NW + w) * ROWS, v1 = v0 + ROWS < n ? v0 + ROWS : n;
+  if (NW > 1 && v0 >= n) return;
   const int64_t kbeg = bptr[v0], kend = bptr[v1];
   if (kbeg == kend) return;
-  // lane < kBndRows: a vertex, its items [q0, q1)
+  // lane < ROWS: a vertex, its items [q0, q1)
   const int64_t own = v0 + lane;
   int64_t q0 = kend, q1 = kend, r0 = 0;
   double bv = 0.;
-  if (lane < kBndRows && own < n) {
+  if (lane < ROWS && own < n) {
     q0 = bptr[own];
     q1 = bptr[own + 1];
     if (q0 < q1) {
@@ -277,14 +289,14 @@ int ffhip_assemble_p1_boundary(ffhip_ctx ctx, ffhip_mesh m, ffhip_mat A, const i
     int *missing = ctx->flag(0);
     const BndRule R = rule(m->dim);
     ctx->tic();
-    if (m->dim == 3)
-      k_p1_boundary<3, true><<<nblocks(m->nv, kBndRows), kWave, 0, s>>>(
-          m->nv, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, c0, cd,
-          A->rowptr, A->colidx, A->vals, nullptr, nullptr, missing);
-    else
-      k_p1_boundary<2, true><<<nblocks(m->nv, kBndRows), kWave, 0, s>>>(
-          m->nv, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, c0, cd,
-          A->rowptr, A->colidx, A->vals, nullptr, nullptr, missing);
+    auto run = [&](auto kernel, int block, int rows) {
+      kernel<<<nblocks(m->nv, rows * (block / kWave)), block, 0, s>>>(
+          m->nv, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, c0, cd, A->rowptr,
+          A->colidx, A->vals, nullptr, nullptr, missing);
+    };
+    if (m->dim == 3) run(k_p1_boundary<3, true, 64, 16>, 64, 16);
+    else if (m->nv <= 1 << 21) run(k_p1_boundary<2, true, 256, 32>, 256, 32);
+    else run(k_p1_boundary<2, true, 256, 64>, 256, 64);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
     const int miss = *missing;
@@ -322,14 +334,15 @@ int ffhip_rhs_p1_boundary(ffhip_ctx ctx, ffhip_mesh m, const int32_t *labels, in
     }
     const BndRule R = rule(m->dim);
     ctx->tic();
-    if (m->dim == 3)
-      k_p1_boundary<3, false><<<nblocks(n, kBndRows), kWave, 0, s>>>(
-          n, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, g0, cd, nullptr,
-          nullptr, nullptr, skip, bd, nullptr);
-    else
-      k_p1_boundary<2, false><<<nblocks(n, kBndRows), kWave, 0, s>>>(
-          n, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, g0, cd, nullptr,
-          nullptr, nullptr, skip, bd, nullptr);
+    auto run = [&](auto kernel, int block, int rows) {
+      kernel<<<nblocks(n, rows * (block / kWave)), block, 0, s>>>(
+          n, m->xyz, m->belems, m->blab, labs.L, m->b2e_ptr, m->b2e, R, kind, g0, cd, nullptr, nullptr,
+          nullptr, skip, bd, nullptr);
+    };
+    if (m->dim == 2 && n <= 1 << 21) run(k_p1_boundary<2, false, 256, 32>, 256, 32);
+    else if (m->dim == 2) run(k_p1_boundary<2, false, 256, 64>, 256, 64);
+    else if (n <= 1 << 22) run(k_p1_boundary<3, false, 64, 16>, 64, 16);
+    else run(k_p1_boundary<3, false, 256, 32>, 256, 32);
     FFHIP_CHECK(hipGetLastError());
     ctx->toc();
     if (!on_device) {
