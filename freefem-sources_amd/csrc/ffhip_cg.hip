@@ -3366,7 +3366,7 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
     auto HN = [&](int i, int j) -> double & { return Hn.get()[(size_t)i * (m + 1) + j]; };
     k_gm_normb<<<G, kBlock, 0, s>>>(n, cg->bw, cg->ntgv > 0 ? cg->wcl : nullptr, cg->pA);
     double normb = std::sqrt(host_sum(cg->pA));
-    double relres = 1e100;
+    double relres = 1e100, rate = std::log(10.);  // decrease per iteration (log), first a fast solve's
     bool noconv = true;
     int iter = 0, nrestart = 0;
     while (noconv) {
@@ -3376,6 +3376,7 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
       g[0] = std::sqrt(host_sum(cg->pA));
       if (normb < 1.e-20 || eps < 0) normb = 1.;
       double inv = 1. / g[0];
+      const double g0 = g[0];
       int it, ahead = 0;  // iterations launched beyond the ones looked at, of the current batch
       int batch = 0;
       const int P = cg->gm_blocks();
@@ -3383,9 +3384,14 @@ int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device, do
       for (it = 0; it < m; it++, iter++) {
         if (ahead == 0) {
           // a batch of iterations in one go, then one copy of what the host
-          // needs of each; those after a convergence are dropped.  Past 2^18
-          // rows an iteration costs more than the wait it saves.
-          batch = std::min(n <= (1 << 18) ? ffhip_cg_s::kGmBatch : 1, m - it);
+          // needs of each; those after a convergence are dropped, so a batch is
+          // no longer than the rest at the rate so far.  (8 from the start, 1000
+          // to 227 k rows: 355 to 465 us for a solve of one iteration that took 285.)
+          // Past 2^18 rows an iteration costs more than the wait it saves.
+          if (it > 0) rate = std::fmax(std::log(std::fabs(g0) / relres) / it, 0.);
+          const double left = std::ceil(std::log((it ? relres : std::fabs(g0)) / (std::fabs(eps) * normb)) / rate);
+          const int most = n <= (1 << 18) ? ffhip_cg_s::kGmBatch : 1;
+          batch = std::min(!(left > 1.) ? 1 : left < most ? (int)left : most, m - it);  // left may be NaN
           cg->gm_basis(it + 1, it + batch);
           batch = std::min(batch, (int)cg->gmV.size() - it);
           const int64_t ld = cg->gm_out();
