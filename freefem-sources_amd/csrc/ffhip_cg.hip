@@ -1355,8 +1355,10 @@ __device__ inline SymRow sym_row(const MatFmt<double> &M, int64_t r) {
   return R;
 }
 // the positions, from the diagonal on, that row r's entries before the diagonal
-// have in the rows of their columns (4 bits each); *ok: all there, with the same value
-__device__ inline uint32_t sym_owners(const MatFmt<double> &M, int64_t r, const SymRow &R, bool &ok) {
+// have in the rows of their columns (4 bits each); bad: not all there (kSymForm),
+// or not with the same value (kSymValues)
+constexpr int kSymForm = 1, kSymValues = 2;
+__device__ inline uint32_t sym_owners(const MatFmt<double> &M, int64_t r, const SymRow &R, int &bad) {
   const int64_t vb = M.ptr[r / kSlice];
   uint32_t pw = 0;
 #pragma unroll 1
@@ -1369,10 +1371,10 @@ __device__ inline uint32_t sym_owners(const MatFmt<double> &M, int64_t r, const 
     int kj = -1;
 #pragma unroll
     for (int q = 0; q < 16; ++q) kj = J.delta(q) == -d ? q : kj;
-    if (kj < 0 || J.L > 16 || kj - J.nl >= kSymHalf) { ok = false; return 0; }
+    if (kj < 0 || J.L > 16 || kj - J.nl >= kSymHalf) { bad = kSymForm; return 0; }
     const double mine = M.val[vb + pair_pos(R.L, k, (int)(r % kSlice))];
     const double theirs = M.val[M.ptr[j / kSlice] + pair_pos(J.L, kj, (int)(j % kSlice))];
-    if (__builtin_bit_cast(uint64_t, mine) != __builtin_bit_cast(uint64_t, theirs)) { ok = false; return 0; }
+    if (__builtin_bit_cast(uint64_t, mine) != __builtin_bit_cast(uint64_t, theirs)) bad = kSymValues;
     pw |= (uint32_t)(kj - J.nl) << (4 * k);
   }
   return pw;
@@ -1382,7 +1384,7 @@ struct SymTables {
   int64_t rep[kSymSlots];             // a row of the pattern
   SymRow row[kSymSlots];
   uint32_t owners[kSymSlots];
-  int bad, count, nl, nu;  // some row does not fit; patterns; most entries before a diagonal, from it on
+  int bad, count, nl, nu;  // some row does not fit (kSymForm, kSymValues); patterns; most entries before a diagonal, from it on
 };
 // every row's slot in the table of patterns.  Once a row fails (or the table
 // fills, as on an unstructured mesh within its first blocks) the rest is left.
@@ -1391,9 +1393,9 @@ __global__ __launch_bounds__(256) void k_sym_rows(MatFmt<double> M, SymTables *T
   const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (r >= M.n || __hip_atomic_load(&T->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   const SymRow R = sym_row(M, r);
-  bool ok = R.L <= 16 && R.nl <= kSymHalf && R.nu <= kSymHalf;
-  const uint32_t pw = ok ? sym_owners(M, r, R, ok) : 0;
-  if (ok) {
+  int bad = R.L <= 16 && R.nl <= kSymHalf && R.nu <= kSymHalf ? 0 : kSymForm;
+  const uint32_t pw = bad ? 0 : sym_owners(M, r, R, bad);
+  if (!bad) {
     unsigned long long h = 0x9e3779b97f4a7c15ull ^ ((unsigned long long)pw << 16 | R.nl << 8 | R.nu);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
@@ -1401,8 +1403,8 @@ __global__ __launch_bounds__(256) void k_sym_rows(MatFmt<double> M, SymTables *T
       h ^= h >> 29;
     }
     h |= 1;
-    ok = false;
-    for (int p = 0; p < 16 && !ok; ++p) {
+    bad = kSymForm;  // until a slot is found
+    for (int p = 0; p < 16 && bad; ++p) {
       const int t = (int)(((h >> 8) + p) & (kSymSlots - 1));
       unsigned long long k = __hip_atomic_load(&T->key[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (k == 0) {
@@ -1416,11 +1418,11 @@ __global__ __launch_bounds__(256) void k_sym_rows(MatFmt<double> M, SymTables *T
       if (k == h) {
         cls[r] = (uint8_t)t;
         owners[r] = pw;
-        ok = true;
+        bad = 0;
       }
     }
   }
-  if (!ok) atomicOr(&T->bad, 1);
+  if (bad) atomicOr(&T->bad, bad);
 }
 // the patterns from their rows
 __global__ __launch_bounds__(kSymSlots) void k_sym_table(MatFmt<double> M, SymTables *T,
@@ -1465,7 +1467,7 @@ __global__ __launch_bounds__(256) void k_sym_fill(MatFmt<double> M, SymTables *T
 #pragma unroll
   for (int g = 0; g < 4; ++g) same &= R.pk[g].x == Q.pk[g].x && R.pk[g].y == Q.pk[g].y;
   if (!same) {  // a hash met twice
-    atomicOr(&T->bad, 1);
+    atomicOr(&T->bad, kSymForm);
     return;
   }
   const int64_t vb = M.ptr[r / kSlice];
@@ -2466,9 +2468,11 @@ struct ffhip_cg_s {
   };
   std::vector<Chunk> graphs;
   int use_graph = 1;
-  // symmetric values of an FP64 kSell16 solver (k_pcg_matvec_sym): 0 not looked
-  // for since the values changed, 1 there, -1 the matrix has not that form
-  int sym = 0, sym_nl = 0, sym_nu = 0;
+  // symmetric values of an FP64 kSell16 solver (k_pcg_matvec_sym)
+  enum Sym { kSymUnknown, kSymThere, kSymNot, kSymNever };  // not looked for since the values
+  // changed; there; not with these values (or no room); the pattern has not that form
+  Sym sym = kSymUnknown;
+  int sym_nl = 0, sym_nu = 0;
   double *symval = nullptr;
   uint8_t *symcls = nullptr;
   SymPattern *symtab = nullptr;
@@ -2897,15 +2901,16 @@ static hipGraphExec_t pcg_chunk_graph(ffhip_cg cg, const double *sval, bool sym)
 // cube(160)) and give 6 to 23 us an iteration: worth it in a solve that has run
 // a while, for a matrix past kSymMinBytes (cube(64), 39 MB, would gain 2 us an
 // iteration for 0.15 ms).  A matrix of another form is seen as one within the
-// search's first blocks, once per solver.
+// search's first blocks, once per solver; values that are not symmetric, or no
+// room for the copy, count until the values change.
 constexpr int kSymAfter = 4 * kChunk;
 constexpr int64_t kSymMinBytes = 64000000;
 static bool sym_build(ffhip_cg cg) {
-  if (cg->sym) return cg->sym > 0;
+  if (cg->sym != cg->kSymUnknown) return cg->sym == cg->kSymThere;
   ffhip_ctx ctx = cg->ctx;
   hipStream_t s = ctx->stream;
   const int64_t n = cg->n;
-  cg->sym = -1;
+  cg->sym = cg->kSymNever;
   // 32-bit byte offsets of the values
   if (cg->fmt != kSell16 || cg->mode != FFHIP_CG_FP64 || cg->matrix_bytes(8) <= kSymMinBytes ||
       cg->S * (kSymHalf * kSlice * 8) >= (int64_t)UINT32_MAX)
@@ -2933,19 +2938,25 @@ static bool sym_build(ffhip_cg cg) {
       fetch(ctx, {{end, &T->bad, sizeof(end)}});
     }
   } catch (const Error &) {  // no room for them: the solve goes on without
-    (void)hipGetLastError();
     (void)hipStreamSynchronize(s);
-    end[0] = 1;
+    end[0] = kSymValues;
   }
   dfree(T);
   dfree(owners);
   if (end[0]) {
+    cg->sym = end[0] & kSymForm ? cg->kSymNever : cg->kSymNot;
+    // the captured chunks that read the buffers go with them
+    auto gone = std::remove_if(cg->graphs.begin(), cg->graphs.end(), [](const ffhip_cg_s::Chunk &c) {
+      if (c.kind == 2) (void)hipGraphExecDestroy(c.exec);
+      return c.kind == 2;
+    });
+    cg->graphs.erase(gone, cg->graphs.end());
     dfree(cg->symval);
     dfree(cg->symcls);
     dfree(cg->symtab);
     return false;
   }
-  cg->sym = 1;
+  cg->sym = cg->kSymThere;
   return true;
 }
 static hipGraphExec_t mix_chunk_graph(ffhip_cg cg, const float *sval32, int par) {
@@ -3193,7 +3204,7 @@ int ffhip_cg_layout(ffhip_cg cg, int *layout, int64_t *entries) {
 int ffhip_cg_update_values(ffhip_cg cg) {
   return guard([&] {
     FFHIP_REQUIRE(cg, FFHIP_ERR_ARG, "ffhip_cg_update_values: null solver");
-    if (cg->sym > 0) cg->sym = 0;
+    if (cg->sym != cg->kSymNever) cg->sym = cg->kSymUnknown;
     cg_setup_jacobi(cg);
     setup_readback(cg);
     cg_fill_values(cg, false);
@@ -3217,7 +3228,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
       return;
     }
     // captured before this solve's first launch (kept for later solves)
-    if (cg->mode == FFHIP_CG_FP64) (void)pcg_chunk_graph(cg, sval, !trans && cg->sym > 0);
+    if (cg->mode == FFHIP_CG_FP64) (void)pcg_chunk_graph(cg, sval, !trans && cg->sym == cg->kSymThere);
     else { (void)mix_chunk_graph(cg, sval32, 0); (void)mix_chunk_graph(cg, sval32, 1); }
     FFHIP_CHECK(hipMemcpyAsync(cg->bw, b, 8 * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
     FFHIP_CHECK(hipMemcpyAsync(cg->xw, x, 8 * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
@@ -3232,7 +3243,7 @@ int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device, doubl
       const int G = cg->grid;
       const MatFmt<double> M = cg->fmt_of(sval);
       const int chunk = kChunk;
-      bool sym = !trans && cg->sym > 0;
+      bool sym = !trans && cg->sym == cg->kSymThere;
       half_from = sym ? 1 : 0;
       hipGraphExec_t gx = pcg_chunk_graph(cg, sval, sym);
       hs.it0 = 1;

@@ -168,3 +168,24 @@ def test_rhs_without_room_for_every_tet(alloc, kind, entries, size, labels):
         assert torch.equal(b, b0)
         b.fill_(float("nan"))
         alloc.drop_cache()
+
+
+def test_half_of_the_values_without_room(alloc):
+    M = ffhip.cube(76, 77, 79)
+    A = ffhip.Matrix.p1(M)
+    A.assemble_p1(ffhip.COEF_SIN3)
+    A.set_bc((1, 2, 3, 4, 5, 6))
+    b = ffhip.rhs_p1(M, 1.0, (1, 2, 3, 4, 5, 6))
+    cg = ffhip.CG(A)
+    x0, st = cg.solve(b, eps=1e-6, trans=True)
+    assert st["iters"] > 64
+    alloc.drop_cache()
+    half = -(-M.nv // 64) * 64 * 8 * 8  # 8 values a row, rounded to 2 MiB by the allocator
+    alloc.fail = lambda size: half <= size <= half + (2 << 20)
+    for _ in range(2):
+        x, st = cg.solve(b, eps=1e-6)
+        assert st["half_from"] == 0 and np.array_equal(x, x0)
+    alloc.fail = lambda size: False
+    cg.update_values()  # looked for again
+    x, st = cg.solve(b, eps=1e-6)
+    assert st["half_from"] == 65 and np.array_equal(x, x0)
