@@ -62,7 +62,7 @@ class Allocator:
         """the library gives its cached blocks back when a request fails"""
         self.fail = lambda size: True
         with pytest.raises(ffhip.FFHipError) as e:
-            ffhip.cube(183, 171, 167)  # larger than any block kept
+            ffhip.cube(390, 380, 400)  # 5.7 GB of tets: larger than any block kept
         assert e.value.code == ERR_HIP
         self.fail = lambda size: False
 
