@@ -48,25 +48,6 @@ __constant__ double c_qt5_pts[7][2];
 __constant__ double c_qt5_w[7];
 
 // ---------------------------------------------------------------- incidence
-__global__ void k_v2e_count(const int32_t *__restrict__ elems, int64_t m,
-                            uint32_t *__restrict__ deg) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m) atomicAdd(&deg[elems[i]], 1u);
-}
-
-// one pass: count and place every incidence into a 32-entry bucket of its
-// dof (lists longer than 32 set *ovf and are rebuilt by count + fill)
-__global__ void k_v2e_bucket(const int32_t *__restrict__ elems, int64_t m,
-                             uint32_t *__restrict__ deg, int32_t *__restrict__ bucket,
-                             int *__restrict__ ovf) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const int32_t v = elems[i];
-  const uint32_t pos = atomicAdd(&deg[v], 1u);
-  if (pos < 32) bucket[32 * (int64_t)v + pos] = (int32_t)i;
-  else atomicOr(ovf, 1);
-}
-
 __global__ void k_u32_to_i64(int64_t n, const uint32_t *__restrict__ a, int64_t *__restrict__ b) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) b[i] = a[i];

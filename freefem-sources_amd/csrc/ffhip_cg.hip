@@ -215,31 +215,22 @@ __device__ inline int64_t uniform(int64_t v) {
 }
 __device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kSlice); }
 
-// Slices of this wave in the streaming mat-vec kernels.  CYCLIC: each XCD's
+// Slices of this wave in the streaming sliced-ELL kernels: each XCD's
 // contiguous slice range is walked by all of its waves together, wave q taking
 // slices q, q + Q, q + 2Q, ... (Q waves on the XCD), so the XCD streams one
 // contiguous window of Q slices at a time and a column's x value, needed by
 // rows up to one window-width apart (the plane neighbours of a 3D mesh), is
 // re-read while still in that XCD's L2 (cube(160) P1: 8 % less HBM fetch, the
-// FP32 mat-vec 6 % faster).  Otherwise each block walks its own contiguous
-// chunk of slices — kept for the [P2,P2,P2] block layout, whose node rows are
-// sorted by length in windows and ran 1.8x slower with the cyclic walk.
-constexpr bool kCyclicSell = true;
-template <bool CYCLIC>
+// FP32 mat-vec 6 % faster than with a contiguous chunk per block).  The
+// [P2,P2,P2] block layout, whose node rows are sorted by length in windows, ran
+// 1.8x slower this way and walks chunks.
 __device__ inline void wave_slices(int64_t S, int64_t &first, int64_t &end, int64_t &stride) {
-  if (CYCLIC) {
-    const int G = gridDim.x, b = blockIdx.x;
-    const int groups = (G % 8) ? 1 : 8;
-    const int grp = b % groups, loc = b / groups, nloc = G / groups;
-    first = (grp * S) / groups + (int64_t)loc * kWavesPerBlock + wave_id();
-    end = ((grp + 1) * S) / groups;
-    stride = (int64_t)nloc * kWavesPerBlock;
-  } else {
-    const int64_t G = gridDim.x, lb = xcd_block_id();
-    first = (lb * S) / G + wave_id();
-    end = ((lb + 1) * S) / G;
-    stride = kWavesPerBlock;
-  }
+  const int G = gridDim.x, b = blockIdx.x;
+  const int groups = (G % 8) ? 1 : 8;
+  const int grp = b % groups, loc = b / groups, nloc = G / groups;
+  first = (grp * S) / groups + (int64_t)loc * kWavesPerBlock + wave_id();
+  end = ((grp + 1) * S) / groups;
+  stride = (int64_t)nloc * kWavesPerBlock;
 }
 
 // the maximum over a wave, in every lane
@@ -533,8 +524,6 @@ __global__ void k_bsr_waves(int64_t S3, const int64_t *__restrict__ sptr, int nw
   wstart[w] = (int32_t)lo;
 }
 
-// flags a row with a column farther than 16 bits from the row index
-// the columns of a row are sorted: its first and last bound the deltas
 // CSR-layout values: A (optionally transposed through tmap) and/or the FP32
 // copy of D^-1/2 A D^-1/2, one 16-lane group per row
 __global__ void k_csr_fill(int64_t n, const int64_t *__restrict__ rowptr,
@@ -706,7 +695,7 @@ struct MatFmt {
   const int16_t *col16;  // kSell16: col - row, packed [group of 4][lane][4] per slice
   const int64_t *ptr16;  // kSell16: slice offsets of col16
   const V *val;          // kBsr3: 9 ents values, entry k of slice s at 9 ptr[s] + 9 64 k (bsr_pos)
-  int64_t nb, ents;      // kBsr3: node rows, slice entries (ptr/len/col: slices, perm: rows)
+  int64_t nb;            // kBsr3: node rows (ptr/len/col: slices, perm: rows)
   const int32_t *perm;   // kBsr3: node row of each sorted position
   const int32_t *wstart; // kBsr3: first slice of each block (share) or wave, and the end, split by entries
   bool share;            // kBsr3: a block's waves take its slices together
@@ -796,7 +785,7 @@ __device__ inline ACC sell16_slice_row(const MatFmt<double> &M, int64_t s, int l
 template <bool NT, class ACC, class F, class P, class E>
 __device__ inline void sell16_walk(const MatFmt<double> &M, F xval, P pre, E epi) {
   int64_t s, s1, ds;
-  wave_slices<kCyclicSell>(M.S, s, s1, ds);
+  wave_slices(M.S, s, s1, ds);
   const int lane = threadIdx.x % kSlice;
   for (; s < s1; s += ds) {
     const int64_t r = s * kSlice + lane;
@@ -845,7 +834,7 @@ __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
                      [&](int64_t r, ACC acc, int, bool row) { if (row) epi(r, acc); });
   } else if constexpr (KIND == kSell || KIND == kSell16) {
     int64_t s0, s1, ds;
-    wave_slices<kCyclicSell>(M.S, s0, s1, ds);
+    wave_slices(M.S, s0, s1, ds);
     const int lane = threadIdx.x % kSlice;
     for (int64_t s = s0; s < s1; s += ds) {
       const int64_t base = uniform(M.ptr[s]) + lane;
@@ -1280,7 +1269,7 @@ __global__ FFHIP_MATVEC_ATTR void k_pcg_matvec_sym(SymFmt M, const double *__res
   const auto at = [](uint32_t r) { return r * 8u + (r / kSlice) * ((NU - 1) * kSlice * 8u); };
   double p_hah = 0.;
   int64_t s, s1, ds;
-  wave_slices<kCyclicSell>(M.S, s, s1, ds);
+  wave_slices(M.S, s, s1, ds);
   const int lane = threadIdx.x % kSlice;
   for (; s < s1; s += ds) {
     const int64_t r = s * kSlice + lane;
@@ -2552,7 +2541,6 @@ struct ffhip_cg_s {
     M.col16 = scol16;
     M.ptr16 = sptr16;
     M.nb = 0;
-    M.ents = ents;
     M.perm = bperm;
     if (fmt == kSell || fmt == kSell16) { M.ptr = sptr; M.len = slen; M.col = scol; }
     else if (fmt == kBsr3) { M.ptr = sptr; M.len = slen; M.col = bcol; M.nb = n / 3; }
@@ -2565,13 +2553,18 @@ struct ffhip_cg_s {
   }
 };
 
-// launch a layout-templated mat-vec kernel with the solver's layout
-#define FFHIP_LAUNCH_FMT(cg, kern, grid, stream, ...)                        \
+// launch a layout-templated mat-vec kernel with the solver's layout (_ROWS: not
+// the 3x3 blocks)
+#define FFHIP_LAUNCH_ROWS(cg, kern, grid, stream, ...)                       \
   do {                                                                       \
     if ((cg)->fmt == kSell) kern<kSell><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__); \
     else if ((cg)->fmt == kSell16) kern<kSell16><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__); \
-    else if ((cg)->fmt == kBsr3) kern<kBsr3><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__); \
     else kern<kCsrV><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__);           \
+  } while (0)
+#define FFHIP_LAUNCH_FMT(cg, kern, grid, stream, ...)                        \
+  do {                                                                       \
+    if ((cg)->fmt == kBsr3) kern<kBsr3><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__); \
+    else FFHIP_LAUNCH_ROWS(cg, kern, grid, stream, __VA_ARGS__);              \
   } while (0)
 
 #define FFHIP_LAUNCH_MATVEC(cg, T, M, x, y, stream)                                          \
@@ -2850,7 +2843,7 @@ static void launch_pcg_chunk(ffhip_cg cg, const double *sval, bool sym, bool mar
                                         cg->xw, cg->pA, cg->pB, cg->st);
     if (marks) cg->mark(4 * c + 1);
     if (fused)
-      FFHIP_LAUNCH_FMT(cg, k_pcg_dir_matvec, G, s, c, M, cg->H[c & 1], cg->CG, cg->G, cg->H[(c + 1) & 1],
+      FFHIP_LAUNCH_ROWS(cg, k_pcg_dir_matvec, G, s, c, M, cg->H[c & 1], cg->CG, cg->G, cg->H[(c + 1) & 1],
                        cg->AH, cg->xw, cg->pA, cg->pB, cg->st);
     else if (sym)
       (cg->sym_nu == 4              ? k_pcg_matvec_sym<3, 4>
@@ -2880,7 +2873,7 @@ static void launch_mix_chunk(ffhip_cg cg, const float *sval32, int par, bool mar
     if (!fused) k_mix_dirvec<<<G, kBlock, 0, s>>>(c, cg->n, pold, cg->r32, pnew, cg->pA, cg->st, cg->ms);
     if (marks) cg->mark(4 * c + 1);
     if (fused)
-      FFHIP_LAUNCH_FMT(cg, k_mix_dir_matvec, G, s, c, M32, pold, cg->r32, pnew, cg->q32, cg->pA, cg->pB, cg->st,
+      FFHIP_LAUNCH_ROWS(cg, k_mix_dir_matvec, G, s, c, M32, pold, cg->r32, pnew, cg->q32, cg->pA, cg->pB, cg->st,
                        cg->ms);
     else
       FFHIP_LAUNCH_FMT(cg, k_mix_matvec, G, s, M32, pnew, cg->q32, cg->pB, cg->st);

@@ -49,11 +49,12 @@ __global__ __launch_bounds__(64) void k_fetch(FetchArgs a, uint32_t *__restrict_
 void fetch(ffhip_ctx ctx, std::initializer_list<Fetch> list) {
   FetchArgs a{};
   int k = 0, words = 0;
+  FFHIP_REQUIRE(list.size() <= 4, FFHIP_ERR_INTERNAL, "fetch: %d values", (int)list.size());
   for (const Fetch &f : list) {
     a.src[k] = static_cast<const uint32_t *>(f.src);
     a.end[k++] = words += f.bytes / 4;
   }
-  FFHIP_REQUIRE(list.size() <= 4 && words <= 64, FFHIP_ERR_INTERNAL, "fetch: %d words", words);
+  FFHIP_REQUIRE(words <= 64, FFHIP_ERR_INTERNAL, "fetch: %d words", words);
   for (; k < 4; ++k) a.end[k] = words;
   k_fetch<<<1, 64, 0, ctx->stream>>>(a, static_cast<uint32_t *>(ctx->pinned_data()));
   FFHIP_CHECK(hipGetLastError());
