@@ -29,6 +29,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -241,10 +242,64 @@ __device__ inline int wave_max(int v) {
 }
 
 // ---------------------------------------------------------------- SELL build
+// What the solver set-up reads back to the host, in one copy: the tgv
+// figures (k_tgv_reduce), the layout sizes (k_setup_sizes) and the columns' order
+// (sample_order).
+struct SetupRb {
+  double ttgv, ntgv;      // the tgv value (0: none) and the count of rows holding it
+  int64_t ents, ents16;   // entries of the sliced layout, of its packed 16-bit deltas
+  int far;                // some column is more than 2^15 from its row
+  // of sampled rows: entries, those whose place in the next row holds the next
+  // column, and those where it holds one within kNear columns
+  int entries, next, near_;
+};
+
+// How far apart the values lie that lanes on consecutive rows gather: 128 pairs of
+// rows (r, r + 1) spread by the golden ratio (an even spread would meet the ends of
+// a box's lines), 16 lanes on the first 16 entries of a pair, every load of the
+// pairs in flight together.  n > 1.
+constexpr int kNear = 64, kOrderBlock = 256;
+__device__ inline void sample_order(int64_t n, const int64_t *__restrict__ rowptr,
+                                    const int32_t *__restrict__ colidx, SetupRb *__restrict__ rb) {
+  __shared__ double lds[kOrderBlock / kWave];
+  constexpr int Q = 8;
+  const int g = threadIdx.x / 16, k = threadIdx.x % 16;
+  int64_t p0[Q], p1[Q], p2[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const uint32_t u = (uint32_t)(g * Q + q) * 2654435769u;
+    const int64_t r = (int64_t)(((uint64_t)u * (uint64_t)(n - 1)) >> 32);
+    p0[q] = rowptr[r];
+    p1[q] = rowptr[r + 1];
+    p2[q] = rowptr[r + 2];
+  }
+  int entries = 0, next = 0, near_ = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const bool in = p0[q] + k < p1[q], both = in && p1[q] + k < p2[q];
+    const int d = both ? colidx[p1[q] + k] - colidx[p0[q] + k] : INT_MAX;
+    entries += in;
+    next += d == 1;
+    near_ += d >= -kNear && d <= kNear;
+  }
+  const double e = block_sum<kOrderBlock>(entries, lds), a = block_sum<kOrderBlock>(next, lds),
+               b = block_sum<kOrderBlock>(near_, lds);
+  if (threadIdx.x != 0) return;
+  rb->entries = (int)e;
+  rb->next = (int)a;
+  rb->near_ = (int)b;
+}
+
 // the widest row of each slice: a wave per slice (a lane per slice walked its 64
-// rows: 13 us for P2 on a 27 x 24 x 21 box, square(200) 11)
-__global__ void k_sell_len(int64_t n, int64_t S, const int64_t *__restrict__ rowptr,
-                           int32_t *__restrict__ len, int64_t *__restrict__ cnt) {
+// rows: 13 us for P2 on a 27 x 24 x 21 box, square(200) 11); with colidx a block past
+// the slices' samples the order of the columns meanwhile
+__global__ __launch_bounds__(kOrderBlock) void k_sell_len(int64_t n, int64_t S, const int64_t *__restrict__ rowptr,
+                                                          const int32_t *__restrict__ colidx, SetupRb *__restrict__ rb,
+                                                          int32_t *__restrict__ len, int64_t *__restrict__ cnt) {
+  if (colidx && blockIdx.x == gridDim.x - 1) {
+    sample_order(n, rowptr, colidx, rb);
+    return;
+  }
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, s = r / kSlice;
   if (s >= S) return;
   const int m = wave_max(r < n ? (int)(rowptr[r + 1] - rowptr[r]) : 0);
@@ -552,17 +607,6 @@ __global__ void k_diag_vals(int64_t n, const int64_t *__restrict__ diag,
   has[i] = s >= 0;
 }
 
-// What the solver set-up reads back to the host, in one copy: the tgv
-// figures (k_tgv_reduce) and the layout sizes (k_setup_sizes).
-struct SetupRb {
-  double ttgv, ntgv;      // the tgv value (0: none) and the count of rows holding it
-  int64_t ents, ents16;   // entries of the sliced layout, of its packed 16-bit deltas
-  int far;                // some column is more than 2^15 from its row
-  // of sampled rows: entries, those whose place in the next row holds the next
-  // column, and those where it holds one within kNear columns
-  int entries, next, near_;
-};
-
 // pass 1: max diagonal; pass 2: count of the max (*top), max of the rest
 // (HashMatrix::gettgv, HashMatrix.cpp:1340-1371)
 __global__ void k_tgv_pass(int64_t n, const double *__restrict__ d, const uint8_t *__restrict__ has,
@@ -619,38 +663,12 @@ __global__ __launch_bounds__(kBlock) void k_tgv_reduce(int GB, const double *__r
 }
 
 // the layout sizes for the host (entries of the sliced layout and of the
-// packed deltas: the last slice offsets), the far-column flag's start and, with
-// sample, how far apart the values lie that lanes on consecutive rows gather
-// (1024 rows, 4 per thread)
-constexpr int kSetupBlock = 256, kNear = 64;
-__global__ __launch_bounds__(kSetupBlock) void k_setup_sizes(
-    SetupRb *__restrict__ rb, const int64_t *__restrict__ ents, const int64_t *__restrict__ ents16, int far,
-    bool sample, int64_t n, const int64_t *__restrict__ rowptr, const int32_t *__restrict__ colidx) {
-  __shared__ double lds[kSetupBlock / kWave];
-  int entries = 0, next = 0, near_ = 0;
-  if (sample) {  // n > 1
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int64_t r = (q * kSetupBlock + threadIdx.x) * (n - 1) / (4 * kSetupBlock);
-      const int64_t p0 = rowptr[r], p1 = rowptr[r + 1], p2 = rowptr[r + 2];
-      const int L = (int)(p1 - p0 < 32 ? p1 - p0 : 32);
-      entries += L;
-      for (int k = 0; k < L && p1 + k < p2; ++k) {
-        const int d = colidx[p1 + k] - colidx[p0 + k];
-        next += d == 1;
-        near_ += d >= -kNear && d <= kNear;
-      }
-    }
-  }
-  const double e = block_sum<kSetupBlock>(entries, lds), m = block_sum<kSetupBlock>(next, lds),
-               w = block_sum<kSetupBlock>(near_, lds);
-  if (threadIdx.x != 0) return;
+// packed deltas: the last slice offsets) and the far-column flag's start
+__global__ void k_setup_sizes(SetupRb *__restrict__ rb, const int64_t *__restrict__ ents,
+                              const int64_t *__restrict__ ents16, int far) {
   rb->ents = ents ? *ents : 0;
   rb->ents16 = ents16 ? *ents16 : 0;
   rb->far = far;
-  rb->entries = (int)e;
-  rb->next = (int)m;
-  rb->near_ = (int)w;
 }
 
 __global__ void k_jacobi(int64_t n, const double *__restrict__ d, const uint8_t *__restrict__ has,
@@ -2516,7 +2534,7 @@ struct ffhip_cg_s {
   // 28.3 / 28.6, 1.03 M 36.7 / 39.9; at random 30 k 20.8 / 20.7, 69 k 23.8 / 25.7, 1.03 M
   // 102 / 230; P2 24 k 21.1 / 18.6, 149 k 41.3 / 41.4.  FP64 systems of one workgroup's
   // size keep the launches' bits of k_pcg_small.
-  // order (kSell16): most sampled entries are followed by the next column (2), by
+  // order (kSell16, sample_order): most sampled entries are followed by the next column (2), by
   // one near it (1), or not (0)
   int order = 0;
   int64_t fuse_small() const { return mode == FFHIP_CG_MIXED ? 1 << 15 : 1 << 14; }
@@ -2617,7 +2635,7 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
     int64_t *cnt = dalloc<int64_t>(S3 + 1);
     k_bsr_len<<<nblk(S3 * kSlice, 256), 256, 0, s>>>(nb, S3, A->nodeptr, cg->bperm, cg->slen, cnt);
     exclusive_scan_i64(ctx, cnt, cg->sptr, S3 + 1);
-    k_setup_sizes<<<1, kSetupBlock, 0, s>>>(cg->rb, cg->sptr + S3, nullptr, 1, false, A->n, A->rowptr, A->colidx);
+    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + S3, nullptr, 1);
     cg->ents = setup_readback(cg).ents;
     dfree(cnt); dfree(tmp); dfree(keys); dfree(skeys); dfree(vals);
     cg->bcol = dalloc<int32_t>(cg->ents);
@@ -2633,15 +2651,15 @@ static void cg_plan_layout(ffhip_cg cg, int layout, bool index32) {
     cg->sptr16 = dalloc<int64_t>(cg->S + 1);
     int64_t *cnt = ar.take<int64_t>(cg->S + 1);
     int64_t *cnt4 = ar.take<int64_t>(cg->S + 1);
-    k_sell_len<<<nblk(cg->S * kSlice, 256), 256, 0, s>>>(A->n, cg->S, A->rowptr, cg->slen, cnt);
+    const bool sample = cg->n > cg->fuse_small() && cg->n <= cg->fuse_large();
+    k_sell_len<<<nblk(cg->S * kSlice, kOrderBlock) + (sample ? 1 : 0), kOrderBlock, 0, s>>>(
+        A->n, cg->S, A->rowptr, sample ? A->colidx : nullptr, cg->rb, cg->slen, cnt);
     exclusive_scan_i64(ctx, cnt, cg->sptr, cg->S + 1);
     // 16-bit column deltas unless index32: the fill checks every delta
     // against 2^15 and falls back to int32 columns (far_pending)
     k_sell_len4<<<nblk(cg->S, 256), 256, 0, s>>>(cg->S, cg->slen, cnt4);
     exclusive_scan_i64(ctx, cnt4, cg->sptr16, cg->S + 1);
-    const bool sample = cg->n > cg->fuse_small() && cg->n <= cg->fuse_large();
-    k_setup_sizes<<<1, kSetupBlock, 0, s>>>(cg->rb, cg->sptr + cg->S, cg->sptr16 + cg->S, index32, sample, A->n,
-                                            A->rowptr, A->colidx);
+    k_setup_sizes<<<1, 1, 0, s>>>(cg->rb, cg->sptr + cg->S, cg->sptr16 + cg->S, index32);
     FFHIP_CHECK(hipGetLastError());
     const SetupRb h = setup_readback(cg);
     cg->ents = h.ents;

@@ -49,6 +49,19 @@ def test_rule(n, box, random):
         assert np.linalg.norm(y[p] - x) <= 1e-8 * np.linalg.norm(x)
 
 
+@pytest.mark.parametrize("mesh", [lambda: ffhip.square(255), lambda: ffhip.square(511), lambda: ffhip.cube(63),
+                                  lambda: ffhip.cube(31, 63, 63), lambda: ffhip.cube(15, 127, 63)])
+def test_lines_of_a_power_of_two(mesh):
+    """65536 to 262144 rows: an even spread of samples would meet the lines' ends"""
+    M = mesh()
+    A = ffhip.Matrix.p1(M)
+    A.assemble_p1(ffhip.COEF_CONST, 1.0)
+    A.set_bc((1, 2, 3))
+    b = ffhip.rhs_p1(M, 1.0, (1, 2, 3))
+    for mode in (ffhip.CG_FP64, ffhip.CG_MIXED):
+        assert solve(A, b, mode)[1] == 1
+
+
 # 68921 and 262144 rows in FP64 and MIXED (2^18 is the limit), 274625 past it
 @pytest.mark.parametrize("n,fused", [(40, 1), (63, 1), (64, 0)])
 def test_shuffled_within_a_few(n, fused):
