@@ -152,7 +152,9 @@ int ffhip_rhs_p1(ffhip_ctx ctx, ffhip_mesh mesh, double f,
  * and on(labels, u=g) rows set to tgv * g with g per
  * dof (gvals, n values: g at the dof's vertex, as AssembleBC evaluates it,
  * problem.cpp:10120-10176) or the constant g0 when gvals is NULL.  fcoef,
- * gvals and b are device pointers when on_device != 0, else host pointers. */
+ * gvals and b are device pointers when on_device != 0, else host pointers.  In
+ * 3D a call takes 8 (CONST, P0), 16 (P1) or 32 bytes a tet of device memory, or
+ * the tets in parts of at least 256 where they do not fit. */
 int ffhip_rhs_p1_form(ffhip_ctx ctx, ffhip_mesh mesh, int kind, double f0,
                       const double *fcoef, const int32_t *labels, int nlab,
                       double tgv, double g0, const double *gvals, double *b,
@@ -242,15 +244,18 @@ int ffhip_mat_read_text(ffhip_ctx ctx, const char *path, ffhip_mat *mat);
  * terms, problem.cpp:6384-6437; Tet_5 is exact for it) applied to u - ud, and
  * the zeroed Dirichlet rows of the adjoint problem.  u, ud, r: device
  * pointers (n doubles); J: host pointer. FreeFEM has no adjoint routine; this
- * is the continuous adjoint of its composed varfs. */
+ * is the continuous adjoint of its composed varfs.  r takes 16 bytes a tet of
+ * device memory during the call, or none, at a slower pace, where they do not
+ * fit. */
 int ffhip_p1_misfit(ffhip_ctx ctx, ffhip_mesh mesh, const double *u,
                     const double *ud, const int32_t *labels, int nlab,
                     double *J, double *r);
 /* ffhip_p1_misfit without any device allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  Its
- * temporaries (the J partials, the label list, the Dirichlet marks) live in a
- * fixed device array of the library, one per device, of 16.8 MB: meshes of
+ * temporaries (the label list, the Dirichlet marks) live in a
+ * fixed device array of the library, one per device, of 16.8 MB, and the J
+ * partials in page-locked memory of the context: meshes of
  * at most 2^24 vertices, at most 64 labels (FFHIP_ERR_ARG beyond).  The
  * mesh's vertex incidence must already exist when r is wanted (any assembly
  * or ffhip_p1_misfit call on the mesh builds it).  Calls that overlap on one
@@ -398,7 +403,12 @@ int ffhip_cg_update_values(ffhip_cg cg);
  * are initialised to b_i/tgv (SetInitWithBC); stop when
  * (g, D^-1 g) < eps^2 (g0, D^-1 g0) for eps > 0, or < eps^2 for eps < 0
  * (CG.cpp:226,247).  itmax <= 0 means n.  b, x: device pointers when
- * on_device != 0, else host.  trans != 0 solves A^T x = b (SolveT). */
+ * on_device != 0, else host.  trans != 0 solves A^T x = b (SolveT).  From its
+ * 65th iteration on an FP64 solve of a large matrix that is symmetric bit for bit
+ * and has rows of few patterns (a box mesh's) reads a copy of half of the values,
+ * 65 bytes a row more device memory, the same bits; where it does not fit, or
+ * after ffhip_cg_update_values with values that are not symmetric, the whole
+ * matrix. */
 int ffhip_cg_solve(ffhip_cg cg, const double *b, double *x, int on_device,
                    double eps, int itmax, double tgv, int trans,
                    ffhip_cg_stats *stats);
@@ -431,7 +441,8 @@ int ffhip_cg_solve_affine(ffhip_cg cg, const double *b, double *x, int on_device
  * means n.  stats: iters = fgmres' iteration count, refinements = restarts,
  * gcg0 = ||b||, gcg = the final |g_{k+1}| / ||b||.  FFHIP_ERR_NOCONV when it
  * does not converge (SolverGMRES, erronerr = 1).  The basis vectors are
- * allocated as a solve first reaches them and kept by the solver. */
+ * allocated as a solve first reaches them, up to 7 ahead where they fit, and kept
+ * by the solver. */
 int ffhip_gmres_solve(ffhip_cg cg, const double *b, double *x, int on_device,
                       double eps, int itmax, int restart, double tgv, int trans,
                       ffhip_cg_stats *stats);
