@@ -78,7 +78,8 @@ constexpr int kU = FFHIP_SELL_U;
 constexpr int kSell = 0;
 constexpr int kCsrV = 1;
 constexpr int kSell16 = 2;  // sliced ELL with 16-bit column deltas (col - row)
-constexpr int kBsr3 = 3;    // 3x3 blocks of the [P2,P2,P2] node rows
+constexpr int kBsr3 = 3;    // 3x3 blocks of the [P2,P2,P2] node rows, a block's waves on a slice together
+constexpr int kBsr3W = 4;   // the same layout, a wave per slice (a kernel of its own: never a solver's fmt)
 // MIXED: the FP32 residual is replaced by the FP64 one once (r32, r32) fell by
 // this factor since the last replacement (every two decades of the residual
 // norm: FP32 recurrences of ill-conditioned systems, e.g. vector P2
@@ -715,8 +716,7 @@ struct MatFmt {
   const V *val;          // kBsr3: 9 ents values, entry k of slice s at 9 ptr[s] + 9 64 k (bsr_pos)
   int64_t nb;            // kBsr3: node rows (ptr/len/col: slices, perm: rows)
   const int32_t *perm;   // kBsr3: node row of each sorted position
-  const int32_t *wstart; // kBsr3: first slice of each block (share) or wave, and the end, split by entries
-  bool share;            // kBsr3: a block's waves take its slices together
+  const int32_t *wstart; // kBsr3: first slice of each block (kBsr3W: wave), and the end, split by entries
   bool nt;  // the matrix's loads bypass the caches
 };
 
@@ -845,7 +845,7 @@ __device__ inline ACC csr_row_sum(const MatFmt<V> &M, int64_t r, bool in, int la
 
 // Calls epi(r, sum_k a_rk X(j_k)) once for every row r of this block's range;
 // for kCsrV only the first lane of each 16-lane group calls it.
-template <bool NT, bool SHARE, int KIND, class V, class ACC, class F, class E>
+template <bool NT, int KIND, class V, class ACC, class F, class E>
 __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
   if constexpr (KIND == kSell16 && sizeof(V) == 8) {
     sell16_walk<NT, ACC>(M, xval, [](int32_t) { return 0; },
@@ -868,9 +868,10 @@ __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
         acc = sell_row<NT, kU, V, ACC, int32_t>(M.col + base, M.val + base, L, r32, xval);
       if (r < M.n) epi(r, acc);
     }
-  } else if constexpr (KIND == kBsr3) {
+  } else if constexpr (KIND == kBsr3 || KIND == kBsr3W) {
+    constexpr bool SHARE = KIND == kBsr3;
     // While there are fewer slices than waves or the matrix stays in the caches
-    // (SHARE), the block's four waves take each slice together, a quarter of its entries each (a wave per slice
+    // (kBsr3), the block's four waves take each slice together, a quarter of its entries each (a wave per slice
     // left one serial chain of 14-32 rounds per SIMD at cube(20), 1077 slices: 50 us,
     // now 29 with the matrix kept in the caches, 41 without; cube(8) 18 -> 9.6 us);
     // their sums meet in LDS, added in entry order, and 192 threads finish the
@@ -1001,14 +1002,12 @@ __device__ inline void matvec_rows_as(const MatFmt<V> &M, F xval, E epi) {
 
 template <int KIND, class V, class ACC, class F, class E>
 __device__ inline void matvec_rows(const MatFmt<V> &M, F xval, E epi) {
-  if constexpr (KIND == kBsr3) {
-    if (!M.share) {  // larger than the caches
-      matvec_rows_as<true, false, KIND, V, ACC>(M, xval, epi);
-      return;
-    }
+  if constexpr (KIND == kBsr3W) {  // larger than the caches
+    matvec_rows_as<true, KIND, V, ACC>(M, xval, epi);
+  } else {
+    if (M.nt) matvec_rows_as<true, KIND, V, ACC>(M, xval, epi);
+    else matvec_rows_as<false, KIND, V, ACC>(M, xval, epi);
   }
-  if (M.nt) matvec_rows_as<true, true, KIND, V, ACC>(M, xval, epi);
-  else matvec_rows_as<false, true, KIND, V, ACC>(M, xval, epi);
 }
 
 // Calls epi(r, sum_k a_rk X(j_k), pre(r), row) for the rows r of this block's
@@ -2564,7 +2563,6 @@ struct ffhip_cg_s {
     else if (fmt == kBsr3) { M.ptr = sptr; M.len = slen; M.col = bcol; M.nb = n / 3; }
     else { M.ptr = A->rowptr; M.len = nullptr; M.col = A->colidx; }
     M.wstart = bwave;
-    M.share = bshare;
     M.val = val;
     M.nt = matrix_bytes(sizeof(V)) > kCachedMatrix;
     return M;
@@ -2581,7 +2579,8 @@ struct ffhip_cg_s {
   } while (0)
 #define FFHIP_LAUNCH_FMT(cg, kern, grid, stream, ...)                        \
   do {                                                                       \
-    if ((cg)->fmt == kBsr3) kern<kBsr3><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__); \
+    if ((cg)->fmt == kBsr3 && (cg)->bshare) kern<kBsr3><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__); \
+    else if ((cg)->fmt == kBsr3) kern<kBsr3W><<<(grid), kBlock, 0, (stream)>>>(__VA_ARGS__); \
     else FFHIP_LAUNCH_ROWS(cg, kern, grid, stream, __VA_ARGS__);              \
   } while (0)
 
@@ -2591,6 +2590,8 @@ struct ffhip_cg_s {
       k_matvec<kSell, T, T><<<(cg)->grid, kBlock, 0, (stream)>>>(M, (const T *)(x), (T *)(y)); \
     else if ((cg)->fmt == kSell16)                                                          \
       k_matvec<kSell16, T, T><<<(cg)->grid, kBlock, 0, (stream)>>>(M, (const T *)(x), (T *)(y)); \
+    else if ((cg)->fmt == kBsr3 && !(cg)->bshare)                                           \
+      k_matvec<kBsr3W, T, T><<<(cg)->grid, kBlock, 0, (stream)>>>(M, (const T *)(x), (T *)(y)); \
     else if ((cg)->fmt == kBsr3)                                                            \
       k_matvec<kBsr3, T, T><<<(cg)->grid, kBlock, 0, (stream)>>>(M, (const T *)(x), (T *)(y)); \
     else                                                                                    \
